@@ -21,6 +21,9 @@ LIB_PATH = os.path.join(LIB_DIR, "libarctic_moe_hip.so")
 # (source, object name, extra flags); the 16-bit grouped GEMM is compiled as four groups of entry points in parallel
 GEMM_PARTS = 4
 SOURCES = [(f, os.path.splitext(f)[0], []) for f in ("api.hip", "router.hip", "permute.hip", "rows.hip", "gemm_f32.hip", "remap.hip")]
+# the default tile shape of the same products: one group per epilogue
+PP_PARTS = 3
+SOURCES = [("gemm_pp.hip", f"gemm_pp_p{i}", [f"-DAMOE_PP_PART={i}"]) for i in range(PP_PARTS)] + SOURCES
 SOURCES = [("gemm_bf16.hip", f"gemm_bf16_p{i}", [f"-DAMOE_GEMM_PART={i}"]) for i in range(GEMM_PARTS)] + SOURCES
 
 HIPCC_FLAGS = [
@@ -59,14 +62,15 @@ def _compile(item) -> str:
     return obj
 
 
-def _check_gemm_assembly(part: int):
-    """Compile one group of gemm_bf16.hip to assembly and run the static check of its inline-assembly
-    LDS reads (asm_check.py); raises, and so fails the build, on a violation.  Returns the numbers of
-    kernels and of transposing reads checked."""
+def _check_gemm_assembly(item):
+    """Compile one group of a 16-bit GEMM source to assembly and run the static check of its
+    inline-assembly LDS traffic (asm_check.py); raises, and so fails the build, on a violation.  Returns
+    the numbers of kernels and of inline transposing reads checked."""
     from . import asm_check
 
-    flags = [f for f in HIPCC_FLAGS if f not in ("-fPIC", "-fvisibility=hidden")] + [f"-DAMOE_GEMM_PART={part}"]
-    asm = asm_check.compile_to_assembly(os.path.join(SRC_DIR, "gemm_bf16.hip"), os.path.join(OBJ_DIR, f"gemm_bf16_p{part}.s"), flags)
+    src, name, extra = item
+    flags = [f for f in HIPCC_FLAGS if f not in ("-fPIC", "-fvisibility=hidden")] + extra
+    asm = asm_check.compile_to_assembly(os.path.join(SRC_DIR, src), os.path.join(OBJ_DIR, f"{name}.s"), flags)
     return asm_check.check_assembly(asm, min_kernels=1, require_tr=False)
 
 
@@ -113,7 +117,7 @@ def build(force: bool = True, jobs: int = 8) -> str:
             return LIB_PATH
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         objs_f = [ex.submit(_compile, item) for item in SOURCES]
-        checks = [ex.submit(_check_gemm_assembly, i) for i in range(GEMM_PARTS)]
+        checks = [ex.submit(_check_gemm_assembly, item) for item in SOURCES if item[0] in ("gemm_bf16.hip", "gemm_pp.hip")]
         objs = [f.result() for f in objs_f]
         # a violation raises here: no library is linked from a source that fails the check
         counts = [c.result() for c in checks]

@@ -31,7 +31,8 @@
 // on one XCD cover one super-tile of gm x gn tiles (shared A and B panels in that XCD's L2),
 // and super-tiles rotate over the XCDs, which keeps them evenly loaded whatever the routing
 // skew.
-#include "amoe_common.h"
+#include "gemm_common.h"
+#include "gemm_launch.h"
 
 // This file is compiled once per group of entry points (-DAMOE_GEMM_PART=0..3), in parallel: the
 // kernels of all groups are instances of the same two templates.
@@ -42,77 +43,11 @@
 #endif
 #define AMOE_PART(n) (AMOE_GEMM_PART < 0 || AMOE_GEMM_PART == (n))
 
-#include <atomic>
-#include <type_traits>
-
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 mfma_bf16x8;
-typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 mfma_f16x8;
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float mfma_f32x16;
-
-// What the kernel needs to know about its 16-bit element type: the MFMA operand vector and
-// instruction, and the conversions of the epilogues (round to nearest even on the way out).
-// Addresses, tiles and the LDS layout only depend on the element size, which the two types share.
-template <typename ET>
-struct Elem16;
-template <>
-struct Elem16<bf16_t> {
-    typedef mfma_bf16x8 frag_t;
-    __device__ static __forceinline__ float lo(uint32_t w) { return bf16_lo(w); }
-    __device__ static __forceinline__ float hi(uint32_t w) { return bf16_hi(w); }
-    __device__ static __forceinline__ uint32_t pack2(float a, float b) { return pack_bf16x2(a, b); }
-    __device__ static __forceinline__ mfma_f32x16 mfma(frag_t a, frag_t b, mfma_f32x16 c)
-    {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-    }
-};
-template <>
-struct Elem16<f16_t> {
-    typedef mfma_f16x8 frag_t;
-    __device__ static __forceinline__ float lo(uint32_t w) { return f16_lo(w); }
-    __device__ static __forceinline__ float hi(uint32_t w) { return f16_hi(w); }
-    __device__ static __forceinline__ uint32_t pack2(float a, float b) { return pack_f16x2(a, b); }
-    __device__ static __forceinline__ mfma_f32x16 mfma(frag_t a, frag_t b, mfma_f32x16 c)
-    {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    }
-};
-
 namespace {
 
 constexpr int BK = 32;      // K extent of one LDS stage
 constexpr int NSTAGE = 4;   // LDS stages: one being consumed, the others landed or in flight.  (5 stages fit
                             // the 160 KB of LDS and were measured: no faster.)
-
-struct GemmArgs {
-    const bf16_t* A;
-    const bf16_t* B;
-    bf16_t* C;
-    bf16_t* C2;
-    const int32_t* a_row_map;
-    const int32_t* b_row_map;  // weight gradient only
-    const float* row_scale;  // gated epilogues: the per-row factor of the gated activation (null = 1)
-    const bf16_t* G;         // gated-backward epilogue: gate_up [R, 2N] of the forward pass
-    float* partials;         // gated-backward epilogue: [n_ntiles][part_stride] row sums, or null
-    int ldg, part_stride;
-    const int32_t* offsets;
-    const int4* tile_map;
-    const int32_t* n_mtiles;
-    int lda, ldb, ldc, ldc2;
-    long long strideB, strideC;
-    int E;
-    int Kd;       // rows mode: reduction length
-    int M;        // wgrad mode: output rows per expert
-    int N;        // output columns
-    int n_ntiles;
-    int n_mt;     // wgrad mode: M tiles per expert
-    int rows_total;  // weight gradient: length of the row maps
-    int gm, gn;   // blocks of one XCD work on super-tiles of gm x gn tiles
-    int sn;       // super-tiles along N
-    int max_mtiles;  // rows mode: entries of tile_map (those past the last tile hold expert -1)
-    int f16;         // host side only: the operands are float16 (launch the f16 instance), else bf16
-};
-
-enum { EPI_STORE = 0, EPI_GATED = 1, EPI_GATED_BWD = 2 };
 
 #if AMOE_PART(3)
 // tile map of a caller that brings its own expert offsets (amoe_emit_tile_map has the layout)
@@ -145,16 +80,7 @@ __device__ __forceinline__ float lane_xor2(float x)
 // 16 zero bytes that masked lanes of a direct-to-LDS load read instead of out-of-range rows
 static __device__ __attribute__((aligned(16))) uint32_t g_zero_chunk[4] = {0u, 0u, 0u, 0u};
 
-// Wave-uniform load of one int32 from memory this kernel never writes: read through the
-// constant address space, which makes it a scalar load (its own counter, tracked by the
-// compiler) instead of a vector load.
-__device__ __forceinline__ int scalar_load_i32(const int32_t* ptr)
-{
-    return *(const __attribute__((address_space(4))) int32_t*)ptr;
-}
-
 typedef const __attribute__((address_space(1))) void* gptr_t;
-typedef __attribute__((address_space(3))) void* lptr_t;
 
 // wave-level half of a workgroup barrier for LDS data: this wave's LDS reads have returned and
 // all but N of its loads have landed; then the hardware barrier.  (No memory fence: LDS is not
@@ -185,47 +111,11 @@ __device__ __forceinline__ void dma16_sbase(const void* base, uint32_t lane_offs
                  : "s"(m0v), "v"(lane_offset), "s"(sb)
                  : "memory");
 }
-// the same for 4 bytes per lane (lane l lands at M0 + 4 l)
-__device__ __forceinline__ void dma4_sbase(const void* base, uint32_t lane_offset, uint32_t lds_addr)
-{
-    // (operands the compiler may hold in vector registers although they are wave-uniform)
-    const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_addr);
-    const uint64_t b64 = (uint64_t)(uintptr_t)base;
-    const uint64_t sb = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b64) |
-                        ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b64 >> 32)) << 32);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-                 :
-                 : "s"(m0v), "v"(lane_offset), "s"(sb)
-                 : "memory");
-}
 // workgroup barrier for data exchanged through LDS by ordinary LDS accesses: this wave's LDS traffic
 // has completed, then the hardware barrier (loads and stores to global memory stay in flight)
 __device__ __forceinline__ void lds_sync()
 {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-// Activation for the bf16 epilogue: the sigmoid's division by the hardware reciprocal (1 ulp; the
-// result is rounded to bf16 next) instead of the ten-instruction IEEE division sequence.
-template <int ACT>
-__device__ __forceinline__ float act_fwd_fast(float g)
-{
-    if (ACT == AMOE_ACT_SILU) return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
-    if (ACT == AMOE_ACT_GPT_OSS) return g * __builtin_amdgcn_rcpf(1.0f + __expf(-1.702f * g));
-    return act_fwd<ACT>(g);
-}
-// act(g) and act'(g) for the backward epilogue, sharing one sigmoid (hardware reciprocal, see above)
-template <int ACT>
-__device__ __forceinline__ void act_both_fast(float g, float& f, float& df)
-{
-    if (ACT == AMOE_ACT_SILU || ACT == AMOE_ACT_GPT_OSS) {
-        const float a = ACT == AMOE_ACT_SILU ? 1.0f : 1.702f;
-        const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-a * g));
-        f = g * sg;
-        df = sg * (1.0f + a * g * (1.0f - sg));
-    } else {
-        f = act_fwd<ACT>(g);
-        df = act_bwd<ACT>(g);
-    }
 }
 using T_ = std::true_type;
 using F_ = std::false_type;
@@ -426,7 +316,7 @@ __device__ __forceinline__ void grouped_gemm_wgrad_body(const GemmArgs& p)
         return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
     };
     auto read_a = [&](const u32x4_t* sa, auto KS, frag_t (&fa)[TM], auto LIVE) {
-        constexpr int ks = decltype(KS)::value;
+        [[maybe_unused]] constexpr int ks = decltype(KS)::value;
 #pragma unroll
         for (int t = 0; t < decltype(LIVE)::value; ++t) {
             fa[t] = __builtin_bit_cast(frag_t, read_tr(sa, std::integral_constant<int, BM / 8>{}, wm * WTM + t * 32, KS));
@@ -813,7 +703,7 @@ __device__ __forceinline__ void grouped_gemm_rows_body(const GemmArgs& p)
         return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
     };
     auto read_a = [&](const u32x4_t* sa, auto KS, frag_t (&fa)[TM], auto LIVE) {
-        constexpr int ks = decltype(KS)::value;
+        [[maybe_unused]] constexpr int ks = decltype(KS)::value;
 #pragma unroll
         for (int t = 0; t < decltype(LIVE)::value; ++t) {
             const int row = wm * WTM + t * 32 + lj;
@@ -1290,41 +1180,6 @@ grouped_gemm_rows_f16_kernel(GemmArgs p)
     grouped_gemm_rows_body<BM, BN, WGM, WGN, B_KC, EPI, ACT, f16_t>(p);
 }
 
-// compute units of the current device (0 if it cannot be read)
-static int device_cu_count()
-{
-    static std::atomic<int> cached[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-    int n = cached[dev].load(std::memory_order_relaxed);
-    if (n == 0) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
-        cached[dev].store(n, std::memory_order_relaxed);
-    }
-    return n;
-}
-
-template <auto KERN, int THREADS, int LDS_BYTES>
-int launch_kernel(const GemmArgs& a, int grid, hipStream_t s)
-{
-    // The LDS limit is an attribute of the kernel on one device: set once per device (bit d of the
-    // mask); setting it twice from racing threads is harmless.
-    static std::atomic<unsigned long long> attr_done{0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 63;   // 63: never cached
-    if (dev == 63 || !(attr_done.load(std::memory_order_relaxed) >> dev & 1ull)) {
-        hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(KERN),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-        if (err != hipSuccess) {
-            amoe_set_error("grouped_gemm: cannot reserve %d bytes of LDS: %s", LDS_BYTES, hipGetErrorString(err));
-            return AMOE_ERR_LAUNCH;
-        }
-        if (dev != 63) attr_done.fetch_or(1ull << dev, std::memory_order_relaxed);
-    }
-    hipLaunchKernelGGL(KERN, dim3(grid), dim3(THREADS), LDS_BYTES, s, a);
-    return amoe_check_launch("grouped_gemm_16bit");
-}
-
 // F16_OK = false leaves the float16 instance of this shape out of the library
 template <int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC, int EPI, int ACT, int MAPS = 0, bool F16_OK = true>
 int launch_cfg(const GemmArgs& a, int grid, hipStream_t s)
@@ -1395,7 +1250,9 @@ int launch_any(const GemmArgs& a, int tile_cfg, int grid, hipStream_t s)
                 return launch_cfg<256, 256, 4, 2, A_KC, B_KC, EPI, ACT, MAPS>(a, grid, s);
             }
         case 2: return launch_cfg<256, 128, 2, 2, A_KC, B_KC, EPI, ACT, MAPS>(a, grid, s);
-        default: return launch_cfg<256, 256, 2, 4, A_KC, B_KC, EPI, ACT, MAPS>(a, grid, s);  // 8 waves, 128x64 per wave
+        default:
+            if constexpr (A_KC) return AMOE_ERR_BAD_ARG;   // (the default of the row-grouped products is in gemm_pp.hip)
+            else return launch_cfg<256, 256, 2, 4, A_KC, B_KC, EPI, ACT, MAPS>(a, grid, s);  // 8 waves, 128x64 per wave
     }
 }
 
@@ -1418,7 +1275,13 @@ static int set_supertiles(GemmArgs& a, long long m_tiles, long long* grid)
     const long long sm = (m_tiles + a.gm - 1) / a.gm;
     const long long supers = sm * a.sn;
     *grid = 8 * ((supers + 7) / 8) * a.gm * a.gn;
-    AMOE_REQUIRE(*grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
+    auto inverse = [](int d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; };
+    a.inv_gm = inverse(a.gm);
+    a.inv_gn = inverse(a.gn);
+    a.inv_sn = inverse(a.sn);
+    a.inv_super = inverse(a.gm * a.gn);
+    // (n / d by multiplication with these is exact while n d < 2^32; every n here is a tile index)
+    AMOE_REQUIRE(*grid < (1ll << 31) / 32 && *grid * a.sn < (1ll << 32), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
     return AMOE_OK;
 }
 
@@ -1471,6 +1334,11 @@ int amoe_tile_map_layout(int R, int E, int dtype, int tile_cfg, void* workspace,
 
 #endif
 
+// the default tile shape (gemm_pp.hip)
+int amoe_pp_gateup_act(const GemmArgs& a, int act, int tiles, hipStream_t s);
+int amoe_pp_rows(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s);
+int amoe_pp_gated_bwd(const GemmArgs& a, int act, int tiles, hipStream_t s);
+
 // rows mode driver shared by the three row-grouped entry points
 template <bool B_KC, int EPI, int ACT>
 static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C,
@@ -1517,6 +1385,11 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
     a.max_mtiles = max_mtiles;
     rc = set_supertiles(a, max_mtiles, &grid);
     if (rc) return rc;
+    if (tile_cfg == 0) {
+        if constexpr (EPI == EPI_GATED) return amoe_pp_gateup_act(a, ACT, (int)grid, s);
+        else if constexpr (EPI == EPI_GATED_BWD) return amoe_pp_gated_bwd(a, ACT, (int)grid, s);
+        else return amoe_pp_rows(a, B_KC, (int)grid, s);
+    }
     return launch_any<true, B_KC, EPI, ACT>(a, tile_cfg, (int)grid, s);
 }
 

@@ -1,0 +1,754 @@
+// The 16-bit grouped GEMMs at the default tile shape, 256 x 256 x 64 on v_mfma_f32_16x16x32, f32 accumulate.
+//
+// 512 threads = two groups of four wavefronts, one wavefront of each group per SIMD.  A K tile is worked off in
+// four phases, one quadrant of the output each; a phase is a memory part (LDS reads of the operands the phase
+// needs, direct-to-LDS loads of the K tile after the next, and, at a tile's end, the epilogue of the quadrant
+// finished one phase before) and an arithmetic part (16 MFMAs back to back).  The second group runs one part
+// behind the first, held there by the workgroup barrier after every part: while one wavefront of a SIMD issues
+// MFMAs, the other does everything else, so reads, loads and the epilogue's conversions and stores sit under
+// the matrix pipe instead of between its bursts.
+#include "gemm_common.h"
+
+#ifndef AMOE_PP_PART
+#define AMOE_PP_PART -1
+#endif
+#define AMOE_PP_PART_IS(n) (AMOE_PP_PART < 0 || AMOE_PP_PART == (n))
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float mfma_f32x4;
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+
+namespace {
+
+constexpr int PP_BM = 256, PP_BN = 256, PP_BK = 64;
+constexpr int PP_THREADS = 512;
+constexpr uint32_t PP_HALF = 128 * PP_BK * 2;        // bytes of a half tile: 128 rows (or columns) of one operand
+constexpr uint32_t PP_STAGE = 4 * PP_HALF;           // A0 A1 B0 B1
+constexpr uint32_t PP_IDX = 2 * PP_STAGE;            // row indices of the next tile, 64 per wavefront
+constexpr uint32_t PP_SCALE = PP_IDX + 8 * 64 * 4;   // row scales of two tiles
+constexpr uint32_t PP_PART = PP_SCALE + 2 * PP_BM * 4;   // row-sum partials, one row of 256 per wave column
+constexpr uint32_t PP_LDS = PP_PART + 4 * PP_BM * 4;
+
+constexpr uint32_t PP_NOWHERE = 0xFFFFFFF0u;         // a load offset past every operand: the lane receives zeros
+constexpr uint32_t PP_DROP = 0x80000000u;            // a store offset past the tile: the lane stores nothing
+
+using T_ = std::true_type;
+using F_ = std::false_type;
+
+typedef uint32_t srd_t __attribute__((ext_vector_type(4)));
+
+template <typename ET>
+struct Mfma16;
+template <>
+struct Mfma16<bf16_t> {
+    __device__ static __forceinline__ mfma_f32x4 run(mfma_bf16x8 a, mfma_bf16x8 b, mfma_f32x4 c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
+};
+template <>
+struct Mfma16<f16_t> {
+    __device__ static __forceinline__ mfma_f32x4 run(mfma_f16x8 a, mfma_f16x8 b, mfma_f32x4 c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+    }
+};
+
+// 16 bytes per lane from global memory straight into LDS (lane l lands at lds_addr + 16 l): a wave-uniform base,
+// a 32-bit byte offset per lane.  Through a buffer descriptor, whose range check returns zeros for PP_NOWHERE:
+// rows past an expert's end, columns past the matrix and the K remainder need no clamping and no masking.
+// Not known to the compiler: the kernel's own vmcnt waits cover it.
+// (lds_addr = lds_base + LDS_OFF is formed in M0 itself)
+template <uint32_t LDS_OFF>
+__device__ __forceinline__ void pp_dma16(const srd_t& d, uint32_t off, uint32_t lds_base)
+{
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds_base), "v"(off), "s"(d), "n"(LDS_OFF)
+                 : "memory", "scc");
+}
+__device__ __forceinline__ srd_t pp_srd(const void* base)
+{
+    const uint64_t b = (uint64_t)(uintptr_t)base;
+    return srd_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b), (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)),
+                 PP_NOWHERE, 0x00020000u};
+}
+// move a descriptor's base on
+__device__ __forceinline__ void pp_advance(srd_t& d, uint32_t bytes)
+{
+    const uint64_t b = (((uint64_t)d[1] << 32) | d[0]) + bytes;
+    d[0] = (uint32_t)b;
+    d[1] = (uint32_t)(b >> 32);
+}
+
+template <int N>
+__device__ __forceinline__ void pp_vmwait()
+{
+    static_assert(N >= 0 && N <= 63, "vmcnt is 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void pp_fence() { __builtin_amdgcn_sched_barrier(0); }
+__device__ __forceinline__ void pp_barrier()
+{
+    pp_fence();
+    __builtin_amdgcn_s_barrier();
+    pp_fence();
+}
+template <typename T>
+__device__ __forceinline__ T pp_lds(uint32_t addr)
+{
+    return *(const __attribute__((address_space(3))) T*)(uintptr_t)addr;
+}
+
+// (x, y) = four consecutive columns each of two 16-column tiles, lane quarter q holding columns 4q..4q+3 of both;
+// afterwards quarter q holds columns 8q..8q+7 of the 32: x the first four of them, y the second four.
+__device__ __forceinline__ void pp_join(uint32_t& x, uint32_t& y)
+{
+    auto a = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    auto b = __builtin_amdgcn_permlane16_swap(a[0], a[1], false, false);
+    x = b[0];
+    y = b[1];
+}
+// sum over the four lane quarters, in every lane
+__device__ __forceinline__ float pp_quarter_sum(float v)
+{
+    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const float s = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+__device__ __forceinline__ void pp_store16(__amdgpu_buffer_rsrc_t d, u32x4_t v, uint32_t off, uint32_t soff)
+{
+    __builtin_amdgcn_raw_buffer_store_b128(v, d, off, soff, 0);
+    // (a 16-byte store reads its data a wait state after it issues, and not only without a scalar offset as the
+    // compiler assumes: with the next instruction writing the first of the four registers, lanes 12-15 of each 16
+    // stored that instruction's result, in about one row of 200)
+    pp_fence();
+    asm volatile("s_nop 1");
+    pp_fence();
+}
+
+// The kernel's arguments, read again from the kernel argument segment at each place that uses them between two
+// K loops: held in scalar registers across the loops they would spill.  (The argument struct is the only one.)
+typedef const __attribute__((address_space(4))) GemmArgs args_t;
+__device__ __forceinline__ args_t& pp_args()
+{
+    auto k = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    return *(args_t*)k;
+}
+// a value the compiler cannot trace: what is derived from it is computed here, not hoisted out of the tile loop
+__device__ __forceinline__ int pp_here(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// ------------------------------------------------------------------ row-grouped products
+// C[rows_e,:] = A[rows_e,:] @ B[e] (B_KC false: B [Kd,N]) or @ B[e]^T (B_KC: B [N,Kd]).
+// Persistent: one workgroup per CU walks its tiles, and the K loops of consecutive tiles form one stream of
+// K tiles -- the loads run two K tiles ahead, across the tile boundary.
+//
+// LDS: a K tile is four half tiles of 128 x 64, two stages.  K-contiguous halves are [row][8 chunks of 16 B],
+// chunk c of row r at c ^ ((r >> 1) & 7); K-strided halves are [k][16 chunks], chunk c of row k at
+// c ^ 2 ((k & 3) | (((k >> 3) & 1) << 2)), read with the transposing LDS read.  Either way the 32 lanes that the
+// LDS serves together meet every bank once.
+//
+// Wave (g, wc): g = group, wc = column quarter.  Quadrant (a, b): tile rows a*128.., columns b*128 + wc*32 ..+31.
+// The rows of a half are dealt to the groups in blocks of 16 (row = (a*4 + i)*32 + g*16 + l), so that a tile with
+// fewer live rows spares both groups the same MFMAs.
+//
+// What bounds it: the memory part of a phase has to fit into the other group's 256 cycles of MFMA, so every
+// instruction in it counts (range tests on the loads, waits chosen by a branch and branches around dead rows each
+// cost 4-6 % of the K loop and are gone from it).  Measured on one MI355X, 131072 rows, N = 2048, bf16 NT: K = 8192
+// 1.50-1.66 PFLOP/s (operands from HBM / from L2); K = 2048 1.23-1.43, K = 768 1.0: what a tile costs beside its K loop
+// is about 5 us, of which half are its stores.  The kernel this one replaced (32-wide K tiles, 32x32x16 MFMAs, all
+// eight waves in step) ran at 1.0-1.1 on the same problems.
+template <bool B_KC, int EPI, int ACT, typename ET>
+__device__ __forceinline__ void pp_rows_body()
+{
+    typedef typename Elem16<ET>::frag_t frag_t;
+    extern __shared__ u32x4_t smem[];
+    const uint32_t lds = (uint32_t)(uintptr_t)(lptr_t)smem;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = wave >> 2, wc = wave & 3;
+    const int l16 = lane & 15, lq = lane >> 4;
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I4 = std::integral_constant<int, 4>;
+    const int Kd = pp_args().Kd;
+    const int KT = max(4, (Kd + PP_BK - 1) / PP_BK);               // K tiles (of a short reduction, the last are empty)
+    const bool ragged_k = Kd < KT * PP_BK;
+
+    // ------------------------------------------------------------ this workgroup's tiles
+    // Virtual blocks b, b + grid, b + 2 grid, ...; virtual block v belongs to XCD v % 8 (the hardware deals
+    // workgroups to the XCDs round-robin) and is slot (v / 8) % (gm gn) of super-tile ((v / 8) / (gm gn)) * 8
+    // + v % 8: the workgroups resident on one XCD work on one super-tile of gm x gn tiles at a time (its gm A
+    // panels and gn B panels are shared in that XCD's L2) and the super-tiles rotate over the XCDs.  Only whole
+    // groups of 8 super-tiles are dealt that way; the up to 7 left over go to the XCDs tile by tile.
+    // (divisions by multiplication with the host's rounded-up reciprocals: exact for the numerators that occur)
+    int vb_next = blockIdx.x;
+    const int n_mtiles = min(scalar_load_i32(pp_args().n_mtiles), pp_args().max_mtiles);
+    auto divide = [](int n, uint32_t inv) -> int { return inv ? (int)(((uint64_t)(uint32_t)n * inv) >> 32) : n; };
+    auto advance = [&](int& pm, int& nt) -> bool {
+        args_t& p = pp_args();
+        const int per_super = p.gm * p.gn;
+        const int supers = (divide(n_mtiles + p.gm - 1, p.inv_gm)) * p.sn;
+        const int vb_rot = (supers >> 3) * 8 * per_super;
+        const int vb_total = supers * per_super;
+        while (vb_next < vb_total) {
+            const int vb = vb_next;
+            vb_next += gridDim.x;
+            int sid, w;
+            if (vb < vb_rot) {
+                const int xcd = vb & 7, q = vb >> 3;
+                sid = divide(q, p.inv_super);
+                w = q - sid * per_super;
+                sid = sid * 8 + xcd;
+            } else {
+                sid = divide(vb, p.inv_super);
+                w = vb - sid * per_super;
+            }
+            const int sm = divide(sid, p.inv_sn), sn_i = sid - sm * p.sn;
+            const int wm = divide(w, p.inv_gn);
+            pm = sm * p.gm + wm;
+            nt = sn_i * p.gn + w - wm * p.gn;
+            if (nt < p.n_ntiles && pm < n_mtiles) return true;
+        }
+        return false;
+    };
+    auto load_entry = [&](int pm) -> int4 {
+        const int32_t* ent = reinterpret_cast<const int32_t*>(pp_args().tile_map + pm);
+        int4 v;
+        v.x = scalar_load_i32(ent);
+        v.y = scalar_load_i32(ent + 1);
+        v.z = scalar_load_i32(ent + 2);
+        v.w = 0;
+        return v;
+    };
+
+    // ------------------------------------------------------------ loads
+    // Thread tid fills chunks tid and tid + 512 of every half tile.
+    // Thread tid's: K-contiguous row tid / 8 (+ 64 j), k (tid % 8 ^ (row / 2) % 8) * 8; K-strided k row tid / 16 (+ 32 j).
+    uint32_t aoff[2][2], boff[2][2];
+    srd_t ad, bd;
+    const int lda = pp_args().lda, ldb = pp_args().ldb, N = pp_args().N;
+    const bf16_t* const A = pp_args().A;
+    const bool gather = pp_args().a_row_map != nullptr;
+    const uint32_t bstep = B_KC ? PP_BK * 2 : (uint32_t)ldb * (PP_BK * 2);
+    auto expert_b = [&](int e) { args_t& p = pp_args(); return p.B + (long long)e * p.strideB; };
+    // a plan without rows (m0 == mend) or columns (n0 >= N) reads nothing
+    auto plan_a = [&](int m0, int mend, const int32_t* map) {     // map: the row map (first tile), else the indices are in LDS
+        const int th = pp_here(tid);
+        const int r = th >> 3, k = ((th & 7) ^ ((r >> 1) & 7)) * 8;
+        // tile row of this thread's chunk in half a: (a*4 + i)*32 + j*16 + l with i = r / 16, l = r % 16
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int row = m0 + (a * 4 + (r >> 4)) * 32 + j * 16 + (r & 15);
+                int gr = row;
+                if (gather)
+                    gr = map ? map[min(row, mend - 1)] : pp_lds<int>(lds + PP_IDX + (uint32_t)(wave * 64 + a * 16 + j * 8 + (r & 7)) * 4u);
+                aoff[a][j] = row < mend && k < Kd ? ((uint32_t)gr * (uint32_t)lda + k) * 2u : PP_NOWHERE;
+            }
+        ad = pp_srd(A);
+    };
+    auto plan_b = [&](const bf16_t* B, int n0) {
+        const int th = pp_here(tid);
+        const int r = th >> 3, kr = th >> 4;
+        const int k = ((th & 7) ^ ((r >> 1) & 7)) * 8;
+        const int col = ((th & 15) ^ (2 * ((kr & 3) | (((kr >> 3) & 1) << 2)))) * 8;
+        bd = pp_srd(B);
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int n = n0 + b * 128 + (B_KC ? r + 64 * j : col);
+                const uint32_t o = B_KC ? (uint32_t)n * (uint32_t)ldb + k : (uint32_t)(kr + 32 * j) * (uint32_t)ldb + n;
+                boff[b][j] = n < N && (B_KC ? k : kr + 32 * j) < Kd ? o * 2u : PP_NOWHERE;
+            }
+    };
+    // the K tile loaded next holds only `left` of its 64 k (none at all if left <= 0)
+    auto cut_k = [&](int left) {
+        const int th = pp_here(tid);
+        const int k = ((th & 7) ^ ((th >> 4) & 7)) * 8, kr = th >> 4;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                if (k >= left) aoff[h][j] = PP_NOWHERE;
+                if ((B_KC ? k : kr + 32 * j) >= left) boff[h][j] = PP_NOWHERE;
+            }
+    };
+    uint32_t fill = lds + (uint32_t)wave * 1024u;                  // this wave's place in the stage being filled
+    auto dma_a = [&](auto A_) {
+        constexpr int a = decltype(A_)::value;
+        pp_dma16<a * PP_HALF>(ad, aoff[a][0], fill);
+        pp_dma16<a * PP_HALF + 8192u>(ad, aoff[a][1], fill);
+    };
+    auto dma_b = [&](auto B_) {
+        constexpr int b = decltype(B_)::value;
+        pp_dma16<(2 + b) * PP_HALF>(bd, boff[b][0], fill);
+        pp_dma16<(2 + b) * PP_HALF + 8192u>(bd, boff[b][1], fill);
+    };
+    auto next_k = [&]() {
+        fill ^= PP_STAGE;
+        pp_advance(ad, PP_BK * 2);
+        pp_advance(bd, bstep);
+    };
+
+    // ------------------------------------------------------------ fragments
+    frag_t fa[4][2], fb0[2][2], fb1[2][2];
+    uint32_t ra[2], rb[2];   // LDS read addresses: A per k step; B per k step (K-contiguous) or per 16-column tile
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const int row = grp * 64 + l16;
+        ra[s] = lds + (uint32_t)(row * 8 + ((s * 4 + lq) ^ ((row >> 1) & 7))) * 16u;
+        if (B_KC) {
+            const int n = wc * 32 + l16;
+            rb[s] = lds + 2 * PP_HALF + (uint32_t)(n * 8 + ((s * 4 + lq) ^ ((n >> 1) & 7))) * 16u;
+        } else {
+            const int k = 8 * lq + (l16 >> 2);
+            const int chunk = (wc * 4 + 2 * s + ((l16 & 3) >> 1)) ^ (2 * ((l16 >> 2) | ((lq & 1) << 2)));
+            rb[s] = lds + 2 * PP_HALF + (uint32_t)(k * 256 + chunk * 16 + (l16 & 1) * 8);
+        }
+    }
+    auto flip = [&]() {
+        ra[0] ^= PP_STAGE;
+        ra[1] ^= PP_STAGE;
+        rb[0] ^= PP_STAGE;
+        rb[1] ^= PP_STAGE;
+    };
+    auto read_a = [&](auto A_, auto N_) {
+#pragma unroll
+        for (int i = 0; i < decltype(N_)::value; ++i)
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                fa[i][s] = __builtin_bit_cast(frag_t, pp_lds<u32x4_t>(ra[s] + decltype(A_)::value * PP_HALF + i * 2048u));
+    };
+    auto read_b = [&](auto B_, frag_t (&fb)[2][2]) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                if (B_KC) {
+                    fb[j][s] = __builtin_bit_cast(frag_t, pp_lds<u32x4_t>(rb[s] + decltype(B_)::value * PP_HALF + j * 2048u));
+                } else {
+                    const uint32_t ad = rb[j] + decltype(B_)::value * PP_HALF + s * 8192u;
+                    typedef __attribute__((address_space(3))) i16x4_t* tr_ptr;
+                    const u32x2_t lo = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)ad));
+                    const u32x2_t hi = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)(ad + 1024u)));
+                    fb[j][s] = __builtin_bit_cast(frag_t, u32x4_t{lo[0], lo[1], hi[0], hi[1]});
+                }
+            }
+    };
+    // FIRST: the quadrant's first K tile, nothing to add to
+    auto mma = [&](auto FIRST, auto N_, mfma_f32x4 (&c)[4][2], const frag_t (&fb)[2][2]) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int i = 0; i < decltype(N_)::value; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    c[i][j] = Mfma16<ET>::run(fb[j][s], fa[i][s], decltype(FIRST)::value && s == 0 ? mfma_f32x4{0.f, 0.f, 0.f, 0.f} : c[i][j]);
+    };
+
+    // ------------------------------------------------------------ tile state
+    int m0, mend, nt, n0;
+    bool have_n, have_nn = false;        // is there a next tile, and one after it
+    int nt_n = 0, nt_nn = 0;
+    int4 tm_n, tm_nn = make_int4(0, 0, 0, 0);
+    const bf16_t* b_n = nullptr;
+    {
+        int pm = 0;
+        nt = 0;
+        if (!advance(pm, nt)) return;
+        const int4 tm = load_entry(pm);
+        m0 = tm.y;
+        mend = tm.z;
+        have_n = advance(pm, nt_n);
+        tm_n = have_n ? load_entry(pm) : make_int4(0, 0, 0, 0);
+        n0 = nt * PP_BN;
+        plan_a(m0, mend, pp_args().a_row_map);
+        plan_b(expert_b(tm.x), n0);
+    }
+    int par = 0;            // row scales: which of the two LDS rows is this tile's
+    bool sums_due = false;  // row-sum partials of the previous tile are complete in LDS and not yet written
+    int sums_m0 = 0, sums_end = 0, sums_nt = 0;
+
+    // ------------------------------------------------------------ epilogue of quadrant (a, b)
+    // Lane (lq, l16) holds columns 4 lq ..+3 of both 16-column tiles j for row l16 of every 16-row block.
+    // What the four quadrants share is worked out during the last K tile but one.
+    bf16_t *e_c, *e_c2;      // this wave's first element of the tile in the outputs (gated backward: d_gate_up, and gate_up)
+    int e_ldc = 0, e_ldc2 = 0, e_cols = 0, e_rows = 0;
+    uint32_t e_off = 0, e_off2 = 0;
+    auto prepare_epilogue = [&]() {
+        args_t& p = pp_args();
+        const int le = pp_here(lane);
+        const int rl = grp * 16 + (le & 15), eq = le >> 4;
+        const int c0 = n0 + wc * 32;
+        e_cols = N - c0;                 // columns of the wave's part that exist, from its first one (N is a multiple of 8)
+        e_rows = mend - m0;
+        if (EPI == EPI_GATED_BWD) {
+            e_ldc = p.ldg;
+            e_c = p.C + (long long)m0 * e_ldc + 2 * c0;
+            e_c2 = const_cast<bf16_t*>(p.G) + (long long)m0 * e_ldc + 2 * c0;
+            e_off = (uint32_t)(rl * e_ldc + 8 * eq) * 2u;
+        } else {
+            e_ldc = p.ldc;
+            e_c = p.C;
+            if (EPI != EPI_GATED || e_c) e_c += (long long)m0 * e_ldc + c0;
+            e_off = (uint32_t)(rl * e_ldc + 8 * eq) * 2u;
+            if (EPI == EPI_GATED) {
+                e_ldc2 = p.ldc2;
+                e_c2 = p.C2 + (long long)m0 * e_ldc2 + (c0 >> 1);
+                e_off2 = (uint32_t)(rl * e_ldc2 + 4 * eq) * 2u;
+            }
+        }
+    };
+    u32x4_t gu[2][4][2];     // gated backward: gate_up of two quadrants, requested ahead of their epilogues
+    auto fetch_gate_up = [&](auto A_, auto B_) {
+        constexpr int a = decltype(A_)::value, b = decltype(B_)::value;
+        if constexpr (EPI == EPI_GATED_BWD) {
+            const int le = pp_here(lane);
+            const int eq = le >> 4, rl = grp * 16 + (le & 15);
+            const __amdgpu_buffer_rsrc_t g = __builtin_amdgcn_make_buffer_rsrc(e_c2, (short)0, (int)PP_DROP, 0x00020000);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const bool ok = b * 128 + 16 * j + 4 * eq < e_cols && (a * 4 + i) * 32 + rl < e_rows;
+                    gu[b][i][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                               g, ok ? e_off + j * 64u : PP_DROP, (a * 4 + i) * (uint32_t)e_ldc * 64u + b * 512u, 0));
+                }
+        }
+    };
+    float dots[4] = {0.f, 0.f, 0.f, 0.f};
+    auto epilogue = [&](auto A_, auto B_, const mfma_f32x4 (&acc)[4][2]) {
+        constexpr int a = decltype(A_)::value, b = decltype(B_)::value;
+        const int le = pp_here(lane);
+        const int eq = le >> 4, rl = grp * 16 + (le & 15);
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc(e_c, (short)0, (int)PP_DROP, 0x00020000);
+        const uint32_t srow = (uint32_t)e_ldc * 64u;           // bytes of 32 rows
+        if constexpr (EPI == EPI_GATED_BWD) {
+            // d_inter is in the accumulators; the (gate, up) pairs of its columns come back from the forward pass
+            auto place = [&](int j, int i) {
+                return b * 128 + 16 * j + 4 * eq < e_cols && (a * 4 + i) * 32 + rl < e_rows ? e_off + j * 64u : PP_DROP;
+            };
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                pp_fence();   // (left alone, the scheduler interleaves the activation chains and their temporaries spill)
+                const float s = pp_lds<float>(lds + PP_SCALE + (uint32_t)(par * PP_BM + (a * 4 + i) * 32 + rl) * 4u);
+                float dot = 0.f;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    u32x4_t o;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float dd = acc[i][j][v];
+                        const float gate = Elem16<ET>::lo(gu[b][i][j][v]), up = Elem16<ET>::hi(gu[b][i][j][v]);
+                        float f, df;
+                        act_both_fast<ACT>(gate, f, df);
+                        dot += dd * up * f;
+                        const float sd = s * dd;
+                        o[v] = Elem16<ET>::pack2(sd * up * df, sd * f);
+                    }
+                    pp_store16(d, o, place(j, i), (a * 4 + i) * srow + b * 512u);
+                    pp_fence();
+                }
+                dots[i] = b == 0 ? dot : dots[i] + dot;
+                asm volatile("" : "+v"(dots[i]));   // (summed up here: put off to its use, the sum holds on to all its terms)
+                if (b == 1) {
+                    const float t = pp_quarter_sum(dots[i]);
+                    if (eq == 0) *(__attribute__((address_space(3))) float*)(uintptr_t)(lds + PP_PART + (uint32_t)(wc * PP_BM + (a * 4 + i) * 32 + rl) * 4u) = t;
+                }
+            }
+            if (b == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        } else {
+            const __amdgpu_buffer_rsrc_t d2 = __builtin_amdgcn_make_buffer_rsrc(EPI == EPI_GATED ? e_c2 : e_c, (short)0, (int)PP_DROP, 0x00020000);
+            const uint32_t srow2 = (uint32_t)e_ldc2 * 64u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                pp_fence();
+                const bool ok = b * 128 + 8 * eq < e_cols && (a * 4 + i) * 32 + rl < e_rows;
+                uint32_t x[2], y[2];
+#pragma unroll
+                for (int v = 0; v < 2; ++v) {
+                    x[v] = Elem16<ET>::pack2(acc[i][0][2 * v], acc[i][0][2 * v + 1]);
+                    y[v] = Elem16<ET>::pack2(acc[i][1][2 * v], acc[i][1][2 * v + 1]);
+                }
+                if constexpr (EPI == EPI_GATED) {
+                    // a packed pair is (gate, up) of one intermediate column
+                    const float s = pp_lds<float>(lds + PP_SCALE + (uint32_t)(par * PP_BM + (a * 4 + i) * 32 + rl) * 4u);
+                    uint32_t hx = Elem16<ET>::pack2(s * Elem16<ET>::hi(x[0]) * act_fwd_fast<ACT>(Elem16<ET>::lo(x[0])),
+                                                    s * Elem16<ET>::hi(x[1]) * act_fwd_fast<ACT>(Elem16<ET>::lo(x[1])));
+                    uint32_t hy = Elem16<ET>::pack2(s * Elem16<ET>::hi(y[0]) * act_fwd_fast<ACT>(Elem16<ET>::lo(y[0])),
+                                                    s * Elem16<ET>::hi(y[1]) * act_fwd_fast<ACT>(Elem16<ET>::lo(y[1])));
+                    pp_join(hx, hy);
+                    __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{hx, hy}, d2, ok ? e_off2 : PP_DROP, (a * 4 + i) * srow2 + b * 128u, 0);
+                }
+                pp_join(x[0], y[0]);
+                pp_join(x[1], y[1]);
+                if (EPI != EPI_GATED || e_c) pp_store16(d, u32x4_t{x[0], x[1], y[0], y[1]}, ok ? e_off : PP_DROP, (a * 4 + i) * srow + b * 256u);
+            }
+        }
+    };
+    // the row sums of a finished tile: each group adds up its own rows' four wave columns
+    auto write_sums = [&]() {
+        if constexpr (EPI == EPI_GATED_BWD) {
+            args_t& p = pp_args();
+            if (sums_due && p.partials) {
+                const int lane = pp_here(tid) & 63;
+                const int w = wc * 32 + (lane & 31);                       // 128 rows of this group
+                const int row = (w >> 4) * 32 + grp * 16 + (w & 15);
+                float t = 0.f;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) t += pp_lds<float>(lds + PP_PART + (uint32_t)(c * PP_BM + row) * 4u);
+                if (lane < 32 && sums_m0 + row < sums_end) p.partials[(long long)sums_nt * p.part_stride + sums_m0 + row] = t;
+            }
+            sums_due = false;
+        }
+    };
+
+    // ------------------------------------------------------------ one tile
+    // The waits: phase n awaits the loads issued in phase n - 5, which the next phase reads after the barrier; ten younger
+    // loads stay in flight.  (Epilogue stores count as well and are not allowed for: letting them stay in flight through
+    // the first K tile was measured and gains nothing.)
+    auto run_tile = [&]() {
+        mfma_f32x4 acc[2][2][4][2];
+        // ---- phase 0 of the first K tile
+        read_a(I0{}, I4{});
+        dma_a(I1{});
+        next_k();
+        {
+            args_t& p = pp_args();
+            const int le = pp_here(lane);
+            if (EPI != EPI_STORE && wave < 4) {
+                const int row = wave * 64 + le;
+                const uint32_t dst = lds + PP_SCALE + (uint32_t)(par * PP_BM + wave * 64) * 4u;
+                if (p.row_scale) {
+                    dma4_sbase(p.row_scale, (uint32_t)min(m0 + row, mend - 1) * 4u, dst);
+                } else {
+                    *(__attribute__((address_space(3))) float*)(uintptr_t)(dst + le * 4u) = 1.0f;
+                }
+            }
+            if (p.a_row_map && have_n) {
+                const int q = le & 31, r = wave * 8 + (q & 7);
+                const int row = ((q >> 4) * 4 + (r >> 4)) * 32 + ((q >> 3) & 1) * 16 + (r & 15);
+                dma4_sbase(p.a_row_map, (uint32_t)min(tm_n.y + row, tm_n.z - 1) * 4u, lds + PP_IDX + (uint32_t)wave * 256u);
+            }
+        }
+        pp_vmwait<10>();
+        pp_barrier();
+        mma(T_{}, I4{}, acc[0][0], fb0);
+        {
+            // the next tile's weights; which tile follows it, and its entry of the tile map
+            b_n = expert_b(tm_n.x);
+            int pm = 0;
+            have_nn = have_n && advance(pm, nt_nn);
+            tm_nn = have_nn ? load_entry(pm) : make_int4(0, 0, 0, 0);
+        }
+        pp_barrier();
+        write_sums();
+        // K tile t (t < KT - 1): phases 1..3, and phase 0 of the next; loads K tile t + 2, with TURN (t = KT - 2) the
+        // next tile's first one
+        auto k_tile = [&](auto FIRST, auto TURN, auto N_) {
+            constexpr bool turn = decltype(TURN)::value;
+            // phase 1
+            read_b(I1{}, fb1);
+            if (turn) plan_b(b_n, have_n ? nt_n * PP_BN : 0x7fffff00);
+            dma_b(I0{});
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(FIRST, I4{}, acc[0][1], fb1);
+            pp_barrier();
+            // phase 2
+            read_a(I1{}, N_);
+            if (turn) {
+                plan_a(tm_n.y, tm_n.z, nullptr);
+            }
+            dma_a(I0{});
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(FIRST, N_, acc[1][0], fb0);
+            pp_barrier();
+            // phase 3
+            flip();
+            read_b(I0{}, fb0);
+            dma_b(I1{});
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(FIRST, N_, acc[1][1], fb1);
+            if (turn) prepare_epilogue();
+            pp_barrier();
+            // phase 0 of the next K tile
+            read_a(I0{}, I4{});
+            dma_a(I1{});
+            next_k();
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(F_{}, I4{}, acc[0][0], fb0);
+            pp_barrier();
+        };
+        if (Kd < 3 * PP_BK) cut_k(Kd - 2 * PP_BK);                      // K tile 2 is loaded next
+        k_tile(T_{}, F_{}, I4{});
+        // The rows of the lower half beyond the last block with a live row are neither read nor multiplied: one copy of
+        // the loop per number of such blocks, one after the other, all but one of them with no iterations (chosen
+        // between by if and else, each copy's registers would be live across the others).
+        const int n1 = min(max(((mend - m0 + 31) >> 5) - 4, 0), 4);
+        int t = 1;
+        for (int part = 0; part < 2; ++part) {
+            const int end = KT - 3 + part;
+            for (const int e = n1 == 4 ? end : 0; t < e; ++t) k_tile(F_{}, F_{}, I4{});
+            for (const int e = n1 == 3 ? end : 0; t < e; ++t) k_tile(F_{}, F_{}, std::integral_constant<int, 3>{});
+            for (const int e = n1 == 2 || n1 == 1 ? end : 0; t < e; ++t) k_tile(F_{}, F_{}, std::integral_constant<int, 2>{});
+            for (const int e = n1 == 0 ? end : 0; t < e; ++t) k_tile(F_{}, F_{}, I0{});
+            if (part == 0 && ragged_k) cut_k(Kd - (KT - 1) * PP_BK);    // K tile KT - 1 is loaded next
+        }
+        k_tile(F_{}, T_{}, I4{});
+        if (Kd < 2 * PP_BK) cut_k(Kd - PP_BK);                          // the next tile's K tile 1 is loaded next
+        // ---- last K tile
+        if constexpr (EPI == EPI_STORE) {
+            // the epilogue of each finished quadrant in the memory part of the phase after it
+            read_b(I1{}, fb1);
+            dma_b(I0{});
+            epilogue(I0{}, I0{}, acc[0][0]);
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(F_{}, I4{}, acc[0][1], fb1);
+            pp_barrier();
+            read_a(I1{}, I4{});
+            dma_a(I0{});
+            epilogue(I0{}, I1{}, acc[0][1]);
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(F_{}, I4{}, acc[1][0], fb0);
+            pp_barrier();
+            flip();
+            read_b(I0{}, fb0);
+            dma_b(I1{});
+            epilogue(I1{}, I0{}, acc[1][0]);
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(F_{}, I4{}, acc[1][1], fb1);
+            pp_barrier();
+            epilogue(I1{}, I1{}, acc[1][1]);
+        } else {
+            // activations are far more vector work than one arithmetic part hides: all four quadrants together, so
+            // that the two wavefronts of a SIMD share its vector unit instead of taking turns at it
+            read_b(I1{}, fb1);
+            dma_b(I0{});
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(F_{}, I4{}, acc[0][1], fb1);
+            pp_barrier();
+            read_a(I1{}, I4{});
+            dma_a(I0{});
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(F_{}, I4{}, acc[1][0], fb0);
+            pp_barrier();
+            flip();
+            dma_b(I1{});
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(F_{}, I4{}, acc[1][1], fb1);
+            fetch_gate_up(I0{}, I0{});
+            fetch_gate_up(I0{}, I1{});
+            pp_barrier();
+            epilogue(I0{}, I0{}, acc[0][0]);
+            fetch_gate_up(I1{}, I0{});
+            epilogue(I0{}, I1{}, acc[0][1]);
+            fetch_gate_up(I1{}, I1{});
+            epilogue(I1{}, I0{}, acc[1][0]);
+            epilogue(I1{}, I1{}, acc[1][1]);
+            read_b(I0{}, fb0);
+        }
+    };
+
+    // ------------------------------------------------------------ the workgroup's tiles
+    dma_b(I0{}); dma_a(I0{}); dma_b(I1{}); dma_a(I1{});
+    next_k();
+    if (Kd < 2 * PP_BK) cut_k(Kd - PP_BK);
+    dma_b(I0{}); dma_a(I0{}); dma_b(I1{});
+    pp_vmwait<12>();
+    pp_barrier();
+    if (grp == 1) pp_barrier();
+    read_b(I0{}, fb0);
+    pp_vmwait<10>();
+    pp_barrier();
+    pp_barrier();
+    for (;;) {
+        run_tile();
+        if (EPI == EPI_GATED_BWD) {
+            sums_due = true;
+            sums_m0 = m0;
+            sums_end = mend;
+            sums_nt = nt;
+        }
+        if (!have_n) break;
+        m0 = tm_n.y;
+        mend = tm_n.z;
+        nt = nt_n;
+        n0 = nt * PP_BN;
+        have_n = have_nn;
+        nt_n = nt_nn;
+        tm_n = tm_nn;
+        par ^= 1;
+    }
+    pp_barrier();
+    write_sums();
+    if (grp == 0) pp_barrier();
+    pp_vmwait<0>();   // (loads past the last tile wrote zeros into LDS: landed before the workgroup leaves)
+}
+
+template <bool B_KC, int EPI, int ACT>
+__global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_rows_bf16_kernel(GemmArgs)
+{
+    pp_rows_body<B_KC, EPI, ACT, bf16_t>();
+}
+template <bool B_KC, int EPI, int ACT>
+__global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_rows_f16_kernel(GemmArgs)
+{
+    pp_rows_body<B_KC, EPI, ACT, f16_t>();
+}
+
+}  // namespace
+
+#include "gemm_launch.h"
+
+template <bool B_KC, int EPI, int ACT>
+static int launch_pp_rows(const GemmArgs& a, int tiles, hipStream_t s)
+{
+    const int cus = device_cu_count();
+    AMOE_REQUIRE(cus > 0, AMOE_ERR_LAUNCH, "grouped_gemm: cannot read the number of compute units");
+    // (a multiple of 8: every XCD then runs the same number of workgroups)
+    const int grid = ((tiles < cus ? tiles : cus) + 7) & ~7;
+    if (a.f16) return launch_kernel<grouped_gemm_pp_rows_f16_kernel<B_KC, EPI, ACT>, PP_THREADS, PP_LDS>(a, grid, s);
+    return launch_kernel<grouped_gemm_pp_rows_bf16_kernel<B_KC, EPI, ACT>, PP_THREADS, PP_LDS>(a, grid, s);
+}
+
+// `tiles`: upper bound of the number of tiles
+#if AMOE_PP_PART_IS(0)
+int amoe_pp_gateup_act(const GemmArgs& a, int act, int tiles, hipStream_t s)
+{
+    AMOE_DISPATCH_ACT(act, return (launch_pp_rows<false, EPI_GATED, ACT>(a, tiles, s)))
+    return AMOE_ERR_BAD_ARG;
+}
+#endif
+#if AMOE_PP_PART_IS(1)
+int amoe_pp_rows(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s)
+{
+    return b_kc ? launch_pp_rows<true, EPI_STORE, 0>(a, tiles, s) : launch_pp_rows<false, EPI_STORE, 0>(a, tiles, s);
+}
+#endif
+#if AMOE_PP_PART_IS(2)
+int amoe_pp_gated_bwd(const GemmArgs& a, int act, int tiles, hipStream_t s)
+{
+    AMOE_DISPATCH_ACT(act, return (launch_pp_rows<true, EPI_GATED_BWD, ACT>(a, tiles, s)))
+    return AMOE_ERR_BAD_ARG;
+}
+#endif

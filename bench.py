@@ -304,14 +304,16 @@ def main():
     fused_bwd = dtype == torch.bfloat16 and c in (0, 1, 2)   # what the layer's backward does
     # the kernel symbol (template instance) each launch resolves to: what rocprofv3 reports
     tile = {1: "128, 128, 2, 2", 2: "256, 128, 2, 2", 3: "256, 256, 2, 2", 5: "256, 256, 4, 2"}.get(c, "256, 256, 2, 4")
+    rows = f"grouped_gemm_rows_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_rows_bf16_kernel<"
     gathered = token_of is not None
     sym = {
+        # grouped_gemm_pp_rows_bf16_kernel<B K-contiguous, epilogue, activation>; other tile shapes:
         # grouped_gemm_rows_bf16_kernel<BM, BN, waves along M, waves along N, B K-contiguous, epilogue, activation>
-        "gemm_gateup_act_fwd": f"grouped_gemm_rows_bf16_kernel<{tile}, false, 1, 0>",
-        "gemm_down_fwd": f"grouped_gemm_rows_bf16_kernel<{tile}, false, 0, 0>",
-        "gemm_dgrad_down": f"grouped_gemm_rows_bf16_kernel<{tile}, true, 0, 0>",
-        "gemm_dgrad_down_gated_bwd": f"grouped_gemm_rows_bf16_kernel<{tile}, true, 2, 0>",
-        "gemm_dgrad_gateup": f"grouped_gemm_rows_bf16_kernel<{tile}, true, 0, 0>",
+        "gemm_gateup_act_fwd": f"{rows}false, 1, 0>",
+        "gemm_down_fwd": f"{rows}false, 0, 0>",
+        "gemm_dgrad_down": f"{rows}true, 0, 0>",
+        "gemm_dgrad_down_gated_bwd": f"{rows}true, 2, 0>",
+        "gemm_dgrad_gateup": f"{rows}true, 0, 0>",
         # grouped_gemm_wgrad_bf16_kernel<BM, BN, waves along M, waves along N, gathered operand>
         "gemm_wgrad_down": f"grouped_gemm_wgrad_bf16_kernel<{tile}, {2 if gathered else 0}>",
         "gemm_wgrad_gateup": f"grouped_gemm_wgrad_bf16_kernel<{tile}, {1 if gathered else 0}>",
