@@ -21,8 +21,8 @@ LIB_PATH = os.path.join(LIB_DIR, "libarctic_moe_hip.so")
 # (source, object name, extra flags); the 16-bit grouped GEMM is compiled as four groups of entry points in parallel
 GEMM_PARTS = 4
 SOURCES = [(f, os.path.splitext(f)[0], []) for f in ("api.hip", "router.hip", "permute.hip", "rows.hip", "gemm_f32.hip", "remap.hip")]
-# the default tile shape of the same products: one group per epilogue
-PP_PARTS = 3
+# the default tile shape of the same products: one group per epilogue, and the weight gradients
+PP_PARTS = 4
 SOURCES = [("gemm_pp.hip", f"gemm_pp_p{i}", [f"-DAMOE_PP_PART={i}"]) for i in range(PP_PARTS)] + SOURCES
 SOURCES = [("gemm_bf16.hip", f"gemm_bf16_p{i}", [f"-DAMOE_GEMM_PART={i}"]) for i in range(GEMM_PARTS)] + SOURCES
 

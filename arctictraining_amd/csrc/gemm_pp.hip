@@ -705,6 +705,357 @@ __device__ __forceinline__ void pp_rows_body()
     pp_vmwait<0>();   // (loads past the last tile wrote zeros into LDS: landed before the workgroup leaves)
 }
 
+// ------------------------------------------------------------------ weight gradients
+// C[e] = A[rows_e,:]^T @ B[rows_e,:]: the reduction runs over the expert's rows, both operands are K-strided.  The same
+// phases and the same persistent stream of K tiles as the row-grouped kernel; a tile is 256 x 256 of one expert's
+// gradient, its number of K tiles that of the expert's rows (three at least, the missing ones empty).
+// MAPS: 1 = the rows of A, 2 = the rows of B are gathered through a row map: the indices of a K tile are fetched by
+// scalar loads a phase before its offsets are worked out beside the MFMAs.
+// Rows past the expert's end read as zeros: an operand that is not gathered has a descriptor that ends with them, a
+// gathered one gets PP_NOWHERE for them.
+template <int MAPS, typename ET>
+__device__ __forceinline__ void pp_wgrad_body()
+{
+    typedef typename Elem16<ET>::frag_t frag_t;
+    extern __shared__ u32x4_t smem[];
+    const uint32_t lds = (uint32_t)(uintptr_t)(lptr_t)smem;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = wave >> 2, wc = wave & 3;
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I4 = std::integral_constant<int, 4>;
+    constexpr bool A_MAP = MAPS == 1, B_MAP = MAPS == 2;
+
+    // ------------------------------------------------------------ this workgroup's tiles
+    // Tiles are numbered expert by expert, inside an expert in strips of gn columns; XCD x (workgroups with
+    // blockIdx % 8 == x) works through chunks x, x + 8, ... of 32 consecutive tiles, so that the workgroups of an XCD
+    // share operand panels in its L2; the tiles left over from the last whole group of chunks are dealt one by one.
+    auto divide = [](int n, uint32_t inv) -> int { return inv ? (int)(((uint64_t)(uint32_t)n * inv) >> 32) : n; };
+    struct Tile { int e, m0, n0, r0, r1; };
+    auto decode = [&](int q, Tile& t) -> bool {       // q-th tile of this XCD
+        args_t& p = pp_args();
+        const int xcd = blockIdx.x & 7;
+        const int per = p.n_mt * p.n_ntiles, total = p.E * per;
+        const int whole = total & ~255;
+        int v = ((q >> 5) << 8) + (xcd << 5) + (q & 31);
+        if (v >= whole) v = whole + ((q - (whole >> 3)) << 3) + xcd;
+        if (v >= total) return false;
+        t.e = divide(v, p.inv_super);
+        const int i = v - t.e * per;
+        const int strip = divide(i, p.inv_sn);
+        const int r = i - strip * p.n_mt * p.gn;
+        const bool last = strip == p.sn - 1;
+        const int mt = divide(r, last ? p.inv_gm : p.inv_gn);
+        const int w = last ? p.n_ntiles - strip * p.gn : p.gn;
+        t.m0 = mt * PP_BM;
+        t.n0 = (strip * p.gn + r - mt * w) * PP_BN;
+        t.r0 = __builtin_amdgcn_readfirstlane(scalar_load_i32(p.offsets + t.e));
+        t.r1 = __builtin_amdgcn_readfirstlane(scalar_load_i32(p.offsets + t.e + 1));
+        return true;
+    };
+
+    // ------------------------------------------------------------ loads
+    // Thread tid fills k rows tid / 16 and tid / 16 + 32 of every half tile.
+    uint32_t aoff[2][2], boff[2][2];
+    uint32_t acol[2], bcol[2];        // byte offsets of its columns in the two halves (PP_NOWHERE outside the matrix)
+    srd_t ad, bd;
+    const uint32_t lda2 = (uint32_t)pp_args().lda * 2u, ldb2 = (uint32_t)pp_args().ldb * 2u;
+    int left = 0;                     // rows of the expert from the K tile loaded next
+    int row_n = 0, left_n = 0;        // gathered: map position of the K tile whose indices are fetched next
+    int idx[2][4];
+    auto add_sat = [](uint32_t a, uint32_t b) { return __builtin_elementwise_add_sat(a, b); };
+    auto fetch_idx = [&]() {
+        if constexpr (MAPS != 0) {
+            args_t& p = pp_args();
+            const int32_t* map = A_MAP ? p.a_row_map : p.b_row_map;
+            typedef int i32x4_t __attribute__((ext_vector_type(4), aligned(4)));
+            const int row = row_n + wave * 4;
+            if (row_n + 64 <= p.rows_total) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const i32x4_t v = *(const __attribute__((address_space(4))) i32x4_t*)(map + row + 32 * j);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) idx[j][q] = v[q];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) idx[j][q] = scalar_load_i32(map + min(row + 32 * j + q, p.rows_total - 1));
+            }
+        }
+    };
+    // offsets of the gathered operand for the K tile whose indices were fetched, of which `rows` rows exist
+    auto gather_offsets = [&](int rows) {
+        if constexpr (MAPS != 0) {
+            const int th = pp_here(tid);
+            const int q = (th >> 4) & 3, kr = th >> 4;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int i01 = q & 1 ? idx[j][1] : idx[j][0], i23 = q & 1 ? idx[j][3] : idx[j][2];
+                const uint32_t o = kr + 32 * j < rows ? (uint32_t)(q & 2 ? i23 : i01) * (A_MAP ? lda2 : ldb2) : PP_NOWHERE;
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (A_MAP) aoff[h][j] = add_sat(o, acol[h]); else boff[h][j] = add_sat(o, bcol[h]);
+            }
+        }
+    };
+    auto limit = [&]() {              // descriptors of the operands that are not gathered end with the expert's rows
+        int some = max(left, 0);
+        asm("" : "+s"(some));         // (a clamp in one step would be a vector instruction)
+        const uint32_t rows = (uint32_t)min(some, PP_BK);
+        if (!A_MAP) ad[2] = rows * lda2;
+        if (!B_MAP) bd[2] = rows * ldb2;
+    };
+    auto plan = [&](const Tile& t) {
+        args_t& p = pp_args();
+        const int th = pp_here(tid);
+        const int kr = th >> 4;
+        const int col = ((th & 15) ^ (2 * ((kr & 3) | (((kr >> 3) & 1) << 2)))) * 8;
+        ad = pp_srd(A_MAP ? p.A : p.A + (long long)t.r0 * p.lda);
+        bd = pp_srd(B_MAP ? p.B : p.B + (long long)t.r0 * p.ldb);
+        left = t.r1 - t.r0;
+        limit();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int m = t.m0 + h * 128 + col, n = t.n0 + h * 128 + col;
+            acol[h] = m < p.M ? (uint32_t)m * 2u : PP_NOWHERE;
+            bcol[h] = n < p.N ? (uint32_t)n * 2u : PP_NOWHERE;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                if (!A_MAP) aoff[h][j] = add_sat((uint32_t)(kr + 32 * j) * lda2, acol[h]);
+                if (!B_MAP) boff[h][j] = add_sat((uint32_t)(kr + 32 * j) * ldb2, bcol[h]);
+            }
+        }
+        gather_offsets(left);
+    };
+    auto next_k = [&]() {             // on to the next K tile of the same tile
+        left -= PP_BK;
+        if (!A_MAP) pp_advance(ad, PP_BK * lda2);
+        if (!B_MAP) pp_advance(bd, PP_BK * ldb2);
+        limit();
+        gather_offsets(left);
+    };
+    uint32_t fill = lds + (uint32_t)wave * 1024u;
+    auto dma_a = [&](auto A_) {
+        constexpr int a = decltype(A_)::value;
+        pp_dma16<a * PP_HALF>(ad, aoff[a][0], fill);
+        pp_dma16<a * PP_HALF + 8192u>(ad, aoff[a][1], fill);
+    };
+    auto dma_b = [&](auto B_) {
+        constexpr int b = decltype(B_)::value;
+        pp_dma16<(2 + b) * PP_HALF>(bd, boff[b][0], fill);
+        pp_dma16<(2 + b) * PP_HALF + 8192u>(bd, boff[b][1], fill);
+    };
+
+    // ------------------------------------------------------------ fragments
+    frag_t fa[4][2], fb0[2][2], fb1[2][2];
+    uint32_t ra[4], rb[2];            // LDS read addresses per 16-column tile
+    {
+        const int l16 = lane & 15, lq = lane >> 4;
+        const int k = 8 * lq + (l16 >> 2), key = 2 * ((l16 >> 2) | ((lq & 1) << 2));
+        const uint32_t base = lds + (uint32_t)(k * 256 + (l16 & 1) * 8);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ra[i] = base + (uint32_t)((grp * 8 + 2 * i + ((l16 & 3) >> 1)) ^ key) * 16u;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) rb[j] = base + 2 * PP_HALF + (uint32_t)((wc * 4 + 2 * j + ((l16 & 3) >> 1)) ^ key) * 16u;
+    }
+    auto flip = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ra[i] ^= PP_STAGE;
+        rb[0] ^= PP_STAGE;
+        rb[1] ^= PP_STAGE;
+    };
+    auto read_tr = [&](uint32_t ad) -> frag_t {
+        typedef __attribute__((address_space(3))) i16x4_t* tr_ptr;
+        const u32x2_t lo = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)ad));
+        const u32x2_t hi = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)(ad + 1024u)));
+        return __builtin_bit_cast(frag_t, u32x4_t{lo[0], lo[1], hi[0], hi[1]});
+    };
+    auto read_a = [&](auto A_, auto N_) {
+#pragma unroll
+        for (int i = 0; i < decltype(N_)::value; ++i)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) fa[i][s] = read_tr(ra[i] + decltype(A_)::value * PP_HALF + s * 8192u);
+    };
+    auto read_b = [&](auto B_, frag_t (&fb)[2][2]) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) fb[j][s] = read_tr(rb[j] + decltype(B_)::value * PP_HALF + s * 8192u);
+    };
+    auto mma = [&](auto FIRST, auto N_, mfma_f32x4 (&c)[4][2], const frag_t (&fb)[2][2]) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int i = 0; i < decltype(N_)::value; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    c[i][j] = Mfma16<ET>::run(fb[j][s], fa[i][s], decltype(FIRST)::value && s == 0 ? mfma_f32x4{0.f, 0.f, 0.f, 0.f} : c[i][j]);
+    };
+
+    // ------------------------------------------------------------ tile state
+    Tile cur, nxt = {0, 0, 0, 0, 0}, far = {0, 0, 0, 0, 0};
+    int q = blockIdx.x >> 3;                       // position of the last tile taken in this XCD's queue
+    const int gq = gridDim.x >> 3;
+    if (!decode(q, cur)) return;
+    bool have_n = decode(q += gq, nxt), have_nn = false;
+
+    bf16_t* e_c;
+    int e_ldc2 = 0, e_cols = 0, e_rows = 0;
+    uint32_t e_off = 0;
+    auto prepare_epilogue = [&]() {
+        args_t& p = pp_args();
+        const int le = pp_here(lane);
+        e_ldc2 = p.ldc * 2;
+        e_c = p.C + (long long)cur.e * p.strideC + (long long)(cur.m0 + grp * 64) * p.ldc + cur.n0 + wc * 32;
+        e_cols = p.N - cur.n0 - wc * 32;
+        e_rows = p.M - cur.m0 - grp * 64;
+        e_off = (uint32_t)((le & 15) * e_ldc2 + 16 * (le >> 4));
+    };
+    auto epilogue = [&](auto A_, auto B_, const mfma_f32x4 (&acc)[4][2]) {
+        constexpr int a = decltype(A_)::value, b = decltype(B_)::value;
+        const int le = pp_here(lane);
+        const int eq = le >> 4, rl = le & 15;
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc(e_c, (short)0, (int)PP_DROP, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            pp_fence();
+            const bool ok = b * 128 + 8 * eq < e_cols && a * 128 + i * 16 + rl < e_rows;
+            uint32_t x[2], y[2];
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                x[v] = Elem16<ET>::pack2(acc[i][0][2 * v], acc[i][0][2 * v + 1]);
+                y[v] = Elem16<ET>::pack2(acc[i][1][2 * v], acc[i][1][2 * v + 1]);
+            }
+            pp_join(x[0], y[0]);
+            pp_join(x[1], y[1]);
+            pp_store16(d, u32x4_t{x[0], x[1], y[0], y[1]}, ok ? e_off : PP_DROP, (uint32_t)((a * 128 + i * 16) * e_ldc2 + b * 256));
+        }
+    };
+
+    auto run_tile = [&]() {
+        mfma_f32x4 acc[2][2][4][2];
+        const int KT = max(3, (cur.r1 - cur.r0 + PP_BK - 1) >> 6);
+        // ---- phase 0 of the first K tile
+        read_a(I0{}, I4{});
+        dma_a(I1{});
+        fill ^= PP_STAGE;
+        pp_vmwait<10>();
+        pp_barrier();
+        mma(T_{}, I4{}, acc[0][0], fb0);
+        next_k();
+        have_nn = have_n && decode(q += gq, far);
+        if (!have_nn) far = Tile{0, 0, 0, 0, 0};
+        pp_barrier();
+        auto k_tile = [&](auto FIRST, auto TURN, auto N_, bool turn_next) {
+            // phase 1
+            read_b(I1{}, fb1);
+            if (decltype(TURN)::value) plan(nxt);
+            dma_b(I0{});
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(FIRST, I4{}, acc[0][1], fb1);
+            pp_barrier();
+            // phase 2
+            read_a(I1{}, N_);
+            dma_a(I0{});
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(FIRST, N_, acc[1][0], fb0);
+            pp_barrier();
+            // phase 3
+            flip();
+            read_b(I0{}, fb0);
+            dma_b(I1{});
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(FIRST, N_, acc[1][1], fb1);
+            row_n = turn_next ? nxt.r0 : row_n + PP_BK;
+            fetch_idx();
+            pp_barrier();
+            // phase 0 of the next K tile
+            read_a(I0{}, I4{});
+            dma_a(I1{});
+            fill ^= PP_STAGE;
+            pp_vmwait<10>();
+            pp_barrier();
+            mma(F_{}, I4{}, acc[0][0], fb0);
+            if (decltype(TURN)::value) prepare_epilogue();
+            next_k();
+            pp_barrier();
+        };
+        // the lower half of the tile lies past the matrix (not told apart without a gathered operand: there the second
+        // copy of the loop spills)
+        const bool half = MAPS != 0 && cur.m0 + 128 >= pp_args().M;
+        k_tile(T_{}, F_{}, I4{}, KT == 3);
+        int t = 1;
+        int full = half ? 0 : KT - 2;
+        asm("" : "+s"(full));       // (left to see that one of the two loops is empty, the compiler branches between them)
+        for (; t < full; ++t) k_tile(F_{}, F_{}, I4{}, t == KT - 3);
+        if constexpr (MAPS != 0)
+            for (; t < KT - 2; ++t) k_tile(F_{}, F_{}, I0{}, t == KT - 3);
+        k_tile(F_{}, T_{}, I4{}, false);
+        // ---- last K tile: the epilogue of each finished quadrant in the memory part of the phase after it
+        read_b(I1{}, fb1);
+        dma_b(I0{});
+        epilogue(I0{}, I0{}, acc[0][0]);
+        pp_vmwait<10>();
+        pp_barrier();
+        mma(F_{}, I4{}, acc[0][1], fb1);
+        pp_barrier();
+        read_a(I1{}, I4{});
+        dma_a(I0{});
+        epilogue(I0{}, I1{}, acc[0][1]);
+        pp_vmwait<10>();
+        pp_barrier();
+        mma(F_{}, I4{}, acc[1][0], fb0);
+        pp_barrier();
+        flip();
+        read_b(I0{}, fb0);
+        dma_b(I1{});
+        epilogue(I1{}, I0{}, acc[1][0]);
+        pp_vmwait<10>();
+        pp_barrier();
+        mma(F_{}, I4{}, acc[1][1], fb1);
+        row_n += PP_BK;
+        fetch_idx();
+        pp_barrier();
+        epilogue(I1{}, I1{}, acc[1][1]);
+    };
+
+    // ------------------------------------------------------------ the workgroup's tiles
+    row_n = cur.r0;
+    fetch_idx();
+    plan(cur);
+    dma_b(I0{}); dma_a(I0{}); dma_b(I1{}); dma_a(I1{});
+    fill ^= PP_STAGE;
+    row_n += PP_BK;
+    fetch_idx();
+    next_k();
+    dma_b(I0{}); dma_a(I0{}); dma_b(I1{});
+    row_n += PP_BK;
+    fetch_idx();
+    pp_vmwait<12>();
+    pp_barrier();
+    if (grp == 1) pp_barrier();
+    read_b(I0{}, fb0);
+    pp_vmwait<10>();
+    pp_barrier();
+    pp_barrier();
+    for (;;) {
+        run_tile();
+        if (!have_n) break;
+        cur = nxt;
+        nxt = far;
+        have_n = have_nn;
+    }
+    if (grp == 0) pp_barrier();
+    pp_vmwait<0>();   // (loads past the last tile wrote zeros into LDS: landed before the workgroup leaves)
+}
+
 template <bool B_KC, int EPI, int ACT>
 __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_rows_bf16_kernel(GemmArgs)
 {
@@ -714,6 +1065,17 @@ template <bool B_KC, int EPI, int ACT>
 __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_rows_f16_kernel(GemmArgs)
 {
     pp_rows_body<B_KC, EPI, ACT, f16_t>();
+}
+
+template <int MAPS>
+__global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_wgrad_bf16_kernel(GemmArgs)
+{
+    pp_wgrad_body<MAPS, bf16_t>();
+}
+template <int MAPS>
+__global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_wgrad_f16_kernel(GemmArgs)
+{
+    pp_wgrad_body<MAPS, f16_t>();
 }
 
 }  // namespace
@@ -750,5 +1112,33 @@ int amoe_pp_gated_bwd(const GemmArgs& a, int act, int tiles, hipStream_t s)
 {
     AMOE_DISPATCH_ACT(act, return (launch_pp_rows<true, EPI_GATED_BWD, ACT>(a, tiles, s)))
     return AMOE_ERR_BAD_ARG;
+}
+#endif
+#if AMOE_PP_PART_IS(3)
+template <int MAPS>
+static int launch_pp_wgrad(const GemmArgs& a, int grid, hipStream_t s)
+{
+    if (a.f16) return launch_kernel<grouped_gemm_pp_wgrad_f16_kernel<MAPS>, PP_THREADS, 2 * PP_STAGE>(a, grid, s);
+    return launch_kernel<grouped_gemm_pp_wgrad_bf16_kernel<MAPS>, PP_THREADS, 2 * PP_STAGE>(a, grid, s);
+}
+
+int amoe_pp_wgrad(GemmArgs a, hipStream_t s)
+{
+    const int cus = device_cu_count();
+    AMOE_REQUIRE(cus > 0, AMOE_ERR_LAUNCH, "grouped_gemm: cannot read the number of compute units");
+    const int strips = (a.n_ntiles + 7) / 8;
+    a.gn = (a.n_ntiles + strips - 1) / strips;
+    a.sn = (a.n_ntiles + a.gn - 1) / a.gn;
+    auto inverse = [](int d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; };
+    const long long per = (long long)a.n_mt * a.n_ntiles, total = per * a.E;
+    AMOE_REQUIRE(total * per < (1ll << 32), AMOE_ERR_UNSUPPORTED, "grouped_gemm_wgrad: too many tiles");
+    a.inv_super = inverse((int)per);
+    a.inv_sn = inverse(a.n_mt * a.gn);
+    a.inv_gn = inverse(a.gn);
+    a.inv_gm = inverse(a.n_ntiles - (a.sn - 1) * a.gn);
+    const int grid = (int)(((total < cus ? total : cus) + 7) & ~7);
+    if (a.a_row_map) return launch_pp_wgrad<1>(a, grid, s);
+    if (a.b_row_map) return launch_pp_wgrad<2>(a, grid, s);
+    return launch_pp_wgrad<0>(a, grid, s);
 }
 #endif

@@ -305,6 +305,7 @@ def main():
     # the kernel symbol (template instance) each launch resolves to: what rocprofv3 reports
     tile = {1: "128, 128, 2, 2", 2: "256, 128, 2, 2", 3: "256, 256, 2, 2", 5: "256, 256, 4, 2"}.get(c, "256, 256, 2, 4")
     rows = f"grouped_gemm_rows_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_rows_bf16_kernel<"
+    wgrad = f"grouped_gemm_wgrad_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_wgrad_bf16_kernel<"
     gathered = token_of is not None
     sym = {
         # grouped_gemm_pp_rows_bf16_kernel<B K-contiguous, epilogue, activation>; other tile shapes:
@@ -314,9 +315,10 @@ def main():
         "gemm_dgrad_down": f"{rows}true, 0, 0>",
         "gemm_dgrad_down_gated_bwd": f"{rows}true, 2, 0>",
         "gemm_dgrad_gateup": f"{rows}true, 0, 0>",
+        # grouped_gemm_pp_wgrad_bf16_kernel<gathered operand>; other tile shapes, and fewer than 256 rows per expert:
         # grouped_gemm_wgrad_bf16_kernel<BM, BN, waves along M, waves along N, gathered operand>
-        "gemm_wgrad_down": f"grouped_gemm_wgrad_bf16_kernel<{tile}, {2 if gathered else 0}>",
-        "gemm_wgrad_gateup": f"grouped_gemm_wgrad_bf16_kernel<{tile}, {1 if gathered else 0}>",
+        "gemm_wgrad_down": f"{wgrad}{2 if gathered else 0}>",
+        "gemm_wgrad_gateup": f"{wgrad}{1 if gathered else 0}>",
     }
     if dtype != torch.bfloat16:
         sym = {k: "grouped_gemm_f32_kernel" for k in sym}

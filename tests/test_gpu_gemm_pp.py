@@ -77,3 +77,35 @@ def test_many_tiles_per_workgroup(ops, gpu_device, E, Kd, N):
     for _ in range(3):
         _check(ops.grouped_gemm_nn(src, w, offs, a_row_map=rows), ref, 1e-2)
         _check(ops.grouped_gemm_nt(src, w.transpose(1, 2).contiguous(), offs, a_row_map=rows), ref, 1e-2)
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 1e-2), (torch.float16, 2e-3)])
+@pytest.mark.parametrize("M,N,counts", [
+    (256, 256, [0, 1, 700, 513, 0, 400]),            # empty and one-row experts, remainders of a K tile
+    (136, 1032, [1100, 64, 65, 0, 200, 900]),        # edges in both extents
+    (1408, 520, [257] * 9 + [0, 600]),               # a last row tile of half height; several tiles per workgroup
+])
+def test_weight_gradient(ops, gpu_device, dtype, tol, M, N, counts):
+    print("pp wgrad", dtype, M, N, flush=True)
+    g = torch.Generator(device=gpu_device).manual_seed(M + N)
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(gpu_device)
+    R, E = sum(counts), len(counts)
+    assert R >= 256 * E   # (below that the default is another tile shape)
+    T = R // 3
+    rows = torch.randint(0, T, (R,), device=gpu_device, generator=g, dtype=torch.int32)
+    rnd = lambda *s: torch.randn(*s, device=gpu_device, generator=g).to(dtype)
+    A, B, As, Bs = rnd(R, M), rnd(R, N), rnd(T, M), rnd(T, N)
+
+    def ref(a, b):
+        return torch.stack([p.float().t() @ q.float() for p, q in zip(a.split(counts), b.split(counts))])
+
+    for got, want in (
+        (ops.grouped_gemm_wgrad(A, B, offs, E), ref(A, B)),
+        (ops.grouped_gemm_wgrad(As, B, offs, E, a_row_map=rows), ref(As[rows.long()], B)),
+        (ops.grouped_gemm_wgrad(A, Bs, offs, E, b_row_map=rows), ref(A, Bs[rows.long()])),
+    ):
+        for e in range(E):
+            if counts[e]:
+                _check(got[e], want[e], tol)
+            else:
+                assert bool((got[e] == 0).all())
