@@ -3,6 +3,7 @@ pointers and the current HIP stream, raise on error.  One function per stage of 
 expert layer, in the order the reference's forward runs them
 (arctic_training/model/moe/moe.py:219-323).
 """
+import ctypes
 from typing import Optional, Tuple
 
 import torch
@@ -406,7 +407,7 @@ def _expert_view(t: torch.Tensor, name: str):
     return t.shape[0], t.shape[1], t.shape[2], (t.stride(0) if t.shape[0] > 1 else t.shape[1] * t.shape[2])
 
 
-def remap_pack(in0: torch.Tensor, in1: Optional[torch.Tensor] = None) -> torch.Tensor:
+def remap_pack(in0: torch.Tensor, in1: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[e][h][G*i+g] = in_g[e][i][h]: gate/up nn.Linear weights [E,I,H] -> interleaved
     expert_gate_up [E,H,2I] (in1 given), or a batched transpose [E,I,H] -> [E,H,I] (in1 None)."""
     lib = _lib.load()
@@ -414,7 +415,11 @@ def remap_pack(in0: torch.Tensor, in1: Optional[torch.Tensor] = None) -> torch.T
     if in1 is not None:
         if _expert_view(in1, "in1") != (E, I, H, es) or in1.dtype != in0.dtype:
             raise RuntimeError("in1 must match in0 in shape, strides and dtype")
-    out = torch.empty((E, H, (2 if in1 is not None else 1) * I), dtype=in0.dtype, device=in0.device)
+    shape = (E, H, (2 if in1 is not None else 1) * I)
+    if out is None:
+        out = torch.empty(shape, dtype=in0.dtype, device=in0.device)
+    elif _chk(out, "out").shape != shape or out.dtype != in0.dtype:
+        raise RuntimeError("out must be [E, H, G*I] of the inputs' dtype")
     rc = lib.amoe_remap_pack(in0.data_ptr(), _ptr(in1), out.data_ptr(), _dtype_code(in0), E, I, H, es, _stream())
     _lib.check(rc, "amoe_remap_pack")
     return out
@@ -442,3 +447,36 @@ def remap_unpack(joint: torch.Tensor, two: bool, out0: Optional[torch.Tensor] = 
                                shape[3], _stream())
     _lib.check(rc, "amoe_remap_unpack")
     return (out0, out1) if two else out0
+
+
+def _pointers(ptrs):
+    return None if ptrs is None else (ctypes.c_void_p * len(ptrs))(*ptrs)
+
+
+def remap_pack_list(in0, in1, out: torch.Tensor, first: int = 0) -> None:
+    """remap_pack from experts that are separate matrices: `in0` / `in1` list the device addresses of dense, 16-byte
+    aligned [I, H] matrices of out's dtype (in1 None: one matrix an expert); they fill out[first : first + len(in0)]."""
+    lib = _lib.load()
+    _chk(out, "out")
+    n, (E, H, GI) = len(in0), out.shape
+    if first < 0 or first + n > E or (in1 is not None and (len(in1) != n or GI % 2)):
+        raise RuntimeError("the lists must name one matrix (of each kind) per expert of out")
+    rc = lib.amoe_remap_pack_list(
+        _pointers(in0), _pointers(in1), out.data_ptr() + first * H * GI * out.element_size(), _dtype_code(out), n,
+        GI if in1 is None else GI // 2, H, _stream(),
+    )
+    _lib.check(rc, "amoe_remap_pack_list")
+
+
+def remap_unpack_list(joint: torch.Tensor, out0, out1, first: int = 0) -> None:
+    """The inverse of remap_pack_list: joint[first : first + len(out0)] into the matrices at `out0` / `out1`."""
+    lib = _lib.load()
+    _chk(joint, "joint")
+    n, (E, H, GI) = len(out0), joint.shape
+    if first < 0 or first + n > E or (out1 is not None and (len(out1) != n or GI % 2)):
+        raise RuntimeError("the lists must name one matrix (of each kind) per expert of joint")
+    rc = lib.amoe_remap_unpack_list(
+        joint.data_ptr() + first * H * GI * joint.element_size(), _pointers(out0), _pointers(out1), _dtype_code(joint), n,
+        GI if out1 is None else GI // 2, H, _stream(),
+    )
+    _lib.check(rc, "amoe_remap_unpack_list")

@@ -8,7 +8,8 @@ can be restored for saving a checkpoint in the original format.
 
 The weight re-layout itself -- transposing each expert's nn.Linear weights and interleaving
 gate / up on the last dimension -- runs in the HIP kernels of csrc/remap.hip through the C ABI
-(`amoe_remap_pack`, `amoe_remap_unpack`); there is no torch or CPU fallback for it.
+(`amoe_remap_pack*`, `amoe_remap_unpack*`), straight from and to the experts' own weights where these
+are dense, aligned and of the parameters' dtype and device; there is no torch or CPU fallback for it.
 
 Three storage formats of the original experts are understood:
   * a ModuleList of per-expert MLPs with `gate_proj`, `up_proj`, `down_proj` nn.Linear modules
@@ -105,9 +106,105 @@ def _experts_is_a_list(experts) -> bool:
     return isinstance(experts, torch.nn.ModuleList)
 
 
-def _stacked_linear_weights(experts, name: str, device) -> torch.Tensor:
-    """[E, out, in] stack of the nn.Linear weights `name` of a ModuleList of experts."""
-    return torch.stack([getattr(ex, name).weight.detach().to(device) for ex in experts]).contiguous()
+# experts per kernel launch when they are separate modules: walking their weights costs the host about as long as the
+# kernels take, so the first launch goes out after a few of them (a quarter of the 128-expert layer)
+_EXPERTS_PER_LAUNCH = 32
+_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def _linear_weight(expert, name: str):
+    """expert.<name>.weight; a plain module's own tables answer at a fifth of the cost of two __getattr__ calls."""
+    sub = expert._modules.get(name)
+    w = sub._parameters.get("weight") if sub is not None else None
+    return w if w is not None else getattr(expert, name).weight
+
+
+def _in_place(w, shape, dtype, index) -> bool:
+    """Whether a kernel on cuda:`index` can read or write the matrix w where it is."""
+    return (
+        type(w) in _PLAIN_TENSORS and w.dtype is dtype and w.get_device() == index and w.is_contiguous()
+        and w.shape == shape and w.data_ptr() % 16 == 0
+    )
+
+
+def _kernel_side(param, device):
+    """param itself if the kernels can work on it, else None: a dense tensor of a dtype they know, on `device`."""
+    ok = param.is_cuda and param.device == device and param.is_contiguous() and param.dtype in ops._DTYPE_CODES
+    return param if ok and param.data_ptr() % 16 == 0 else None
+
+
+def _indexed(device) -> torch.device:
+    device = torch.device(device)
+    return torch.device("cuda", torch.cuda.current_device()) if device.type == "cuda" and device.index is None else device
+
+
+def _pack_into(param, sources, device) -> None:
+    """param <- pack(sources): one or two [E, I, H] tensors."""
+    device = _indexed(device)
+    direct = _kernel_side(param, device)
+    if direct is None or direct.dtype != sources[0].dtype:
+        param.copy_(ops.remap_pack(*sources))
+        return
+    ops.remap_pack(sources[0], sources[1] if len(sources) > 1 else None, out=param.detach())
+    torch.autograd.graph.increment_version(param)
+
+
+def _pack_experts_into(param, experts, names, device) -> None:
+    """param [E, H, G*I] <- pack of the weights `names` (G of them, [I, H] each) of a ModuleList of experts."""
+    (E, H, GI), experts = param.shape, list(experts)
+    shape = torch.Size((GI // len(names), H))
+    if len(experts) != E:
+        raise RuntimeError(f"{len(experts)} experts cannot fill parameters of {E}")
+    device = _indexed(device)
+    out = _kernel_side(param, device)
+    if out is None:  # packed beside it, in the weights' own dtype
+        out = torch.empty(param.shape, dtype=_linear_weight(experts[0], names[0]).dtype, device=device)
+    dense, dtype, index = out.detach(), out.dtype, device.index
+    for first in range(0, E, _EXPERTS_PER_LAUNCH):
+        lists, held = [], []
+        for name in names:
+            ptrs = []
+            for ex in experts[first : first + _EXPERTS_PER_LAUNCH]:
+                w = _linear_weight(ex, name)
+                if not _in_place(w, shape, dtype, index):
+                    w = w.detach().to(device).to(dtype).contiguous()
+                    if w.shape != shape:
+                        raise RuntimeError(f"{name} of shape {tuple(w.shape)}: expected {tuple(shape)}")
+                    w = w if w.data_ptr() % 16 == 0 else w.clone()
+                    held.append(w)
+                ptrs.append(w.data_ptr())
+            lists.append(ptrs)
+        ops.remap_pack_list(lists[0], lists[1] if len(lists) > 1 else None, dense, first)
+    if out is param:
+        torch.autograd.graph.increment_version(param)
+    else:
+        param.copy_(out)
+
+
+def _unpack_into_experts(experts, names, joint) -> None:
+    """The inverse: the weights `names` of every expert <- unpack(joint [E, H, G*I]), each where it lies if it can be."""
+    (E, H, GI), experts = joint.shape, list(experts)
+    shape = torch.Size((GI // len(names), H))
+    if len(experts) > E:
+        raise RuntimeError(f"parameters of {E} experts cannot fill {len(experts)}")
+    dtype, index = joint.dtype, joint.get_device()
+    for first in range(0, len(experts), _EXPERTS_PER_LAUNCH):
+        lists, copies, written = [], [], []
+        for name in names:
+            ptrs = []
+            for ex in experts[first : first + _EXPERTS_PER_LAUNCH]:
+                w = _linear_weight(ex, name)
+                if _in_place(w, shape, dtype, index):
+                    written.append(w)
+                    ptrs.append(w.data_ptr())
+                else:
+                    copies.append((w, torch.empty(shape, dtype=dtype, device=joint.device)))
+                    ptrs.append(copies[-1][1].data_ptr())
+            lists.append(ptrs)
+        ops.remap_unpack_list(joint, lists[0], lists[1] if len(lists) > 1 else None, first)
+        torch.autograd.graph.increment_version(written)
+        for w, x in copies:
+            w.copy_(x)
 
 
 @torch.no_grad()
@@ -116,9 +213,8 @@ def fill_arctic_moe_from_orig_mlp(arctic_moe: ArcticMoE, orig_mlp, device) -> No
     experts = orig_mlp.experts
     arctic_moe.router_gate.copy_(orig_mlp.gate.weight.detach().to(device))
     if _experts_is_a_list(experts):
-        gate = _stacked_linear_weights(experts, "gate_proj", device)  # [E, I, H]
-        up = _stacked_linear_weights(experts, "up_proj", device)
-        down = _stacked_linear_weights(experts, "down_proj", device)  # [E, H, I]
+        _pack_experts_into(arctic_moe.expert_gate_up, experts, ("gate_proj", "up_proj"), device)
+        _pack_experts_into(arctic_moe.expert_down, experts, ("down_proj",), device)
     else:
         fused = experts.gate_up_proj.detach().to(device)
         down = experts.down_proj.detach().to(device).contiguous()
@@ -126,10 +222,10 @@ def fill_arctic_moe_from_orig_mlp(arctic_moe: ArcticMoE, orig_mlp, device) -> No
         if getattr(arctic_moe._config, "fused_gate_up_interleaved", False):
             # gpt-oss: gate / up already interleaved; at most a batched transpose is needed
             if _interleaved_is_transposed(arctic_moe._config, fused.shape, H, I2):
-                arctic_moe.expert_gate_up.copy_(ops.remap_pack(fused.contiguous()))
+                _pack_into(arctic_moe.expert_gate_up, (fused.contiguous(),), device)
             else:
                 arctic_moe.expert_gate_up.copy_(fused)
-            arctic_moe.expert_down.copy_(ops.remap_pack(down))
+            _pack_into(arctic_moe.expert_down, (down,), device)
             return
         if tuple(fused.shape[-2:]) != (I2, H):
             raise ValueError(
@@ -137,9 +233,8 @@ def fill_arctic_moe_from_orig_mlp(arctic_moe: ArcticMoE, orig_mlp, device) -> No
                 "a tensor that interleaves gate and up (gpt-oss) needs fused_gate_up_interleaved=True in the config"
             )
         inter = fused.shape[1] // 2
-        gate, up = fused[:, :inter, :], fused[:, inter:, :]
-    arctic_moe.expert_gate_up.copy_(ops.remap_pack(gate, up))
-    arctic_moe.expert_down.copy_(ops.remap_pack(down))
+        _pack_into(arctic_moe.expert_gate_up, (fused[:, :inter, :], fused[:, inter:, :]), device)
+        _pack_into(arctic_moe.expert_down, (down,), device)
     if arctic_moe._config.use_shared_expert:
         sh = orig_mlp.shared_expert
         g = sh.gate_proj.weight.detach().to(device)[None].contiguous()
@@ -155,13 +250,10 @@ def fill_orig_mlp_from_arctic_moe(orig_mlp, arctic_moe: ArcticMoE) -> None:
     experts = orig_mlp.experts
     orig_mlp.gate.weight.copy_(arctic_moe.router_gate)
     gate_up = arctic_moe.expert_gate_up.detach().contiguous()
-    down = ops.remap_unpack(arctic_moe.expert_down.detach().contiguous(), two=False)  # [E, H, I]
+    down_joint = arctic_moe.expert_down.detach().contiguous()
     if _experts_is_a_list(experts):
-        gate, up = ops.remap_unpack(gate_up, two=True)
-        for i, ex in enumerate(experts):
-            ex.gate_proj.weight.copy_(gate[i])
-            ex.up_proj.weight.copy_(up[i])
-            ex.down_proj.weight.copy_(down[i])
+        _unpack_into_experts(experts, ("gate_proj", "up_proj"), gate_up)
+        _unpack_into_experts(experts, ("down_proj",), down_joint)
     elif getattr(arctic_moe._config, "fused_gate_up_interleaved", False):
         fused = experts.gate_up_proj
         H, I2 = arctic_moe.model_dim, 2 * arctic_moe.intermediate_dim
@@ -169,7 +261,7 @@ def fill_orig_mlp_from_arctic_moe(orig_mlp, arctic_moe: ArcticMoE) -> None:
             fused.copy_(ops.remap_unpack(gate_up, two=False))
         else:
             fused.copy_(gate_up)
-        experts.down_proj.copy_(down)
+        experts.down_proj.copy_(ops.remap_unpack(down_joint, two=False))
     else:
         fused = experts.gate_up_proj
         inter = fused.shape[1] // 2
@@ -178,7 +270,7 @@ def fill_orig_mlp_from_arctic_moe(orig_mlp, arctic_moe: ArcticMoE) -> None:
         else:
             gate, up = ops.remap_unpack(gate_up, two=True)
             fused.copy_(torch.cat((gate, up), dim=1))
-        experts.down_proj.copy_(down)
+        experts.down_proj.copy_(ops.remap_unpack(down_joint, two=False))
     if arctic_moe._config.use_shared_expert:
         sh = orig_mlp.shared_expert
         g, u = ops.remap_unpack(arctic_moe.shared_expert_gate_up.detach()[None].contiguous(), two=True)

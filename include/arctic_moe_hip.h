@@ -278,6 +278,16 @@ int amoe_remap_pack(const void* in0, const void* in1, void* out, int dtype, int 
 int amoe_remap_unpack(const void* in, void* out0, void* out1, int dtype, int E, int I, int H,
                       long long out_expert_stride, void* stream);
 
+/*
+ * The two re-layouts with the per-expert side as E separate dense [I, H] matrices: in0 / in1 (out0 / out1) are
+ * host arrays of E device pointers, 16-byte aligned, in1 (out1) null for one matrix per expert.  A ModuleList of
+ * experts is packed from (unpacked into) its own weights, with no stacked copy.
+ */
+int amoe_remap_pack_list(const void* const* in0, const void* const* in1, void* out, int dtype, int E, int I, int H,
+                         void* stream);
+int amoe_remap_unpack_list(const void* in, void* const* out0, void* const* out1, int dtype, int E, int I, int H,
+                           void* stream);
+
 #ifdef __cplusplus
 }
 #endif

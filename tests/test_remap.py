@@ -142,6 +142,54 @@ def test_hip_remap_headline_shape_round_trip(ops, gpu_device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,E,I,H", [(torch.bfloat16, 1, 8, 72), (torch.float16, 33, 24, 64), (torch.float32, 131, 4, 68)])
+def test_hip_remap_of_separate_experts(ops, gpu_device, dtype, E, I, H):
+    """Lists of matrices (one launch each, and more experts than one launch takes), and the same through a ModuleList
+    some of whose weights the kernels cannot use where they lie."""
+    from arctictraining_amd import remap as R
+
+    print("remap list", dtype, E, I, H, flush=True)
+    g = torch.Generator().manual_seed(E + I + H)
+    gate, up = torch.randn(E, I, H, generator=g).to(dtype), torch.randn(E, I, H, generator=g).to(dtype)
+    gu = torch.from_numpy(RO.pack_gate_up(gate.float().numpy(), up.float().numpy())).to(dtype)
+    on = [[w.to(gpu_device).clone() for w in m] for m in (gate, up)]
+    ptrs = [[w.data_ptr() for w in m] for m in on]
+    out = torch.zeros(E, H, 2 * I, dtype=dtype, device=gpu_device)
+    ops.remap_pack_list(*ptrs, out)
+    assert torch.equal(out.cpu(), gu)
+    back = [[torch.zeros_like(w) for w in m] for m in on]
+    ops.remap_unpack_list(out, *[[w.data_ptr() for w in m] for m in back])
+    assert all(torch.equal(a, b) for x, y in zip(on, back) for a, b in zip(x, y))
+
+    def module(w, e):
+        if e % 5 == 1:    # not contiguous
+            w = w.t().contiguous().t()
+        elif e % 5 == 2:  # not 16-byte aligned
+            w = torch.cat((w.new_zeros(1), w.flatten()))[1:].view(w.shape)
+        elif e % 5 == 3:  # elsewhere, in another type that holds the same values
+            w = w.cpu().double()
+        m = torch.nn.Module()
+        m.weight = torch.nn.Parameter(w, requires_grad=False)
+        return m
+
+    def expert(e):
+        m = torch.nn.Module()
+        m.gate_proj, m.up_proj = module(on[0][e], e), module(on[1][e], e)
+        return m
+
+    experts = torch.nn.ModuleList(expert(e) for e in range(E))
+    param = torch.nn.Parameter(torch.zeros_like(out), requires_grad=False)
+    before = param._version
+    R._pack_experts_into(param, experts, ("gate_proj", "up_proj"), gpu_device)
+    assert torch.equal(param.cpu(), gu) and param._version > before
+    want = [(m.gate_proj.weight.clone(), m.up_proj.weight.clone()) for m in experts]
+    for m in experts:
+        m.gate_proj.weight.zero_(), m.up_proj.weight.zero_()
+    R._unpack_into_experts(experts, ("gate_proj", "up_proj"), param.detach())
+    assert all(torch.equal(m.gate_proj.weight, a) and torch.equal(m.up_proj.weight, b) for m, (a, b) in zip(experts, want))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("as_list", [False, True])
 def test_install_and_restore_hooks(gpu_device, as_list):
     """A one-layer stand-in for a HF MoE model: install ArcticMoE from its block, compare the
