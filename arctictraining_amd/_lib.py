@@ -83,6 +83,32 @@ SIGNATURES = {
         _c_int,
         [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, ctypes.c_longlong, _c_void_p],
     ),
+    "amoe_layer_sizes": (_c_int, [_c_void_p, _c_int, _c_int, _c_void_p]),
+    "amoe_layer_fwd": (
+        _c_int,
+        [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+         _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_void_p],
+    ),
+    "amoe_layer_bwd": (
+        _c_int,
+        [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_void_p,
+         _c_void_p, _c_void_p, _c_void_p, _c_void_p],
+    ),
+    "amoe_layer_bwd_shared": (
+        _c_int,
+        [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+         _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p],
+    ),
+    "amoe_layer_bwd_input": (
+        _c_int,
+        [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+         _c_void_p, _c_void_p, _c_void_p, _c_void_p],
+    ),
+    "amoe_dense_wgrad": (
+        _c_int,
+        [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
+         _c_void_p],
+    ),
     "amoe_remap_pack_list": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p]),
     "amoe_remap_unpack_list": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p]),
     "amoe_gated_act_bwd": (

@@ -23,16 +23,19 @@ gather_rows_kernel(const T* __restrict__ x, const int32_t* __restrict__ token_of
 }
 
 // dst[t,:] = (addend ? addend[t,:] : 0) + sum_k w[t,k] * src[row_of[t,k],:]   (w == null -> 1)
-template <typename T, int KMAX>
+// SHARED adds what a shared expert gives the gradient of the input: second[t,:] + coef[t] * vec[:]
+template <typename T, int KMAX, bool SHARED>
 __global__ void __launch_bounds__(kBlock)
 gather_reduce_kernel(const T* __restrict__ src, const int32_t* __restrict__ row_of, const float* __restrict__ w,
-                     const T* __restrict__ addend, T* __restrict__ dst, int n_tokens, int K, int H)
+                     const T* __restrict__ addend, T* __restrict__ dst, int n_tokens, int K, int H,
+                     const T* __restrict__ second, const T* __restrict__ coef, const T* __restrict__ vec)
 {
     constexpr int V = ElemTraits<T>::kVec;
     const int nvec = H / V;
     for (int t = blockIdx.x; t < n_tokens; t += gridDim.x) {
         int rows[KMAX];
         float wk[KMAX];
+        const float c = SHARED ? ElemTraits<T>::load1(coef + t) : 0.f;
 #pragma unroll
         for (int k = 0; k < KMAX; ++k) {
             bool ok = k < K;
@@ -47,6 +50,13 @@ gather_reduce_kernel(const T* __restrict__ src, const int32_t* __restrict__ row_
             } else {
 #pragma unroll
                 for (int j = 0; j < V; ++j) acc[j] = 0.f;
+            }
+            if (SHARED) {
+                float a[V], b[V];
+                ElemTraits<T>::unpack(reinterpret_cast<const u32x4_t*>(second + (size_t)t * H)[i], a);
+                ElemTraits<T>::unpack(reinterpret_cast<const u32x4_t*>(vec)[i], b);
+#pragma unroll
+                for (int j = 0; j < V; ++j) acc[j] += a[j] + c * b[j];
             }
 #pragma unroll
             for (int k = 0; k < KMAX; ++k) {
@@ -172,7 +182,7 @@ gated_act_bwd_kernel(const T* __restrict__ gu, const T* __restrict__ d_inter, co
         if (d_scale_tk) {
             dot = wave_sum(dot);
             if (lane == 0) {
-                const int f = slot_of[r];
+                const int f = slot_of ? slot_of[r] : r;   // (null: one slot per row, in row order)
                 const int k = f / n_tokens;
                 d_scale_tk[(size_t)(f - k * n_tokens) * K + k] = dot;
             }
@@ -180,17 +190,70 @@ gated_act_bwd_kernel(const T* __restrict__ gu, const T* __restrict__ d_inter, co
     }
 }
 
-// d_scores[t,k] = sum_p partials[p][row_of[t,k]]  (fixed order over p)
+// d_scores[t,k] = sum_p partials[p][row_of[t,k]] (+ extra[row_of[t,k]])  (fixed order over p), added to what d_scores
+// holds if `accumulate`
 __global__ void __launch_bounds__(kBlock)
-score_grad_gather_kernel(const float* __restrict__ partials, int n_parts, long long part_stride,
-                         const int32_t* __restrict__ row_of, float* __restrict__ d_scores, int n_slots)
+score_grad_gather_kernel(const float* __restrict__ partials, int n_parts, long long part_stride, const float* __restrict__ extra,
+                         const int32_t* __restrict__ row_of, float* __restrict__ d_scores, int n_slots, int accumulate)
 {
     const int s = blockIdx.x * kBlock + threadIdx.x;
     if (s >= n_slots) return;
     const int row = row_of[s];
-    float tot = 0.f;
+    float tot = accumulate ? d_scores[s] : 0.f;
     for (int p = 0; p < n_parts; ++p) tot += partials[p * part_stride + row];
+    if (extra) tot += extra[row];
     d_scores[s] = tot;
+}
+
+// sig[t] = sigmoid(<x[t,:], w>), rounded to the element type after the product and after the sigmoid as the library's
+// two steps round (moe.py:311-312); one wavefront per token
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+shared_gate_kernel(const T* __restrict__ x, const T* __restrict__ w, float* __restrict__ sig, int n_tokens, int H)
+{
+    constexpr int V = ElemTraits<T>::kVec;
+    const int lane = threadIdx.x & 63;
+    const int t = blockIdx.x * (kBlock / AMOE_WAVE) + (threadIdx.x >> 6);
+    if (t >= n_tokens) return;
+    float dot = 0.f;
+    for (int i = lane; i < H / V; i += AMOE_WAVE) {
+        float a[V], b[V];
+        ElemTraits<T>::unpack(reinterpret_cast<const u32x4_t*>(x + (size_t)t * H)[i], a);
+        ElemTraits<T>::unpack(reinterpret_cast<const u32x4_t*>(w)[i], b);
+#pragma unroll
+        for (int j = 0; j < V; ++j) dot += a[j] * b[j];
+    }
+    dot = ElemTraits<T>::round(wave_sum(dot));
+    if (lane == 0) sig[t] = ElemTraits<T>::round(1.0f / (1.0f + expf(-dot)));
+}
+
+// d_pre[t] = d_sig[t] * sig[t] * (1 - sig[t])
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+shared_gate_bwd_kernel(const float* __restrict__ d_sig, const float* __restrict__ sig, T* __restrict__ d_pre, int n_tokens)
+{
+    const int t = blockIdx.x * kBlock + threadIdx.x;
+    if (t < n_tokens) ElemTraits<T>::store1(d_pre + t, d_sig[t] * sig[t] * (1.0f - sig[t]));
+}
+
+// out[i] = sum_p parts[p][i] in float32, one rounding
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+sum_parts_kernel(const T* __restrict__ parts, int n_parts, T* __restrict__ out, long long n_vec)
+{
+    constexpr int V = ElemTraits<T>::kVec;
+    const u32x4_t* src = reinterpret_cast<const u32x4_t*>(parts);
+    for (long long i = blockIdx.x * (long long)kBlock + threadIdx.x; i < n_vec; i += (long long)gridDim.x * kBlock) {
+        float acc[V] = {};
+#pragma unroll 4
+        for (int p = 0; p < n_parts; ++p) {
+            float f[V];
+            ElemTraits<T>::unpack(src[p * n_vec + i], f);
+#pragma unroll
+            for (int j = 0; j < V; ++j) acc[j] += f[j];
+        }
+        reinterpret_cast<u32x4_t*>(out)[i] = ElemTraits<T>::pack(acc);
+    }
 }
 
 int check_rows(const char* what, int dtype, int rows, int H)
@@ -218,23 +281,20 @@ AMOE_EXPORT int amoe_gather_rows_fwd(const void* x, const int32_t* token_of, voi
     return amoe_check_launch("gather_rows_fwd");
 }
 
-template <typename T>
+template <typename T, bool SHARED>
 static void launch_gather_reduce(const void* src, const int32_t* row_of, const float* w, const void* addend, void* dst,
-                                 int T_, int K, int H, hipStream_t s)
+                                 int T_, int K, int H, hipStream_t s, const void* second = nullptr, const void* coef = nullptr,
+                                 const void* vec = nullptr)
 {
     dim3 grid(row_grid(T_)), block(kBlock);
-    if (K <= 2)
-        hipLaunchKernelGGL((gather_reduce_kernel<T, 2>), grid, block, 0, s, (const T*)src, row_of, w, (const T*)addend,
-                           (T*)dst, T_, K, H);
-    else if (K <= 4)
-        hipLaunchKernelGGL((gather_reduce_kernel<T, 4>), grid, block, 0, s, (const T*)src, row_of, w, (const T*)addend,
-                           (T*)dst, T_, K, H);
-    else if (K <= 8)
-        hipLaunchKernelGGL((gather_reduce_kernel<T, 8>), grid, block, 0, s, (const T*)src, row_of, w, (const T*)addend,
-                           (T*)dst, T_, K, H);
-    else
-        hipLaunchKernelGGL((gather_reduce_kernel<T, AMOE_MAX_TOPK>), grid, block, 0, s, (const T*)src, row_of, w,
-                           (const T*)addend, (T*)dst, T_, K, H);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, (const T*)src, row_of, w, (const T*)addend, (T*)dst, T_, K, H, (const T*)second,
+                           (const T*)coef, (const T*)vec);
+    };
+    if (K <= 2) go(gather_reduce_kernel<T, 2, SHARED>);
+    else if (K <= 4) go(gather_reduce_kernel<T, 4, SHARED>);
+    else if (K <= 8) go(gather_reduce_kernel<T, 8, SHARED>);
+    else go(gather_reduce_kernel<T, AMOE_MAX_TOPK, SHARED>);
 }
 
 AMOE_EXPORT int amoe_gather_rows_bwd(const void* d_xp, const int32_t* row_of, const void* addend, void* dx, int dtype,
@@ -245,7 +305,7 @@ AMOE_EXPORT int amoe_gather_rows_bwd(const void* d_xp, const int32_t* row_of, co
     if (rc) return rc;
     AMOE_REQUIRE(K > 0 && K <= AMOE_MAX_TOPK, AMOE_ERR_UNSUPPORTED, "gather_rows_bwd: K=%d outside 1..%d", K,
                  AMOE_MAX_TOPK);
-    AMOE_DISPATCH_ELEM(dtype, launch_gather_reduce<ELEM>(d_xp, row_of, nullptr, addend, dx, T, K, H, (hipStream_t)stream))
+    AMOE_DISPATCH_ELEM(dtype, (launch_gather_reduce<ELEM, false>(d_xp, row_of, nullptr, addend, dx, T, K, H, (hipStream_t)stream)))
     return amoe_check_launch("gather_rows_bwd");
 }
 
@@ -256,7 +316,7 @@ AMOE_EXPORT int amoe_combine_fwd(const void* moe_out, const int32_t* row_of, con
     int rc = check_rows("combine_fwd", dtype, T, H);
     if (rc) return rc;
     AMOE_REQUIRE(K > 0 && K <= AMOE_MAX_TOPK, AMOE_ERR_UNSUPPORTED, "combine_fwd: K=%d outside 1..%d", K, AMOE_MAX_TOPK);
-    AMOE_DISPATCH_ELEM(dtype, launch_gather_reduce<ELEM>(moe_out, row_of, scores, nullptr, y, T, K, H, (hipStream_t)stream))
+    AMOE_DISPATCH_ELEM(dtype, (launch_gather_reduce<ELEM, false>(moe_out, row_of, scores, nullptr, y, T, K, H, (hipStream_t)stream)))
     return amoe_check_launch("combine_fwd");
 }
 
@@ -287,6 +347,26 @@ int amoe_launch_gated_act_fwd(const void* gu, const float* row_scale, void* inte
     return amoe_check_launch("gated_act_fwd");
 }
 
+static void launch_act_bwd(const void* gate_up, const void* d_inter, const float* row_scale, const int32_t* slot_of, void* d_gate_up,
+                           float* d_row_scale, int dtype, int R, int I, int T, int K, int act, hipStream_t s)
+{
+    const int rows_per_block = kBlock / AMOE_WAVE;
+    const int grid = (R + rows_per_block - 1) / rows_per_block < 65536 ? (R + rows_per_block - 1) / rows_per_block : 65536;
+    AMOE_DISPATCH_ACT(act, {
+        AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL((gated_act_bwd_kernel<ELEM, ACT>), dim3(grid), dim3(kBlock), 0, s,
+                                                     (const ELEM*)gate_up, (const ELEM*)d_inter, row_scale, slot_of, T, K,
+                                                     (ELEM*)d_gate_up, d_row_scale, R, I))
+    })
+}
+
+// the same with the gradient of row_scale in row order (a shared expert: one row per token)
+int amoe_launch_gated_act_bwd_rows(const void* gate_up, const void* d_inter, const float* row_scale, void* d_gate_up, float* d_scale,
+                                   int dtype, int R, int I, int act, hipStream_t s)
+{
+    launch_act_bwd(gate_up, d_inter, row_scale, nullptr, d_gate_up, d_scale, dtype, R, I, R, 1, act, s);
+    return amoe_check_launch("gated_act_bwd");
+}
+
 AMOE_EXPORT int amoe_gated_act_bwd(const void* gate_up, const void* d_inter, const float* row_scale,
                                    const int32_t* slot_of, void* d_gate_up, float* d_row_scale, int dtype, int R, int I,
                                    int T, int K, int act, void* stream)
@@ -301,15 +381,55 @@ AMOE_EXPORT int amoe_gated_act_bwd(const void* gate_up, const void* d_inter, con
         AMOE_REQUIRE(T > 0 && K > 0 && (long long)T * K == (long long)R, AMOE_ERR_BAD_ARG,
                      "gated_act_bwd: T*K must equal R (T=%d K=%d R=%d)", T, K, R);
     }
-    const int rows_per_block = kBlock / AMOE_WAVE;
-    const int grid = (R + rows_per_block - 1) / rows_per_block < 65536 ? (R + rows_per_block - 1) / rows_per_block : 65536;
-    hipStream_t s = (hipStream_t)stream;
-    AMOE_DISPATCH_ACT(act, {
-        AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL((gated_act_bwd_kernel<ELEM, ACT>), dim3(grid), dim3(kBlock), 0, s,
-                                                     (const ELEM*)gate_up, (const ELEM*)d_inter, row_scale, slot_of, T, K,
-                                                     (ELEM*)d_gate_up, d_row_scale, R, I))
-    })
+    launch_act_bwd(gate_up, d_inter, row_scale, slot_of, d_gate_up, d_row_scale, dtype, R, I, T, K, act, (hipStream_t)stream);
     return amoe_check_launch("gated_act_bwd");
+}
+
+int amoe_launch_score_grad(const float* partials, int n_parts, const float* extra, const int32_t* row_of, float* d_scores,
+                           int n_slots, bool accumulate, hipStream_t s)
+{
+    hipLaunchKernelGGL(score_grad_gather_kernel, dim3((n_slots + kBlock - 1) / kBlock), dim3(kBlock), 0, s, partials, n_parts,
+                       (long long)n_slots, extra, row_of, d_scores, n_slots, (int)accumulate);
+    return amoe_check_launch("score_grad_gather");
+}
+
+int amoe_launch_shared_gate(const void* x, const void* w, float* sig, int dtype, int T, int H, hipStream_t s)
+{
+    int rc = check_rows("shared_gate", dtype, T, H);
+    if (rc) return rc;
+    const dim3 grid((T + kBlock / AMOE_WAVE - 1) / (kBlock / AMOE_WAVE));
+    AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL(shared_gate_kernel<ELEM>, grid, dim3(kBlock), 0, s, (const ELEM*)x, (const ELEM*)w,
+                                                 sig, T, H))
+    return amoe_check_launch("shared_gate");
+}
+
+int amoe_launch_shared_gate_bwd(const float* d_sig, const float* sig, void* d_pre, int dtype, int T, hipStream_t s)
+{
+    AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL(shared_gate_bwd_kernel<ELEM>, dim3((T + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
+                                                 d_sig, sig, (ELEM*)d_pre, T))
+    return amoe_check_launch("shared_gate_bwd");
+}
+
+// dx[t,:] = dense[t,:] + sum_k d_xp[row_of[t,k],:]  (+ shared[t,:] + d_pre[t] * gate[:] with a shared expert)
+int amoe_launch_input_grad(const void* d_xp, const int32_t* row_of, const void* dense, const void* shared, const void* d_pre,
+                           const void* gate, void* dx, int dtype, int T, int K, int H, hipStream_t s)
+{
+    if (!shared) return amoe_gather_rows_bwd(d_xp, row_of, dense, dx, dtype, T, K, H, s);
+    int rc = check_rows("input_grad", dtype, T, H);
+    if (rc) return rc;
+    AMOE_DISPATCH_ELEM(dtype, (launch_gather_reduce<ELEM, true>(d_xp, row_of, nullptr, dense, dx, T, K, H, s, shared, d_pre, gate)))
+    return amoe_check_launch("input_grad");
+}
+
+int amoe_launch_sum_parts(const void* parts, int n_parts, void* out, int dtype, long long n, hipStream_t s)
+{
+    const int vec = dtype != AMOE_F32 ? 8 : 4;
+    AMOE_REQUIRE(n % vec == 0, AMOE_ERR_UNSUPPORTED, "sum_parts: %lld elements are no multiple of %d", n, vec);
+    const long long blocks = (n / vec + kBlock - 1) / kBlock;
+    const dim3 grid((unsigned)(blocks < 8192 ? blocks : 8192));
+    AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL(sum_parts_kernel<ELEM>, grid, dim3(kBlock), 0, s, (const ELEM*)parts, n_parts,
+                                                 (ELEM*)out, n / vec))
+    return amoe_check_launch("sum_parts");
 }
 
 AMOE_EXPORT int amoe_score_grad_gather(const float* partials, int n_parts, const int32_t* row_of, float* d_scores, int T,
@@ -318,8 +438,5 @@ AMOE_EXPORT int amoe_score_grad_gather(const float* partials, int n_parts, const
     AMOE_REQUIRE(partials && row_of && d_scores, AMOE_ERR_BAD_ARG, "score_grad_gather: null pointer");
     AMOE_REQUIRE(n_parts > 0 && T > 0 && K > 0, AMOE_ERR_BAD_ARG, "score_grad_gather: sizes must be positive");
     AMOE_REQUIRE((long long)T * K < (1ll << 31), AMOE_ERR_UNSUPPORTED, "score_grad_gather: T*K does not fit int32");
-    const int n = T * K;
-    hipLaunchKernelGGL(score_grad_gather_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, (hipStream_t)stream,
-                       partials, n_parts, (long long)n, row_of, d_scores, n);
-    return amoe_check_launch("score_grad_gather");
+    return amoe_launch_score_grad(partials, n_parts, nullptr, row_of, d_scores, T * K, false, (hipStream_t)stream);
 }

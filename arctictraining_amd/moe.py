@@ -9,6 +9,9 @@ The whole routed-expert computation is one torch.autograd.Function whose forward
 backward call the kernels stage by stage with no host synchronisation.
 """
 import contextlib
+import ctypes
+import functools
+import math
 import time
 from collections import OrderedDict, defaultdict
 from dataclasses import dataclass
@@ -18,7 +21,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import ops
+from . import _lib, ops
 
 
 @dataclass(kw_only=True)
@@ -91,6 +94,11 @@ class PhaseTimers:
         else:
             self.times[name] = 0
 
+    def skip(self, names):
+        """What start and stop of each leave behind while switched off."""
+        for name in names:
+            self.times[name] = 0
+
     def elapsed(self, name):
         return self.times[name]
 
@@ -152,6 +160,12 @@ def _token_ids(T: int, device) -> torch.Tensor:
     return _INDEX_CACHE.get((T, "ids", str(device)), lambda: torch.arange(T, dtype=torch.int32, device=device))
 
 
+def _dense_splits(T: int, Kd: int, N: int, dtype, tile: int = 256) -> int:
+    """Chunks of the tokens for the weight gradient [Kd,N] of a dense (not routed) linear map."""
+    tiles = -(-Kd // tile) * -(-N // tile)
+    return max(1, min(16, 512 // tiles, T // 256)) if dtype != torch.float32 else 1
+
+
 def _dense_weight_grad(a: torch.Tensor, b: torch.Tensor, tile_cfg: int = 0, tile: int = 256) -> torch.Tensor:
     """C [Kd,N] = a^T [Kd,T] @ b [T,N]: the weight gradient of a dense (not routed) linear map.
 
@@ -160,14 +174,8 @@ def _dense_weight_grad(a: torch.Tensor, b: torch.Tensor, tile_cfg: int = 0, tile
     C[s] = a[chunk s]^T @ b[chunk s].  The kernel accumulates each partial product in float32 and
     stores it in the operands' 16-bit type; the (at most 16) partials are then added in float32
     and the sum is rounded once more."""
-    T, Kd = a.shape
-    N = b.shape[1]
-    tiles = -(-Kd // tile) * -(-N // tile)
-    splits = max(1, min(16, 512 // tiles, T // 256)) if a.dtype != torch.float32 else 1
-    part = ops.grouped_gemm_wgrad(a, b, _token_offsets(T, splits, a.device), splits, tile_cfg=tile_cfg)
-    if splits == 1:
-        return part[0]
-    return part.sum(dim=0, dtype=torch.float32).to(a.dtype)
+    splits = _dense_splits(a.shape[0], a.shape[1], b.shape[1], a.dtype, tile)
+    return ops.dense_wgrad(a, b, _token_offsets(a.shape[0], splits, a.device), tile_cfg=tile_cfg)
 
 
 def _router_weight_grad(d_logits: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
@@ -177,6 +185,20 @@ def _router_weight_grad(d_logits: torch.Tensor, x: torch.Tensor) -> torch.Tensor
     if x.dtype == torch.float32 or E % 8 or T < 16 * 32:
         return torch.matmul(d_logits.t(), x)
     return _dense_weight_grad(d_logits, x, tile_cfg=1, tile=128)  # 128x128 tiles
+
+
+def _replayed(replay, E: int, opts) -> torch.Tensor:
+    """The replayed assignments as int32."""
+    assign = replay.to(torch.int32).contiguous()
+    if opts.get("check_replay", True) and not torch.cuda.is_current_stream_capturing():
+        # The reference's one_hot(..., num_classes=E) raises on an expert id outside [0, E)
+        # (moe.py:374).  The same error here, at the price of one host synchronisation per replayed
+        # forward; `ArcticMoE.check_replay = False` (and a HIP graph capture, which cannot
+        # synchronise) skips it, the permutation kernels then clamp such ids for memory safety.
+        bad = ((assign < 0) | (assign >= E)).any()
+        if bool(bad):
+            raise RuntimeError(f"routing_replay_assignments holds expert ids outside [0, {E})")
+    return assign
 
 
 def _route(x, router_gate, replay, opts):
@@ -190,17 +212,7 @@ def _route(x, router_gate, replay, opts):
     timers.start("router")
     logits = torch.matmul(x, router_gate.t())  # plain library GEMM, moe.py:233
     probs, topk_idx, scores = ops.router_topk_fwd(logits, K, opts["normalize"])
-    assign = topk_idx
-    if replay is not None:
-        assign = replay.to(torch.int32).contiguous()
-        if opts.get("check_replay", True) and not torch.cuda.is_current_stream_capturing():
-            # The reference's one_hot(..., num_classes=E) raises on an expert id outside [0, E)
-            # (moe.py:374).  The same error here, at the price of one host synchronisation per replayed
-            # forward; `ArcticMoE.check_replay = False` (and a HIP graph capture, which cannot
-            # synchronise) skips it, the permutation kernels then clamp such ids for memory safety.
-            bad = ((assign < 0) | (assign >= E)).any()
-            if bool(bad):
-                raise RuntimeError(f"routing_replay_assignments holds expert ids outside [0, {E})")
+    assign = topk_idx if replay is None else _replayed(replay, E, opts)
     # the row-grouped GEMMs of a step share one tile map: the permutation plan builds it (its
     # scan kernel holds the offsets), the workspace is kept for backward
     ws = ops.gemm_workspace(T * K, E, x.device)
@@ -209,176 +221,185 @@ def _route(x, router_gate, replay, opts):
     return logits, probs, topk_idx, scores, ws, plan
 
 
+@functools.lru_cache(maxsize=64)
+def _layer_config(E, K, H, I, act, dtype, normalize, tile_cfg, shared):
+    return (ctypes.c_int32 * 9)(E, K, H, I, act, dtype, normalize, tile_cfg, shared)
+
+
+# byte offsets and element counts inside the saved buffer, in the order the library lists them
+_SAVED_FIELDS = ("probs", "scores", "scores_perm", "topk_idx", "counts", "offsets", "token_of", "slot_of", "row_of")
+
+
+@functools.lru_cache(maxsize=256)
+def _layer_sizes(config_key, T: int, keep: bool):
+    out = (ctypes.c_longlong * (4 + len(_SAVED_FIELDS)))()
+    _lib.check(_lib.load().amoe_layer_sizes(_layer_config(*config_key), T, int(keep), out), "amoe_layer_sizes")
+    return tuple(out)
+
+
+def _saved_view(saved, name, config_key, T: int):
+    """One of _SAVED_FIELDS as a tensor over the saved buffer."""
+    E, K = config_key[:2]
+    shape = {"probs": (T, E), "scores": (T, K), "topk_idx": (T, K), "counts": (E,), "offsets": (E + 1,), "row_of": (T, K)}.get(name, (T * K,))
+    dtype = torch.float32 if name in ("probs", "scores", "scores_perm") else torch.int32
+    start = _layer_sizes(config_key, T, True)[3 + _SAVED_FIELDS.index(name)]
+    return saved[start : start + 4 * math.prod(shape)].view(dtype).view(shape)
+
+
+def _check_operand(t, name, like, shape) -> None:
+    """t has to be dense, of `like`'s type, on the current device (like's), and of the given shape."""
+    if t.dtype is not like.dtype or t.get_device() != like.get_device() or not t.is_contiguous():
+        ops._chk(t, name, like.dtype)
+    if t.shape != shape:
+        raise RuntimeError(f"{name} must be {list(shape)}, got {list(t.shape)}")
+
+
+def _layer_forward(x, router_gate, w_gate_up, w_down, shared, replay, opts, keep: bool):
+    """Router linear map, then the whole layer in one native call (moe.py:231-233, 340-411, 176-193, 450-461).  Returns y,
+    the buffer of what backward reads (keep) or of what a caller that only runs forward may look at, and the
+    config key."""
+    T, H = x.shape
+    E, K = opts["num_experts"], opts["top_k"]
+    ops._chk(x, "x")
+    _check_operand(w_gate_up, "w_gate_up", x, (E, H, w_gate_up.shape[-1]))
+    I = w_gate_up.shape[2] // 2
+    _check_operand(w_down, "w_down", x, (E, I, H))
+    sh_gate_up, sh_down, sh_out_gate = shared
+    all_rows = None
+    if sh_gate_up is not None:
+        _check_operand(sh_gate_up, "shared_expert_gate_up", x, (H, 2 * I))
+        _check_operand(sh_down, "shared_expert_down", x, (I, H))
+        _check_operand(sh_out_gate, "shared_expert_output_gate", x, (H, 1))
+        all_rows = _token_offsets(T, 1, x.device)
+    timers: PhaseTimers = opts["timers"]
+    key = (E, K, H, I, opts["act"], ops._dtype_code(x), opts["normalize"], opts["tile_cfg"], all_rows is not None)
+    sizes = _layer_sizes(key, T, keep)
+    if timers.wall_clock_breakdown:
+        timers.start("router")
+    logits = torch.matmul(x, router_gate.t())  # plain library GEMM, moe.py:233
+    assign = None if replay is None else _replayed(replay, E, opts)
+    y = torch.empty_like(x)
+    buf = torch.empty(sizes[0] + (0 if keep else sizes[1]), dtype=torch.uint8, device=x.device)
+    base = buf.data_ptr()
+    scratch = torch.empty(sizes[1], dtype=torch.uint8, device=x.device) if keep else None
+
+    def run(stages):
+        _lib.check(
+            _lib.load().amoe_layer_fwd(
+                _layer_config(*key), T, x.data_ptr(), logits.data_ptr(), ops._dtype_code(logits), ops._ptr(assign),
+                w_gate_up.data_ptr(), w_down.data_ptr(), ops._ptr(sh_gate_up), ops._ptr(sh_down), ops._ptr(sh_out_gate),
+                ops._ptr(all_rows), base, keep, scratch.data_ptr() if keep else base + sizes[0], y.data_ptr(), stages, ops._stream(),
+            ),
+            "amoe_layer_fwd",
+        )
+
+    if not timers.wall_clock_breakdown:
+        run(_STAGE_ALL)
+        timers.skip(_PHASES)
+    else:
+        for name, stage in zip(_PHASES, (1, 2, 4, 8)):
+            if name != "router":
+                if name == "shared-expert" and all_rows is None:
+                    continue
+                timers.start(name)
+            run(stage)
+            timers.stop(name)
+    cap = opts.get("capture")
+    if cap is not None:
+        cap.update(logits=logits, **{n: _saved_view(buf, n, key, T).clone() for n in _SAVED_FIELDS if n != "scores_perm"})
+    return y, buf, key
+
+
+_STAGE_ALL = 15
+_PHASES = ("router", "groupGeMM", "shared-expert", "moe-combine")
+
+
 class _ExpertLayerFn(torch.autograd.Function):
     """router top-k -> permutation -> grouped gated FFN -> weighted combine, and the
     gradients of all of it (the autograd of moe.py:231-233, 340-411, 176-193, 450-461 plus
-    the load-balance hook :393-406)."""
+    the load-balance hook :393-406).  A shared expert (moe.py:305-314) runs through the same
+    kernels as one more expert that owns every token, the sigmoid of its output gate in the role of
+    the routing score."""
 
     @staticmethod
     def forward(ctx, x, router_gate, w_gate_up, w_down, sh_gate_up, sh_down, sh_out_gate, replay, opts):
-        T, H = x.shape
-        E, K = opts["num_experts"], opts["top_k"]
-        timers: PhaseTimers = opts["timers"]
-        cfg = opts["tile_cfg"]
-        logits, probs, topk_idx, scores, ws, (counts, offsets, token_of, slot_of, row_of, scores_perm) = _route(
-            x, router_gate, replay, opts
+        y, saved, key = _layer_forward(
+            x, router_gate, w_gate_up, w_down, (sh_gate_up, sh_down, sh_out_gate), replay, opts, keep=True
         )
-
-        # The gather x[token_of] (moe.py:356) happens inside the GEMMs' A loads: the routed copy
-        # of the activations is never written.  The score of a routed row multiplies the expert's intermediate activation (epilogue of
-        # the gate_up GEMM) instead of its output: the down projection is linear, so
-        # (s * inter) @ W_down == s * (inter @ W_down), and the combine becomes a plain sum.
-        timers.start("groupGeMM")
-        gate_up, inter_s = ops.grouped_gemm_gateup_act_fwd(
-            x, w_gate_up, offsets, opts["act"], a_row_map=token_of, n_rows=T * K, tile_cfg=cfg, row_scale=scores_perm,
-            workspace=ws, map_ready=True,
-        )
-        out_s = ops.grouped_gemm_nn(inter_s, w_down, offsets, tile_cfg=cfg, workspace=ws, map_ready=True)
-        timers.stop("groupGeMM")
-
-        # Shared expert (moe.py:305-314): a dense gated FFN over all T tokens, its output scaled per
-        # token by sigmoid(x @ w_out_gate).  It runs through the same kernels as one more expert that
-        # owns every token, the sigmoid in the role of the routing score; its output joins the
-        # combine as the addend of the per-token sum.
-        shared = sh_gate_up is not None
-        sh_gu = sh_inter_s = sh_sig = sh_out = None
-        if shared:
-            timers.start("shared-expert")
-            all_rows = _token_offsets(T, 1, x.device)
-            sh_sig = torch.sigmoid(torch.matmul(x, sh_out_gate)).float().reshape(T)
-            sh_gu, sh_inter_s = ops.grouped_gemm_gateup_act_fwd(
-                x, sh_gate_up.unsqueeze(0), all_rows, opts["act"], tile_cfg=cfg, row_scale=sh_sig
-            )
-            sh_out = ops.grouped_gemm_nn(sh_inter_s, sh_down.unsqueeze(0), all_rows, tile_cfg=cfg)
-            timers.stop("shared-expert")
-
-        timers.start("moe-combine")
-        # y[t] = sum_k out_s[row_of[t,k]] (+ the shared expert's row t)
-        y = ops.gather_rows_bwd(out_s, row_of, addend=sh_out) if shared else ops.combine_fwd(out_s, row_of, None)
-        timers.stop("moe-combine")
-
-        ctx.opts = opts
-        ctx.shared = shared
-        ctx.gemm_ws = ws
-        ctx.save_for_backward(
-            x, router_gate, w_gate_up, w_down, probs, topk_idx, counts, offsets, row_of, token_of, slot_of, scores_perm,
-            gate_up, inter_s, sh_gate_up, sh_down, sh_out_gate, sh_gu, sh_inter_s, sh_sig,
-        )
+        ctx.opts, ctx.key = opts, key
+        ctx.save_for_backward(x, router_gate, w_gate_up, w_down, sh_gate_up, sh_down, sh_out_gate, saved)
+        ctx.set_materialize_grads(False)  # no zero-filled gradient for an output the loss does not use
+        if not opts["want_scores"]:
+            return y
         # scores in routed-row order, in the model dtype, as the reference returns them (moe.py:323,
         # only when return_router_scores); they stay attached to the graph like the reference's
-        if opts["want_scores"]:
-            scores_out = scores_perm.to(x.dtype)
-        else:
-            scores_out = scores_perm.new_empty(0)
-            ctx.mark_non_differentiable(scores_out)
-        ctx.set_materialize_grads(False)  # no zero-filled gradient for an output the loss does not use
-        cap = opts.get("capture")
-        if cap is not None:
-            cap.update(logits=logits, probs=probs, topk_idx=topk_idx, scores=scores, counts=counts, offsets=offsets,
-                       token_of=token_of, slot_of=slot_of, row_of=row_of)
-        return y, scores_out
+        return y, _saved_view(saved, "scores_perm", key, x.shape[0]).to(x.dtype, copy=True)
 
     @staticmethod
-    def backward(ctx, dy, ds_perm):
-        (x, router_gate, w_gate_up, w_down, probs, topk_idx, counts, offsets, row_of, token_of, slot_of, scores_perm,
-         gate_up, inter_s, sh_gate_up, sh_down, sh_out_gate, sh_gu, sh_inter_s, sh_sig) = ctx.saved_tensors
-        opts = ctx.opts
-        E, K = opts["num_experts"], opts["top_k"]
-        T = x.shape[0]
-        R = T * K
-        cfg = opts["tile_cfg"]
+    def backward(ctx, dy, ds_perm=None):
+        x, router_gate, w_gate_up, w_down, sh_gate_up, sh_down, sh_out_gate, saved = ctx.saved_tensors
+        opts, key = ctx.opts, ctx.key
         if dy is None and ds_perm is None:  # neither output took part in the loss
             return (None,) * 9
+        (T, H), (E, K, _, I) = x.shape, key[:4]
         dy = torch.zeros_like(x) if dy is None else dy.contiguous()
-
-        # The two expert weight gradients run on a second stream beside the chain of data gradients.
-        # Fork: the side stream sees everything the main stream has queued so far (dy, the saved
-        # tensors); join (below): the main stream waits for it before this function returns, so the
-        # tensors either stream reads outlive the kernels that read them.
-        main = side = None
-        if x.is_cuda and opts.get("overlap_weight_grads", True):
-            main, side = torch.cuda.current_stream(), _side_stream(x.device)
-            side.wait_stream(main)
-
-        def on_side(fn):
-            if side is None:
-                return fn()
-            with torch.cuda.stream(side):
-                out = fn()
-            if not torch.cuda.is_current_stream_capturing():
-                out.record_stream(main)   # allocated from the side stream's pool, consumed on the main stream
-            return out
-
-        # d(out_s)[r] = dy[token_of[r]]: the rows of dy are gathered inside the GEMMs' loads
-        ws = ctx.gemm_ws  # still holds the forward's tile map
-        fused = x.dtype != torch.float32 and cfg in (0, 1, 2)
-        if fused:
-            # data gradient of the down projection with the gated-activation backward as its
-            # epilogue: d_inter is never written; the score gradients come back as per-N-tile row sums
-            d_gate_up, parts = ops.grouped_gemm_nt_gated_bwd(
-                dy, w_down, offsets, gate_up, opts["act"], row_scale=scores_perm, a_row_map=token_of, n_rows=R, tile_cfg=cfg,
-                workspace=ws, map_ready=True,
-            )
-            if ds_perm is not None:  # gradient of the returned scores [R] (row order): one more partial
-                parts = torch.cat((parts, ds_perm.float().reshape(1, R)))
-                ds_perm = None
-            d_scores = ops.score_grad_gather(parts, row_of)
-        else:
-            d_inter_s = ops.grouped_gemm_nt(dy, w_down, offsets, a_row_map=token_of, n_rows=R, tile_cfg=cfg, workspace=ws,
-                                            map_ready=True)
-            # gated-activation backward, with the score multiply: also yields d_scores [T,K]
-            d_gate_up, d_scores = ops.gated_act_bwd(
-                gate_up, d_inter_s, opts["act"], row_scale=scores_perm, slot_of=slot_of, tk=(T, K)
-            )
-        # (queued after the data gradient above, which it does not depend on: its workgroups take the
-        # compute units as that kernel's last tiles finish)
-        d_w_down = None
-        if ctx.needs_input_grad[3]:
-            d_w_down = on_side(lambda: ops.grouped_gemm_wgrad(inter_s, dy, offsets, E, tile_cfg=cfg, b_row_map=token_of))
-        d_w_gate_up = None
-        if ctx.needs_input_grad[2]:
-            if side is not None:
-                side.wait_stream(main)   # d_gate_up
-            d_w_gate_up = on_side(lambda: ops.grouped_gemm_wgrad(x, d_gate_up, offsets, E, tile_cfg=cfg, a_row_map=token_of))
+        ops._chk(dy, "dy", x.dtype)
+        lib, config, stream, need = _lib.load(), _layer_config(*key), ops._stream(), ctx.needs_input_grad
+        cfg, shared = key[7], sh_gate_up is not None
+        scratch = torch.empty(_layer_sizes(key, T, True)[2], dtype=torch.uint8, device=x.device)
+        d_w_gate_up = torch.empty_like(w_gate_up) if need[2] else None
+        d_w_down = torch.empty_like(w_down) if need[3] else None
+        d_logits = torch.empty((T, E), dtype=x.dtype, device=x.device)
         if ds_perm is not None:
-            # gradient of the returned scores [R] (row order), taken back to the slots [T,K]
-            d_scores = d_scores + ds_perm.float()[row_of.long()]
-
-        d_logits = ops.router_bwd(
-            d_scores, probs, topk_idx, counts, x.dtype, opts["normalize"], opts["loss_coeff"] / T / opts["ep_size"]
+            ds_perm = ds_perm.float().contiguous()
+        # The two expert weight gradients run on a second stream beside the chain of data gradients.  It
+        # starts on them behind everything the main stream has queued up to their operands, and the main
+        # stream waits for it at the end, so the tensors either stream uses outlive the kernels that use them.
+        side = _side_stream(x.device).cuda_stream if opts["overlap_weight_grads"] and (need[2] or need[3]) else None
+        _lib.check(
+            lib.amoe_layer_bwd(
+                config, T, x.data_ptr(), dy.data_ptr(), w_down.data_ptr(), saved.data_ptr(), scratch.data_ptr(), ops._ptr(ds_perm),
+                opts["loss_coeff"] / T / opts["ep_size"], ops._ptr(d_w_gate_up), ops._ptr(d_w_down), d_logits.data_ptr(), stream, side,
+            ),
+            "amoe_layer_bwd",
         )
-        d_router_gate = _router_weight_grad(d_logits, x) if ctx.needs_input_grad[1] else None
+        d_router_gate = _router_weight_grad(d_logits, x) if need[1] else None
         cap = opts.get("capture")
         if cap is not None:
-            cap.update(d_scores=d_scores, d_logits=d_logits)
+            start = _layer_sizes(key, T, True)[-1]
+            cap.update(d_logits=d_logits, d_scores=scratch[start : start + 4 * T * K].view(torch.float32).view(T, K).clone())
 
-        d_sh_gate_up = d_sh_down = d_sh_out_gate = d_sh_gu = d_pre = None
-        if ctx.shared:
-            # the same chain for the expert that owns every token; the "score" gradient comes
-            # back per token and goes on through the sigmoid
+        d_sh_gate_up = d_sh_down = d_sh_out_gate = d_pre = all_rows = None
+        if shared:
             all_rows = _token_offsets(T, 1, x.device)
-            d_sh_inter_s = ops.grouped_gemm_nt(dy, sh_down.unsqueeze(0), all_rows, tile_cfg=cfg)
-            if ctx.needs_input_grad[5]:
-                d_sh_down = _dense_weight_grad(sh_inter_s, dy, tile_cfg=cfg)
-            d_sh_gu, d_sig = ops.gated_act_bwd(
-                sh_gu, d_sh_inter_s, opts["act"], row_scale=sh_sig, slot_of=_token_ids(T, x.device), tk=(T, 1)
+            d_pre = torch.empty((T, 1), dtype=x.dtype, device=x.device)
+            n_gu, n_dn = _dense_splits(T, H, 2 * I, x.dtype), _dense_splits(T, I, H, x.dtype)
+            d_sh_gate_up = torch.empty_like(sh_gate_up) if need[4] else None
+            d_sh_down = torch.empty_like(sh_down) if need[5] else None
+            parts = torch.empty(max(2 * n_gu, n_dn) * H * I, dtype=x.dtype, device=x.device) if max(n_gu, n_dn) > 1 else None
+            _lib.check(
+                lib.amoe_layer_bwd_shared(
+                    config, T, x.data_ptr(), dy.data_ptr(), sh_down.data_ptr(), all_rows.data_ptr(), saved.data_ptr(),
+                    scratch.data_ptr(), ops._ptr(parts), _token_offsets(T, n_gu, x.device).data_ptr(), n_gu, ops._ptr(d_sh_gate_up),
+                    _token_offsets(T, n_dn, x.device).data_ptr(), n_dn, ops._ptr(d_sh_down), d_pre.data_ptr(), stream,
+                ),
+                "amoe_layer_bwd_shared",
             )
-            if ctx.needs_input_grad[4]:
-                d_sh_gate_up = _dense_weight_grad(x, d_sh_gu, tile_cfg=cfg)
-            d_pre = (d_sig.reshape(T) * sh_sig * (1.0 - sh_sig)).to(x.dtype).unsqueeze(1)  # [T,1]
-            if ctx.needs_input_grad[6]:
+            if need[6]:
                 d_sh_out_gate = torch.matmul(x.t(), d_pre)
 
-        dx = None
-        if ctx.needs_input_grad[0]:
-            d_xp = ops.grouped_gemm_nt(d_gate_up, w_gate_up, offsets, tile_cfg=cfg, workspace=ws, map_ready=True)
-            dx_dense = torch.matmul(d_logits, router_gate)
-            if ctx.shared:
-                dx_dense.addmm_(d_pre, sh_out_gate.t())
-                dx_dense += ops.grouped_gemm_nt(d_sh_gu, sh_gate_up.unsqueeze(0), all_rows, tile_cfg=cfg)
-            dx = ops.gather_rows_bwd(d_xp, row_of, addend=dx_dense)
-        if side is not None:
-            main.wait_stream(side)
+        dx = dx_router = None
+        if need[0]:
+            dx = torch.empty_like(x)
+            dx_router = torch.matmul(d_logits, router_gate)
+        if dx is not None or side is not None:
+            _lib.check(
+                lib.amoe_layer_bwd_input(
+                    config, T, w_gate_up.data_ptr(), ops._ptr(sh_gate_up), ops._ptr(sh_out_gate), ops._ptr(all_rows),
+                    saved.data_ptr(), scratch.data_ptr(), ops._ptr(dx_router), ops._ptr(d_pre), ops._ptr(dx), stream, side,
+                ),
+                "amoe_layer_bwd_input",
+            )
         return dx, d_router_gate, d_w_gate_up, d_w_down, d_sh_gate_up, d_sh_down, d_sh_out_gate, None, None
 
 
@@ -615,11 +636,22 @@ class ArcticMoE(nn.Module):
         if getattr(self._config, "use_shared_expert", False):
             shared = (self.shared_expert_gate_up, self.shared_expert_down, self.shared_expert_output_gate)
         # the kernels are launched on the current device's current stream: make x's device current
-        with torch.cuda.device(x.device) if x.is_cuda else contextlib.nullcontext():
-            layer_fn = _ExpertLayerFn if self.is_gated else _UngatedExpertLayerFn
-            output, scores = layer_fn.apply(
-                x, self.router_gate, self.expert_gate_up, self.expert_down, *shared, replay, opts
-            )
+        elsewhere = x.is_cuda and x.device.index != torch.cuda.current_device()
+        with torch.cuda.device(x.device) if elsewhere else contextlib.nullcontext():
+            if self.is_gated:
+                output, scores = self._run_gated(x, shared, replay, opts)
+            else:
+                output, scores = _UngatedExpertLayerFn.apply(
+                    x, self.router_gate, self.expert_gate_up, self.expert_down, *shared, replay, opts
+                )
         output = output.reshape(orig_shape)
         self.timers.stop("amoe e2e")
         return (output, scores) if getattr(self._config, "return_router_scores", False) else output
+
+    def _run_gated(self, x, shared, replay, opts):
+        weights = (self.router_gate, self.expert_gate_up, self.expert_down)
+        if torch.is_grad_enabled():
+            out = _ExpertLayerFn.apply(x, *weights, *shared, replay, opts)
+            return out if opts["want_scores"] else (out, None)
+        y, saved, key = _layer_forward(x, *weights, shared, replay, opts, keep=False)
+        return y, _saved_view(saved, "scores_perm", key, x.shape[0]).to(x.dtype, copy=True) if opts["want_scores"] else None

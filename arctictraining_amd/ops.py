@@ -43,7 +43,8 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # (the handle alone: a torch.cuda.Stream object of the current stream costs the host some 2 us a call)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def router_topk_fwd(logits: torch.Tensor, top_k: int, normalize: bool):
@@ -364,6 +365,26 @@ def grouped_gemm_wgrad(A, B, offsets, num_experts: int, tile_cfg: int = 0, a_row
         num_experts, Kd, N, tile_cfg, _stream()
     )
     _lib.check(rc, "amoe_grouped_gemm_wgrad")
+    return C
+
+
+def dense_wgrad(A, B, chunk_offsets: torch.Tensor, tile_cfg: int = 0) -> torch.Tensor:
+    """C [Kd,N] = A [T,Kd]^T @ B [T,N]; the chunks of the tokens that chunk_offsets [splits+1] names are multiplied side
+    by side and the partial products added in float32."""
+    lib = _lib.load()
+    _chk(A, "A")
+    _chk(B, "B", A.dtype)
+    _chk(chunk_offsets, "chunk_offsets", torch.int32)
+    T, Kd = A.shape
+    N = B.shape[1]
+    splits = chunk_offsets.numel() - 1
+    C = torch.empty((Kd, N), dtype=A.dtype, device=A.device)
+    parts = torch.empty((splits, Kd, N), dtype=A.dtype, device=A.device) if splits > 1 else None
+    rc = lib.amoe_dense_wgrad(
+        A.data_ptr(), B.data_ptr(), chunk_offsets.data_ptr(), splits, _ptr(parts), C.data_ptr(), _dtype_code(A), T, Kd, N, tile_cfg,
+        _stream()
+    )
+    _lib.check(rc, "amoe_dense_wgrad")
     return C
 
 

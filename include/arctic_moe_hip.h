@@ -257,6 +257,52 @@ int amoe_gated_act_bwd(const void* gate_up, const void* d_inter, const float* ro
                        void* stream);
 
 /*
+ * The gated layer's forward and backward as a few calls, the stages above run over two buffers of the caller's.
+ *   config: int32[9] on the HOST = {E, K, H, I, act, dtype, normalize, tile_cfg, shared}
+ *   amoe_layer_sizes fills out (long long[13], host): the bytes of the saved buffer (what backward reads; with keep = 0
+ *   what forward alone needs of it), of forward's scratch and of backward's scratch; then the byte offsets inside the
+ *   saved buffer of probs, scores, scores_perm, topk_idx, counts, offsets, token_of, slot_of, row_of (the
+ *   layouts of amoe_router_topk_fwd and amoe_permute_plan), and that of d_scores [T,K] f32 inside backward's scratch.
+ *   amoe_layer_fwd: y [T,H] from x [T,H] and logits [T,E] (of logits_dtype); assign [T,K] i32 or null replaces the
+ *   selected experts.  stages: which of the AMOE_STAGE_* steps to run, in this order.  With config.shared: the shared
+ *   expert's gate_up [H,2I], down [I,H] and output gate [H,1] (moe.py:305-314), all_rows = int32 {0, T} on the device.
+ *   amoe_layer_bwd: d_logits [T,E] and, where not null, the experts' weight gradients (on side_stream if that is not
+ *   null) from dy [T,H]; d_scores_rows [R] f32 or null: gradient of the row-ordered scores; saved made with keep = 1.
+ *   amoe_layer_bwd_shared: the shared expert's weight gradients where not null, and d_pre [T] (gradient in front
+ *   of its sigmoid).  *_chunks / *_splits / parts: see amoe_dense_wgrad; parts holds the larger of the two.
+ *   amoe_layer_bwd_input: dx [T,H] (skipped if null) from dx_router [T,H] = d_logits @ router weights and what the
+ *   calls before left in scratch; then `stream` waits for side_stream.  The three share one scratch, in this order.
+ */
+#define AMOE_STAGE_ROUTE 1
+#define AMOE_STAGE_EXPERTS 2
+#define AMOE_STAGE_SHARED 4
+#define AMOE_STAGE_COMBINE 8
+#define AMOE_STAGE_ALL 15
+int amoe_layer_sizes(const int32_t* config, int T, int keep, long long* out);
+int amoe_layer_fwd(const int32_t* config, int T, const void* x, const void* logits, int logits_dtype, const int32_t* assign,
+                   const void* w_gate_up, const void* w_down, const void* sh_gate_up, const void* sh_down,
+                   const void* sh_out_gate, const int32_t* all_rows, void* saved, int keep, void* scratch, void* y, int stages,
+                   void* stream);
+int amoe_layer_bwd(const int32_t* config, int T, const void* x, const void* dy, const void* w_down, const void* saved,
+                   void* scratch, const float* d_scores_rows, float lb_coeff, void* d_w_gate_up, void* d_w_down,
+                   void* d_logits, void* stream, void* side_stream);
+int amoe_layer_bwd_shared(const int32_t* config, int T, const void* x, const void* dy, const void* sh_down,
+                          const int32_t* all_rows, const void* saved, void* scratch, void* parts,
+                          const int32_t* gate_up_chunks, int gate_up_splits, void* d_sh_gate_up,
+                          const int32_t* down_chunks, int down_splits, void* d_sh_down, void* d_pre, void* stream);
+int amoe_layer_bwd_input(const int32_t* config, int T, const void* w_gate_up, const void* sh_gate_up,
+                         const void* sh_out_gate, const int32_t* all_rows, const void* saved, void* scratch,
+                         const void* dx_router, const void* d_pre, void* dx, void* stream, void* side_stream);
+
+/*
+ * Weight gradient of a linear map that every token takes: C [Kd,N] = A [T,Kd]^T @ B [T,N].  The tokens are cut into
+ * `splits` chunks, chunk_offsets [splits+1] i32 on the device; parts [splits][Kd][N] in the operands' type holds the
+ * partial products (unused for splits = 1), which are added in float32.
+ */
+int amoe_dense_wgrad(const void* A, const void* B, const int32_t* chunk_offsets, int splits, void* parts, void* C, int dtype,
+                     int T, int Kd, int N, int tile_cfg, void* stream);
+
+/*
  * Expert-weight re-layout, checkpoint format -> ArcticMoE parameters.  Replaces the torch
  * stack / view / transpose sequence of remap_orig_moe_mlp_params_to_arctic_moe
  * (arctic_training/model/moe/utils.py:232-266):

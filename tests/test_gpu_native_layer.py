@@ -1,0 +1,54 @@
+"""The layer as native calls: its own small kernels at their edges, and forward alone against forward for backward."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,Kd,N,splits", [(5, 8, 16, 1), (300, 40, 264, 3), (4096, 256, 8, 16)])
+def test_dense_weight_gradient(gpu_device, dtype, T, Kd, N, splits):
+    from arctictraining_amd import moe, ops
+
+    print("dense_wgrad", dtype, T, Kd, N, splits, flush=True)
+    g = torch.Generator(gpu_device).manual_seed(T + N)
+    a = torch.randn(T, Kd, device=gpu_device, generator=g).to(dtype)
+    b = torch.randn(T, N, device=gpu_device, generator=g).to(dtype)
+    got = ops.dense_wgrad(a, b, moe._token_offsets(T, splits, gpu_device))
+    ref = a.double().t() @ b.double()
+    tol = {torch.bfloat16: 1e-2, torch.float16: 2e-3, torch.float32: 1e-5}[dtype]
+    assert (got.double() - ref).norm() <= tol * ref.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("T", [1, 7, 260])
+def test_forward_alone_equals_forward_for_backward(gpu_device, dtype, shared, T):
+    from arctictraining_amd import ArcticMoE, MoEConfig
+
+    print("layer", dtype, shared, T, flush=True)
+    torch.manual_seed(T)
+    cfg = MoEConfig(act_fn=F.silu, input_dtype=dtype, intermediate_dim=72, model_dim=136, normalize_topk_scores=True, num_experts=5,
+                    top_k=2, use_shared_expert=shared, return_router_scores=True)
+    with gpu_device:
+        layer = ArcticMoE(cfg)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, 0.1)
+    x = torch.randn(T, 136, device=gpu_device).to(dtype)
+    y, scores = layer(x)
+    with torch.no_grad():
+        y0, scores0 = layer(x)
+        # the shared expert's part against a plain computation of it
+        if shared:
+            plain = ArcticMoE(MoEConfig(**{**cfg.__dict__, "use_shared_expert": False})).to(gpu_device)
+            for n, p in plain.named_parameters():
+                p.copy_(getattr(layer, n))
+            h = x.float() @ layer.shared_expert_gate_up.float()
+            want = (F.silu(h[:, 0::2]) * h[:, 1::2]) @ layer.shared_expert_down.float()
+            want = want * torch.sigmoid(x.float() @ layer.shared_expert_output_gate.float())
+            got = y0.float() - plain(x)[0].float()
+            assert (got - want).norm() <= (2e-2 if dtype == torch.bfloat16 else 1e-5) * (want.norm() + y0.float().norm())
+    assert torch.equal(y, y0) and torch.equal(scores, scores0)
+    assert y.requires_grad and not y0.requires_grad
