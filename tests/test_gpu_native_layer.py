@@ -29,14 +29,14 @@ def test_forward_alone_equals_forward_for_backward(gpu_device, dtype, shared, T)
 
     print("layer", dtype, shared, T, flush=True)
     torch.manual_seed(T)
-    cfg = MoEConfig(act_fn=F.silu, input_dtype=dtype, intermediate_dim=72, model_dim=136, normalize_topk_scores=True, num_experts=5,
+    cfg = MoEConfig(act_fn=F.silu, input_dtype=dtype, intermediate_dim=96, model_dim=160, normalize_topk_scores=True, num_experts=5,
                     top_k=2, use_shared_expert=shared, return_router_scores=True)
     with gpu_device:
         layer = ArcticMoE(cfg)
     with torch.no_grad():
         for p in layer.parameters():
             p.normal_(0.0, 0.1)
-    x = torch.randn(T, 136, device=gpu_device).to(dtype)
+    x = torch.randn(T, 160, device=gpu_device).to(dtype)
     y, scores = layer(x)
     with torch.no_grad():
         y0, scores0 = layer(x)
