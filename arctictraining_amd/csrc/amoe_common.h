@@ -268,8 +268,9 @@ __device__ __forceinline__ void amoe_emit_tile_map(const int32_t* row_end, int r
         const int first_tile = lo ? tscan[lo - 1] : 0;
         const int row0 = lo ? row_end[lo - 1] : 0;
         const int tiles = tscan[lo] - first_tile;
-        // the expert's rows in tiles of equal height, a multiple of the 32 rows at which the kernels skip work
-        const int height = ((row_end[lo] - row0 + tiles - 1) / tiles + 31) & ~31;
+        // the expert's rows in tiles of equal height, a multiple of the 32 rows at which the kernels skip work (bm < 32: of bm)
+        const int round = bm < 32 ? bm : 32;
+        const int height = ((row_end[lo] - row0 + tiles - 1) / tiles + round - 1) & ~(round - 1);
         const int first = row0 + (mt - first_tile) * height;
         const int last = first + height < row_end[lo] ? first + height : row_end[lo];
         tile_map[mt] = make_int4(lo, row_base + first, row_base + last, 0);

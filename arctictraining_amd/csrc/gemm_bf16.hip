@@ -1284,8 +1284,25 @@ static int set_supertiles(GemmArgs& a, long long m_tiles, long long* grid)
     return AMOE_OK;
 }
 
-// workspace: [0,16) tile count, then one int4 per M tile for the smallest tile height (64)
+// workspace: [0,16) tile count, then one int4 per M tile
 static inline int ws_max_mtiles(int R, int E, int bm) { return R / bm + E + 1; }
+
+// Tile height of the row-grouped products: that of the tile shape, and with the default one a lower one where an
+// expert has few rows on average (gemm_skinny.hip reads the weights once per such tile and is bound by that).
+// 128 experts of 2048 x 768, A B[e] of both products, this tile height against 256 rows: 1 row an expert 142 against
+// 160 us, 4 rows 219 / 230, 8 rows 232 / 230, 16 rows 248 / 236; 64 experts of 2048 x 1408 (whose 256-column tiles fill
+// the last round of workgroups badly) 8 rows 209 / 236, 16 rows 219 / 239; 32 experts of 1024 x 1024 8 rows 39 / 50.
+// Uneven loads set the limits: where a sixteenth of the experts has half of the rows, their low tiles read the weights
+// again, at 6 rows an expert and 16-row tiles 13 % in the products with B^T (153 / 135 us), at 8 and 32-row tiles
+// nothing (135 / 136), at 12 again 14 %.
+static inline int rows_tile_height(int R, int E, int tile_cfg)
+{
+    if (tile_cfg == 0) {
+        if (R <= 4ll * E) return 16;
+        if (R <= 8ll * E) return 32;
+    }
+    return pick_cfg(tile_cfg).bm;
+}
 
 int amoe_build_tile_map(const int32_t* offsets, int R, int E, int bm, void* workspace, size_t workspace_bytes,
                         const int4** tile_map, const int32_t** n_mtiles, int* max_mtiles, hipStream_t s, bool ready);
@@ -1294,7 +1311,9 @@ int amoe_build_tile_map(const int32_t* offsets, int R, int E, int bm, void* work
 AMOE_EXPORT size_t amoe_grouped_gemm_workspace_bytes(int R, int E)
 {
     if (R <= 0 || E <= 0) return 0;
-    return 16 + sizeof(int4) * (size_t)ws_max_mtiles(R, E, 64);
+    // (64: the tile height of the float32 kernels)
+    const int low = rows_tile_height(R, E, 0);
+    return 16 + sizeof(int4) * (size_t)ws_max_mtiles(R, E, low < 64 ? low : 64);
 }
 
 // ready: the workspace already holds the map for these arguments (AMOE_TILE_MAP_READY); nothing is launched
@@ -1324,7 +1343,7 @@ int amoe_tile_map_layout(int R, int E, int dtype, int tile_cfg, void* workspace,
     AMOE_REQUIRE(R > 0 && E > 0 && E <= AMOE_MAX_EXPERTS, AMOE_ERR_BAD_ARG, "tile map: bad sizes R=%d E=%d", R, E);
     AMOE_REQUIRE(workspace_bytes >= amoe_grouped_gemm_workspace_bytes(R, E), AMOE_ERR_WORKSPACE,
                  "tile map: workspace %zu < %zu bytes", workspace_bytes, amoe_grouped_gemm_workspace_bytes(R, E));
-    *bm = dtype == AMOE_F32 ? 64 : pick_cfg(shape).bm;
+    *bm = dtype == AMOE_F32 ? 64 : rows_tile_height(R, E, shape);
     *max_mtiles = ws_max_mtiles(R, E, *bm);
     *n_mtiles = (int32_t*)workspace;
     *tile_map = (int4*)((char*)workspace + 16);
@@ -1338,6 +1357,9 @@ int amoe_pp_gateup_act(const GemmArgs& a, int act, int tiles, hipStream_t s);
 int amoe_pp_rows(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s);
 int amoe_pp_gated_bwd(const GemmArgs& a, int act, int tiles, hipStream_t s);
 int amoe_pp_wgrad(GemmArgs a, hipStream_t s);
+// few rows per expert (gemm_skinny.hip)
+int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s);
+int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s);
 
 // rows mode driver shared by the three row-grouped entry points
 template <bool B_KC, int EPI, int ACT>
@@ -1354,7 +1376,8 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
                  AMOE_ERR_UNSUPPORTED, "grouped_gemm: operand of 4 GiB or more (R=%d, K=%d, N=%d)", R, Kred, N);
     GemmArgs a = {};
     int max_mtiles = 0;
-    int rc = amoe_build_tile_map(offsets, R, E, tc.bm, workspace, workspace_bytes, &a.tile_map, &a.n_mtiles,
+    const int bm = rows_tile_height(R, E, tile_cfg);
+    int rc = amoe_build_tile_map(offsets, R, E, bm, workspace, workspace_bytes, &a.tile_map, &a.n_mtiles,
                                  &max_mtiles, s, map_ready);
     if (rc) return rc;
     a.A = (const bf16_t*)A;
@@ -1383,6 +1406,11 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
     a.n_mt = 0;
     long long grid = 0;
     a.max_mtiles = max_mtiles;
+    if (bm < tc.bm) {
+        if constexpr (EPI == EPI_GATED) return amoe_skinny_gateup_act(a, ACT, bm, s);
+        else if constexpr (EPI == EPI_STORE && !B_KC) return amoe_skinny_nn(a, bm, s);
+        // (the products with B^T run on the default kernel, which takes tiles of any height up to its own)
+    }
     rc = set_supertiles(a, max_mtiles, &grid);
     if (rc) return rc;
     if (tile_cfg == 0) {

@@ -1,0 +1,214 @@
+// The 16-bit grouped products C[rows_e,:] = A[rows_e,:] @ B[e] where an expert has a few rows (decoding, short prompts).
+//
+// Bound by reading the weights once: with 256-row tiles eight wavefronts wait at the same barriers for the same stage,
+// a tile has one workgroup's loads in flight, and one token of K = 8 experts fills 48 compute units.  Here a wavefront
+// streams its part of the weights straight into registers: no LDS and no barrier before the last sum, so every wavefront
+// on a compute unit has its own two 8 KB steps in flight.
+//
+// A workgroup owns MT x 16 rows of an expert and 16 * CPL columns, its NW wavefronts take every NW-th step of 32 k.
+// Lane (lq, l16) loads, for each of the 8 k of its quarter lq, the CPL columns l16 * CPL .. of the row of B (256 or 128
+// contiguous bytes per row and quarter); byte permutes of two such rows give the MFMA operands: fragment j holds column
+// l16 * CPL + j.  The wavefronts' partial sums meet in LDS, in a fixed order.
+//
+// One MI355X, bf16, gate_up and down product, against 256-row tiles: 128 experts of 2048 x 768, 1 row an expert 105 and
+// 55 -> 99 and 43 us, 4 rows 152 and 78 -> 145 and 74 (5.5 TB/s, what a read of that size reaches); 8 experts of
+// 4096 x 14336, 1 row 292 and 184 -> 256 and 129, 4 rows 334 and 195 -> 330 and 149; 16 experts of 512 x 512, 4 rows 17
+// and 12 -> 11 and 9.  A 64-row form at 32 rows an expert of the first took 222 and 90 us (one-tile workgroups of 256 rows
+// 204 and 83) and is not kept.
+#include "gemm_common.h"
+#include "gemm_launch.h"
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float sk_f32x4;
+
+namespace {
+
+constexpr uint32_t SK_NOWHERE = 0xFFFFFFF0u;   // a load offset past every operand: the lane receives zeros
+
+template <typename ET>
+struct MfmaSkinny;
+template <>
+struct MfmaSkinny<bf16_t> {
+    __device__ static __forceinline__ sk_f32x4 run(u32x4_t a, u32x4_t b, sk_f32x4 c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mfma_bf16x8, a), __builtin_bit_cast(mfma_bf16x8, b), c, 0, 0, 0);
+    }
+};
+template <>
+struct MfmaSkinny<f16_t> {
+    __device__ static __forceinline__ sk_f32x4 run(u32x4_t a, u32x4_t b, sk_f32x4 c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mfma_f16x8, a), __builtin_bit_cast(mfma_f16x8, b), c, 0, 0, 0);
+    }
+};
+
+template <int MT, int CPL, int NW, int EPI, int ACT, typename ET>
+__device__ __forceinline__ void skinny_body(const GemmArgs& p)
+{
+    constexpr int W = CPL / 2, H = CPL / 4;           // dwords of a lane's row, groups of four columns
+    __shared__ sk_f32x4 red[NW][4 * H * 64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lq = lane >> 4;
+
+    const int pm = blockIdx.x / p.n_ntiles;
+    const int n0 = (blockIdx.x - pm * p.n_ntiles) * 16 * CPL;
+    if (pm >= min(scalar_load_i32(p.n_mtiles), p.max_mtiles)) return;
+    const int32_t* ent = reinterpret_cast<const int32_t*>(p.tile_map + pm);
+    const int e = scalar_load_i32(ent), m0 = scalar_load_i32(ent + 1), mend = scalar_load_i32(ent + 2);
+
+    const int steps = p.Kd / 32;                      // (the reduction length is a multiple of 32)
+    const uint32_t row_bytes = (uint32_t)p.ldb * 2u;
+    const __amdgpu_buffer_rsrc_t bd = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t*>(p.B) + (long long)e * p.strideB, (short)0, (int)((uint32_t)p.Kd * row_bytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t ad = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.A), (short)0, (int)SK_NOWHERE, 0x00020000);
+    const int n = n0 + l16 * CPL;
+    const uint32_t boff = n < p.N ? (uint32_t)(lq * 8) * row_bytes + (uint32_t)n * 2u : SK_NOWHERE;
+    uint32_t aoff[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int row = m0 + i * 16 + l16;
+        const int src = row < mend && p.a_row_map ? p.a_row_map[row] : row;
+        aoff[i] = row < mend ? ((uint32_t)src * (uint32_t)p.lda + lq * 8) * 2u : SK_NOWHERE;
+    }
+
+    struct Step {
+        uint32_t b[8][W];
+        u32x4_t a[MT];
+    };
+    // a step past the last loads zeros
+    auto load = [&](Step& s, int step) {
+        const bool live = step < steps;
+        const uint32_t sb = live ? (uint32_t)step * 32u * row_bytes : 0u, sa = live ? (uint32_t)step * 64u : 0u;
+        const uint32_t vb = live ? boff : SK_NOWHERE;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if constexpr (CPL == 8) {
+                const u32x4_t v = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(bd, vb, sb + k * row_bytes, 0));
+#pragma unroll
+                for (int w = 0; w < 4; ++w) s.b[k][w] = v[w];
+            } else {
+                const u32x2_t v = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(bd, vb, sb + k * row_bytes, 0));
+                s.b[k][0] = v[0];
+                s.b[k][1] = v[1];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            s.a[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ad, live ? aoff[i] : SK_NOWHERE, sa, 0));
+    };
+    sk_f32x4 acc[MT][CPL];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < CPL; ++j) acc[i][j] = sk_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const Step& s) {
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            u32x4_t f0, f1;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                f0[k] = __builtin_amdgcn_perm(s.b[2 * k + 1][w], s.b[2 * k][w], 0x05040100u);
+                f1[k] = __builtin_amdgcn_perm(s.b[2 * k + 1][w], s.b[2 * k][w], 0x07060302u);
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                acc[i][2 * w] = MfmaSkinny<ET>::run(f0, s.a[i], acc[i][2 * w]);
+                acc[i][2 * w + 1] = MfmaSkinny<ET>::run(f1, s.a[i], acc[i][2 * w + 1]);
+            }
+        }
+    };
+
+    const int rounds = (steps + NW - 1) / NW;
+    Step s0, s1;
+    load(s0, wave);
+    for (int r = 0; r < rounds; r += 2) {
+        load(s1, (r + 1) * NW + wave);
+        multiply(s0);
+        load(s0, (r + 2) * NW + wave);
+        multiply(s1);
+    }
+
+    // the wavefronts' sums, 16 rows at a time.  Lane (lq, l16) holds columns (4 lq + v) * CPL + j of row l16.
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        if (m0 + i * 16 >= mend) break;
+        if (i) __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+                red[wave][(v * H + h) * 64 + lane] =
+                    sk_f32x4{acc[i][4 * h][v], acc[i][4 * h + 1][v], acc[i][4 * h + 2][v], acc[i][4 * h + 3][v]};
+        __syncthreads();
+        for (int u = tid; u < 4 * H * 64; u += NW * 64) {
+            sk_f32x4 c = red[0][u];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) c += red[w][u];
+            const int l = u & 63, q = u >> 6;
+            const int row = m0 + i * 16 + (l & 15);
+            const int col = n0 + ((l >> 4) * 4 + q / H) * CPL + (q % H) * 4;
+            if (row < mend && col < p.N) {
+                const uint32_t x = Elem16<ET>::pack2(c[0], c[1]), y = Elem16<ET>::pack2(c[2], c[3]);
+                if (EPI != EPI_GATED || p.C) *reinterpret_cast<u32x2_t*>(p.C + (long long)row * p.ldc + col) = u32x2_t{x, y};
+                if constexpr (EPI == EPI_GATED) {
+                    const float s = p.row_scale ? p.row_scale[row] : 1.0f;
+                    *reinterpret_cast<uint32_t*>(p.C2 + (long long)row * p.ldc2 + (col >> 1)) =
+                        Elem16<ET>::pack2(s * Elem16<ET>::hi(x) * act_fwd_fast<ACT>(Elem16<ET>::lo(x)),
+                                          s * Elem16<ET>::hi(y) * act_fwd_fast<ACT>(Elem16<ET>::lo(y)));
+                }
+            }
+        }
+    }
+}
+
+// (at least 4 wavefronts per SIMD with 16 rows, 3 with 32)
+template <int MT, int CPL, int NW, int EPI, int ACT>
+__global__ void __launch_bounds__(NW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_bf16_kernel(GemmArgs p)
+{
+    skinny_body<MT, CPL, NW, EPI, ACT, bf16_t>(p);
+}
+template <int MT, int CPL, int NW, int EPI, int ACT>
+__global__ void __launch_bounds__(NW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_f16_kernel(GemmArgs p)
+{
+    skinny_body<MT, CPL, NW, EPI, ACT, f16_t>(p);
+}
+
+template <int MT, int CPL, int NW, int EPI, int ACT>
+int launch_skinny(GemmArgs a, int m_tiles, hipStream_t s)
+{
+    a.n_ntiles = (a.N + 16 * CPL - 1) / (16 * CPL);
+    const long long grid = (long long)m_tiles * a.n_ntiles;
+    AMOE_REQUIRE(grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
+    if (a.f16)
+        hipLaunchKernelGGL((grouped_gemm_skinny_f16_kernel<MT, CPL, NW, EPI, ACT>), dim3((int)grid), dim3(NW * 64), 0, s, a);
+    else
+        hipLaunchKernelGGL((grouped_gemm_skinny_bf16_kernel<MT, CPL, NW, EPI, ACT>), dim3((int)grid), dim3(NW * 64), 0, s, a);
+    return amoe_check_launch("grouped_gemm_skinny");
+}
+
+// bm: height of the map's tiles; R rows of a.E experts
+template <int EPI, int ACT>
+int launch_height(const GemmArgs& a, int bm, hipStream_t s)
+{
+    const int R = a.M;
+    // every expert with a row has at most rows / bm + 1 tiles
+    int m_tiles = R / bm + (a.E < R ? a.E : R);
+    if (m_tiles > R) m_tiles = R;
+    if (m_tiles > a.max_mtiles) m_tiles = a.max_mtiles;
+    AMOE_REQUIRE(bm == 16 || bm == 32, AMOE_ERR_UNSUPPORTED, "grouped_gemm: no kernel for tiles of %d rows", bm);
+    if (bm == 32) return launch_skinny<2, 8, 4, EPI, ACT>(a, m_tiles, s);
+    // too few tiles of 128 columns for the compute units (one token): half as wide, twice as many wavefronts each
+    const int cus = device_cu_count();
+    if ((long long)m_tiles * ((a.N + 127) / 128) < cus) return launch_skinny<1, 4, 8, EPI, ACT>(a, m_tiles, s);
+    return launch_skinny<1, 8, 4, EPI, ACT>(a, m_tiles, s);
+}
+
+}  // namespace
+
+int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s)
+{
+    AMOE_DISPATCH_ACT(act, return (launch_height<EPI_GATED, ACT>(a, bm, s)))
+    return AMOE_ERR_BAD_ARG;
+}
+
+int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s) { return launch_height<EPI_STORE, 0>(a, bm, s); }
