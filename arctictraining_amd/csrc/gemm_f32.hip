@@ -1,8 +1,15 @@
 // Ragged grouped GEMMs in float32 on v_mfma_f32_32x32x2_f32 (full-precision FMA in the
-// matrix core).  One 64x64x16 kernel serves the three layouts; operands are staged in LDS
+// matrix core).  One 64x64 kernel serves the three layouts; operands are staged in LDS
 // K-major ([k][m]) so that the one-float-per-lane MFMA operands are read conflict-free
 // whatever the layout in memory.  This is the path of the small float32 configuration; the
-// bf16 kernels are the performance path.
+// 16-bit kernels are the performance path.
+//
+// What bounds it: with 2 to 9 small workgroups per compute unit, the wait for a stage's loads between two barriers.
+// The next stage's loads are therefore issued before this one's MFMAs and go into the other of two LDS stages, one
+// barrier per stage.  32 k a stage in the row products, 16 in the weight gradients (in which twice as many workgroups
+// share a compute unit; 32 is 4-10 % slower there).  One MI355X, 8 experts x 512 rows, 512 x 2048 and 1024 x 512: A B
+// 96 and 72 -> 99 and 57 us, A B^T 56 and 127 -> 53 and 108 us; 32 rows an expert 28 and 36 -> 21 and 32, 24 and 77
+// -> 19 and 58.  Dealing each XCD a contiguous eighth of the tiles changed none of these figures.
 #include "amoe_common.h"
 
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float mfma_f32x16;
@@ -12,7 +19,7 @@ int amoe_build_tile_map(const int32_t* offsets, int R, int E, int bm, void* work
 
 namespace {
 
-constexpr int BM = 64, BN = 64, BK = 16, NT = 256, PAD = 4;
+constexpr int BM = 64, BN = 64, NT = 256, PAD = 4;
 
 struct GemmArgsF32 {
     const float* A;
@@ -33,8 +40,9 @@ __global__ void __launch_bounds__(NT)
 grouped_gemm_f32_kernel(GemmArgsF32 p)
 {
     constexpr bool WGRAD = !A_KC;
-    __shared__ float As[BK][BM + PAD];
-    __shared__ float Bs[BK][BN + PAD];
+    constexpr int BK = WGRAD ? 16 : 32, NV = BK / 16;   // k of a stage; vectors of either operand per thread
+    __shared__ float As[2][BK][BM + PAD];
+    __shared__ float Bs[2][BK][BN + PAD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int lj = lane & 31, lg = lane >> 5;
@@ -63,7 +71,7 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
     const float* Ab = WGRAD ? p.A + (long long)r0 * p.lda : p.A;
     const float* Bb = WGRAD ? p.B + (long long)r0 * p.ldb : p.B + (long long)e * p.strideB;
 
-    // per-thread source coordinates
+    // per-thread source coordinates: NV vectors of either operand per stage, 16 apart in k
     long long a_src;
     int a_col = 0, b_col = 0;  // column offsets of the gathered weight-gradient operands
     int a_k;  // k offset inside the tile
@@ -97,46 +105,57 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
     for (int v = 0; v < 16; ++v) acc[v] = 0.f;
 
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < k_len; k0 += BK) {
-        f32x4_t va, vb;
-        if (A_KC) {
-            va = (k0 + a_k < k_len) ? *reinterpret_cast<const f32x4_t*>(Ab + a_src + k0) : zero4;
-        } else if (p.a_row_map) {
-            va = (k0 + a_k < k_len) ? *reinterpret_cast<const f32x4_t*>(
-                                          p.A + (long long)p.a_row_map[r0 + k0 + a_k] * p.lda + a_col)
-                                    : zero4;
-        } else {
-            va = (k0 + a_k < k_len) ? *reinterpret_cast<const f32x4_t*>(Ab + a_src + (long long)k0 * p.lda) : zero4;
-        }
-        if (B_KC) {
-            vb = (k0 + b_k < k_len) ? *reinterpret_cast<const f32x4_t*>(Bb + b_src + k0) : zero4;
-        } else if (WGRAD && p.b_row_map) {
-            vb = (k0 + b_k < k_len) ? *reinterpret_cast<const f32x4_t*>(
-                                          p.B + (long long)p.b_row_map[r0 + k0 + b_k] * p.ldb + b_col)
-                                    : zero4;
-        } else {
-            vb = (k0 + b_k < k_len) ? *reinterpret_cast<const f32x4_t*>(Bb + b_src + (long long)k0 * p.ldb) : zero4;
-        }
-        __syncthreads();  // previous step's reads are done
-        if (A_KC) {
-            const int m = tid >> 2;
+    f32x4_t va[NV], vb[NV];
+    auto fetch = [&](int k0) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) As[a_k + i][m] = va[i];
-        } else {
-            *reinterpret_cast<f32x4_t*>(&As[a_k][(tid & 15) * 4]) = va;
+        for (int h = 0; h < NV; ++h) {
+            const int kh = k0 + h * 16;
+            if (kh + a_k >= k_len) {
+                va[h] = zero4;
+            } else if (A_KC) {
+                va[h] = *reinterpret_cast<const f32x4_t*>(Ab + a_src + kh);
+            } else if (p.a_row_map) {
+                va[h] = *reinterpret_cast<const f32x4_t*>(p.A + (long long)p.a_row_map[r0 + kh + a_k] * p.lda + a_col);
+            } else {
+                va[h] = *reinterpret_cast<const f32x4_t*>(Ab + a_src + (long long)kh * p.lda);
+            }
+            if (kh + b_k >= k_len) {
+                vb[h] = zero4;
+            } else if (B_KC) {
+                vb[h] = *reinterpret_cast<const f32x4_t*>(Bb + b_src + kh);
+            } else if (WGRAD && p.b_row_map) {
+                vb[h] = *reinterpret_cast<const f32x4_t*>(p.B + (long long)p.b_row_map[r0 + kh + b_k] * p.ldb + b_col);
+            } else {
+                vb[h] = *reinterpret_cast<const f32x4_t*>(Bb + b_src + (long long)kh * p.ldb);
+            }
         }
-        if (B_KC) {
-            const int n = tid >> 2;
+    };
+    fetch(0);
+    int stage = 0;
+    for (int k0 = 0; k0 < k_len; k0 += BK, stage ^= 1) {
+        // (the stage written here was last read before the barrier of the step in between)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) Bs[b_k + i][n] = vb[i];
-        } else {
-            *reinterpret_cast<f32x4_t*>(&Bs[b_k][(tid & 15) * 4]) = vb;
+        for (int h = 0; h < NV; ++h) {
+            const int ka = a_k + h * 16, kb = b_k + h * 16;
+            if (A_KC) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) As[stage][ka + i][tid >> 2] = va[h][i];
+            } else {
+                *reinterpret_cast<f32x4_t*>(&As[stage][ka][(tid & 15) * 4]) = va[h];
+            }
+            if (B_KC) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) Bs[stage][kb + i][tid >> 2] = vb[h][i];
+            } else {
+                *reinterpret_cast<f32x4_t*>(&Bs[stage][kb][(tid & 15) * 4]) = vb[h];
+            }
         }
         __syncthreads();
+        if (k0 + BK < k_len) fetch(k0 + BK);
 #pragma unroll
         for (int kb = 0; kb < BK; kb += 2) {
-            const float a = As[kb + lg][wm * 32 + lj];
-            const float b = Bs[kb + lg][wn * 32 + lj];
+            const float a = As[stage][kb + lg][wm * 32 + lj];
+            const float b = Bs[stage][kb + lg][wn * 32 + lj];
             acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
         }
     }
