@@ -52,9 +52,14 @@ __device__ __forceinline__ void skinny_body(const GemmArgs& p)
 
     const int pm = blockIdx.x / p.n_ntiles;
     const int n0 = (blockIdx.x - pm * p.n_ntiles) * 16 * CPL;
-    if (pm >= min(scalar_load_i32(p.n_mtiles), p.max_mtiles)) return;
-    const int32_t* ent = reinterpret_cast<const int32_t*>(p.tile_map + pm);
-    const int e = scalar_load_i32(ent), m0 = scalar_load_i32(ent + 1), mend = scalar_load_i32(ent + 2);
+    int e = 0, m0 = pm * 16 * MT, mend = p.M;         // without a map: one expert that has all p.M rows
+    if (p.tile_map) {
+        if (pm >= min(scalar_load_i32(p.n_mtiles), p.max_mtiles)) return;
+        const int32_t* ent = reinterpret_cast<const int32_t*>(p.tile_map + pm);
+        e = scalar_load_i32(ent);
+        m0 = scalar_load_i32(ent + 1);
+        mend = scalar_load_i32(ent + 2);
+    }
 
     const int steps = p.Kd / 32;                      // (the reduction length is a multiple of 32)
     const uint32_t row_bytes = (uint32_t)p.ldb * 2u;
@@ -203,7 +208,61 @@ int launch_height(const GemmArgs& a, int bm, hipStream_t s)
     return launch_skinny<1, 8, 4, EPI, ACT>(a, m_tiles, s);
 }
 
+// ------------------------------------------------------------------ the router's linear map for few tokens
+// logits [T,E] = x [T,H] @ w [E,H]^T, both operands K-contiguous and read straight into MFMA operands.  A workgroup is a
+// 16 x 16 tile, its 16 wavefronts share the reduction (every 16th step of 32 k).  Bound by latency: the tile's
+// steps are requested all at once.
+// (The caller's rule for using it holds the measurements.)
+constexpr int kLogitWaves = 16;
+
+template <typename ET>
+__global__ void __launch_bounds__(kLogitWaves * 64)
+router_logits_kernel(const ET* __restrict__ x, const ET* __restrict__ w, ET* __restrict__ logits, int T, int E, int H)
+{
+    __shared__ sk_f32x4 red[kLogitWaves][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int l16 = lane & 15, lq = lane >> 4;
+    const int n_et = (E + 15) >> 4;
+    const int t0 = (int)(blockIdx.x / n_et) * 16, e0 = (int)(blockIdx.x % n_et) * 16;
+    // (rows past the last are copies of it; their products are not stored)
+    const ET* const xr = x + (size_t)min(t0 + l16, T - 1) * H + lq * 8;
+    const ET* const wr = w + (size_t)min(e0 + l16, E - 1) * H + lq * 8;
+    sk_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int k = wave * 32; k < H; k += kLogitWaves * 32)
+        acc = MfmaSkinny<ET>::run(*reinterpret_cast<const u32x4_t*>(wr + k), *reinterpret_cast<const u32x4_t*>(xr + k), acc);
+    red[wave][lane] = acc;
+    __syncthreads();
+    // thread (q, l, v): logit of token l and expert 4 q + v
+    if (threadIdx.x < 256) {
+        const int l = threadIdx.x & 63, v = threadIdx.x >> 6;
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < kLogitWaves; ++i) sum += red[i][l][v];
+        const int t = t0 + (l & 15), e = e0 + (l >> 4) * 4 + v;
+        if (t < T && e < E) ElemTraits<ET>::store1(logits + (size_t)t * E + e, sum);
+    }
+}
+
 }  // namespace
+
+AMOE_EXPORT int amoe_router_logits(const void* x, const void* w, void* logits, int dtype, int T, int E, int H, void* stream)
+{
+    AMOE_REQUIRE(x && w && logits, AMOE_ERR_BAD_ARG, "router_logits: null pointer");
+    AMOE_REQUIRE(T > 0 && E > 0 && H > 0, AMOE_ERR_BAD_ARG, "router_logits: sizes must be positive (T=%d E=%d H=%d)", T, E, H);
+    AMOE_REQUIRE(dtype == AMOE_BF16 || dtype == AMOE_F16, AMOE_ERR_UNSUPPORTED, "router_logits: bf16 and float16 only");
+    AMOE_REQUIRE(H % 32 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0, AMOE_ERR_UNSUPPORTED,
+                 "router_logits: H=%d must be a multiple of 32, the operands aligned to 16 bytes", H);
+    const long long grid = (long long)((T + 15) / 16) * ((E + 15) / 16);
+    AMOE_REQUIRE(grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "router_logits: grid too large");
+    if (dtype == AMOE_F16)
+        hipLaunchKernelGGL((router_logits_kernel<f16_t>), dim3((int)grid), dim3(kLogitWaves * 64), 0, (hipStream_t)stream,
+                           (const f16_t*)x, (const f16_t*)w, (f16_t*)logits, T, E, H);
+    else
+        hipLaunchKernelGGL((router_logits_kernel<bf16_t>), dim3((int)grid), dim3(kLogitWaves * 64), 0, (hipStream_t)stream,
+                           (const bf16_t*)x, (const bf16_t*)w, (bf16_t*)logits, T, E, H);
+    return amoe_check_launch("router_logits");
+}
 
 int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s)
 {
@@ -212,3 +271,28 @@ int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s)
 }
 
 int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s) { return launch_height<EPI_STORE, 0>(a, bm, s); }
+
+// out [T,H] = d_logits [T,E] @ w [E,H], the router's part of the gradient of the input: the product above with one
+// expert that has every row.
+AMOE_EXPORT int amoe_router_input_grad(const void* d_logits, const void* w, void* out, int dtype, int T, int E, int H, void* stream)
+{
+    AMOE_REQUIRE(d_logits && w && out, AMOE_ERR_BAD_ARG, "router_input_grad: null pointer");
+    AMOE_REQUIRE(T > 0 && E > 0 && H > 0, AMOE_ERR_BAD_ARG, "router_input_grad: sizes must be positive (T=%d E=%d H=%d)", T, E, H);
+    AMOE_REQUIRE(dtype == AMOE_BF16 || dtype == AMOE_F16, AMOE_ERR_UNSUPPORTED, "router_input_grad: bf16 and float16 only");
+    AMOE_REQUIRE(E % 32 == 0 && H % 8 == 0 && ((uintptr_t)d_logits | (uintptr_t)w | (uintptr_t)out) % 16 == 0, AMOE_ERR_UNSUPPORTED,
+                 "router_input_grad: E=%d must be a multiple of 32, H=%d of 8, the operands aligned to 16 bytes", E, H);
+    AMOE_REQUIRE((unsigned long long)T * E * 2ull < (1ull << 31) && (unsigned long long)E * H * 2ull < (1ull << 31), AMOE_ERR_UNSUPPORTED,
+                 "router_input_grad: operand of 2 GiB or more");
+    GemmArgs a = {};
+    a.A = (const bf16_t*)d_logits;
+    a.B = (const bf16_t*)w;
+    a.C = (bf16_t*)out;
+    a.f16 = dtype == AMOE_F16;
+    a.lda = E;
+    a.ldb = a.ldc = a.N = H;
+    a.E = 1;
+    a.Kd = E;
+    a.M = T;
+    if (T <= 16) return launch_skinny<1, 4, 8, EPI_STORE, 0>(a, 1, (hipStream_t)stream);
+    return launch_skinny<2, 8, 4, EPI_STORE, 0>(a, (T + 31) / 32, (hipStream_t)stream);
+}

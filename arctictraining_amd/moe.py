@@ -178,11 +178,51 @@ def _dense_weight_grad(a: torch.Tensor, b: torch.Tensor, tile_cfg: int = 0, tile
     return ops.dense_wgrad(a, b, _token_offsets(a.shape[0], splits, a.device), tile_cfg=tile_cfg)
 
 
+# The router's three products.  Up to this many tokens a pass is bound by the host, and a call of torch.matmul costs it
+# 19 us against 8 us of a launch of the kernels here, which take as long on the GPU (128 experts, H = 2048, 200 tokens:
+# logits 6.0 us against 5.7, input gradient 4.9 against 4.4); at 1024 tokens the library is the faster (6.5 us against
+# 9.8, 5.6 against 8.1).
+_ROUTER_KERNEL_TOKENS = 256
+
+
+def _router_kernel_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether a product of a [T, .] with the router's weight may run on the package's kernels: few tokens, both dense,
+    of one 16-bit type, on one device, aligned, and no autocast that would change a type."""
+    return (
+        a.shape[0] <= _ROUTER_KERNEL_TOKENS
+        and a.dtype in (torch.bfloat16, torch.float16)
+        and w.dtype is a.dtype
+        and a.is_contiguous()
+        and w.is_contiguous()
+        and w.get_device() == a.get_device()
+        and (a.data_ptr() | w.data_ptr()) % 16 == 0
+        and not torch.is_autocast_enabled("cuda")
+    )
+
+
+def _router_logits(x: torch.Tensor, router_gate: torch.Tensor) -> torch.Tensor:
+    """x [T,H] @ router_gate [E,H]^T (moe.py:233)."""
+    # (longer rows are more than 8 steps in a row for a wavefront of the kernel: H = 7168 14.6 us against 7.7)
+    if _router_kernel_fits(x, router_gate) and x.shape[1] == router_gate.shape[1] <= 4096 and x.shape[1] % 32 == 0:
+        return ops.router_logits(x, router_gate)
+    return torch.matmul(x, router_gate.t())
+
+
+def _router_input_grad(d_logits: torch.Tensor, router_gate: torch.Tensor) -> torch.Tensor:
+    """d_logits [T,E] @ router_gate [E,H] (autograd of moe.py:233)."""
+    E, H = router_gate.shape
+    if E % 32 == 0 and H % 8 == 0 and _router_kernel_fits(d_logits, router_gate):
+        return ops.router_input_grad(d_logits, router_gate)
+    return torch.matmul(d_logits, router_gate)
+
+
 def _router_weight_grad(d_logits: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """dW_router [E,H] = d_logits^T [E,T] @ x [T,H] (autograd of moe.py:233): skinny (E rows) and
-    deep (T), the library GEMM leaves most of the chip idle on it."""
+    deep (T), the library GEMM leaves most of the chip idle on it (128 experts, H = 2048: 4096 tokens 34 us
+    against 13; few tokens: 19 us of host time against 10).  In between, beside the experts' weight gradients on the
+    second stream, the library's is the better one (a step of 509 tokens 953 us against 962)."""
     T, E = d_logits.shape
-    if x.dtype == torch.float32 or E % 8 or T < 16 * 32:
+    if x.dtype == torch.float32 or E % 8 or _ROUTER_KERNEL_TOKENS < T < 512:
         return torch.matmul(d_logits.t(), x)
     return _dense_weight_grad(d_logits, x, tile_cfg=1, tile=128)  # 128x128 tiles
 
@@ -210,7 +250,7 @@ def _route(x, router_gate, replay, opts):
     E, K = opts["num_experts"], opts["top_k"]
     timers: PhaseTimers = opts["timers"]
     timers.start("router")
-    logits = torch.matmul(x, router_gate.t())  # plain library GEMM, moe.py:233
+    logits = _router_logits(x, router_gate)
     probs, topk_idx, scores = ops.router_topk_fwd(logits, K, opts["normalize"])
     assign = topk_idx if replay is None else _replayed(replay, E, opts)
     # the row-grouped GEMMs of a step share one tile map: the permutation plan builds it (its
@@ -276,7 +316,7 @@ def _layer_forward(x, router_gate, w_gate_up, w_down, shared, replay, opts, keep
     sizes = _layer_sizes(key, T, keep)
     if timers.wall_clock_breakdown:
         timers.start("router")
-    logits = torch.matmul(x, router_gate.t())  # plain library GEMM, moe.py:233
+    logits = _router_logits(x, router_gate)
     assign = None if replay is None else _replayed(replay, E, opts)
     y = torch.empty_like(x)
     buf = torch.empty(sizes[0] + (0 if keep else sizes[1]), dtype=torch.uint8, device=x.device)
@@ -391,7 +431,7 @@ class _ExpertLayerFn(torch.autograd.Function):
         dx = dx_router = None
         if need[0]:
             dx = torch.empty_like(x)
-            dx_router = torch.matmul(d_logits, router_gate)
+            dx_router = _router_input_grad(d_logits, router_gate)
         if dx is not None or side is not None:
             _lib.check(
                 lib.amoe_layer_bwd_input(
@@ -504,7 +544,7 @@ class _UngatedExpertLayerFn(torch.autograd.Function):
         dx = None
         if ctx.needs_input_grad[0]:
             d_xp = ops.grouped_gemm_nt(d_inter, w_up, offsets, tile_cfg=cfg, workspace=ws, map_ready=True)
-            dx_dense = torch.matmul(d_logits, router_gate)
+            dx_dense = _router_input_grad(d_logits, router_gate)
             if ctx.shared:
                 dx_dense.addmm_(d_pre, sh_out_gate.t())
                 dx_dense.addmm_(d_sh_inter, sh_up.t())

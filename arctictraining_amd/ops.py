@@ -63,6 +63,34 @@ def router_topk_fwd(logits: torch.Tensor, top_k: int, normalize: bool):
     return probs, idx, scores
 
 
+def router_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x [T,H] @ w [E,H]^T in bf16 or float16, H a multiple of 32."""
+    _chk(x, "x")
+    _chk(w, "w", x.dtype)
+    (T, H), E = x.shape, w.shape[0]
+    if w.shape[1] != H:
+        raise RuntimeError(f"w must be [E, {H}], got {list(w.shape)}")
+    logits = torch.empty((T, E), dtype=x.dtype, device=x.device)
+    rc = _lib.load().amoe_router_logits(x.data_ptr(), w.data_ptr(), logits.data_ptr(), _dtype_code(x), T, E, H, _stream())
+    _lib.check(rc, "amoe_router_logits")
+    return logits
+
+
+def router_input_grad(d_logits: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """d_logits [T,E] @ w [E,H] in bf16 or float16, E a multiple of 32 and H of 8."""
+    _chk(d_logits, "d_logits")
+    _chk(w, "w", d_logits.dtype)
+    (T, E), H = d_logits.shape, w.shape[1]
+    if w.shape[0] != E:
+        raise RuntimeError(f"w must be [{E}, H], got {list(w.shape)}")
+    out = torch.empty((T, H), dtype=w.dtype, device=w.device)
+    rc = _lib.load().amoe_router_input_grad(
+        d_logits.data_ptr(), w.data_ptr(), out.data_ptr(), _dtype_code(w), T, E, H, _stream()
+    )
+    _lib.check(rc, "amoe_router_input_grad")
+    return out
+
+
 def router_bwd(d_scores, probs, topk_idx, counts, out_dtype, normalize: bool, lb_coeff: float) -> torch.Tensor:
     lib = _lib.load()
     _chk(d_scores, "d_scores", torch.float32)

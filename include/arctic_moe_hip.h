@@ -65,6 +65,17 @@ int amoe_router_topk_fwd(const void* logits, int dtype, int T, int E, int K, int
                          int32_t* topk_idx, float* scores, void* stream);
 
 /*
+ * The router's linear map for few tokens: logits [T,E] = x [T,H] @ w [E,H]^T (moe.py:233), bf16 or float16, sums in
+ * float32.  H has to be a multiple of 32 and the operands aligned to 16 bytes (AMOE_ERR_UNSUPPORTED otherwise).
+ */
+int amoe_router_logits(const void* x, const void* w, void* logits, int dtype, int T, int E, int H, void* stream);
+
+/*
+ * Its input gradient for few tokens: out [T,H] = d_logits [T,E] @ w [E,H], bf16 or float16; E a multiple of 32, H of 8.
+ */
+int amoe_router_input_grad(const void* d_logits, const void* w, void* out, int dtype, int T, int E, int H, void* stream);
+
+/*
  * Router backward.  Replaces top_k_gating_bwd (top_k_gating.h:24-28,
  * top_k_gating_cuda.cu:243-294) plus the load-balance hook moe.py:393-406.
  *   d_scores [T,K] f32, probs [T,E] f32, topk_idx [T,K], counts [E] i32 (routed rows per
