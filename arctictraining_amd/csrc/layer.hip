@@ -9,6 +9,10 @@
 #include <mutex>
 #include <vector>
 
+int amoe_launch_route(const void* logits, int logits_dtype, int T, int K, int E, int normalize, float* probs, int32_t* topk_idx,
+                      float* scores, int32_t* counts, int32_t* offsets, int32_t* token_of, int32_t* slot_of, int32_t* row_of,
+                      float* scores_perm, void* workspace, size_t workspace_bytes, void* gemm_workspace,
+                      size_t gemm_workspace_bytes, int dtype, int tile_cfg, hipStream_t s);
 int amoe_launch_score_grad(const float* partials, int n_parts, const float* extra, const int32_t* row_of, float* d_scores,
                            int n_slots, bool accumulate, hipStream_t s);
 int amoe_launch_shared_gate(const void* x, const void* w, float* sig, int dtype, int T, int H, hipStream_t s);
@@ -219,11 +223,17 @@ AMOE_EXPORT int amoe_layer_fwd(const int32_t* config, int T, const void* x, cons
     const FwdScratch f = cut_fwd(c, T, scratch);
     const int R = T * c.K, ready = c.tile_cfg | AMOE_TILE_MAP_READY;
     if (stages & AMOE_STAGE_ROUTE) {
-        AMOE_TRY(amoe_router_topk_fwd(logits, logits_dtype, T, c.E, c.K, c.normalize, s.probs, s.topk_idx, s.scores, stream));
         // the row-grouped products share one tile map: the plan builds it, backward uses it again
-        AMOE_TRY(amoe_permute_plan_tiled(assign ? assign : s.topk_idx, s.scores, T, c.K, c.E, s.counts, s.offsets, s.token_of,
-                                         s.slot_of, s.row_of, s.scores_perm, f.plan_ws, f.plan_ws_bytes, s.gemm_ws,
-                                         s.gemm_ws_bytes, c.dtype, c.tile_cfg, stream));
+        if (assign) {
+            AMOE_TRY(amoe_router_topk_fwd(logits, logits_dtype, T, c.E, c.K, c.normalize, s.probs, s.topk_idx, s.scores, stream));
+            AMOE_TRY(amoe_permute_plan_tiled(assign, s.scores, T, c.K, c.E, s.counts, s.offsets, s.token_of, s.slot_of, s.row_of,
+                                             s.scores_perm, f.plan_ws, f.plan_ws_bytes, s.gemm_ws, s.gemm_ws_bytes, c.dtype,
+                                             c.tile_cfg, stream));
+        } else {
+            AMOE_TRY(amoe_launch_route(logits, logits_dtype, T, c.K, c.E, c.normalize, s.probs, s.topk_idx, s.scores, s.counts,
+                                       s.offsets, s.token_of, s.slot_of, s.row_of, s.scores_perm, f.plan_ws, f.plan_ws_bytes,
+                                       s.gemm_ws, s.gemm_ws_bytes, c.dtype, c.tile_cfg, (hipStream_t)stream));
+        }
     }
     if (stages & AMOE_STAGE_EXPERTS) {
         // the rows x[token_of] are gathered inside the product's loads; a row's score multiplies its intermediate

@@ -50,3 +50,29 @@ def test_refused(gpu_device):
         assert moe._router_logits(x, odd.clone()).dtype == torch.float16
     with pytest.raises(RuntimeError):
         moe._router_logits(x, odd.float())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("E,K", [(5, 1), (64, 8), (65, 16), (128, 8), (300, 3), (512, 16)])
+@pytest.mark.parametrize("T", [1, 5, 16, 17])
+def test_route_in_one_launch(gpu_device, dtype, E, K, T):
+    """The layer's routing of a few tokens equals the stages on their own (whole numbers exactly)."""
+    from arctictraining_amd import ArcticMoE, MoEConfig, ops
+
+    if K > E:
+        pytest.skip("top_k above the number of experts")
+    print("route", dtype, E, K, T, flush=True)
+    torch.manual_seed(E + T)
+    with gpu_device:
+        layer = ArcticMoE(MoEConfig(act_fn=F.silu, input_dtype=dtype, intermediate_dim=32, model_dim=32, normalize_topk_scores=T % 2 == 0,
+                                    num_experts=E, top_k=K))
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, 0.1)
+        layer.capture = got = {}
+        layer(torch.randn(T, 32, device=gpu_device).to(dtype))
+        probs, idx, scores = ops.router_topk_fwd(got["logits"], K, T % 2 == 0)
+        counts, offsets, token_of, slot_of, row_of, _ = ops.permute_plan(idx, E, scores)
+    for name, want in dict(probs=probs, topk_idx=idx, scores=scores, counts=counts, offsets=offsets, token_of=token_of, slot_of=slot_of,
+                           row_of=row_of).items():
+        assert torch.equal(got[name], want), name
