@@ -178,18 +178,19 @@ def _dense_weight_grad(a: torch.Tensor, b: torch.Tensor, tile_cfg: int = 0, tile
     return ops.dense_wgrad(a, b, _token_offsets(a.shape[0], splits, a.device), tile_cfg=tile_cfg)
 
 
-# The router's three products.  Up to this many tokens a pass is bound by the host, and a call of torch.matmul costs it
-# 19 us against 8 us of a launch of the kernels here, which take as long on the GPU (128 experts, H = 2048, 200 tokens:
-# logits 6.0 us against 5.7, input gradient 4.9 against 4.4); at 1024 tokens the library is the faster (6.5 us against
-# 9.8, 5.6 against 8.1).
-_ROUTER_KERNEL_TOKENS = 256
+# The router's products on the package's kernels, up to this many (16 x 16 tiles of logits) * H: a pass with so few tokens
+# (256 at 128 experts and H = 2048) is usually bound by the host, and a call of torch.matmul costs it 19 us against 8 us of
+# a launch of the kernels, which take about as long on the GPU (logits, then input gradient, against the library: 128
+# experts, H = 2048, 200 tokens 6.0 / 5.7 us, 4.9 / 4.4, at 1024 tokens 9.8 / 6.5, 8.1 / 5.6; 64 experts, H = 512, 2048
+# tokens 4.4 / 5.7, 5.2 / 4.3).
+_ROUTER_KERNEL_WORK = 1 << 18
 
 
 def _router_kernel_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether a product of a [T, .] with the router's weight may run on the package's kernels: few tokens, both dense,
-    of one 16-bit type, on one device, aligned, and no autocast that would change a type."""
+    """Whether a product of a [T, .] with the router's weight w [E,H] may run on the package's kernels: few tokens, both
+    dense, of one 16-bit type, on one device, aligned, and no autocast that would change a type."""
     return (
-        a.shape[0] <= _ROUTER_KERNEL_TOKENS
+        -(-a.shape[0] // 16) * -(-w.shape[0] // 16) * w.shape[1] <= _ROUTER_KERNEL_WORK
         and a.dtype in (torch.bfloat16, torch.float16)
         and w.dtype is a.dtype
         and a.is_contiguous()
@@ -222,7 +223,7 @@ def _router_weight_grad(d_logits: torch.Tensor, x: torch.Tensor) -> torch.Tensor
     against 13; few tokens: 19 us of host time against 10).  In between, beside the experts' weight gradients on the
     second stream, the library's is the better one (a step of 509 tokens 953 us against 962)."""
     T, E = d_logits.shape
-    if x.dtype == torch.float32 or E % 8 or _ROUTER_KERNEL_TOKENS < T < 512:
+    if x.dtype == torch.float32 or E % 8 or 256 < T < 512:
         return torch.matmul(d_logits.t(), x)
     return _dense_weight_grad(d_logits, x, tile_cfg=1, tile=128)  # 128x128 tiles
 
