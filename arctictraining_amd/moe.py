@@ -367,7 +367,7 @@ class _ExpertLayerFn(torch.autograd.Function):
         y, saved, key = _layer_forward(
             x, router_gate, w_gate_up, w_down, (sh_gate_up, sh_down, sh_out_gate), replay, opts, keep=True
         )
-        ctx.opts, ctx.key = opts, key
+        ctx.opts, ctx.key, ctx.device = opts, key, x.device
         ctx.save_for_backward(x, router_gate, w_gate_up, w_down, sh_gate_up, sh_down, sh_out_gate, saved)
         ctx.set_materialize_grads(False)  # no zero-filled gradient for an output the loss does not use
         if not opts["want_scores"]:
@@ -378,10 +378,25 @@ class _ExpertLayerFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy, ds_perm=None):
-        x, router_gate, w_gate_up, w_down, sh_gate_up, sh_down, sh_out_gate, saved = ctx.saved_tensors
-        opts, key = ctx.opts, ctx.key
         if dy is None and ds_perm is None:  # neither output took part in the loss
             return (None,) * 9
+        # The two expert weight gradients run on a second stream beside the chain of data gradients.  It
+        # starts on them behind everything the main stream has queued up to their operands, and the main
+        # stream waits for it at the end, so the tensors either stream uses outlive the kernels that use them.
+        overlap = ctx.opts["overlap_weight_grads"] and (ctx.needs_input_grad[2] or ctx.needs_input_grad[3])
+        side = _side_stream(ctx.device) if overlap else None
+        try:
+            return _ExpertLayerFn._backward(ctx, dy, ds_perm, None if side is None else side.cuda_stream)
+        except BaseException:
+            # (memory may run out between the fork and the join: what is freed here is used again on the main stream)
+            if side is not None:
+                torch.cuda.current_stream(side.device).wait_stream(side)
+            raise
+
+    @staticmethod
+    def _backward(ctx, dy, ds_perm, side):
+        x, router_gate, w_gate_up, w_down, sh_gate_up, sh_down, sh_out_gate, saved = ctx.saved_tensors
+        opts, key = ctx.opts, ctx.key
         (T, H), (E, K, _, I) = x.shape, key[:4]
         dy = torch.zeros_like(x) if dy is None else dy.contiguous()
         ops._chk(dy, "dy", x.dtype)
@@ -393,10 +408,6 @@ class _ExpertLayerFn(torch.autograd.Function):
         d_logits = torch.empty((T, E), dtype=x.dtype, device=x.device)
         if ds_perm is not None:
             ds_perm = ds_perm.float().contiguous()
-        # The two expert weight gradients run on a second stream beside the chain of data gradients.  It
-        # starts on them behind everything the main stream has queued up to their operands, and the main
-        # stream waits for it at the end, so the tensors either stream uses outlive the kernels that use them.
-        side = _side_stream(x.device).cuda_stream if opts["overlap_weight_grads"] and (need[2] or need[3]) else None
         _lib.check(
             lib.amoe_layer_bwd(
                 config, T, x.data_ptr(), dy.data_ptr(), w_down.data_ptr(), saved.data_ptr(), scratch.data_ptr(), ops._ptr(ds_perm),

@@ -52,3 +52,33 @@ def test_forward_alone_equals_forward_for_backward(gpu_device, dtype, shared, T)
             assert (got - want).norm() <= (2e-2 if dtype == torch.bfloat16 else 1e-5) * (want.norm() + y0.float().norm())
     assert torch.equal(y, y0) and torch.equal(scores, scores0)
     assert y.requires_grad and not y0.requires_grad
+
+
+def test_failure_in_backward_joins_the_second_stream(gpu_device, monkeypatch):
+    """An error between the fork and the join of the second stream: the main stream still waits for it."""
+    from arctictraining_amd import ArcticMoE, MoEConfig, moe
+
+    with gpu_device:
+        layer = ArcticMoE(MoEConfig(act_fn=F.silu, input_dtype=torch.bfloat16, intermediate_dim=32, model_dim=64,
+                                    normalize_topk_scores=True, num_experts=4, top_k=2))
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, 0.1)
+    x = torch.randn(8, 64, device=gpu_device).bfloat16().requires_grad_(True)
+    waited = []
+    wait = torch.cuda.Stream.wait_stream
+
+    def spy(self, other):
+        waited.append(other.cuda_stream)
+        return wait(self, other)
+
+    def fail(*a):
+        raise RuntimeError("planted on the host")
+
+    y = layer(x)
+    monkeypatch.setattr(torch.cuda.Stream, "wait_stream", spy)
+    monkeypatch.setattr(moe, "_router_input_grad", fail)
+    with pytest.raises(RuntimeError, match="planted on the host"):
+        y.sum().backward()
+    assert moe._side_stream(x.device).cuda_stream in waited
+    torch.cuda.synchronize()
