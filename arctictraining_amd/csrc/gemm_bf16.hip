@@ -1406,6 +1406,12 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
     a.n_mt = 0;
     long long grid = 0;
     a.max_mtiles = max_mtiles;
+    // a map that is there already may have been built for another bound of the rows, and then with tiles of another
+    // height: the workspace limits their number
+    if (map_ready && tile_cfg == 0) {
+        const size_t fit = (workspace_bytes - 16) / sizeof(int4);
+        a.max_mtiles = fit < (1u << 20) ? (int)fit : 1 << 20;
+    }
     if (bm < tc.bm) {
         if constexpr (EPI == EPI_GATED) return amoe_skinny_gateup_act(a, ACT, bm, s);
         else if constexpr (EPI == EPI_STORE && !B_KC) return amoe_skinny_nn(a, bm, s);

@@ -42,24 +42,12 @@ struct MfmaSkinny<f16_t> {
 };
 
 template <int MT, int CPL, int NW, int EPI, int ACT, typename ET>
-__device__ __forceinline__ void skinny_body(const GemmArgs& p)
+__device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[NW][CPL * 64], int e, int m0, int mend, int n0)
 {
     constexpr int W = CPL / 2, H = CPL / 4;           // dwords of a lane's row, groups of four columns
-    __shared__ sk_f32x4 red[NW][4 * H * 64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, lq = lane >> 4;
-
-    const int pm = blockIdx.x / p.n_ntiles;
-    const int n0 = (blockIdx.x - pm * p.n_ntiles) * 16 * CPL;
-    int e = 0, m0 = pm * 16 * MT, mend = p.M;         // without a map: one expert that has all p.M rows
-    if (p.tile_map) {
-        if (pm >= min(scalar_load_i32(p.n_mtiles), p.max_mtiles)) return;
-        const int32_t* ent = reinterpret_cast<const int32_t*>(p.tile_map + pm);
-        e = scalar_load_i32(ent);
-        m0 = scalar_load_i32(ent + 1);
-        mend = scalar_load_i32(ent + 2);
-    }
 
     const int steps = p.Kd / 32;                      // (the reduction length is a multiple of 32)
     const uint32_t row_bytes = (uint32_t)p.ldb * 2u;
@@ -166,6 +154,30 @@ __device__ __forceinline__ void skinny_body(const GemmArgs& p)
     }
 }
 
+// A map's tile is 16 * MT rows where the launch's own rule built it; the taller tiles of a map that was built for another
+// bound of the rows are walked in parts.
+template <int MT, int CPL, int NW, int EPI, int ACT, typename ET>
+__device__ __forceinline__ void skinny_body(const GemmArgs& p)
+{
+    __shared__ sk_f32x4 red[NW][CPL * 64];
+    const int pm = blockIdx.x / p.n_ntiles;
+    const int n0 = (blockIdx.x - pm * p.n_ntiles) * 16 * CPL;
+    int e = 0, m0 = pm * 16 * MT, mend = min(m0 + 16 * MT, p.M);   // without a map: one expert that has all p.M rows
+    if (p.tile_map) {
+        if (pm >= min(scalar_load_i32(p.n_mtiles), p.max_mtiles)) return;
+        const int32_t* ent = reinterpret_cast<const int32_t*>(p.tile_map + pm);
+        e = scalar_load_i32(ent);
+        m0 = scalar_load_i32(ent + 1);
+        mend = scalar_load_i32(ent + 2);
+    }
+    skinny_tile<MT, CPL, NW, EPI, ACT, ET>(p, red, e, m0, mend, n0);
+#pragma unroll 1
+    for (m0 += 16 * MT; m0 < mend; m0 += 16 * MT) {
+        __syncthreads();   // (the sums are read before the next part's are written)
+        skinny_tile<MT, CPL, NW, EPI, ACT, ET>(p, red, e, m0, mend, n0);
+    }
+}
+
 // (at least 4 wavefronts per SIMD with 16 rows, 3 with 32)
 template <int MT, int CPL, int NW, int EPI, int ACT>
 __global__ void __launch_bounds__(NW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_bf16_kernel(GemmArgs p)
@@ -196,8 +208,8 @@ template <int EPI, int ACT>
 int launch_height(const GemmArgs& a, int bm, hipStream_t s)
 {
     const int R = a.M;
-    // every expert with a row has at most rows / bm + 1 tiles
-    int m_tiles = R / bm + (a.E < R ? a.E : R);
+    // every expert with a row has at most rows / 16 + 1 tiles, whatever rule built the map
+    int m_tiles = R / 16 + (a.E < R ? a.E : R);
     if (m_tiles > R) m_tiles = R;
     if (m_tiles > a.max_mtiles) m_tiles = a.max_mtiles;
     AMOE_REQUIRE(bm == 16 || bm == 32, AMOE_ERR_UNSUPPORTED, "grouped_gemm: no kernel for tiles of %d rows", bm);

@@ -59,3 +59,32 @@ def test_few_rows(gpu_device, dtype, kind, Kd, N):
         check(inter, scale[:, None] * gu[:, 1::2].float() * fn(gu[:, 0::2].float()))
         only = ops.grouped_gemm_gateup_act_fwd(src, w, offs, act, a_row_map=rows, row_scale=scale, want_gate_up=False)
         assert only[0] is None and torch.equal(only[1], inter)
+
+
+@pytest.mark.parametrize("plan_rows,call_rows", [(4, 8), (4, 40), (8, 4), (40, 4), (40, 8)])
+def test_map_of_another_bound(gpu_device, plan_rows, call_rows):
+    """A tile map built for one bound of the rows serves a product that states another one: the same expert offsets,
+    the rows past the last expert's unused."""
+    from arctictraining_amd import ops
+
+    E, Kd, N = 24, 96, 264
+    bound = [plan_rows * E, call_rows * E]
+    counts = [(e * 5) % 8 if min(bound) > 4 * E else (e * 5) % 5 for e in range(E)]
+    counts[3] += min(bound) - sum(counts)
+    print("map of another bound", plan_rows, call_rows, counts, flush=True)
+    assert min(counts) >= 0
+    g = torch.Generator(device=gpu_device).manual_seed(plan_rows)
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(gpu_device)
+    x = torch.randn(max(bound), Kd, device=gpu_device, generator=g).bfloat16()
+    w = (torch.randn(E, Kd, N, device=gpu_device, generator=g) * 0.05).bfloat16()
+    ws = ops.gemm_workspace(64 * E, E, gpu_device)   # (large enough for both)
+    ops.grouped_gemm_nn(x[: bound[0]].contiguous(), w, offs, workspace=ws)
+    a = x[: bound[1]].contiguous()
+    n = sum(counts)
+    ref = torch.cat([p.float() @ w[e].float() for e, p in enumerate(a[:n].split(counts))])
+    for got in (
+        ops.grouped_gemm_nn(a, w, offs, workspace=ws, map_ready=True)[:n],
+        ops.grouped_gemm_nt(a, w.transpose(1, 2).contiguous(), offs, workspace=ws, map_ready=True)[:n],
+        ops.grouped_gemm_gateup_act_fwd(a, w, offs, workspace=ws, map_ready=True)[0][:n],
+    ):
+        assert (got.float() - ref).norm() <= 1e-2 * ref.norm()
