@@ -203,8 +203,9 @@ def _router_kernel_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 def _router_logits(x: torch.Tensor, router_gate: torch.Tensor) -> torch.Tensor:
     """x [T,H] @ router_gate [E,H]^T (moe.py:233)."""
-    # (longer rows are more than 8 steps in a row for a wavefront of the kernel: H = 7168 14.6 us against 7.7)
-    if _router_kernel_fits(x, router_gate) and x.shape[1] == router_gate.shape[1] <= 4096 and x.shape[1] % 32 == 0:
+    # (longer rows are more than 12 steps in a row for a wavefront of the kernel: 64 tokens, H = 7168 11.8 us against 7.5,
+    # H = 5728 7.5 against 13.0)
+    if _router_kernel_fits(x, router_gate) and x.shape[1] == router_gate.shape[1] <= 6144 and x.shape[1] % 32 == 0:
         return ops.router_logits(x, router_gate)
     return torch.matmul(x, router_gate.t())
 
