@@ -229,8 +229,12 @@ def _router_weight_grad(d_logits: torch.Tensor, x: torch.Tensor) -> torch.Tensor
     return _dense_weight_grad(d_logits, x, tile_cfg=1, tile=128)  # 128x128 tiles
 
 
-def _replayed(replay, E: int, opts) -> torch.Tensor:
-    """The replayed assignments as int32."""
+def _replayed(replay, T: int, opts) -> torch.Tensor:
+    """The replayed assignments as int32 [T,K] on the current device: the kernels read them at that shape."""
+    E, K = opts["num_experts"], opts["top_k"]
+    if tuple(replay.shape) != (T, K):
+        raise RuntimeError(f"routing_replay_assignments must be [{T}, {K}] (tokens, top_k), got {list(replay.shape)}")
+    ops._chk(replay, "routing_replay_assignments", contiguous=False)
     assign = replay.to(torch.int32).contiguous()
     if opts.get("check_replay", True) and not torch.cuda.is_current_stream_capturing():
         # The reference's one_hot(..., num_classes=E) raises on an expert id outside [0, E)
@@ -254,7 +258,7 @@ def _route(x, router_gate, replay, opts):
     timers.start("router")
     logits = _router_logits(x, router_gate)
     probs, topk_idx, scores = ops.router_topk_fwd(logits, K, opts["normalize"])
-    assign = topk_idx if replay is None else _replayed(replay, E, opts)
+    assign = topk_idx if replay is None else _replayed(replay, T, opts)
     # the row-grouped GEMMs of a step share one tile map: the permutation plan builds it (its
     # scan kernel holds the offsets), the workspace is kept for backward
     ws = ops.gemm_workspace(T * K, E, x.device)
@@ -319,7 +323,7 @@ def _layer_forward(x, router_gate, w_gate_up, w_down, shared, replay, opts, keep
     if timers.wall_clock_breakdown:
         timers.start("router")
     logits = _router_logits(x, router_gate)
-    assign = None if replay is None else _replayed(replay, E, opts)
+    assign = None if replay is None else _replayed(replay, T, opts)
     y = torch.empty_like(x)
     buf = torch.empty(sizes[0] + (0 if keep else sizes[1]), dtype=torch.uint8, device=x.device)
     base = buf.data_ptr()

@@ -1,0 +1,51 @@
+"""What the layer refuses before an address reaches the library (the kernels trust the shapes they are told)."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from arctictraining_amd import ArcticMoE, MoEConfig, _lib, moe, ops
+
+T, H, E, K = 8, 32, 4, 2
+
+
+class _Library:
+    """Stands where the native library does: every entry point succeeds and notes that it was reached."""
+
+    def __init__(self):
+        self.reached = []
+
+    def __getattr__(self, name):
+        return lambda *a: self.reached.append(name) or 0
+
+
+@pytest.fixture
+def on_host(monkeypatch):
+    """The layer on CPU tensors: its input and the logits pass for GPU tensors, the library is a stub."""
+    lib = _Library()
+    check = ops._chk
+    monkeypatch.setattr(ops, "_chk", lambda t, name, *a, **k: t if name in ("x", "logits") else check(t, name, *a, **k))
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(_lib, "load", lambda: lib)
+    monkeypatch.setattr(moe, "_layer_sizes", lambda *a: (4096,) * 13)
+    return lib
+
+
+def _layer(gated=True, **options):
+    layer = ArcticMoE(MoEConfig(act_fn=F.silu, input_dtype=torch.float32, intermediate_dim=32, model_dim=H, normalize_topk_scores=True,
+                                num_experts=E, top_k=K, is_gated=gated, **options))
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.zero_()
+    return layer
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("shape", [(T, K), (T - 1, K), (T, K - 1), (T, K + 1), (1, T, K), (T * K,)])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_replayed_assignments(on_host, gated, shape, dtype):
+    """A tensor in host memory and one of another shape than [tokens, top_k] end in an error, checked ids or not."""
+    layer = _layer(gated, enable_routing_replay=True)
+    for layer.check_replay in (True, False):
+        with torch.no_grad(), pytest.raises(RuntimeError, match="routing_replay_assignments"):
+            layer(torch.zeros(T, H), torch.zeros(shape, dtype=dtype))
+    assert "amoe_layer_fwd" not in on_host.reached
