@@ -210,6 +210,24 @@ def _router_logits(x: torch.Tensor, router_gate: torch.Tensor) -> torch.Tensor:
     return torch.matmul(x, router_gate.t())
 
 
+def _layer_logits(x: torch.Tensor, router_gate: torch.Tensor, opts) -> torch.Tensor:
+    """_router_logits of a layer with E experts: at most E columns, one for each row of router_gate."""
+    logits, E = _router_logits(x, router_gate), opts["num_experts"]
+    if logits.shape[1] > E:   # (their counts, weights and gradients do not exist)
+        raise RuntimeError(f"router_gate must have one row for each of at most {E} experts, got {list(router_gate.shape)}")
+    return logits
+
+
+def _padded_logits(logits: torch.Tensor, opts) -> torch.Tensor:
+    """What the native layer reads, [T,E]: an expert that the router leaves out has a probability of 0."""
+    E, K = opts["num_experts"], opts["top_k"]
+    if logits.shape[1] == E:
+        return logits
+    if logits.shape[1] < K:
+        raise RuntimeError(f"router_gate must have at least top_k = {K} rows, got {logits.shape[1]}")
+    return F.pad(logits, (0, E - logits.shape[1]), value=float("-inf"))
+
+
 def _router_input_grad(d_logits: torch.Tensor, router_gate: torch.Tensor) -> torch.Tensor:
     """d_logits [T,E] @ router_gate [E,H] (autograd of moe.py:233)."""
     E, H = router_gate.shape
@@ -256,7 +274,7 @@ def _route(x, router_gate, replay, opts):
     E, K = opts["num_experts"], opts["top_k"]
     timers: PhaseTimers = opts["timers"]
     timers.start("router")
-    logits = _router_logits(x, router_gate)
+    logits = _layer_logits(x, router_gate, opts)
     probs, topk_idx, scores = ops.router_topk_fwd(logits, K, opts["normalize"])
     assign = topk_idx if replay is None else _replayed(replay, T, opts)
     # the row-grouped GEMMs of a step share one tile map: the permutation plan builds it (its
@@ -322,7 +340,8 @@ def _layer_forward(x, router_gate, w_gate_up, w_down, shared, replay, opts, keep
     sizes = _layer_sizes(key, T, keep)
     if timers.wall_clock_breakdown:
         timers.start("router")
-    logits = _router_logits(x, router_gate)
+    routed = _layer_logits(x, router_gate, opts)
+    logits = ops._chk(_padded_logits(routed, opts), "logits")
     assign = None if replay is None else _replayed(replay, T, opts)
     y = torch.empty_like(x)
     buf = torch.empty(sizes[0] + (0 if keep else sizes[1]), dtype=torch.uint8, device=x.device)
@@ -352,7 +371,7 @@ def _layer_forward(x, router_gate, w_gate_up, w_down, shared, replay, opts, keep
             timers.stop(name)
     cap = opts.get("capture")
     if cap is not None:
-        cap.update(logits=logits, **{n: _saved_view(buf, n, key, T).clone() for n in _SAVED_FIELDS if n != "scores_perm"})
+        cap.update(logits=routed, **{n: _saved_view(buf, n, key, T).clone() for n in _SAVED_FIELDS if n != "scores_perm"})
     return y, buf, key
 
 
@@ -420,6 +439,8 @@ class _ExpertLayerFn(torch.autograd.Function):
             ),
             "amoe_layer_bwd",
         )
+        if router_gate.shape[0] != E:
+            d_logits = d_logits[:, : router_gate.shape[0]].contiguous()
         d_router_gate = _router_weight_grad(d_logits, x) if need[1] else None
         cap = opts.get("capture")
         if cap is not None:

@@ -82,3 +82,34 @@ def test_failure_in_backward_joins_the_second_stream(gpu_device, monkeypatch):
         y.sum().backward()
     assert moe._side_stream(x.device).cuda_stream in waited
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("T", [3, 70])
+def test_router_of_fewer_experts(gpu_device, gated, T):
+    """A router_gate with fewer rows than the layer has experts: the layer of the first experts alone."""
+    from arctictraining_amd import ArcticMoE, MoEConfig
+
+    print("router of fewer experts", gated, T, flush=True)
+    torch.manual_seed(T)
+
+    def layer(E):
+        return ArcticMoE(MoEConfig(act_fn=F.silu, input_dtype=torch.bfloat16, intermediate_dim=32, model_dim=64, normalize_topk_scores=True,
+                                   num_experts=E, top_k=2, is_gated=gated, loss_coeff=0.5)).to(gpu_device)
+
+    few, wide = layer(5), layer(8)
+    with torch.no_grad():
+        for n, p in few.named_parameters():
+            p.normal_(0.0, 0.1)
+            getattr(wide, n).normal_(0.0, 0.1)[:5].copy_(p)
+    wide.router_gate = torch.nn.Parameter(few.router_gate.detach().clone())
+    x, dy = torch.randn(2, T, 64, device=gpu_device).bfloat16()
+    out = []
+    for m in (few, wide):
+        xg = x.clone().requires_grad_(True)
+        y = m(xg)
+        y.backward(dy)
+        out.append((y.detach(), xg.grad, *(p.grad[:5] for p in m.parameters())))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+    for p in (wide.expert_gate_up, wide.expert_down):
+        assert bool((p.grad[5:] == 0).all())

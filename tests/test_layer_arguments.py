@@ -1,4 +1,6 @@
 """What the layer refuses before an address reaches the library (the kernels trust the shapes they are told)."""
+import ctypes
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -49,3 +51,31 @@ def test_replayed_assignments(on_host, gated, shape, dtype):
         with torch.no_grad(), pytest.raises(RuntimeError, match="routing_replay_assignments"):
             layer(torch.zeros(T, H), torch.zeros(shape, dtype=dtype))
     assert "amoe_layer_fwd" not in on_host.reached
+
+
+@pytest.mark.parametrize("gated", [True, False])
+def test_router_of_more_experts_than_the_layer_has(on_host, gated):
+    """Its logits would choose experts that have no weights."""
+    layer = _layer(gated)
+    layer.router_gate = torch.nn.Parameter(torch.zeros(E + 1, H))
+    with torch.no_grad(), pytest.raises(RuntimeError, match="router_gate"):
+        layer(torch.zeros(T, H))
+    assert not on_host.reached
+
+
+def test_router_of_fewer_experts(on_host, monkeypatch):
+    """The kernels read logits [tokens, experts]: the experts that the router leaves out get -inf, a probability of 0."""
+    layer = _layer()
+    layer.router_gate = torch.nn.Parameter(torch.ones(E - 1, H))
+    seen = {}
+
+    def forward(config, tokens, x, logits, *rest):
+        seen["logits"] = torch.frombuffer((ctypes.c_float * (tokens * E)).from_address(logits), dtype=torch.float32).clone()
+        return 0
+
+    monkeypatch.setattr(on_host, "amoe_layer_fwd", forward, raising=False)
+    with torch.no_grad():
+        layer(torch.ones(T, H))
+    want = torch.full((T, E), float("-inf"))
+    want[:, : E - 1] = H
+    assert torch.equal(seen["logits"].view(T, E), want)
