@@ -391,7 +391,7 @@ class _ExpertLayerFn(torch.autograd.Function):
         y, saved, key = _layer_forward(
             x, router_gate, w_gate_up, w_down, (sh_gate_up, sh_down, sh_out_gate), replay, opts, keep=True
         )
-        ctx.opts, ctx.key, ctx.device = opts, key, x.device
+        ctx.opts, ctx.key, ctx.device, ctx.tokens = opts, key, x.device, x.shape[0]
         ctx.save_for_backward(x, router_gate, w_gate_up, w_down, sh_gate_up, sh_down, sh_out_gate, saved)
         ctx.set_materialize_grads(False)  # no zero-filled gradient for an output the loss does not use
         if not opts["want_scores"]:
@@ -420,12 +420,24 @@ class _ExpertLayerFn(torch.autograd.Function):
     @staticmethod
     def _backward(ctx, dy, ds_perm, side):
         x, router_gate, w_gate_up, w_down, sh_gate_up, sh_down, sh_out_gate, saved = ctx.saved_tensors
-        opts, key = ctx.opts, ctx.key
-        (T, H), (E, K, _, I) = x.shape, key[:4]
+        opts, key, T = ctx.opts, ctx.key, ctx.tokens
+        E, K, H, I = key[:4]
+        # (what a saved-tensor hook returned, read below at the shapes of the forward pass)
+        if ops._dtype_code(ops._chk(x, "x")) != key[5] or x.shape != (T, H):
+            raise RuntimeError(f"saved x must come back as the forward pass had it, got {x.dtype} {list(x.shape)}")
+        _check_operand(w_gate_up, "saved w_gate_up", x, (E, H, 2 * I))
+        _check_operand(w_down, "saved w_down", x, (E, I, H))
+        if sh_gate_up is not None:
+            _check_operand(sh_gate_up, "saved shared_expert_gate_up", x, (H, 2 * I))
+            _check_operand(sh_down, "saved shared_expert_down", x, (I, H))
+            _check_operand(sh_out_gate, "saved shared_expert_output_gate", x, (H, 1))
+        ops._chk(saved, "saved routing and activations", torch.uint8)
+        if saved.numel() != _layer_sizes(key, T, True)[0]:
+            raise RuntimeError("saved routing and activations must come back at their size")
         dy = torch.zeros_like(x) if dy is None else dy.contiguous()
         ops._chk(dy, "dy", x.dtype)
         lib, config, stream, need = _lib.load(), _layer_config(*key), ops._stream(), ctx.needs_input_grad
-        cfg, shared = key[7], sh_gate_up is not None
+        shared = sh_gate_up is not None
         scratch = torch.empty(_layer_sizes(key, T, True)[2], dtype=torch.uint8, device=x.device)
         d_w_gate_up = torch.empty_like(w_gate_up) if need[2] else None
         d_w_down = torch.empty_like(w_down) if need[3] else None

@@ -22,10 +22,10 @@ class _Library:
 
 @pytest.fixture
 def on_host(monkeypatch):
-    """The layer on CPU tensors: its input and the logits pass for GPU tensors, the library is a stub."""
+    """The layer on CPU tensors: its input, the logits and the incoming gradient pass for GPU tensors, the library is a stub."""
     lib = _Library()
     check = ops._chk
-    monkeypatch.setattr(ops, "_chk", lambda t, name, *a, **k: t if name in ("x", "logits") else check(t, name, *a, **k))
+    monkeypatch.setattr(ops, "_chk", lambda t, name, *a, **k: t if name in ("x", "logits", "dy") else check(t, name, *a, **k))
     monkeypatch.setattr(ops, "_stream", lambda: 0)
     monkeypatch.setattr(_lib, "load", lambda: lib)
     monkeypatch.setattr(moe, "_layer_sizes", lambda *a: (4096,) * 13)
@@ -79,3 +79,29 @@ def test_router_of_fewer_experts(on_host, monkeypatch):
     want = torch.full((T, E), float("-inf"))
     want[:, : E - 1] = H
     assert torch.equal(seen["logits"].view(T, E), want)
+
+
+@pytest.mark.parametrize("unpack", [lambda t: t.half(), lambda t: t[..., :-1], lambda t: t.transpose(0, -1)],
+                         ids=["type", "shape", "strides"])
+@pytest.mark.parametrize("which", range(6))
+def test_saved_tensors_come_back_as_they_were(on_host, unpack, which):
+    """Backward reads what the unpack hook returns: another type, shape or layout ends in an error."""
+    layer = _layer(use_shared_expert=True)
+    layer.overlap_weight_grads = False
+    saved = [None, layer.expert_gate_up, layer.expert_down, layer.shared_expert_gate_up, layer.shared_expert_down,
+             layer.shared_expert_output_gate][which]
+    x = torch.zeros(T, H, requires_grad=True)
+    planted = []
+
+    def hook(t):
+        if t.shape == (x if which == 0 else saved).shape:
+            planted.append(unpack(t))
+            return planted[-1]
+        return t
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, hook):
+        y = layer(x)
+    ops_reached = len(on_host.reached)
+    with pytest.raises(RuntimeError, match="must"):
+        y.sum().backward()
+    assert planted and len(on_host.reached) == ops_reached
