@@ -146,7 +146,7 @@ AMOE_EXPORT int amoe_grouped_gemm_wgrad(const void* A, const int32_t* a_row_map,
     const char* what = "grouped_gemm_wgrad";
     AMOE_REQUIRE(A && B && offsets && C, AMOE_ERR_BAD_ARG, "%s: null pointer", what);
     AMOE_REQUIRE(!(a_row_map && b_row_map), AMOE_ERR_UNSUPPORTED, "%s: at most one operand may be gathered", what);
-    int rc = check_gemm_common(what, dtype, R, E, Kd, N, tile_cfg);
+    int rc = check_gemm_common(what, dtype, R, E, Kd, N, tile_cfg < 0 ? tile_cfg : tile_cfg & ~AMOE_SOURCE_BELOW_4GIB);
     if (rc) return rc;
     const int vec = dtype != AMOE_F32 ? 8 : 4;
     AMOE_REQUIRE(Kd % vec == 0 && N % vec == 0, AMOE_ERR_UNSUPPORTED, "%s: extents (%d, %d) must be multiples of %d",

@@ -1486,7 +1486,8 @@ int amoe_bf16_gated_bwd_parts(int I, int tile_cfg)
 int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map,
                     const int32_t* offsets, void* C, int R, int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype)
 {
-    tile_cfg &= ~AMOE_TILE_MAP_READY;   // no tile map in the weight gradient
+    const bool offsets32 = !(a_row_map || b_row_map) || (tile_cfg & AMOE_SOURCE_BELOW_4GIB);
+    tile_cfg &= ~(AMOE_TILE_MAP_READY | AMOE_SOURCE_BELOW_4GIB);   // no tile map in the weight gradient
     TileCfg tc = pick_cfg(tile_cfg);
     GemmArgs a = {};
     a.f16 = dtype == AMOE_F16;
@@ -1506,15 +1507,15 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
     a.N = N;
     a.n_ntiles = (N + tc.bn - 1) / tc.bn;
     a.n_mt = (Kd + tc.bm - 1) / tc.bm;
-    // The default kernel addresses a gathered operand (at most R source rows) with 32-bit byte offsets and numbers its
-    // tiles in 32 bits; operands beyond that keep the kernel with 64-bit addresses.
+    // The default kernel addresses a gathered operand with 32-bit byte offsets and numbers its tiles in 32 bits; where the
+    // caller does not vouch for the operand's size (the length of the map says nothing about it), and beyond that many
+    // tiles, the kernel with 64-bit addresses runs.
     const long long per = (long long)a.n_mt * a.n_ntiles;
     if (tile_cfg == 0) {
         // Below 256 rows per expert the product is bound by the gradients' stores, and a tile of the default kernel is
         // never done in less than three K tiles: the 32-wide K tiles and one-tile workgroups of shape 5 are faster there
         // (128 experts of 2048 x 1536: 32 rows 0.19 against 0.21 ms, 188 rows equal, 375 rows 0.43 against 0.40).
-        const int ld = a_row_map ? Kd : N;
-        if (R >= 256ll * E && (!(a_row_map || b_row_map) || (unsigned long long)R * ld * 2ull < (1ull << 32)) && per * per * E < (1ll << 32))
+        if (R >= 256ll * E && offsets32 && per * per * E < (1ll << 32))
             return amoe_pp_wgrad(a, s);
         tile_cfg = 5;
     }

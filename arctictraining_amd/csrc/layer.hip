@@ -285,12 +285,16 @@ AMOE_EXPORT int amoe_layer_bwd(const int32_t* config, int T, const void* x, cons
     OrderEvent event;
     if (overlap) AMOE_REQUIRE(event.order(main, side), AMOE_ERR_LAUNCH, "layer_bwd: cannot order the second stream after the first");
     void* const wstream = overlap ? side_stream : stream;
+    // (the rows that are gathered are the T tokens')
+    const auto gathered = [&](int width) {
+        return c.tile_cfg | ((size_t)T * width * c.esz() < (1ull << 32) ? AMOE_SOURCE_BELOW_4GIB : 0);
+    };
     if (d_w_down)
-        AMOE_TRY(amoe_grouped_gemm_wgrad(s.inter, nullptr, dy, s.token_of, s.offsets, d_w_down, c.dtype, R, c.E, c.I, c.H, c.tile_cfg,
-                                         wstream));
+        AMOE_TRY(amoe_grouped_gemm_wgrad(s.inter, nullptr, dy, s.token_of, s.offsets, d_w_down, c.dtype, R, c.E, c.I, c.H,
+                                         gathered(c.H), wstream));
     if (d_w_gate_up)
         AMOE_TRY(amoe_grouped_gemm_wgrad(x, s.token_of, w.d_gate_up, nullptr, s.offsets, d_w_gate_up, c.dtype, R, c.E, c.H, 2 * c.I,
-                                         c.tile_cfg, wstream));
+                                         gathered(c.H), wstream));
     if (c.fused_bwd())
         AMOE_TRY(amoe_launch_score_grad(w.parts, amoe_gated_bwd_score_parts(c.I, c.tile_cfg), d_scores_rows, s.row_of, w.d_scores, R,
                                         false, main));

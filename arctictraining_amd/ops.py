@@ -14,6 +14,7 @@ F32, BF16, F16 = 0, 1, 2
 _DTYPE_CODES = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 ACT_SILU, ACT_GELU, ACT_RELU, ACT_GPT_OSS = 0, 1, 2, 3
 TILE_MAP_READY = 0x100  # AMOE_TILE_MAP_READY
+SOURCE_BELOW_4GIB = 0x200  # AMOE_SOURCE_BELOW_4GIB
 
 
 def _dtype_code(t) -> int:
@@ -385,6 +386,9 @@ def grouped_gemm_wgrad(A, B, offsets, num_experts: int, tile_cfg: int = 0, a_row
     R = a_row_map.numel() if a_row_map is not None else A.shape[0]
     if b_row_map is None and a_row_map is not None and B.shape[0] != R:
         raise RuntimeError("B must have one row per routed row")
+    source = A if a_row_map is not None else B if b_row_map is not None else None
+    if source is not None and source.numel() * source.element_size() < 1 << 32:
+        tile_cfg |= SOURCE_BELOW_4GIB
     Kd = A.shape[1]
     N = B.shape[1]
     C = torch.empty((num_experts, Kd, N), dtype=A.dtype, device=A.device)

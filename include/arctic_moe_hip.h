@@ -248,8 +248,11 @@ int amoe_score_grad_gather(const float* score_partials, int n_parts, const int32
  * expert).  A [R,Kd], B [R,N], C [E,Kd,N].  The autograd of moe.py:59 w.r.t. B[e].
  * One of the operands may be gathered: with a_row_map [R], row r of A is read from
  * A[a_row_map[r],:] (A then has as many rows as the map addresses); likewise b_row_map for B.
- * tile_cfg: 0 default, or 1, 2, 3, 5 (other tile shapes, for tuning).
+ * tile_cfg: 0 default, or 1, 2, 3, 5 (other tile shapes, for tuning).  AMOE_SOURCE_BELOW_4GIB may be OR-ed into it: the
+ * gathered operand, all rows that the map may address, is smaller than 4 GiB, and the default kernel, which addresses it
+ * with 32-bit byte offsets, may run (without it a gathered operand may have any size).
  */
+#define AMOE_SOURCE_BELOW_4GIB 0x200
 int amoe_grouped_gemm_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map,
                             const int32_t* offsets, void* C, int dtype, int R, int E, int Kd, int N, int tile_cfg,
                             void* stream);

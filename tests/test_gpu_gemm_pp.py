@@ -109,3 +109,29 @@ def test_weight_gradient(ops, gpu_device, dtype, tol, M, N, counts):
                 _check(got[e], want[e], tol)
             else:
                 assert bool((got[e] == 0).all())
+
+
+@pytest.mark.parametrize("operand", ["A", "B"])
+def test_weight_gradient_gathered_from_4_gib(ops, gpu_device, operand):
+    """A gathered operand of more than 4 GiB behind a short row map: the rows past 4 GiB are the ones that are read."""
+    print("pp wgrad of 4 GiB", operand, flush=True)
+    M, N, counts = 264, 256, [300, 0, 500]
+    width = M if operand == "A" else N
+    R, T = sum(counts), (1 << 32) // (2 * width) + 1000
+    g = torch.Generator(device=gpu_device).manual_seed(1)
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(gpu_device)
+    rnd = lambda *s: torch.randn(*s, device=gpu_device, generator=g).bfloat16()
+    source = torch.zeros(T, width, device=gpu_device, dtype=torch.bfloat16)
+    rows = (T - 1 - torch.arange(R, device=gpu_device)).to(torch.int32)
+    dense = rnd(R, width)
+    source[rows.long()] = dense
+    other = rnd(R, N if operand == "A" else M)
+    if operand == "A":
+        got, (a, b) = ops.grouped_gemm_wgrad(source, other, offs, 3, a_row_map=rows), (dense, other)
+    else:
+        got, (a, b) = ops.grouped_gemm_wgrad(other, source, offs, 3, b_row_map=rows), (other, dense)
+    for e, (p, q) in enumerate(zip(a.split(counts), b.split(counts))):
+        if counts[e]:
+            _check(got[e], p.float().t() @ q.float(), 1e-2)
+        else:
+            assert bool((got[e] == 0).all())
