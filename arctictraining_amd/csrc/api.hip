@@ -31,6 +31,7 @@ int amoe_bf16_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void*
                            const void* gate_up, const float* row_scale, void* d_gate_up, float* partials, int R, int E,
                            int I, int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype);
 int amoe_bf16_gated_bwd_parts(int I, int tile_cfg);
+size_t amoe_rows_map_bytes(int R, int E, int dtype, int tile_cfg);
 int amoe_f32_rows(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int R, int E,
                   int Kred, int N, int ldb, long long strideB, bool b_kc, void* workspace, size_t workspace_bytes,
                   bool map_ready, hipStream_t s);
@@ -87,8 +88,8 @@ AMOE_EXPORT int amoe_grouped_gemm_gateup_act_fwd(const void* xp, const int32_t* 
                  "%s: an operand exceeds 2^32 elements", what);
     rc = check_gemm_dims(what, dtype, H, 2 * I);
     if (rc) return rc;
-    AMOE_REQUIRE(workspace_bytes >= amoe_grouped_gemm_workspace_bytes(R, E), AMOE_ERR_WORKSPACE,
-                 "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_grouped_gemm_workspace_bytes(R, E));
+    AMOE_REQUIRE(workspace_bytes >= amoe_rows_map_bytes(R, E, dtype, tile_cfg), AMOE_ERR_WORKSPACE,
+                 "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_rows_map_bytes(R, E, dtype, tile_cfg));
     hipStream_t s = (hipStream_t)stream;
     if (dtype != AMOE_F32)
         return amoe_bf16_gateup_act(xp, a_row_map, w_gate_up, offsets, gate_up, inter, row_scale, R, E, H, I, act, workspace,
@@ -111,8 +112,8 @@ AMOE_EXPORT int amoe_grouped_gemm_nn(const void* A, const int32_t* a_row_map, co
     if (rc) return rc;
     rc = check_gemm_dims(what, dtype, Kd, N);
     if (rc) return rc;
-    AMOE_REQUIRE(workspace_bytes >= amoe_grouped_gemm_workspace_bytes(R, E), AMOE_ERR_WORKSPACE,
-                 "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_grouped_gemm_workspace_bytes(R, E));
+    AMOE_REQUIRE(workspace_bytes >= amoe_rows_map_bytes(R, E, dtype, tile_cfg), AMOE_ERR_WORKSPACE,
+                 "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_rows_map_bytes(R, E, dtype, tile_cfg));
     hipStream_t s = (hipStream_t)stream;
     if (dtype != AMOE_F32)
         return amoe_bf16_nn(A, a_row_map, B, offsets, C, R, E, Kd, N, workspace, workspace_bytes, tile_cfg, s, dtype);
@@ -130,8 +131,8 @@ AMOE_EXPORT int amoe_grouped_gemm_nt(const void* A, const int32_t* a_row_map, co
     if (rc) return rc;
     rc = check_gemm_dims(what, dtype, N, Kd);  // the reduction runs over N here
     if (rc) return rc;
-    AMOE_REQUIRE(workspace_bytes >= amoe_grouped_gemm_workspace_bytes(R, E), AMOE_ERR_WORKSPACE,
-                 "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_grouped_gemm_workspace_bytes(R, E));
+    AMOE_REQUIRE(workspace_bytes >= amoe_rows_map_bytes(R, E, dtype, tile_cfg), AMOE_ERR_WORKSPACE,
+                 "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_rows_map_bytes(R, E, dtype, tile_cfg));
     hipStream_t s = (hipStream_t)stream;
     if (dtype != AMOE_F32)
         return amoe_bf16_nt(A, a_row_map, B, offsets, C, R, E, Kd, N, workspace, workspace_bytes, tile_cfg, s, dtype);
@@ -178,8 +179,8 @@ AMOE_EXPORT int amoe_grouped_gemm_nt_gated_bwd(const void* dy, const int32_t* a_
     AMOE_REQUIRE((long long)R * 2 * I < (1ll << 32), AMOE_ERR_UNSUPPORTED, "%s: an operand exceeds 2^32 elements", what);
     rc = check_gemm_dims(what, dtype, H, I);  // the reduction runs over H
     if (rc) return rc;
-    AMOE_REQUIRE(workspace_bytes >= amoe_grouped_gemm_workspace_bytes(R, E), AMOE_ERR_WORKSPACE,
-                 "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_grouped_gemm_workspace_bytes(R, E));
+    AMOE_REQUIRE(workspace_bytes >= amoe_rows_map_bytes(R, E, dtype, tile_cfg), AMOE_ERR_WORKSPACE,
+                 "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_rows_map_bytes(R, E, dtype, tile_cfg));
     return amoe_bf16_nt_gated_bwd(dy, a_row_map, w_down, offsets, gate_up, row_scale, d_gate_up, score_partials, R, E, I, H,
                                   act, workspace, workspace_bytes, tile_cfg, (hipStream_t)stream, dtype);
 }

@@ -34,6 +34,8 @@
 #include "gemm_common.h"
 #include "gemm_launch.h"
 
+#include <algorithm>
+
 // This file is compiled once per group of entry points (-DAMOE_GEMM_PART=0..3), in parallel: the
 // kernels of all groups are instances of the same two templates.
 //   0: gate_up forward with the gated activation   1: plain row-grouped products (NN, NT)
@@ -1307,24 +1309,33 @@ static inline int rows_tile_height(int R, int E, int tile_cfg)
 int amoe_build_tile_map(const int32_t* offsets, int R, int E, int bm, void* workspace, size_t workspace_bytes,
                         const int4** tile_map, const int32_t** n_mtiles, int* max_mtiles, hipStream_t s, bool ready);
 
+static inline size_t map_bytes(int max_mtiles) { return 16 + sizeof(int4) * (size_t)max_mtiles; }
+
 #if AMOE_PART(3)
+// What any of the products needs for any number of rows up to R: a workspace made for the largest call serves the
+// smaller ones, some of which have more tiles.  (64: the tile height of the float32 kernels)
 AMOE_EXPORT size_t amoe_grouped_gemm_workspace_bytes(int R, int E)
 {
     if (R <= 0 || E <= 0) return 0;
-    // (64: the tile height of the float32 kernels)
-    const int low = rows_tile_height(R, E, 0);
-    return 16 + sizeof(int4) * (size_t)ws_max_mtiles(R, E, low < 64 ? low : 64);
+    const int lowest = (int)std::min<long long>(R, 4ll * E);
+    return map_bytes(std::max(ws_max_mtiles(R, E, 64), ws_max_mtiles(lowest, E, 16)));
+}
+
+// What one call needs: R rows, this type and tile shape
+size_t amoe_rows_map_bytes(int R, int E, int dtype, int tile_cfg)
+{
+    return map_bytes(ws_max_mtiles(R, E, dtype == AMOE_F32 ? 64 : rows_tile_height(R, E, tile_cfg & ~AMOE_TILE_MAP_READY)));
 }
 
 // ready: the workspace already holds the map for these arguments (AMOE_TILE_MAP_READY); nothing is launched
 int amoe_build_tile_map(const int32_t* offsets, int R, int E, int bm, void* workspace, size_t workspace_bytes,
                         const int4** tile_map, const int32_t** n_mtiles, int* max_mtiles, hipStream_t s, bool ready)
 {
-    AMOE_REQUIRE(workspace_bytes >= amoe_grouped_gemm_workspace_bytes(R, E), AMOE_ERR_WORKSPACE,
-                 "grouped_gemm: workspace %zu < %zu bytes", workspace_bytes, amoe_grouped_gemm_workspace_bytes(R, E));
     int32_t* cnt = (int32_t*)workspace;
     int4* map = (int4*)((char*)workspace + 16);
     *max_mtiles = ws_max_mtiles(R, E, bm);
+    AMOE_REQUIRE(workspace_bytes >= map_bytes(*max_mtiles), AMOE_ERR_WORKSPACE, "grouped_gemm: workspace %zu < %zu bytes",
+                 workspace_bytes, map_bytes(*max_mtiles));
     *tile_map = map;
     *n_mtiles = cnt;
     if (ready) return AMOE_OK;
@@ -1341,10 +1352,10 @@ int amoe_tile_map_layout(int R, int E, int dtype, int tile_cfg, void* workspace,
     const int shape = tile_cfg & ~AMOE_TILE_MAP_READY;
     AMOE_REQUIRE(tile_cfg >= 0 && shape <= 5 && shape != 4, AMOE_ERR_BAD_ARG, "tile map: bad tile_cfg %d", tile_cfg);
     AMOE_REQUIRE(R > 0 && E > 0 && E <= AMOE_MAX_EXPERTS, AMOE_ERR_BAD_ARG, "tile map: bad sizes R=%d E=%d", R, E);
-    AMOE_REQUIRE(workspace_bytes >= amoe_grouped_gemm_workspace_bytes(R, E), AMOE_ERR_WORKSPACE,
-                 "tile map: workspace %zu < %zu bytes", workspace_bytes, amoe_grouped_gemm_workspace_bytes(R, E));
     *bm = dtype == AMOE_F32 ? 64 : rows_tile_height(R, E, shape);
     *max_mtiles = ws_max_mtiles(R, E, *bm);
+    AMOE_REQUIRE(workspace_bytes >= map_bytes(*max_mtiles), AMOE_ERR_WORKSPACE, "tile map: workspace %zu < %zu bytes",
+                 workspace_bytes, map_bytes(*max_mtiles));
     *n_mtiles = (int32_t*)workspace;
     *tile_map = (int4*)((char*)workspace + 16);
     return AMOE_OK;

@@ -163,7 +163,8 @@ int amoe_combine_fwd(const void* moe_out, const int32_t* row_of, const float* sc
 int amoe_combine_bwd(const void* dy, const void* moe_out, const int32_t* row_of, const float* scores,
                      void* d_moe_out, float* d_scores, int dtype, int T, int K, int H, void* stream);
 
-/* workspace every grouped GEMM below needs (tile map built on the device from offsets) */
+/* workspace every grouped GEMM below needs for up to R rows (tile map built on the device from offsets); never less for
+ * more rows: a workspace made for the largest call serves the smaller ones */
 size_t amoe_grouped_gemm_workspace_bytes(int R, int E);
 
 /*

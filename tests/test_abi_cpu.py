@@ -127,6 +127,29 @@ def test_gemm_argument_errors(lib):
     assert lib.amoe_grouped_gemm_gateup_act_fwd(P, None, P, P, None, None, P, 0, 128, 4, 64, 64, 0, P, big, 0, None) == -2
 
 
+@pytest.mark.parametrize("E", [1, 8, 24, 128, 512])
+def test_workspace_of_the_largest_call_serves_smaller_ones(lib, E):
+    """The bytes never fall with more rows, and what a call accepts is a workspace of any larger call (each call below is
+    refused by a check that comes after the workspace's, -2 and not -3)."""
+    sizes = [lib.amoe_grouped_gemm_workspace_bytes(R, E) for R in range(1, 20 * E)]
+    assert sizes == sorted(sizes)
+
+    def product(R, size, dtype=1, cfg=0):   # (weights of 4 GiB)
+        return lib.amoe_grouped_gemm_nn(P, None, P, P, P, dtype, R, E, 65536, 32768, P, size, cfg, None)
+
+    def f32(R, size):                       # (float32 without its gate_up buffer)
+        return lib.amoe_grouped_gemm_gateup_act_fwd(P, None, P, P, None, None, P, 0, R, E, 64, 64, 0, P, size, 0, None)
+
+    for R in (1, E, 4 * E, 4 * E + 1, 6 * E, 8 * E, 8 * E + 1, 12 * E):
+        for larger in (R, R + 1, 4 * E + 1, 8 * E, 8 * E + 1, 19 * E):
+            if larger >= R:
+                size = sizes[min(larger, len(sizes)) - 1]
+                assert product(R, size) == -2 and product(R, size, dtype=2, cfg=1) == -2 and f32(R, size) == -2
+        # float32 and the other tile shapes have no low tiles to hold
+        assert f32(R, 16 + 16 * (R // 64 + E + 1)) == -2 and product(R, 16 + 16 * (R // 256 + E + 1), cfg=5) == -2
+        assert f32(R, 16 * (R // 64 + E + 1)) == -3 and product(R, 16 * (R // 256 + E + 1), cfg=5) == -3
+
+
 def test_gated_bwd_gemm_argument_errors(lib):
     big = 1 << 20
     f = lib.amoe_grouped_gemm_nt_gated_bwd
