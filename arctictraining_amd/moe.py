@@ -20,6 +20,7 @@ from typing import Any, Optional
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib, ops
 
@@ -740,7 +741,8 @@ class ArcticMoE(nn.Module):
 
     def _run_gated(self, x, shared, replay, opts):
         weights = (self.router_gate, self.expert_gate_up, self.expert_down)
-        if torch.is_grad_enabled():
+        # (forward-mode runs without gradients too: inside a dual level the autograd function decides on the tangents)
+        if torch.is_grad_enabled() or getattr(forward_ad, "_current_level", 0) >= 0:
             out = _ExpertLayerFn.apply(x, *weights, *shared, replay, opts)
             return out if opts["want_scores"] else (out, None)
         y, saved, key = _layer_forward(x, *weights, shared, replay, opts, keep=False)

@@ -105,3 +105,27 @@ def test_saved_tensors_come_back_as_they_were(on_host, unpack, which):
     with pytest.raises(RuntimeError, match="must"):
         y.sum().backward()
     assert planted and len(on_host.reached) == ops_reached
+
+
+@pytest.mark.parametrize("dual", ["x", "expert_down"])
+def test_forward_mode_without_gradients(monkeypatch, dual):
+    """The layer has no forward-mode derivative: a tangent ends in an error also where gradients are switched off, and is
+    not dropped.  An open dual level without a tangent changes nothing."""
+    import torch.autograd.forward_ad as fwAD
+
+    layer = _layer()
+    key = (E, K, H, 32, 0, 0, True, 0, False)
+    monkeypatch.setattr(moe, "_layer_forward", lambda x, *a, **k: (x + 1, torch.zeros(64, dtype=torch.uint8), key))
+    x = torch.zeros(T, H)
+    with torch.no_grad(), fwAD.dual_level():
+        assert torch.equal(layer(x), x + 1)
+        if dual == "x":
+            x = fwAD.make_dual(x, torch.ones(T, H))
+        else:
+            tangent = fwAD.make_dual(layer.expert_down.detach(), torch.ones_like(layer.expert_down))
+            del layer.expert_down
+            layer.expert_down = tangent
+        with pytest.raises(NotImplementedError, match="jvp"):
+            layer(x)
+    with torch.no_grad():
+        assert torch.equal(layer(torch.zeros(T, H)), torch.ones(T, H))
