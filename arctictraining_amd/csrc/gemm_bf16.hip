@@ -1297,6 +1297,11 @@ static inline int ws_max_mtiles(int R, int E, int bm) { return R / bm + E + 1; }
 // Uneven loads set the limits: where a sixteenth of the experts has half of the rows, their low tiles read the weights
 // again, at 6 rows an expert and 16-row tiles 13 % in the products with B^T (153 / 135 us), at 8 and 32-row tiles
 // nothing (135 / 136), at 12 again 14 %.
+// Loads that are more uneven than that gain: the rows of 4 an expert all on top_k = 8 of 128 experts of 2048 x 768, gate_up
+// and down products 34 / 48 us, those with B^T 63 / 62; all on one expert 26 / 60 and 62 / 77 (more workgroups than 256-row
+// tiles make, and the weights that they read again are in the caches).  What is lost is a launch of a few tiles more than
+// there are compute units: half of 3 rows an expert on a sixteenth of 64 experts of 2048 x 1408, one product 84 / 51 us,
+// the four 316 / 324.  Tiles of their own for the products with B^T, of 32 or 128 rows, win these and lose 2-6 % elsewhere.
 static inline int rows_tile_height(int R, int E, int tile_cfg)
 {
     if (tile_cfg == 0) {
