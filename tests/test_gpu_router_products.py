@@ -11,7 +11,7 @@ TOL = {torch.bfloat16: 4e-3, torch.float16: 5e-4}
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("T", [1, 15, 16, 17, 33, 256])
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 33, 256, 300, 511, 513])
 @pytest.mark.parametrize("E,H", [(1, 32), (8, 544), (60, 1024), (128, 2048), (32, 4096), (512, 96)])
 def test_products(gpu_device, dtype, T, E, H):
     from arctictraining_amd import moe, ops
