@@ -162,7 +162,8 @@ __device__ __forceinline__ int pp_here(int v)
 // instruction in it counts (range tests on the loads, waits chosen by a branch and branches around dead rows each
 // cost 4-6 % of the K loop and are gone from it).  Measured on one MI355X, 131072 rows, N = 2048, bf16 NT: K = 8192
 // 1.50-1.66 PFLOP/s (operands from HBM / from L2); K = 2048 1.23-1.43, K = 768 1.0: what a tile costs beside its K loop
-// is about 5 us, of which half are its stores.  The kernel this one replaced (32-wide K tiles, 32x32x16 MFMAs, all
+// is about 5 us, of which half are its stores.  The gated epilogues cost more: the gate_up product of K = 2048 runs at
+// 0.96-1.08 (128 uneven / even experts; the library's plain product of that size at 1.0), the gated backward one at 0.87.  The kernel this one replaced (32-wide K tiles, 32x32x16 MFMAs, all
 // eight waves in step) ran at 1.0-1.1 on the same problems.
 template <bool B_KC, int EPI, int ACT, typename ET>
 __device__ __forceinline__ void pp_rows_body()

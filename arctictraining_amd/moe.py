@@ -5,8 +5,9 @@ HIP kernels reached through the C ABI of libarctic_moe_hip.so.
 Same constructor argument, parameter names / shapes / layouts (they are checkpoint keys,
 arctic_training/model/moe/utils.py:563-566), forward signature and return type as the
 reference, so the trainer's `layer.mlp = ArcticMoE(config)` (utils.py:320) works unchanged.
-The whole routed-expert computation is one torch.autograd.Function whose forward and
-backward call the kernels stage by stage with no host synchronisation.
+The whole routed-expert computation of a gated layer is one torch.autograd.Function: forward is one
+native call, backward three at most, over one saved and one scratch buffer; a layer without a gate calls the
+kernels stage by stage.  Neither synchronises with the host.
 """
 import contextlib
 import ctypes
@@ -155,10 +156,6 @@ def _token_offsets(T: int, parts: int, device) -> torch.Tensor:
         (T, parts, str(device)),
         lambda: (torch.arange(parts + 1, dtype=torch.int64, device=device) * T // parts).to(torch.int32),
     )
-
-
-def _token_ids(T: int, device) -> torch.Tensor:
-    return _INDEX_CACHE.get((T, "ids", str(device)), lambda: torch.arange(T, dtype=torch.int32, device=device))
 
 
 def _dense_splits(T: int, Kd: int, N: int, dtype, tile: int = 256) -> int:
