@@ -208,22 +208,15 @@ def _router_logits(x: torch.Tensor, router_gate: torch.Tensor) -> torch.Tensor:
     return torch.matmul(x, router_gate.t())
 
 
-def _layer_logits(x: torch.Tensor, router_gate: torch.Tensor, opts) -> torch.Tensor:
-    """_router_logits of a layer with E experts: at most E columns, one for each row of router_gate."""
-    logits, E = _router_logits(x, router_gate), opts["num_experts"]
-    if logits.shape[1] > E:   # (their counts, weights and gradients do not exist)
-        raise RuntimeError(f"router_gate must have one row for each of at most {E} experts, got {list(router_gate.shape)}")
-    return logits
-
-
-def _padded_logits(logits: torch.Tensor, opts) -> torch.Tensor:
-    """What the native layer reads, [T,E]: an expert that the router leaves out has a probability of 0."""
-    E, K = opts["num_experts"], opts["top_k"]
-    if logits.shape[1] == E:
-        return logits
-    if logits.shape[1] < K:
-        raise RuntimeError(f"router_gate must have at least top_k = {K} rows, got {logits.shape[1]}")
-    return F.pad(logits, (0, E - logits.shape[1]), value=float("-inf"))
+def _fit_logits(logits: torch.Tensor, opts, pad: bool = True) -> torch.Tensor:
+    """The logits of a router_gate that has not one row for each of the layer's experts, as the kernels read them: [T,E],
+    an expert that the router leaves out with a probability of 0 (not padded for the stages, which take E from them)."""
+    n, E, K = logits.shape[1], opts["num_experts"], opts["top_k"]
+    if n > E:   # (their counts, weights and gradients do not exist)
+        raise RuntimeError(f"router_gate must have one row for each of at most {E} experts, got {n}")
+    if n < K:
+        raise RuntimeError(f"router_gate must have at least top_k = {K} rows, got {n}")
+    return F.pad(logits, (0, E - n), value=float("-inf")) if pad else logits
 
 
 def _router_input_grad(d_logits: torch.Tensor, router_gate: torch.Tensor) -> torch.Tensor:
@@ -272,7 +265,7 @@ def _route(x, router_gate, replay, opts):
     E, K = opts["num_experts"], opts["top_k"]
     timers: PhaseTimers = opts["timers"]
     timers.start("router")
-    logits = _layer_logits(x, router_gate, opts)
+    logits = _fit_logits(_router_logits(x, router_gate), opts, pad=False)
     probs, topk_idx, scores = ops.router_topk_fwd(logits, K, opts["normalize"])
     assign = topk_idx if replay is None else _replayed(replay, T, opts)
     # the row-grouped GEMMs of a step share one tile map: the permutation plan builds it (its
@@ -338,8 +331,9 @@ def _layer_forward(x, router_gate, w_gate_up, w_down, shared, replay, opts, keep
     sizes = _layer_sizes(key, T, keep)
     if timers.wall_clock_breakdown:
         timers.start("router")
-    routed = _layer_logits(x, router_gate, opts)
-    logits = ops._chk(_padded_logits(routed, opts), "logits")
+    logits = routed = _router_logits(x, router_gate)
+    if routed.shape != (T, E) or not routed.is_contiguous():
+        logits = _fit_logits(routed, opts).contiguous()
     assign = None if replay is None else _replayed(replay, T, opts)
     y = torch.empty_like(x)
     buf = torch.empty(sizes[0] + (0 if keep else sizes[1]), dtype=torch.uint8, device=x.device)
