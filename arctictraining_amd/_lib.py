@@ -111,6 +111,11 @@ SIGNATURES = {
         [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
          _c_void_p],
     ),
+    "amoe_column_grad_workspace_bytes": (_c_size_t, [_c_int, _c_int]),
+    "amoe_column_grad": (
+        _c_int,
+        [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_size_t, _c_void_p],
+    ),
     "amoe_remap_pack_list": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p]),
     "amoe_remap_unpack_list": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p]),
     "amoe_gated_act_bwd": (

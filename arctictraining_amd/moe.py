@@ -468,7 +468,7 @@ class _ExpertLayerFn(torch.autograd.Function):
                 "amoe_layer_bwd_shared",
             )
             if need[6]:
-                d_sh_out_gate = torch.matmul(x.t(), d_pre)
+                d_sh_out_gate = ops.column_grad(x, d_pre)
 
         dx = dx_router = None
         if need[0]:
@@ -581,7 +581,7 @@ class _UngatedExpertLayerFn(torch.autograd.Function):
             if ctx.needs_input_grad[4]:
                 d_sh_up = torch.matmul(x.t(), d_sh_inter)
             if ctx.needs_input_grad[6]:
-                d_sh_out_gate = torch.matmul(x.t(), d_pre)
+                d_sh_out_gate = ops.column_grad(x, d_pre)
 
         dx = None
         if ctx.needs_input_grad[0]:

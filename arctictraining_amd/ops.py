@@ -450,6 +450,21 @@ def gated_act_bwd(
     return d_gu if slot_of is None else (d_gu, d_scale)
 
 
+def column_grad(x: torch.Tensor, coef: torch.Tensor) -> torch.Tensor:
+    """x [T,H]^T @ coef [T,1] -> [H,1]: the weight gradient of a linear map onto one column."""
+    _chk(x, "x")
+    _chk(coef, "coef", x.dtype)
+    T, H = x.shape
+    if coef.numel() != T:
+        raise RuntimeError(f"coef must hold {T} values, got {list(coef.shape)}")
+    lib = _lib.load()
+    out = torch.empty((H, 1), dtype=x.dtype, device=x.device)
+    ws = torch.empty(lib.amoe_column_grad_workspace_bytes(T, H), dtype=torch.uint8, device=x.device)
+    rc = lib.amoe_column_grad(x.data_ptr(), coef.data_ptr(), out.data_ptr(), _dtype_code(x), T, H, ws.data_ptr(), ws.numel(), _stream())
+    _lib.check(rc, "amoe_column_grad")
+    return out
+
+
 def _expert_view(t: torch.Tensor, name: str):
     """[E, I, H] tensor whose experts may be strided (a slice of a fused tensor) but whose
     [I, H] matrices are dense; returns (E, I, H, expert stride in elements)."""

@@ -318,6 +318,15 @@ int amoe_dense_wgrad(const void* A, const void* B, const int32_t* chunk_offsets,
                      int T, int Kd, int N, int tile_cfg, void* stream);
 
 /*
+ * Weight gradient of a linear map of every token onto one column (a shared expert's output gate):
+ * out [H] = sum_t coef[t] * x[t,:], x [T,H] and coef [T] and out of one type, summed in float32 in a fixed order.
+ * H is a multiple of 8 (float32: 4).
+ */
+size_t amoe_column_grad_workspace_bytes(int T, int H);
+int amoe_column_grad(const void* x, const void* coef, void* out, int dtype, int T, int H, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
+/*
  * Expert-weight re-layout, checkpoint format -> ArcticMoE parameters.  Replaces the torch
  * stack / view / transpose sequence of remap_orig_moe_mlp_params_to_arctic_moe
  * (arctic_training/model/moe/utils.py:232-266):

@@ -21,6 +21,24 @@ def test_dense_weight_gradient(gpu_device, dtype, T, Kd, N, splits):
     assert (got.double() - ref).norm() <= tol * ref.norm()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H", [(1, 8), (63, 520), (65, 512), (4096, 2048), (4097, 1032), (9556, 320)])
+def test_gradient_of_one_column(gpu_device, dtype, T, H):
+    """One rounding of the result (2^-9, 2^-12, 2^-24 of the value) and the order of float32 sums."""
+    from arctictraining_amd import ops
+
+    print("column_grad", dtype, T, H, flush=True)
+    g = torch.Generator(gpu_device).manual_seed(T + H)
+    x = torch.randn(T, H, device=gpu_device, generator=g).to(dtype)
+    coef = torch.randn(T, 1, device=gpu_device, generator=g).to(dtype)
+    got = ops.column_grad(x, coef)
+    ref = x.double().t() @ coef.double()
+    assert got.shape == (H, 1) and got.dtype == dtype
+    assert (got.double() - ref).norm() <= {torch.bfloat16: 4e-3, torch.float16: 5e-4, torch.float32: 2e-6}[dtype] * ref.norm()
+    with pytest.raises(RuntimeError):
+        ops.column_grad(x, coef[:0])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shared", [False, True])
 @pytest.mark.parametrize("T", [1, 7, 260])
