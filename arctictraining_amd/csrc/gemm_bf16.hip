@@ -1318,7 +1318,7 @@ static inline size_t map_bytes(int max_mtiles) { return 16 + sizeof(int4) * (siz
 
 #if AMOE_PART(3)
 // What any of the products needs for any number of rows up to R: a workspace made for the largest call serves the
-// smaller ones, some of which have more tiles.  (64: the tile height of the float32 kernels)
+// smaller ones, some of which have more tiles.  (64: no tile of another type or shape is lower)
 AMOE_EXPORT size_t amoe_grouped_gemm_workspace_bytes(int R, int E)
 {
     if (R <= 0 || E <= 0) return 0;
@@ -1329,7 +1329,7 @@ AMOE_EXPORT size_t amoe_grouped_gemm_workspace_bytes(int R, int E)
 // What one call needs: R rows, this type and tile shape
 size_t amoe_rows_map_bytes(int R, int E, int dtype, int tile_cfg)
 {
-    return map_bytes(ws_max_mtiles(R, E, dtype == AMOE_F32 ? 64 : rows_tile_height(R, E, tile_cfg & ~AMOE_TILE_MAP_READY)));
+    return map_bytes(ws_max_mtiles(R, E, dtype == AMOE_F32 ? 128 : rows_tile_height(R, E, tile_cfg & ~AMOE_TILE_MAP_READY)));
 }
 
 // ready: the workspace already holds the map for these arguments (AMOE_TILE_MAP_READY); nothing is launched
@@ -1349,7 +1349,7 @@ int amoe_build_tile_map(const int32_t* offsets, int R, int E, int bm, void* work
 }
 
 // Where the tile map of a row-grouped GEMM lives inside its workspace and how tall its tiles are, for a
-// caller that builds the map itself (the permutation plan): the float32 kernels use 64-row tiles.
+// caller that builds the map itself (the permutation plan): the float32 kernels use 128-row tiles.
 int amoe_tile_map_layout(int R, int E, int dtype, int tile_cfg, void* workspace, size_t workspace_bytes, int4** tile_map,
                          int32_t** n_mtiles, int* bm, int* max_mtiles)
 {
@@ -1357,7 +1357,7 @@ int amoe_tile_map_layout(int R, int E, int dtype, int tile_cfg, void* workspace,
     const int shape = tile_cfg & ~AMOE_TILE_MAP_READY;
     AMOE_REQUIRE(tile_cfg >= 0 && shape <= 5 && shape != 4, AMOE_ERR_BAD_ARG, "tile map: bad tile_cfg %d", tile_cfg);
     AMOE_REQUIRE(R > 0 && E > 0 && E <= AMOE_MAX_EXPERTS, AMOE_ERR_BAD_ARG, "tile map: bad sizes R=%d E=%d", R, E);
-    *bm = dtype == AMOE_F32 ? 64 : rows_tile_height(R, E, shape);
+    *bm = dtype == AMOE_F32 ? 128 : rows_tile_height(R, E, shape);
     *max_mtiles = ws_max_mtiles(R, E, *bm);
     AMOE_REQUIRE(workspace_bytes >= map_bytes(*max_mtiles), AMOE_ERR_WORKSPACE, "tile map: workspace %zu < %zu bytes",
                  workspace_bytes, map_bytes(*max_mtiles));
