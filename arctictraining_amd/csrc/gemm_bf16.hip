@@ -1326,10 +1326,10 @@ AMOE_EXPORT size_t amoe_grouped_gemm_workspace_bytes(int R, int E)
     return map_bytes(std::max(ws_max_mtiles(R, E, 64), ws_max_mtiles(lowest, E, 16)));
 }
 
-// What one call needs: R rows, this type and tile shape
+// What one call asks for: R rows, this type and tile shape (float32: what its 64-row tiles needed, its 128-row ones use less)
 size_t amoe_rows_map_bytes(int R, int E, int dtype, int tile_cfg)
 {
-    return map_bytes(ws_max_mtiles(R, E, dtype == AMOE_F32 ? 128 : rows_tile_height(R, E, tile_cfg & ~AMOE_TILE_MAP_READY)));
+    return map_bytes(ws_max_mtiles(R, E, dtype == AMOE_F32 ? 64 : rows_tile_height(R, E, tile_cfg & ~AMOE_TILE_MAP_READY)));
 }
 
 // ready: the workspace already holds the map for these arguments (AMOE_TILE_MAP_READY); nothing is launched
