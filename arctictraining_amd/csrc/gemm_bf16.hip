@@ -1359,8 +1359,8 @@ int amoe_tile_map_layout(int R, int E, int dtype, int tile_cfg, void* workspace,
     AMOE_REQUIRE(R > 0 && E > 0 && E <= AMOE_MAX_EXPERTS, AMOE_ERR_BAD_ARG, "tile map: bad sizes R=%d E=%d", R, E);
     *bm = dtype == AMOE_F32 ? 128 : rows_tile_height(R, E, shape);
     *max_mtiles = ws_max_mtiles(R, E, *bm);
-    AMOE_REQUIRE(workspace_bytes >= map_bytes(*max_mtiles), AMOE_ERR_WORKSPACE, "tile map: workspace %zu < %zu bytes",
-                 workspace_bytes, map_bytes(*max_mtiles));
+    AMOE_REQUIRE(workspace_bytes >= amoe_rows_map_bytes(R, E, dtype, shape), AMOE_ERR_WORKSPACE, "tile map: workspace %zu < %zu bytes",
+                 workspace_bytes, amoe_rows_map_bytes(R, E, dtype, shape));
     *n_mtiles = (int32_t*)workspace;
     *tile_map = (int4*)((char*)workspace + 16);
     return AMOE_OK;

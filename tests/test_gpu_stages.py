@@ -621,3 +621,40 @@ def test_permute_plan_builds_the_gemm_tile_map(ops, gpu_device, dtype, cfg):
     A2 = torch.randn(R, N, generator=g).to(dtype).to(gpu_device)
     assert torch.equal(ops.grouped_gemm_nt(A2, B, offs, tile_cfg=cfg, workspace=ws, map_ready=True),
                        ops.grouped_gemm_nt(A2, B, offs, tile_cfg=cfg))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("copies", [1, 40])
+def test_gelu_of_the_epilogues(gpu_device, dtype, copies):
+    """gelu and its derivative over the range where they are not 0 or g, the lower tail included, through products that
+    hand the epilogues g itself.  One rounding of the result (of 8 or 11 significant bits: 2^-8, 2^-11 of it at most)
+    and 1e-5 of the tail's value."""
+    from arctictraining_amd import ops
+
+    print("gelu epilogues", dtype, copies, flush=True)
+    g = torch.linspace(-6 if dtype == torch.bfloat16 else -3, 12, 2048).to(dtype)
+    H, I, R = 32, 64, 32
+    w = torch.zeros(1, H, 2 * I, dtype=dtype)
+    w[0, 1, 1::2] = 1.0                       # up = 1
+    wd = torch.zeros(1, I, H, dtype=dtype)
+    wd[0, :, 0] = 1.0                         # d_inter = 1
+    for part in g.view(-1, R):
+        x = torch.zeros(R, H, dtype=dtype)
+        x[:, 0], x[:, 1] = part, 1.0
+        x = x.repeat(copies, 1).to(gpu_device)
+        w[0, 0, 0::2] = 1.0                   # gate = the row's value
+        off = torch.tensor([0, R * copies], dtype=torch.int32, device=gpu_device)
+        gu, inter = ops.grouped_gemm_gateup_act_fwd(x, w.to(gpu_device), off, ops.ACT_GELU)
+        dy = torch.zeros(R * copies, H, dtype=dtype, device=gpu_device)
+        dy[:, 0] = 1.0
+        dg, _ = ops.grouped_gemm_nt_gated_bwd(dy, wd.to(gpu_device), off, gu, ops.ACT_GELU)
+        v = part.double().repeat(copies).view(-1, 1)
+        phi = torch.special.ndtr(v)
+        ref = v * phi
+        eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) + 1e-5
+        tiny = 1e-7 if dtype == torch.float16 else 0.0   # (float16 below its normal range)
+        assert ((inter.cpu().double() - ref).abs() <= eps * ref.abs() + tiny).all()
+        d = phi + v * torch.exp(-v * v / 2) * 0.3989422804014327
+        got = dg.cpu().double()
+        assert ((got[:, 0::2] - d).abs() <= eps * d.abs() + 1e-6).all()
+        assert ((got[:, 1::2] - ref).abs() <= eps * ref.abs() + tiny).all()
