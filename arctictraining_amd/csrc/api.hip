@@ -26,7 +26,7 @@ int amoe_bf16_nn(const void* A, const int32_t* a_row_map, const void* B, const i
 int amoe_bf16_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int R, int E,
                  int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype);
 int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map,
-                    const int32_t* offsets, void* C, int R, int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype);
+                    const int32_t* offsets, void* C, int R, int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype, int lda, bool out32);
 int amoe_bf16_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down, const int32_t* offsets,
                            const void* gate_up, const float* row_scale, void* d_gate_up, float* partials, int R, int E,
                            int I, int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype);
@@ -153,7 +153,7 @@ AMOE_EXPORT int amoe_grouped_gemm_wgrad(const void* A, const int32_t* a_row_map,
     AMOE_REQUIRE(Kd % vec == 0 && N % vec == 0, AMOE_ERR_UNSUPPORTED, "%s: extents (%d, %d) must be multiples of %d",
                  what, Kd, N, vec);
     hipStream_t s = (hipStream_t)stream;
-    if (dtype != AMOE_F32) return amoe_bf16_wgrad(A, a_row_map, B, b_row_map, offsets, C, R, E, Kd, N, tile_cfg, s, dtype);
+    if (dtype != AMOE_F32) return amoe_bf16_wgrad(A, a_row_map, B, b_row_map, offsets, C, R, E, Kd, N, tile_cfg, s, dtype, Kd, false);
     return amoe_f32_wgrad(A, a_row_map, B, b_row_map, offsets, C, R, E, Kd, N, s);
 }
 

@@ -127,7 +127,8 @@ using F_ = std::false_type;
 // K-strided ([k][column] in LDS, transposing reads).
 // MAPS: 1 = the rows of A, 2 = the rows of B are gathered through a row map
 // ET: the 16-bit element type (bf16_t or f16_t); GemmArgs names its pointers bf16_t for both
-template <int BM, int BN, int WGM, int WGN, int MAPS, typename ET>
+// OUT32: C is float32 (partial sums)
+template <int BM, int BN, int WGM, int WGN, int MAPS, typename ET, bool OUT32 = false>
 __device__ __forceinline__ void grouped_gemm_wgrad_body(const GemmArgs& p)
 {
     typedef typename Elem16<ET>::frag_t frag_t;
@@ -185,7 +186,7 @@ __device__ __forceinline__ void grouped_gemm_wgrad_body(const GemmArgs& p)
         const int c = tid + NT * i;
         constexpr int CPR = BM / 8;
         const int krow = c / CPR, mc = (c % CPR) ^ ((krow & 3) << 2);
-        const int col = min(m0 + mc * 8, p.M - 8);
+        const int col = min(m0 + mc * 8, p.lda - 8);
         aoff[i] = A_MAP ? (uint32_t)col : (uint32_t)krow * (uint32_t)p.lda + col;
         a_kr[i] = krow;
     }
@@ -517,6 +518,19 @@ __device__ __forceinline__ void grouped_gemm_wgrad_body(const GemmArgs& p)
     // row r and the odd lane with those of row r+1: three VALU operations per 4-byte store.
     // Addresses are a wave-uniform row base (scalar arithmetic) plus one per-lane 32-bit offset;
     // tiles that lie entirely inside the matrix take the FULL form without per-store bounds tests.
+    if constexpr (OUT32) {
+        float* const C32 = reinterpret_cast<float*>(p.C) + (long long)e * p.strideC;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int row = m0 + wm * WTM + i * 32 + 8 * (v >> 2) + 4 * lg + (v & 3), col = n0 + wn * WTN + j * 32 + lj;
+                    if (row < mend && col < p.N) C32[(long long)row * p.ldc + col] = acc[i][j][v];
+                }
+        return;
+    }
     bf16_t* Cb = p.C + (long long)e * p.strideC;
     const int odd1 = lj & 1;
     const uint32_t swap_sel = odd1 ? 0x03020706u : 0x05040100u;
@@ -1169,6 +1183,14 @@ grouped_gemm_wgrad_f16_kernel(GemmArgs p)
     grouped_gemm_wgrad_body<BM, BN, WGM, WGN, MAPS, f16_t>(p);
 }
 
+// partial sums in float32
+template <typename ET>
+__global__ void __launch_bounds__(256)
+grouped_gemm_wgrad_parts_kernel(GemmArgs p)
+{
+    grouped_gemm_wgrad_body<128, 128, 2, 2, 0, ET, true>(p);
+}
+
 template <int BM, int BN, int WGM, int WGN, bool B_KC, int EPI, int ACT>
 __global__ void __launch_bounds__(WGM * WGN * 64)
 grouped_gemm_rows_bf16_kernel(GemmArgs p)
@@ -1499,8 +1521,10 @@ int amoe_bf16_gated_bwd_parts(int I, int tile_cfg)
     return (I + tc.bn - 1) / tc.bn;
 }
 
+// lda: elements from one row of A to the next, a multiple of 8; the Kd of the output may be fewer (not with tile_cfg 0)
+// out32: C is float32 (tile_cfg 1, nothing gathered)
 int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map,
-                    const int32_t* offsets, void* C, int R, int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype)
+                    const int32_t* offsets, void* C, int R, int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype, int lda, bool out32)
 {
     const bool offsets32 = !(a_row_map || b_row_map) || (tile_cfg & AMOE_SOURCE_BELOW_4GIB);
     tile_cfg &= ~(AMOE_TILE_MAP_READY | AMOE_SOURCE_BELOW_4GIB);   // no tile map in the weight gradient
@@ -1514,7 +1538,7 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
     a.b_row_map = b_row_map;
     a.rows_total = R;
     a.offsets = offsets;
-    a.lda = Kd;
+    a.lda = lda;
     a.ldb = N;
     a.ldc = N;
     a.strideC = (long long)Kd * N;
@@ -1538,6 +1562,12 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
     long long grid = 0;
     int rc = set_supertiles(a, (long long)E * a.n_mt, &grid);
     if (rc) return rc;
+    if (out32) {
+        constexpr int lds_bytes = NSTAGE * (128 + 128) * BK * 2;
+        AMOE_REQUIRE(tile_cfg == 1 && !a_row_map && !b_row_map, AMOE_ERR_BAD_ARG, "grouped_gemm_wgrad: float32 sums of gathered rows");
+        if (a.f16) return launch_kernel<grouped_gemm_wgrad_parts_kernel<f16_t>, 256, lds_bytes>(a, (int)grid, s);
+        return launch_kernel<grouped_gemm_wgrad_parts_kernel<bf16_t>, 256, lds_bytes>(a, (int)grid, s);
+    }
     if (a_row_map) return launch_any<false, false, EPI_STORE, 0, 1>(a, tile_cfg, (int)grid, s);
     if (b_row_map) return launch_any<false, false, EPI_STORE, 0, 2>(a, tile_cfg, (int)grid, s);
     return launch_any<false, false, EPI_STORE, 0>(a, tile_cfg, (int)grid, s);

@@ -61,7 +61,7 @@ struct GemmArgs {
     int N;        // output columns
     int n_ntiles;
     int n_mt;     // wgrad mode: M tiles per expert
-    int rows_total;  // weight gradient: length of the row maps
+    int rows_total;  // weight gradient: length of the row maps; gemm_skinny.hip: rows of B (0: Kd)
     int gm, gn;   // blocks of one XCD work on super-tiles of gm x gn tiles
     int sn;       // super-tiles along N
     uint32_t inv_gm, inv_gn, inv_sn, inv_super;   // ceil(2^32 / gm), .. gn, sn, gm gn (0 for a divisor of 1)

@@ -52,7 +52,8 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[N
     const int steps = p.Kd / 32;                      // (the reduction length is a multiple of 32)
     const uint32_t row_bytes = (uint32_t)p.ldb * 2u;
     const __amdgpu_buffer_rsrc_t bd = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<bf16_t*>(p.B) + (long long)e * p.strideB, (short)0, (int)((uint32_t)p.Kd * row_bytes), 0x00020000);
+        const_cast<bf16_t*>(p.B) + (long long)e * p.strideB, (short)0, (int)((uint32_t)(p.rows_total ? p.rows_total : p.Kd) * row_bytes),
+        0x00020000);
     const __amdgpu_buffer_rsrc_t ad = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.A), (short)0, (int)SK_NOWHERE, 0x00020000);
     const int n = n0 + l16 * CPL;
     const uint32_t boff = n < p.N ? (uint32_t)(lq * 8) * row_bytes + (uint32_t)n * 2u : SK_NOWHERE;
@@ -285,26 +286,34 @@ int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s)
 int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s) { return launch_height<EPI_STORE, 0>(a, bm, s); }
 
 // out [T,H] = d_logits [T,E] @ w [E,H], the router's part of the gradient of the input: the product above with one
-// expert that has every row.
-AMOE_EXPORT int amoe_router_input_grad(const void* d_logits, const void* w, void* out, int dtype, int T, int E, int H, void* stream)
+// expert that has every row.  ld: elements from one row of d_logits to the next; those past E are zero, and the rows of w
+// that they would meet read as zeros.
+AMOE_EXPORT int amoe_router_input_grad_rows(const void* d_logits, int ld, const void* w, void* out, int dtype, int T, int E, int H,
+                                            void* stream)
 {
     AMOE_REQUIRE(d_logits && w && out, AMOE_ERR_BAD_ARG, "router_input_grad: null pointer");
     AMOE_REQUIRE(T > 0 && E > 0 && H > 0, AMOE_ERR_BAD_ARG, "router_input_grad: sizes must be positive (T=%d E=%d H=%d)", T, E, H);
+    AMOE_REQUIRE(ld >= E, AMOE_ERR_BAD_ARG, "router_input_grad: rows of %d elements for %d experts", ld, E);
     AMOE_REQUIRE(dtype == AMOE_BF16 || dtype == AMOE_F16, AMOE_ERR_UNSUPPORTED, "router_input_grad: bf16 and float16 only");
-    AMOE_REQUIRE(E % 32 == 0 && H % 8 == 0 && ((uintptr_t)d_logits | (uintptr_t)w | (uintptr_t)out) % 16 == 0, AMOE_ERR_UNSUPPORTED,
-                 "router_input_grad: E=%d must be a multiple of 32, H=%d of 8, the operands aligned to 16 bytes", E, H);
-    AMOE_REQUIRE((unsigned long long)T * E * 2ull < (1ull << 31) && (unsigned long long)E * H * 2ull < (1ull << 31), AMOE_ERR_UNSUPPORTED,
+    AMOE_REQUIRE(ld % 32 == 0 && H % 8 == 0 && ((uintptr_t)d_logits | (uintptr_t)w | (uintptr_t)out) % 16 == 0, AMOE_ERR_UNSUPPORTED,
+                 "router_input_grad: E=%d must be a multiple of 32, H=%d of 8, the operands aligned to 16 bytes", ld, H);
+    AMOE_REQUIRE((unsigned long long)T * ld * 2ull < (1ull << 31) && (unsigned long long)E * H * 2ull < (1ull << 31), AMOE_ERR_UNSUPPORTED,
                  "router_input_grad: operand of 2 GiB or more");
     GemmArgs a = {};
     a.A = (const bf16_t*)d_logits;
     a.B = (const bf16_t*)w;
     a.C = (bf16_t*)out;
     a.f16 = dtype == AMOE_F16;
-    a.lda = E;
+    a.lda = a.Kd = ld;
+    a.rows_total = E;
     a.ldb = a.ldc = a.N = H;
     a.E = 1;
-    a.Kd = E;
     a.M = T;
     if (T <= 16) return launch_skinny<1, 4, 8, EPI_STORE, 0>(a, 1, (hipStream_t)stream);
     return launch_skinny<2, 8, 4, EPI_STORE, 0>(a, (T + 31) / 32, (hipStream_t)stream);
+}
+
+AMOE_EXPORT int amoe_router_input_grad(const void* d_logits, const void* w, void* out, int dtype, int T, int E, int H, void* stream)
+{
+    return amoe_router_input_grad_rows(d_logits, E, w, out, dtype, T, E, H, stream);
 }

@@ -21,7 +21,11 @@ int amoe_launch_input_grad(const void* d_xp, const int32_t* row_of, const void* 
                            const void* gate, void* dx, int dtype, int T, int K, int H, hipStream_t s);
 int amoe_launch_gated_act_bwd_rows(const void* gate_up, const void* d_inter, const float* row_scale, void* d_gate_up, float* d_scale,
                                    int dtype, int R, int I, int act, hipStream_t s);
-int amoe_launch_sum_parts(const void* parts, int n_parts, void* out, int dtype, long long n, hipStream_t s);
+int amoe_launch_router_bwd(const float* d_scores, const float* probs, const int32_t* topk_idx, const int32_t* counts, int dtype, int T,
+                           int E, int K, int normalize, float lb_coeff, void* d_logits, int ld, hipStream_t s);
+int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map, const int32_t* offsets, void* C, int R,
+                    int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype, int lda, bool out32);
+int amoe_launch_sum_parts(const void* parts, int n_parts, void* out, int parts_dtype, int dtype, long long n, hipStream_t s);
 
 namespace {
 
@@ -256,9 +260,22 @@ AMOE_EXPORT int amoe_layer_fwd(const int32_t* config, int T, const void* x, cons
     return AMOE_OK;
 }
 
-AMOE_EXPORT int amoe_layer_bwd(const int32_t* config, int T, const void* x, const void* dy, const void* w_down, const void* saved,
-                               void* scratch, const float* d_scores_rows, float lb_coeff, void* d_w_gate_up, void* d_w_down,
-                               void* d_logits, void* stream, void* side_stream)
+// The forward pass that forms the logits [T,E] itself, of 16-bit x with rows of a multiple of 32.
+AMOE_EXPORT int amoe_layer_fwd_router(const int32_t* config, int T, const void* x, const void* router_gate, void* logits,
+                                      const int32_t* assign, const void* w_gate_up, const void* w_down, const void* sh_gate_up,
+                                      const void* sh_down, const void* sh_out_gate, const int32_t* all_rows, void* saved, int keep,
+                                      void* scratch, void* y, int stages, void* stream)
+{
+    Shape c;
+    AMOE_TRY(read_shape("layer_fwd_router", config, T, &c));
+    if (stages & AMOE_STAGE_ROUTE) AMOE_TRY(amoe_router_logits(x, router_gate, logits, c.dtype, T, c.E, c.H, stream));
+    return amoe_layer_fwd(config, T, x, logits, c.dtype, assign, w_gate_up, w_down, sh_gate_up, sh_down, sh_out_gate, all_rows, saved,
+                          keep, scratch, y, stages, stream);
+}
+
+static int layer_bwd(const int32_t* config, int T, const void* x, const void* dy, const void* w_down, const void* saved, void* scratch,
+                     const float* d_scores_rows, float lb_coeff, void* d_w_gate_up, void* d_w_down, void* d_logits, int ld, void* stream,
+                     void* side_stream)
 {
     Shape c;
     AMOE_TRY(read_shape("layer_bwd", config, T, &c));
@@ -300,7 +317,39 @@ AMOE_EXPORT int amoe_layer_bwd(const int32_t* config, int T, const void* x, cons
                                         false, main));
     else if (d_scores_rows)
         AMOE_TRY(amoe_launch_score_grad(nullptr, 0, d_scores_rows, s.row_of, w.d_scores, R, true, main));
-    return amoe_router_bwd(w.d_scores, s.probs, s.topk_idx, s.counts, c.dtype, T, c.E, c.K, c.normalize, lb_coeff, d_logits, stream);
+    return amoe_launch_router_bwd(w.d_scores, s.probs, s.topk_idx, s.counts, c.dtype, T, c.E, c.K, c.normalize, lb_coeff, d_logits,
+                                  ld ? ld : c.E, main);
+}
+
+AMOE_EXPORT int amoe_layer_bwd(const int32_t* config, int T, const void* x, const void* dy, const void* w_down, const void* saved,
+                               void* scratch, const float* d_scores_rows, float lb_coeff, void* d_w_gate_up, void* d_w_down,
+                               void* d_logits, void* stream, void* side_stream)
+{
+    return layer_bwd(config, T, x, dy, w_down, saved, scratch, d_scores_rows, lb_coeff, d_w_gate_up, d_w_down, d_logits, 0, stream,
+                     side_stream);
+}
+
+// The same with rows of d_logits that are a multiple of 32 long, whatever E is (what is past E: zeros), so that the
+// router's gradients run on kernels that read 8 or 32 elements at a time, and with the router's weight gradient [E,H] in
+// the same call (see amoe_dense_wgrad for the chunks; the parts [splits][E][H] are float32).
+AMOE_EXPORT int amoe_layer_bwd_router(const int32_t* config, int T, const void* x, const void* dy, const void* w_down, const void* saved,
+                                      void* scratch, const float* d_scores_rows, float lb_coeff, void* d_w_gate_up, void* d_w_down,
+                                      void* d_logits, const int32_t* chunk_offsets, int splits, void* parts, void* d_router_gate,
+                                      void* stream, void* side_stream)
+{
+    Shape c;
+    AMOE_TRY(read_shape("layer_bwd_router", config, T, &c));
+    AMOE_REQUIRE(c.dtype != AMOE_F32, AMOE_ERR_UNSUPPORTED, "layer_bwd_router: bf16 and float16 only");
+    AMOE_REQUIRE(c.H % 8 == 0, AMOE_ERR_UNSUPPORTED, "layer_bwd_router: H=%d must be a multiple of 8", c.H);
+    const int ld = (c.E + 31) / 32 * 32;
+    AMOE_TRY(layer_bwd(config, T, x, dy, w_down, saved, scratch, d_scores_rows, lb_coeff, d_w_gate_up, d_w_down, d_logits, ld, stream,
+                       side_stream));
+    if (!d_router_gate) return AMOE_OK;
+    AMOE_REQUIRE(chunk_offsets && splits > 0 && (splits == 1 || parts), AMOE_ERR_BAD_ARG, "layer_bwd_router: null pointer");
+    AMOE_TRY(amoe_bf16_wgrad(d_logits, nullptr, x, nullptr, chunk_offsets, splits > 1 ? parts : d_router_gate, T, splits, c.E, c.H, 1,
+                             (hipStream_t)stream, c.dtype, ld, splits > 1));
+    if (splits == 1) return AMOE_OK;
+    return amoe_launch_sum_parts(parts, splits, d_router_gate, AMOE_F32, c.dtype, (long long)c.E * c.H, (hipStream_t)stream);
 }
 
 // C [Kd,N] = A [T,Kd]^T @ B [T,N], the weight gradient of a map that every token takes: few output tiles and a deep
@@ -313,7 +362,7 @@ AMOE_EXPORT int amoe_dense_wgrad(const void* A, const void* B, const int32_t* ch
     AMOE_TRY(amoe_grouped_gemm_wgrad(A, nullptr, B, nullptr, chunk_offsets, splits > 1 ? parts : C, dtype, T, splits, Kd, N, tile_cfg,
                                      stream));
     if (splits == 1) return AMOE_OK;
-    return amoe_launch_sum_parts(parts, splits, C, dtype, (long long)Kd * N, (hipStream_t)stream);
+    return amoe_launch_sum_parts(parts, splits, C, dtype, dtype, (long long)Kd * N, (hipStream_t)stream);
 }
 
 AMOE_EXPORT int amoe_layer_bwd_shared(const int32_t* config, int T, const void* x, const void* dy, const void* sh_down,

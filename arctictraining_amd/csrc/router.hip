@@ -28,7 +28,7 @@ template <typename T, int VPT>
 __global__ void __launch_bounds__(kTokensPerBlock * AMOE_WAVE)
 router_bwd_kernel(const float* __restrict__ d_scores, const float* __restrict__ probs,
                   const int32_t* __restrict__ topk_idx, const int32_t* __restrict__ counts, int n_tokens, int E,
-                  int K, int normalize, float lb_coeff, T* __restrict__ d_logits)
+                  int K, int normalize, float lb_coeff, T* __restrict__ d_logits, int ld)
 {
     const int lane = threadIdx.x & 63;
     const int t = blockIdx.x * kTokensPerBlock + (threadIdx.x >> 6);
@@ -76,11 +76,11 @@ router_bwd_kernel(const float* __restrict__ d_scores, const float* __restrict__ 
 #pragma unroll
     for (int j = 0; j < VPT; ++j) part += p[j] * dp[j];
     const float inner = wave_sum(part);
-    T* out = d_logits + (size_t)t * E;
+    T* out = d_logits + (size_t)t * ld;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         int e = lane + 64 * j;
-        if (e < E) ElemTraits<T>::store1(out + e, p[j] * (dp[j] - inner));
+        if (e < ld) ElemTraits<T>::store1(out + e, e < E ? p[j] * (dp[j] - inner) : 0.f);
     }
 }
 
@@ -111,19 +111,26 @@ AMOE_EXPORT int amoe_router_topk_fwd(const void* logits, int dtype, int T, int E
     return amoe_check_launch("router_topk_fwd");
 }
 
-AMOE_EXPORT int amoe_router_bwd(const float* d_scores, const float* probs, const int32_t* topk_idx,
-                                const int32_t* counts, int dtype, int T, int E, int K, int normalize, float lb_coeff,
-                                void* d_logits, void* stream)
+// ld: elements from one row of d_logits to the next, at most 32 past E; those past E are set to zero
+int amoe_launch_router_bwd(const float* d_scores, const float* probs, const int32_t* topk_idx, const int32_t* counts, int dtype, int T,
+                           int E, int K, int normalize, float lb_coeff, void* d_logits, int ld, hipStream_t s)
 {
     AMOE_REQUIRE(d_scores && probs && topk_idx && counts && d_logits, AMOE_ERR_BAD_ARG, "router_bwd: null pointer");
     AMOE_REQUIRE(dtype == AMOE_F32 || dtype == AMOE_BF16 || dtype == AMOE_F16, AMOE_ERR_BAD_ARG, "router_bwd: bad dtype %d", dtype);
     int rc = check_router_shape(T, E, K);
     if (rc) return rc;
+    AMOE_REQUIRE(ld >= E && ld <= (E + 31) / 32 * 32, AMOE_ERR_BAD_ARG, "router_bwd: rows of %d elements for %d experts", ld, E);
     dim3 grid((T + kTokensPerBlock - 1) / kTokensPerBlock), block(kTokensPerBlock * AMOE_WAVE);
-    hipStream_t s = (hipStream_t)stream;
     ROUTER_DISPATCH_VPT(E, {
         AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL((router_bwd_kernel<ELEM, VPT>), grid, block, 0, s, d_scores, probs,
-                                                     topk_idx, counts, T, E, K, normalize, lb_coeff, (ELEM*)d_logits))
+                                                     topk_idx, counts, T, E, K, normalize, lb_coeff, (ELEM*)d_logits, ld))
     })
     return amoe_check_launch("router_bwd");
+}
+
+AMOE_EXPORT int amoe_router_bwd(const float* d_scores, const float* probs, const int32_t* topk_idx,
+                                const int32_t* counts, int dtype, int T, int E, int K, int normalize, float lb_coeff,
+                                void* d_logits, void* stream)
+{
+    return amoe_launch_router_bwd(d_scores, probs, topk_idx, counts, dtype, T, E, K, normalize, lb_coeff, d_logits, E, (hipStream_t)stream);
 }

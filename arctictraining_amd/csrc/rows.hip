@@ -292,18 +292,19 @@ column_sum_kernel(const float* __restrict__ parts, int n_parts, T* __restrict__ 
 inline int column_grad_chunk(int T) { return T <= 64 * 64 ? 64 : (T + 63) / 64; }
 
 // out[i] = sum_p parts[p][i] in float32, one rounding
-template <typename T>
+template <typename P, typename T>
 __global__ void __launch_bounds__(kBlock)
-sum_parts_kernel(const T* __restrict__ parts, int n_parts, T* __restrict__ out, long long n_vec)
+sum_parts_kernel(const P* __restrict__ parts, int n_parts, T* __restrict__ out, long long n_vec)
 {
-    constexpr int V = ElemTraits<T>::kVec;
+    constexpr int V = ElemTraits<T>::kVec, W = V / ElemTraits<P>::kVec;
     const u32x4_t* src = reinterpret_cast<const u32x4_t*>(parts);
     for (long long i = blockIdx.x * (long long)kBlock + threadIdx.x; i < n_vec; i += (long long)gridDim.x * kBlock) {
         float acc[V] = {};
 #pragma unroll 4
         for (int p = 0; p < n_parts; ++p) {
             float f[V];
-            ElemTraits<T>::unpack(src[p * n_vec + i], f);
+#pragma unroll
+            for (int w = 0; w < W; ++w) ElemTraits<P>::unpack(src[(p * n_vec + i) * W + w], f + w * ElemTraits<P>::kVec);
 #pragma unroll
             for (int j = 0; j < V; ++j) acc[j] += f[j];
         }
@@ -476,14 +477,20 @@ int amoe_launch_input_grad(const void* d_xp, const int32_t* row_of, const void* 
     return amoe_check_launch("input_grad");
 }
 
-int amoe_launch_sum_parts(const void* parts, int n_parts, void* out, int dtype, long long n, hipStream_t s)
+int amoe_launch_sum_parts(const void* parts, int n_parts, void* out, int parts_dtype, int dtype, long long n, hipStream_t s)
 {
     const int vec = dtype != AMOE_F32 ? 8 : 4;
     AMOE_REQUIRE(n % vec == 0, AMOE_ERR_UNSUPPORTED, "sum_parts: %lld elements are no multiple of %d", n, vec);
     const long long blocks = (n / vec + kBlock - 1) / kBlock;
     const dim3 grid((unsigned)(blocks < 8192 ? blocks : 8192));
-    AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL(sum_parts_kernel<ELEM>, grid, dim3(kBlock), 0, s, (const ELEM*)parts, n_parts,
-                                                 (ELEM*)out, n / vec))
+    if (parts_dtype == AMOE_F32) {
+        AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL((sum_parts_kernel<float, ELEM>), grid, dim3(kBlock), 0, s, (const float*)parts,
+                                                     n_parts, (ELEM*)out, n / vec))
+    } else {
+        AMOE_REQUIRE(parts_dtype == dtype, AMOE_ERR_BAD_ARG, "sum_parts: parts of another type");
+        AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL((sum_parts_kernel<ELEM, ELEM>), grid, dim3(kBlock), 0, s, (const ELEM*)parts,
+                                                     n_parts, (ELEM*)out, n / vec))
+    }
     return amoe_check_launch("sum_parts");
 }
 

@@ -186,12 +186,12 @@ _ROUTER_KERNEL_WORK = 1 << 18
 
 def _router_kernel_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether a product of a [T, .] with the router's weight w [E,H] may run on the package's kernels: few tokens, both
-    dense, of one 16-bit type, on one device, aligned, and no autocast that would change a type."""
+    dense (a: its rows), of one 16-bit type, on one device, aligned, and no autocast that would change a type."""
     return (
         -(-a.shape[0] // 16) * -(-w.shape[0] // 16) * w.shape[1] <= _ROUTER_KERNEL_WORK
         and a.dtype in (torch.bfloat16, torch.float16)
         and w.dtype is a.dtype
-        and a.is_contiguous()
+        and a.stride(1) == 1
         and w.is_contiguous()
         and w.get_device() == a.get_device()
         and (a.data_ptr() | w.data_ptr()) % 16 == 0
@@ -203,9 +203,18 @@ def _router_logits(x: torch.Tensor, router_gate: torch.Tensor) -> torch.Tensor:
     """x [T,H] @ router_gate [E,H]^T (moe.py:233)."""
     # (longer rows are more than 12 steps in a row for a wavefront of the kernel: 64 tokens, H = 7168 11.8 us against 7.5,
     # H = 5728 7.5 against 13.0)
-    if _router_kernel_fits(x, router_gate) and x.shape[1] == router_gate.shape[1] <= 6144 and x.shape[1] % 32 == 0:
+    if _router_logits_fit(x, router_gate):
         return ops.router_logits(x, router_gate)
     return torch.matmul(x, router_gate.t())
+
+
+def _router_logits_fit(x: torch.Tensor, router_gate: torch.Tensor) -> bool:
+    return (
+        x.shape[1] == router_gate.shape[1] <= 6144
+        and x.shape[1] % 32 == 0
+        and x.is_contiguous()
+        and _router_kernel_fits(x, router_gate)
+    )
 
 
 def _fit_logits(logits: torch.Tensor, opts, pad: bool = True) -> torch.Tensor:
@@ -219,10 +228,11 @@ def _fit_logits(logits: torch.Tensor, opts, pad: bool = True) -> torch.Tensor:
     return F.pad(logits, (0, E - n), value=float("-inf")) if pad else logits
 
 
-def _router_input_grad(d_logits: torch.Tensor, router_gate: torch.Tensor) -> torch.Tensor:
-    """d_logits [T,E] @ router_gate [E,H] (autograd of moe.py:233)."""
+def _router_input_grad(d_logits: torch.Tensor, router_gate: torch.Tensor, padded: bool = False) -> torch.Tensor:
+    """d_logits [T,E] @ router_gate [E,H] (autograd of moe.py:233).  padded: the rows of d_logits are a multiple of 32 elements
+    apart, with zeros between them."""
     E, H = router_gate.shape
-    if E % 32 == 0 and H % 8 == 0 and _router_kernel_fits(d_logits, router_gate):
+    if (padded or (E % 32 == 0 and d_logits.is_contiguous())) and H % 8 == 0 and _router_kernel_fits(d_logits, router_gate):
         return ops.router_input_grad(d_logits, router_gate)
     return torch.matmul(d_logits, router_gate)
 
@@ -301,6 +311,19 @@ def _saved_view(saved, name, config_key, T: int):
     return saved[start : start + 4 * math.prod(shape)].view(dtype).view(shape)
 
 
+@functools.lru_cache(maxsize=256)
+def _overlap_pays(config_key, T: int) -> bool:
+    """Whether the expert weight gradients go on the second stream.  The events that order the streams cost the host 40-60 us a
+    step; a step that the GPU takes less time for than the host is longer by that much (20 of 60 steps drawn over the sizes of
+    this layer: 12-39 %), one that it takes longer for is mostly 3-15 % shorter with the second stream.  The line lies where
+    the products at 800 TFLOP/s (float32 100) and the weights, read twice and their gradients written, at 3 TB/s make 150 us:
+    T=556 H=1760 E=8 K=6 I=672 (129 us) 268 us with it, 228 without; T=95 H=2336 E=12 K=2 I=1536 (188) 274 and 299."""
+    E, K, H, I, dtype, shared = *config_key[:4], config_key[5], config_key[8]
+    size, rate = (4, 1e8) if dtype == ops.F32 else (2, 8e8)
+    rows = T * K + (T if shared else 0)
+    return 18.0 * rows * H * I / rate + 6.0 * size * (E + (1 if shared else 0)) * H * I / 3e6 > 150.0
+
+
 def _check_operand(t, name, like, shape) -> None:
     """t has to be dense, of `like`'s type, on the current device (like's), and of the given shape."""
     if t.dtype is not like.dtype or t.get_device() != like.get_device() or not t.is_contiguous():
@@ -331,21 +354,30 @@ def _layer_forward(x, router_gate, w_gate_up, w_down, shared, replay, opts, keep
     sizes = _layer_sizes(key, T, keep)
     if timers.wall_clock_breakdown:
         timers.start("router")
-    logits = routed = _router_logits(x, router_gate)
-    if routed.shape != (T, E) or not routed.is_contiguous():
-        logits = _fit_logits(routed, opts).contiguous()
+    # few tokens: the logits are formed inside the native call, behind its scratch; else the library's product
+    native = router_gate.shape[0] == E and _router_logits_fit(x, router_gate)
+    if not native:
+        logits = routed = _router_logits(x, router_gate)
+        if routed.shape != (T, E) or not routed.is_contiguous():
+            logits = _fit_logits(routed, opts).contiguous()
     assign = None if replay is None else _replayed(replay, T, opts)
     y = torch.empty_like(x)
-    buf = torch.empty(sizes[0] + (0 if keep else sizes[1]), dtype=torch.uint8, device=x.device)
+    extra = T * E * x.element_size() if native else 0
+    buf = torch.empty(sizes[0] + (0 if keep else sizes[1] + extra), dtype=torch.uint8, device=x.device)
     base = buf.data_ptr()
-    scratch = torch.empty(sizes[1], dtype=torch.uint8, device=x.device) if keep else None
+    scratch = torch.empty(sizes[1] + extra, dtype=torch.uint8, device=x.device) if keep else None
+    scratch_ptr = scratch.data_ptr() if keep else base + sizes[0]
 
     def run(stages):
+        if native:
+            call, routing = _lib.load().amoe_layer_fwd_router, (router_gate.data_ptr(), scratch_ptr + sizes[1])
+        else:
+            call, routing = _lib.load().amoe_layer_fwd, (logits.data_ptr(), ops._dtype_code(logits))
         _lib.check(
-            _lib.load().amoe_layer_fwd(
-                _layer_config(*key), T, x.data_ptr(), logits.data_ptr(), ops._dtype_code(logits), ops._ptr(assign),
+            call(
+                _layer_config(*key), T, x.data_ptr(), *routing, ops._ptr(assign),
                 w_gate_up.data_ptr(), w_down.data_ptr(), ops._ptr(sh_gate_up), ops._ptr(sh_down), ops._ptr(sh_out_gate),
-                ops._ptr(all_rows), base, keep, scratch.data_ptr() if keep else base + sizes[0], y.data_ptr(), stages, ops._stream(),
+                ops._ptr(all_rows), base, keep, scratch_ptr, y.data_ptr(), stages, ops._stream(),
             ),
             "amoe_layer_fwd",
         )
@@ -363,6 +395,9 @@ def _layer_forward(x, router_gate, w_gate_up, w_down, shared, replay, opts, keep
             timers.stop(name)
     cap = opts.get("capture")
     if cap is not None:
+        if native:
+            at = sizes[1] if keep else sizes[0] + sizes[1]
+            routed = (scratch if keep else buf)[at : at + extra].view(x.dtype).view(T, E).clone()
         cap.update(logits=routed, **{n: _saved_view(buf, n, key, T).clone() for n in _SAVED_FIELDS if n != "scores_perm"})
     return y, buf, key
 
@@ -400,13 +435,14 @@ class _ExpertLayerFn(torch.autograd.Function):
         # starts on them behind everything the main stream has queued up to their operands, and the main
         # stream waits for it at the end, so the tensors either stream uses outlive the kernels that use them.
         overlap = ctx.opts["overlap_weight_grads"] and (ctx.needs_input_grad[2] or ctx.needs_input_grad[3])
-        side = _side_stream(ctx.device) if overlap else None
+        side = _side_stream(ctx.device) if overlap and _overlap_pays(ctx.key, ctx.tokens) else None
         try:
             return _ExpertLayerFn._backward(ctx, dy, ds_perm, None if side is None else side.cuda_stream)
         except BaseException:
-            # (memory may run out between the fork and the join: what is freed here is used again on the main stream)
-            if side is not None:
-                torch.cuda.current_stream(side.device).wait_stream(side)
+            # (memory may run out between the fork and the join: what is freed here is used again on the main stream; of a
+            # second stream without work the wait is nothing)
+            if overlap:
+                torch.cuda.current_stream(ctx.device).wait_stream(_side_stream(ctx.device))
             raise
 
     @staticmethod
@@ -433,19 +469,38 @@ class _ExpertLayerFn(torch.autograd.Function):
         scratch = torch.empty(_layer_sizes(key, T, True)[2], dtype=torch.uint8, device=x.device)
         d_w_gate_up = torch.empty_like(w_gate_up) if need[2] else None
         d_w_down = torch.empty_like(w_down) if need[3] else None
-        d_logits = torch.empty((T, E), dtype=x.dtype, device=x.device)
         if ds_perm is not None:
             ds_perm = ds_perm.float().contiguous()
-        _lib.check(
-            lib.amoe_layer_bwd(
-                config, T, x.data_ptr(), dy.data_ptr(), w_down.data_ptr(), saved.data_ptr(), scratch.data_ptr(), ops._ptr(ds_perm),
-                opts["loss_coeff"] / T / opts["ep_size"], ops._ptr(d_w_gate_up), ops._ptr(d_w_down), d_logits.data_ptr(), stream, side,
-            ),
-            "amoe_layer_bwd",
-        )
-        if router_gate.shape[0] != E:
-            d_logits = d_logits[:, : router_gate.shape[0]].contiguous()
-        d_router_gate = _router_weight_grad(d_logits, x) if need[1] else None
+        bwd = (config, T, x.data_ptr(), dy.data_ptr(), w_down.data_ptr(), saved.data_ptr(), scratch.data_ptr(), ops._ptr(ds_perm),
+               opts["loss_coeff"] / T / opts["ep_size"], ops._ptr(d_w_gate_up), ops._ptr(d_w_down))
+        # 16 bits: rows of d_logits of a multiple of 32 (zeros past E), whatever E is, and the router's weight gradient in
+        # the same call
+        padded = x.dtype is not torch.float32 and router_gate.shape == (E, H) and router_gate.dtype is x.dtype
+        d_router_gate = None
+        if padded:
+            d_logits = torch.empty((T, -(-E // 32) * 32), dtype=x.dtype, device=x.device)
+            chunks = parts = None
+            splits = 1
+            if need[1]:
+                d_router_gate = torch.empty((E, H), dtype=x.dtype, device=x.device)
+                splits = _dense_splits(T, E, H, x.dtype, 128)
+                chunks = _token_offsets(T, splits, x.device)
+                parts = torch.empty(splits * E * H, dtype=torch.float32, device=x.device) if splits > 1 else None
+            _lib.check(
+                lib.amoe_layer_bwd_router(
+                    *bwd, d_logits.data_ptr(), ops._ptr(chunks), splits, ops._ptr(parts), ops._ptr(d_router_gate), stream, side
+                ),
+                "amoe_layer_bwd",
+            )
+            if d_logits.shape[1] != E:
+                d_logits = d_logits[:, :E]
+        else:
+            d_logits = torch.empty((T, E), dtype=x.dtype, device=x.device)
+            _lib.check(lib.amoe_layer_bwd(*bwd, d_logits.data_ptr(), stream, side), "amoe_layer_bwd")
+            if router_gate.shape[0] != E:
+                d_logits = d_logits[:, : router_gate.shape[0]].contiguous()
+            if need[1]:
+                d_router_gate = _router_weight_grad(d_logits, x)
         cap = opts.get("capture")
         if cap is not None:
             start = _layer_sizes(key, T, True)[-1]
@@ -473,7 +528,7 @@ class _ExpertLayerFn(torch.autograd.Function):
         dx = dx_router = None
         if need[0]:
             dx = torch.empty_like(x)
-            dx_router = _router_input_grad(d_logits, router_gate)
+            dx_router = _router_input_grad(d_logits, router_gate, padded)
         if dx is not None or side is not None:
             _lib.check(
                 lib.amoe_layer_bwd_input(
@@ -605,7 +660,8 @@ class ArcticMoE(nn.Module):
         tile_cfg: tile shape of the grouped GEMMs (0 = the library's default; 1, 2, 3, 5 for tuning)
         check_replay: raise on a replayed expert id outside [0, E), as the reference's one_hot does
                 (one host synchronisation per replayed forward; skipped under graph capture)
-        overlap_weight_grads: run the two expert weight gradients of the backward on a second stream
+        overlap_weight_grads: run the two expert weight gradients of the backward on a second stream where the step is long
+                enough for it to pay
         capture: a dict that receives the routing intermediates of each forward (tests)
     """
 

@@ -78,15 +78,18 @@ def router_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def router_input_grad(d_logits: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """d_logits [T,E] @ w [E,H] in bf16 or float16, E a multiple of 32 and H of 8."""
-    _chk(d_logits, "d_logits")
+    """d_logits [T,E] @ w [E,H] in bf16 or float16, H a multiple of 8; the rows of d_logits are a multiple of 32 elements
+    apart, what stands between them (E no such multiple) is zeros."""
+    _chk(d_logits, "d_logits", contiguous=False)
     _chk(w, "w", d_logits.dtype)
     (T, E), H = d_logits.shape, w.shape[1]
     if w.shape[0] != E:
         raise RuntimeError(f"w must be [{E}, H], got {list(w.shape)}")
+    if d_logits.stride(1) != 1 or (T > 1 and d_logits.stride(0) < E):
+        raise RuntimeError("d_logits must have dense rows")
     out = torch.empty((T, H), dtype=w.dtype, device=w.device)
-    rc = _lib.load().amoe_router_input_grad(
-        d_logits.data_ptr(), w.data_ptr(), out.data_ptr(), _dtype_code(w), T, E, H, _stream()
+    rc = _lib.load().amoe_router_input_grad_rows(
+        d_logits.data_ptr(), d_logits.stride(0), w.data_ptr(), out.data_ptr(), _dtype_code(w), T, E, H, _stream()
     )
     _lib.check(rc, "amoe_router_input_grad")
     return out

@@ -74,6 +74,8 @@ int amoe_router_logits(const void* x, const void* w, void* logits, int dtype, in
  * Its input gradient for few tokens: out [T,H] = d_logits [T,E] @ w [E,H], bf16 or float16; E a multiple of 32, H of 8.
  */
 int amoe_router_input_grad(const void* d_logits, const void* w, void* out, int dtype, int T, int E, int H, void* stream);
+/* the same with rows of d_logits `ld` elements long (a multiple of 32), zeros past E, for any E */
+int amoe_router_input_grad_rows(const void* d_logits, int ld, const void* w, void* out, int dtype, int T, int E, int H, void* stream);
 
 /*
  * Router backward.  Replaces top_k_gating_bwd (top_k_gating.h:24-28,
@@ -281,8 +283,11 @@ int amoe_gated_act_bwd(const void* gate_up, const void* d_inter, const float* ro
  *   amoe_layer_fwd: y [T,H] from x [T,H] and logits [T,E] (of logits_dtype); assign [T,K] i32 or null replaces the
  *   selected experts.  stages: which of the AMOE_STAGE_* steps to run, in this order.  With config.shared: the shared
  *   expert's gate_up [H,2I], down [I,H] and output gate [H,1] (moe.py:305-314), all_rows = int32 {0, T} on the device.
+ *   amoe_layer_fwd_router: the same from the router's weights [E,H]; it writes the logits [T,E] (see amoe_router_logits).
  *   amoe_layer_bwd: d_logits [T,E] and, where not null, the experts' weight gradients (on side_stream if that is not
  *   null) from dy [T,H]; d_scores_rows [R] f32 or null: gradient of the row-ordered scores; saved made with keep = 1.
+ *   amoe_layer_bwd_router: the same in 16 bits with d_logits [T, E rounded up to 32], zeros past E, and the router's weight
+ *   gradient [E,H] where not null; chunk_offsets and splits as in amoe_dense_wgrad, parts [splits][E][H] in float32.
  *   amoe_layer_bwd_shared: the shared expert's weight gradients where not null, and d_pre [T] (gradient in front
  *   of its sigmoid).  *_chunks / *_splits / parts: see amoe_dense_wgrad; parts holds the larger of the two.
  *   amoe_layer_bwd_input: dx [T,H] (skipped if null) from dx_router [T,H] = d_logits @ router weights and what the
@@ -298,9 +303,17 @@ int amoe_layer_fwd(const int32_t* config, int T, const void* x, const void* logi
                    const void* w_gate_up, const void* w_down, const void* sh_gate_up, const void* sh_down,
                    const void* sh_out_gate, const int32_t* all_rows, void* saved, int keep, void* scratch, void* y, int stages,
                    void* stream);
+int amoe_layer_fwd_router(const int32_t* config, int T, const void* x, const void* router_gate, void* logits,
+                          const int32_t* assign, const void* w_gate_up, const void* w_down, const void* sh_gate_up,
+                          const void* sh_down, const void* sh_out_gate, const int32_t* all_rows, void* saved, int keep,
+                          void* scratch, void* y, int stages, void* stream);
 int amoe_layer_bwd(const int32_t* config, int T, const void* x, const void* dy, const void* w_down, const void* saved,
                    void* scratch, const float* d_scores_rows, float lb_coeff, void* d_w_gate_up, void* d_w_down,
                    void* d_logits, void* stream, void* side_stream);
+int amoe_layer_bwd_router(const int32_t* config, int T, const void* x, const void* dy, const void* w_down, const void* saved,
+                          void* scratch, const float* d_scores_rows, float lb_coeff, void* d_w_gate_up, void* d_w_down,
+                          void* d_logits, const int32_t* chunk_offsets, int splits, void* parts, void* d_router_gate,
+                          void* stream, void* side_stream);
 int amoe_layer_bwd_shared(const int32_t* config, int T, const void* x, const void* dy, const void* sh_down,
                           const int32_t* all_rows, const void* saved, void* scratch, void* parts,
                           const int32_t* gate_up_chunks, int gate_up_splits, void* d_sh_gate_up,

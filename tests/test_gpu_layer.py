@@ -334,6 +334,20 @@ def test_weight_gradients_on_the_second_stream_match_the_serial_order(gpu_device
                 assert torch.equal(serial[k], both[k]), f"{k}, seed {seed}, repetition {rep}"
 
 
+def test_second_stream_at_any_size(gpu_device, monkeypatch):
+    """The comparison with the serial order above and the graph capture below, on the second stream also where the layer would
+    not use it."""
+    from arctictraining_amd import moe
+
+    monkeypatch.setattr(moe, "_overlap_pays", lambda *a: True)
+    used = []
+    stream = moe._side_stream
+    monkeypatch.setattr(moe, "_side_stream", lambda device: used.append(device) or stream(device))
+    test_weight_gradients_on_the_second_stream_match_the_serial_order(gpu_device)
+    test_layer_under_hip_graph_capture(gpu_device)
+    assert len(used) > 10
+
+
 def test_module_surface(gpu_device):
     """Names, shapes and attributes the reference's callers rely on (moe.py:91-130,
     utils.py:61-68, 350-369, 449-461)."""

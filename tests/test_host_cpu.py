@@ -48,6 +48,16 @@ def test_layer_without_gate_parameter_shapes():
     assert tuple(gated.expert_gate_up.shape) == (4, 8, 12)
 
 
+def test_second_stream_only_for_long_steps():
+    """The layer's key is (E, K, H, I, act, dtype, normalize, tile_cfg, shared)."""
+    assert moe._overlap_pays((128, 8, 2048, 768, 0, 1, True, 0, False), 16384)
+    assert moe._overlap_pays((128, 8, 2048, 768, 0, 1, True, 0, False), 64)      # (the weights alone)
+    assert moe._overlap_pays((8, 2, 512, 1024, 0, 0, True, 0, False), 2048)
+    assert not moe._overlap_pays((46, 2, 640, 288, 0, 1, True, 0, False), 68)
+    assert not moe._overlap_pays((8, 2, 512, 1024, 0, 0, True, 0, False), 64)
+    assert moe._overlap_pays((5, 1, 864, 11648, 0, 2, True, 0, True), 744)
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU: --gpus above 1 exits with a message and without touching a device."""
     import os
