@@ -1184,11 +1184,15 @@ grouped_gemm_wgrad_f16_kernel(GemmArgs p)
 }
 
 // partial sums in float32
-template <typename ET>
 __global__ void __launch_bounds__(256)
-grouped_gemm_wgrad_parts_kernel(GemmArgs p)
+grouped_gemm_wgrad_parts_bf16_kernel(GemmArgs p)
 {
-    grouped_gemm_wgrad_body<128, 128, 2, 2, 0, ET, true>(p);
+    grouped_gemm_wgrad_body<128, 128, 2, 2, 0, bf16_t, true>(p);
+}
+__global__ void __launch_bounds__(256)
+grouped_gemm_wgrad_parts_f16_kernel(GemmArgs p)
+{
+    grouped_gemm_wgrad_body<128, 128, 2, 2, 0, f16_t, true>(p);
 }
 
 template <int BM, int BN, int WGM, int WGN, bool B_KC, int EPI, int ACT>
@@ -1565,8 +1569,8 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
     if (out32) {
         constexpr int lds_bytes = NSTAGE * (128 + 128) * BK * 2;
         AMOE_REQUIRE(tile_cfg == 1 && !a_row_map && !b_row_map, AMOE_ERR_BAD_ARG, "grouped_gemm_wgrad: float32 sums of gathered rows");
-        if (a.f16) return launch_kernel<grouped_gemm_wgrad_parts_kernel<f16_t>, 256, lds_bytes>(a, (int)grid, s);
-        return launch_kernel<grouped_gemm_wgrad_parts_kernel<bf16_t>, 256, lds_bytes>(a, (int)grid, s);
+        if (a.f16) return launch_kernel<grouped_gemm_wgrad_parts_f16_kernel, 256, lds_bytes>(a, (int)grid, s);
+        return launch_kernel<grouped_gemm_wgrad_parts_bf16_kernel, 256, lds_bytes>(a, (int)grid, s);
     }
     if (a_row_map) return launch_any<false, false, EPI_STORE, 0, 1>(a, tile_cfg, (int)grid, s);
     if (b_row_map) return launch_any<false, false, EPI_STORE, 0, 2>(a, tile_cfg, (int)grid, s);
