@@ -20,7 +20,7 @@ LIB_PATH = os.path.join(LIB_DIR, "libarctic_moe_hip.so")
 
 # (source, object name, extra flags); the 16-bit grouped GEMM is compiled as four groups of entry points in parallel
 GEMM_PARTS = 4
-SOURCES = [(f, os.path.splitext(f)[0], []) for f in ("api.hip", "router.hip", "permute.hip", "rows.hip", "layer.hip", "gemm_skinny.hip", "gemm_f32.hip", "remap.hip")]
+SOURCES = [(f, os.path.splitext(f)[0], []) for f in ("api.hip", "router.hip", "permute.hip", "rows.hip", "layer.hip", "gemm_skinny.hip", "gemm_split.hip", "gemm_f32.hip", "remap.hip")]
 # the default tile shape of the same products: one group per epilogue, and the weight gradients
 PP_PARTS = 4
 SOURCES = [("gemm_pp.hip", f"gemm_pp_p{i}", [f"-DAMOE_PP_PART={i}"]) for i in range(PP_PARTS)] + SOURCES

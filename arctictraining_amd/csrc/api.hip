@@ -20,16 +20,19 @@ AMOE_EXPORT const char* amoe_last_error(void) { return g_err; }
 // implemented in gemm_bf16.hip / gemm_f32.hip / rows.hip
 int amoe_bf16_gateup_act(const void* xp, const int32_t* a_row_map, const void* w, const int32_t* offsets, void* gate_up,
                          void* inter, const float* row_scale, int R, int E, int H, int I, int act, void* workspace, size_t workspace_bytes,
-                         int tile_cfg, hipStream_t s, int dtype);
+                         int tile_cfg, hipStream_t s, int dtype, float* split, size_t split_bytes);
 int amoe_bf16_nn(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int R, int E,
-                 int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype);
+                 int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype, float* split,
+                 size_t split_bytes);
 int amoe_bf16_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int R, int E,
-                 int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype);
+                 int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype, float* split,
+                 size_t split_bytes);
 int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map,
                     const int32_t* offsets, void* C, int R, int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype, int lda, bool out32);
 int amoe_bf16_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down, const int32_t* offsets,
                            const void* gate_up, const float* row_scale, void* d_gate_up, float* partials, int R, int E,
-                           int I, int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype);
+                           int I, int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype,
+                           float* split, size_t split_bytes);
 int amoe_bf16_gated_bwd_parts(int I, int tile_cfg);
 size_t amoe_rows_map_bytes(int R, int E, int dtype, int tile_cfg);
 int amoe_f32_rows(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int R, int E,
@@ -73,11 +76,11 @@ int check_gemm_dims(const char* what, int dtype, int red, int other)
 
 }  // namespace
 
-AMOE_EXPORT int amoe_grouped_gemm_gateup_act_fwd(const void* xp, const int32_t* a_row_map, const void* w_gate_up,
+int amoe_run_gateup_act_fwd(const void* xp, const int32_t* a_row_map, const void* w_gate_up,
                                                  const int32_t* offsets, const float* row_scale, void* gate_up,
                                                  void* inter, int dtype, int R,
                                                  int E, int H, int I, int act, void* workspace, size_t workspace_bytes,
-                                                 int tile_cfg, void* stream)
+                                                 int tile_cfg, void* stream, float* split, size_t split_bytes)
 {
     const char* what = "grouped_gemm_gateup_act_fwd";
     AMOE_REQUIRE(xp && w_gate_up && offsets && inter && workspace, AMOE_ERR_BAD_ARG, "%s: null pointer", what);
@@ -93,7 +96,7 @@ AMOE_EXPORT int amoe_grouped_gemm_gateup_act_fwd(const void* xp, const int32_t* 
     hipStream_t s = (hipStream_t)stream;
     if (dtype != AMOE_F32)
         return amoe_bf16_gateup_act(xp, a_row_map, w_gate_up, offsets, gate_up, inter, row_scale, R, E, H, I, act, workspace,
-                                    workspace_bytes, tile_cfg, s, dtype);
+                                    workspace_bytes, tile_cfg, s, dtype, split, split_bytes);
     AMOE_REQUIRE(gate_up, AMOE_ERR_UNSUPPORTED, "%s: the f32 path needs the gate_up buffer", what);
     AMOE_REQUIRE(I % 4 == 0, AMOE_ERR_UNSUPPORTED, "%s: f32 intermediate size %d must be a multiple of 4", what, I);
     rc = amoe_f32_rows(xp, a_row_map, w_gate_up, offsets, gate_up, R, E, H, 2 * I, 2 * I, (long long)H * 2 * I, false,
@@ -102,9 +105,18 @@ AMOE_EXPORT int amoe_grouped_gemm_gateup_act_fwd(const void* xp, const int32_t* 
     return amoe_launch_gated_act_fwd(gate_up, row_scale, inter, dtype, R, I, act, s);
 }
 
-AMOE_EXPORT int amoe_grouped_gemm_nn(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
+AMOE_EXPORT int amoe_grouped_gemm_gateup_act_fwd(const void* xp, const int32_t* a_row_map, const void* w_gate_up,
+                                                 const int32_t* offsets, const float* row_scale, void* gate_up,
+                                                 void* inter, int dtype, int R,
+                                                 int E, int H, int I, int act, void* workspace, size_t workspace_bytes,
+                                                 int tile_cfg, void* stream)
+{
+    return amoe_run_gateup_act_fwd(xp, a_row_map, w_gate_up, offsets, row_scale, gate_up, inter, dtype, R, E, H, I, act, workspace, workspace_bytes, tile_cfg, stream, nullptr, 0);
+}
+
+int amoe_run_nn(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
                                      void* C, int dtype, int R, int E, int Kd, int N, void* workspace,
-                                     size_t workspace_bytes, int tile_cfg, void* stream)
+                                     size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes)
 {
     const char* what = "grouped_gemm_nn";
     AMOE_REQUIRE(A && B && offsets && C && workspace, AMOE_ERR_BAD_ARG, "%s: null pointer", what);
@@ -116,14 +128,21 @@ AMOE_EXPORT int amoe_grouped_gemm_nn(const void* A, const int32_t* a_row_map, co
                  "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_rows_map_bytes(R, E, dtype, tile_cfg));
     hipStream_t s = (hipStream_t)stream;
     if (dtype != AMOE_F32)
-        return amoe_bf16_nn(A, a_row_map, B, offsets, C, R, E, Kd, N, workspace, workspace_bytes, tile_cfg, s, dtype);
+        return amoe_bf16_nn(A, a_row_map, B, offsets, C, R, E, Kd, N, workspace, workspace_bytes, tile_cfg, s, dtype, split, split_bytes);
     return amoe_f32_rows(A, a_row_map, B, offsets, C, R, E, Kd, N, N, (long long)Kd * N, false, workspace,
                          workspace_bytes, (tile_cfg & AMOE_TILE_MAP_READY) != 0, s);
 }
 
-AMOE_EXPORT int amoe_grouped_gemm_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
+AMOE_EXPORT int amoe_grouped_gemm_nn(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
                                      void* C, int dtype, int R, int E, int Kd, int N, void* workspace,
                                      size_t workspace_bytes, int tile_cfg, void* stream)
+{
+    return amoe_run_nn(A, a_row_map, B, offsets, C, dtype, R, E, Kd, N, workspace, workspace_bytes, tile_cfg, stream, nullptr, 0);
+}
+
+int amoe_run_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
+                                     void* C, int dtype, int R, int E, int Kd, int N, void* workspace,
+                                     size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes)
 {
     const char* what = "grouped_gemm_nt";
     AMOE_REQUIRE(A && B && offsets && C && workspace, AMOE_ERR_BAD_ARG, "%s: null pointer", what);
@@ -135,9 +154,16 @@ AMOE_EXPORT int amoe_grouped_gemm_nt(const void* A, const int32_t* a_row_map, co
                  "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_rows_map_bytes(R, E, dtype, tile_cfg));
     hipStream_t s = (hipStream_t)stream;
     if (dtype != AMOE_F32)
-        return amoe_bf16_nt(A, a_row_map, B, offsets, C, R, E, Kd, N, workspace, workspace_bytes, tile_cfg, s, dtype);
+        return amoe_bf16_nt(A, a_row_map, B, offsets, C, R, E, Kd, N, workspace, workspace_bytes, tile_cfg, s, dtype, split, split_bytes);
     return amoe_f32_rows(A, a_row_map, B, offsets, C, R, E, /*Kred=*/N, /*N out=*/Kd, /*ldb=*/N, (long long)Kd * N, true,
                          workspace, workspace_bytes, (tile_cfg & AMOE_TILE_MAP_READY) != 0, s);
+}
+
+AMOE_EXPORT int amoe_grouped_gemm_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
+                                     void* C, int dtype, int R, int E, int Kd, int N, void* workspace,
+                                     size_t workspace_bytes, int tile_cfg, void* stream)
+{
+    return amoe_run_nt(A, a_row_map, B, offsets, C, dtype, R, E, Kd, N, workspace, workspace_bytes, tile_cfg, stream, nullptr, 0);
 }
 
 AMOE_EXPORT int amoe_grouped_gemm_wgrad(const void* A, const int32_t* a_row_map, const void* B,
@@ -163,11 +189,11 @@ AMOE_EXPORT int amoe_gated_bwd_score_parts(int I, int tile_cfg)
     return amoe_bf16_gated_bwd_parts(I, tile_cfg);
 }
 
-AMOE_EXPORT int amoe_grouped_gemm_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down,
+int amoe_run_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down,
                                                const int32_t* offsets, const void* gate_up, const float* row_scale,
                                                void* d_gate_up, float* score_partials, int dtype, int R, int E, int I,
                                                int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg,
-                                               void* stream)
+                                               void* stream, float* split, size_t split_bytes)
 {
     const char* what = "grouped_gemm_nt_gated_bwd";
     AMOE_REQUIRE(dy && w_down && offsets && gate_up && d_gate_up && workspace, AMOE_ERR_BAD_ARG, "%s: null pointer", what);
@@ -182,5 +208,14 @@ AMOE_EXPORT int amoe_grouped_gemm_nt_gated_bwd(const void* dy, const int32_t* a_
     AMOE_REQUIRE(workspace_bytes >= amoe_rows_map_bytes(R, E, dtype, tile_cfg), AMOE_ERR_WORKSPACE,
                  "%s: workspace %zu < %zu bytes", what, workspace_bytes, amoe_rows_map_bytes(R, E, dtype, tile_cfg));
     return amoe_bf16_nt_gated_bwd(dy, a_row_map, w_down, offsets, gate_up, row_scale, d_gate_up, score_partials, R, E, I, H,
-                                  act, workspace, workspace_bytes, tile_cfg, (hipStream_t)stream, dtype);
+                                  act, workspace, workspace_bytes, tile_cfg, (hipStream_t)stream, dtype, split, split_bytes);
+}
+
+AMOE_EXPORT int amoe_grouped_gemm_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down,
+                                               const int32_t* offsets, const void* gate_up, const float* row_scale,
+                                               void* d_gate_up, float* score_partials, int dtype, int R, int E, int I,
+                                               int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg,
+                                               void* stream)
+{
+    return amoe_run_nt_gated_bwd(dy, a_row_map, w_down, offsets, gate_up, row_scale, d_gate_up, score_partials, dtype, R, E, I, H, act, workspace, workspace_bytes, tile_cfg, stream, nullptr, 0);
 }

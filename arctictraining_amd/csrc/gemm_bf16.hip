@@ -1399,15 +1399,20 @@ int amoe_pp_gateup_act(const GemmArgs& a, int act, int tiles, hipStream_t s);
 int amoe_pp_rows(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s);
 int amoe_pp_gated_bwd(const GemmArgs& a, int act, int tiles, hipStream_t s);
 int amoe_pp_wgrad(GemmArgs a, hipStream_t s);
+// few tiles of a deep reduction (gemm_split.hip)
+int amoe_split_count(int R, int E, int K, int N);
+int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, int tiles, hipStream_t s);
 // few rows per expert (gemm_skinny.hip)
 int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s);
 int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s);
 
 // rows mode driver shared by the three row-grouped entry points
+// split, split_bytes: where the parts of a reduction that is cut into parts go (null: it is not cut)
 template <bool B_KC, int EPI, int ACT>
 static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C,
                          void* C2, const float* row_scale, int R, int E, int Kred, int N, int ldb, long long strideB, void* workspace,
-                         size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype, const void* G = nullptr, float* partials = nullptr)
+                         size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype, float* split, size_t split_bytes, const void* G = nullptr,
+                         float* partials = nullptr)
 {
     const bool map_ready = (tile_cfg & AMOE_TILE_MAP_READY) != 0;
     tile_cfg &= ~AMOE_TILE_MAP_READY;
@@ -1459,8 +1464,21 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
         else if constexpr (EPI == EPI_STORE && !B_KC) return amoe_skinny_nn(a, bm, s);
         // (the products with B^T run on the default kernel, which takes tiles of any height up to its own)
     }
+    const int splits = tile_cfg == 0 && split && bm == tc.bm ? amoe_split_count(R, E, Kred, N) : 1;
+    if (splits > 1) {
+        AMOE_REQUIRE(split_bytes >= (size_t)splits * R * N * sizeof(float), AMOE_ERR_WORKSPACE, "grouped_gemm: %zu bytes for %d parts",
+                     split_bytes, splits);
+        auto inverse = [](int d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; };
+        a.split_out = split;
+        a.splits = splits;
+        a.n_real = a.n_ntiles;
+        a.inv_splits = inverse(splits);
+        a.inv_real = inverse(a.n_real);
+        a.n_ntiles *= splits;
+    }
     rc = set_supertiles(a, max_mtiles, &grid);
     if (rc) return rc;
+    if (splits > 1) return amoe_split_rows(a, B_KC, EPI, ACT, (int)grid, s);
     if (tile_cfg == 0) {
         if constexpr (EPI == EPI_GATED) return amoe_pp_gateup_act(a, ACT, (int)grid, s);
         else if constexpr (EPI == EPI_GATED_BWD) return amoe_pp_gated_bwd(a, ACT, (int)grid, s);
@@ -1472,11 +1490,11 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
 #if AMOE_PART(0)
 int amoe_bf16_gateup_act(const void* xp, const int32_t* a_row_map, const void* w, const int32_t* offsets, void* gate_up,
                          void* inter, const float* row_scale, int R, int E, int H, int I, int act, void* workspace, size_t workspace_bytes,
-                         int tile_cfg, hipStream_t s, int dtype)
+                         int tile_cfg, hipStream_t s, int dtype, float* split, size_t split_bytes)
 {
     AMOE_DISPATCH_ACT(act, return (run_rows_bf16<false, EPI_GATED, ACT>(xp, a_row_map, w, offsets, gate_up, inter, row_scale, R, E, H,
                                                                         2 * I, 2 * I, (long long)H * 2 * I, workspace,
-                                                                        workspace_bytes, tile_cfg, s, dtype)))
+                                                                        workspace_bytes, tile_cfg, s, dtype, split, split_bytes)))
     return AMOE_ERR_BAD_ARG;
 }
 
@@ -1484,18 +1502,21 @@ int amoe_bf16_gateup_act(const void* xp, const int32_t* a_row_map, const void* w
 
 #if AMOE_PART(1)
 int amoe_bf16_nn(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int R, int E,
-                 int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype)
+                 int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype, float* split,
+                 size_t split_bytes)
 {
     return run_rows_bf16<false, EPI_STORE, 0>(A, a_row_map, B, offsets, C, nullptr, nullptr, R, E, Kd, N, N, (long long)Kd * N,
-                                              workspace, workspace_bytes, tile_cfg, s, dtype);
+                                              workspace, workspace_bytes, tile_cfg, s, dtype, split, split_bytes);
 }
 
 // C[rows_e, :Kd] = A[rows_e, :N] @ B[e]^T with B [E, Kd, N]: the reduction runs over N
 int amoe_bf16_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int R, int E,
-                 int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype)
+                 int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype, float* split,
+                 size_t split_bytes)
 {
     return run_rows_bf16<true, EPI_STORE, 0>(A, a_row_map, B, offsets, C, nullptr, nullptr, R, E, /*Kred=*/N, /*N out=*/Kd,
-                                             /*ldb=*/N, (long long)Kd * N, workspace, workspace_bytes, tile_cfg, s, dtype);
+                                             /*ldb=*/N, (long long)Kd * N, workspace, workspace_bytes, tile_cfg, s, dtype, split,
+                                             split_bytes);
 }
 
 #endif
@@ -1506,12 +1527,13 @@ int amoe_bf16_nt(const void* A, const int32_t* a_row_map, const void* B, const i
 // activation as its epilogue.  The reduction runs over H, the output columns are the I intermediate columns.
 int amoe_bf16_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down, const int32_t* offsets,
                            const void* gate_up, const float* row_scale, void* d_gate_up, float* partials, int R, int E,
-                           int I, int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype)
+                           int I, int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype,
+                           float* split, size_t split_bytes)
 {
     AMOE_DISPATCH_ACT(act, return (run_rows_bf16<true, EPI_GATED_BWD, ACT>(dy, a_row_map, w_down, offsets, d_gate_up, nullptr,
                                                                            row_scale, R, E, /*Kred=*/H, /*N out=*/I, /*ldb=*/H,
                                                                            (long long)I * H, workspace, workspace_bytes,
-                                                                           tile_cfg, s, dtype, gate_up, partials)))
+                                                                           tile_cfg, s, dtype, split, split_bytes, gate_up, partials)))
     return AMOE_ERR_BAD_ARG;
 }
 

@@ -66,10 +66,13 @@ struct GemmArgs {
     int sn;       // super-tiles along N
     uint32_t inv_gm, inv_gn, inv_sn, inv_super;   // ceil(2^32 / gm), .. gn, sn, gm gn (0 for a divisor of 1)
     int max_mtiles;  // rows mode: entries of tile_map (those past the last tile hold expert -1)
+    float* split_out;   // EPI_PART: partial sums [splits][M][N]
+    int splits, n_real;  // EPI_PART: parts of the reduction, N tiles of one part (n_ntiles counts the tiles of all)
+    uint32_t inv_splits, inv_real;   // ceil(2^32 / splits), .. n_real (0 for a divisor of 1)
     int f16;         // host side only: the operands are float16 (launch the f16 instance), else bf16
 };
 
-enum { EPI_STORE = 0, EPI_GATED = 1, EPI_GATED_BWD = 2 };
+enum { EPI_STORE = 0, EPI_GATED = 1, EPI_GATED_BWD = 2, EPI_PART = 3 };
 
 namespace {
 

@@ -179,9 +179,25 @@ __device__ __forceinline__ void pp_rows_body()
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I4 = std::integral_constant<int, 4>;
+    constexpr bool PART = EPI == EPI_PART;
+    auto divide = [](int n, uint32_t inv) -> int { return inv ? (int)(((uint64_t)(uint32_t)n * inv) >> 32) : n; };
     const int Kd = pp_args().Kd;
-    const int KT = max(4, (Kd + PP_BK - 1) / PP_BK);               // K tiles (of a short reduction, the last are empty)
-    const bool ragged_k = Kd < KT * PP_BK;
+    const int KT_all = (Kd + PP_BK - 1) / PP_BK;
+    // K tiles (of a short reduction, the last are empty).  EPI_PART: a part's, and part i has those from i KT_all / splits on, one
+    // fewer in some (the launch sees to it that there are four at least)
+    const int KT = PART ? divide(KT_all + pp_args().splits - 1, pp_args().inv_splits) : max(4, KT_all);
+    const bool ragged_k = PART || Kd < KT * PP_BK;
+    struct Part { int i, k0, kd; };                                // number, first k and length
+    auto part_of = [&](int& nt) -> Part {                          // N tile of all parts -> of its part
+        if constexpr (PART) {
+            args_t& p = pp_args();
+            const int i = divide(nt, p.inv_real);
+            nt -= i * p.n_real;
+            const int t0 = divide(i * KT_all, p.inv_splits), t1 = divide((i + 1) * KT_all, p.inv_splits);
+            return {i, t0 * PP_BK, min(t1 * PP_BK, Kd) - t0 * PP_BK};
+        }
+        return {0, 0, Kd};
+    };
 
     // ------------------------------------------------------------ this workgroup's tiles
     // Virtual blocks b, b + grid, b + 2 grid, ...; virtual block v belongs to XCD v % 8 (the hardware deals
@@ -192,7 +208,6 @@ __device__ __forceinline__ void pp_rows_body()
     // (divisions by multiplication with the host's rounded-up reciprocals: exact for the numerators that occur)
     int vb_next = blockIdx.x;
     const int n_mtiles = min(scalar_load_i32(pp_args().n_mtiles), pp_args().max_mtiles);
-    auto divide = [](int n, uint32_t inv) -> int { return inv ? (int)(((uint64_t)(uint32_t)n * inv) >> 32) : n; };
     auto advance = [&](int& pm, int& nt) -> bool {
         args_t& p = pp_args();
         const int per_super = p.gm * p.gn;
@@ -241,7 +256,7 @@ __device__ __forceinline__ void pp_rows_body()
     const uint32_t bstep = B_KC ? PP_BK * 2 : (uint32_t)ldb * (PP_BK * 2);
     auto expert_b = [&](int e) { args_t& p = pp_args(); return p.B + (long long)e * p.strideB; };
     // a plan without rows (m0 == mend) or columns (n0 >= N) reads nothing
-    auto plan_a = [&](int m0, int mend, const int32_t* map) {     // map: the row map (first tile), else the indices are in LDS
+    auto plan_a = [&](int m0, int mend, const int32_t* map, int k0) {     // map: the row map (first tile), else the indices are in LDS
         const int th = pp_here(tid);
         const int r = th >> 3, k = ((th & 7) ^ ((r >> 1) & 7)) * 8;
         // tile row of this thread's chunk in half a: (a*4 + i)*32 + j*16 + l with i = r / 16, l = r % 16
@@ -256,13 +271,15 @@ __device__ __forceinline__ void pp_rows_body()
                 aoff[a][j] = row < mend && k < Kd ? ((uint32_t)gr * (uint32_t)lda + k) * 2u : PP_NOWHERE;
             }
         ad = pp_srd(A);
+        if constexpr (PART) pp_advance(ad, (uint32_t)k0 * 2u);
     };
-    auto plan_b = [&](const bf16_t* B, int n0) {
+    auto plan_b = [&](const bf16_t* B, int n0, int k0) {
         const int th = pp_here(tid);
         const int r = th >> 3, kr = th >> 4;
         const int k = ((th & 7) ^ ((r >> 1) & 7)) * 8;
         const int col = ((th & 15) ^ (2 * ((kr & 3) | (((kr >> 3) & 1) << 2)))) * 8;
         bd = pp_srd(B);
+        if constexpr (PART) pp_advance(bd, B_KC ? (uint32_t)k0 * 2u : (uint32_t)k0 * ((uint32_t)ldb * 2u));
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
@@ -359,6 +376,7 @@ __device__ __forceinline__ void pp_rows_body()
 
     // ------------------------------------------------------------ tile state
     int m0, mend, nt, n0;
+    Part part, part_n;                   // this tile's part of the reduction, the next one's
     bool have_n, have_nn = false;        // is there a next tile, and one after it
     int nt_n = 0, nt_nn = 0;
     int4 tm_n, tm_nn = make_int4(0, 0, 0, 0);
@@ -372,9 +390,10 @@ __device__ __forceinline__ void pp_rows_body()
         mend = tm.z;
         have_n = advance(pm, nt_n);
         tm_n = have_n ? load_entry(pm) : make_int4(0, 0, 0, 0);
+        part = part_of(nt);
         n0 = nt * PP_BN;
-        plan_a(m0, mend, pp_args().a_row_map);
-        plan_b(expert_b(tm.x), n0);
+        plan_a(m0, mend, pp_args().a_row_map, part.k0);
+        plan_b(expert_b(tm.x), n0, part.k0);
     }
     int par = 0;            // row scales: which of the two LDS rows is this tile's
     bool sums_due = false;  // row-sum partials of the previous tile are complete in LDS and not yet written
@@ -393,7 +412,11 @@ __device__ __forceinline__ void pp_rows_body()
         const int c0 = n0 + wc * 32;
         e_cols = N - c0;                 // columns of the wave's part that exist, from its first one (N is a multiple of 8)
         e_rows = mend - m0;
-        if (EPI == EPI_GATED_BWD) {
+        if (PART) {
+            e_ldc = p.N * 2;             // in elements of 16 bits, as below
+            e_c = reinterpret_cast<bf16_t*>(p.split_out + ((long long)part.i * p.M + m0) * p.N + c0);
+            e_off = (uint32_t)(rl * p.N + 4 * eq) * 4u;
+        } else if (EPI == EPI_GATED_BWD) {
             e_ldc = p.ldg;
             e_c = p.C + (long long)m0 * e_ldc + 2 * c0;
             e_c2 = const_cast<bf16_t*>(p.G) + (long long)m0 * e_ldc + 2 * c0;
@@ -434,7 +457,17 @@ __device__ __forceinline__ void pp_rows_body()
         const int eq = le >> 4, rl = grp * 16 + (le & 15);
         const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc(e_c, (short)0, (int)PP_DROP, 0x00020000);
         const uint32_t srow = (uint32_t)e_ldc * 64u;           // bytes of 32 rows
-        if constexpr (EPI == EPI_GATED_BWD) {
+        if constexpr (PART) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                pp_fence();
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const bool ok = b * 128 + 16 * j + 4 * eq < e_cols && (a * 4 + i) * 32 + rl < e_rows;
+                    pp_store16(d, __builtin_bit_cast(u32x4_t, acc[i][j]), ok ? e_off + j * 64u : PP_DROP, (a * 4 + i) * srow + b * 512u);
+                }
+            }
+        } else if constexpr (EPI == EPI_GATED_BWD) {
             // d_inter is in the accumulators; the (gate, up) pairs of its columns come back from the forward pass
             auto place = [&](int j, int i) {
                 return b * 128 + 16 * j + 4 * eq < e_cols && (a * 4 + i) * 32 + rl < e_rows ? e_off + j * 64u : PP_DROP;
@@ -527,7 +560,7 @@ __device__ __forceinline__ void pp_rows_body()
         {
             args_t& p = pp_args();
             const int le = pp_here(lane);
-            if (EPI != EPI_STORE && wave < 4) {
+            if (EPI != EPI_STORE && !PART && wave < 4) {
                 const int row = wave * 64 + le;
                 const uint32_t dst = lds + PP_SCALE + (uint32_t)(par * PP_BM + wave * 64) * 4u;
                 if (p.row_scale) {
@@ -548,6 +581,7 @@ __device__ __forceinline__ void pp_rows_body()
         {
             // the next tile's weights; which tile follows it, and its entry of the tile map
             b_n = expert_b(tm_n.x);
+            part_n = part_of(nt_n);
             int pm = 0;
             have_nn = have_n && advance(pm, nt_nn);
             tm_nn = have_nn ? load_entry(pm) : make_int4(0, 0, 0, 0);
@@ -560,7 +594,7 @@ __device__ __forceinline__ void pp_rows_body()
             constexpr bool turn = decltype(TURN)::value;
             // phase 1
             read_b(I1{}, fb1);
-            if (turn) plan_b(b_n, have_n ? nt_n * PP_BN : 0x7fffff00);
+            if (turn) plan_b(b_n, have_n ? nt_n * PP_BN : 0x7fffff00, have_n ? part_n.k0 : 0);
             dma_b(I0{});
             pp_vmwait<10>();
             pp_barrier();
@@ -569,7 +603,7 @@ __device__ __forceinline__ void pp_rows_body()
             // phase 2
             read_a(I1{}, N_);
             if (turn) {
-                plan_a(tm_n.y, tm_n.z, nullptr);
+                plan_a(tm_n.y, tm_n.z, nullptr, have_n ? part_n.k0 : 0);
             }
             dma_a(I0{});
             pp_vmwait<10>();
@@ -594,25 +628,25 @@ __device__ __forceinline__ void pp_rows_body()
             mma(F_{}, I4{}, acc[0][0], fb0);
             pp_barrier();
         };
-        if (Kd < 3 * PP_BK) cut_k(Kd - 2 * PP_BK);                      // K tile 2 is loaded next
+        if (!PART && Kd < 3 * PP_BK) cut_k(Kd - 2 * PP_BK);             // K tile 2 is loaded next
         k_tile(T_{}, F_{}, I4{});
         // The rows of the lower half beyond the last block with a live row are neither read nor multiplied: one copy of
         // the loop per number of such blocks, one after the other, all but one of them with no iterations (chosen
         // between by if and else, each copy's registers would be live across the others).
         const int n1 = min(max(((mend - m0 + 31) >> 5) - 4, 0), 4);
         int t = 1;
-        for (int part = 0; part < 2; ++part) {
-            const int end = KT - 3 + part;
+        for (int half = 0; half < 2; ++half) {
+            const int end = KT - 3 + half;
             for (const int e = n1 == 4 ? end : 0; t < e; ++t) k_tile(F_{}, F_{}, I4{});
             for (const int e = n1 == 3 ? end : 0; t < e; ++t) k_tile(F_{}, F_{}, std::integral_constant<int, 3>{});
             for (const int e = n1 == 2 || n1 == 1 ? end : 0; t < e; ++t) k_tile(F_{}, F_{}, std::integral_constant<int, 2>{});
             for (const int e = n1 == 0 ? end : 0; t < e; ++t) k_tile(F_{}, F_{}, I0{});
-            if (part == 0 && ragged_k) cut_k(Kd - (KT - 1) * PP_BK);    // K tile KT - 1 is loaded next
+            if (half == 0 && ragged_k) cut_k((PART ? part.kd : Kd) - (KT - 1) * PP_BK);    // K tile KT - 1 is loaded next
         }
         k_tile(F_{}, T_{}, I4{});
-        if (Kd < 2 * PP_BK) cut_k(Kd - PP_BK);                          // the next tile's K tile 1 is loaded next
+        if (!PART && Kd < 2 * PP_BK) cut_k(Kd - PP_BK);                 // the next tile's K tile 1 is loaded next
         // ---- last K tile
-        if constexpr (EPI == EPI_STORE) {
+        if constexpr (EPI == EPI_STORE || PART) {
             // the epilogue of each finished quadrant in the memory part of the phase after it
             read_b(I1{}, fb1);
             dma_b(I0{});
@@ -673,7 +707,7 @@ __device__ __forceinline__ void pp_rows_body()
     // ------------------------------------------------------------ the workgroup's tiles
     dma_b(I0{}); dma_a(I0{}); dma_b(I1{}); dma_a(I1{});
     next_k();
-    if (Kd < 2 * PP_BK) cut_k(Kd - PP_BK);
+    if (!PART && Kd < 2 * PP_BK) cut_k(Kd - PP_BK);
     dma_b(I0{}); dma_a(I0{}); dma_b(I1{});
     pp_vmwait<12>();
     pp_barrier();
@@ -694,6 +728,7 @@ __device__ __forceinline__ void pp_rows_body()
         m0 = tm_n.y;
         mend = tm_n.z;
         nt = nt_n;
+        part = part_n;
         n0 = nt * PP_BN;
         have_n = have_nn;
         nt_n = nt_nn;
@@ -1103,6 +1138,10 @@ int amoe_pp_gateup_act(const GemmArgs& a, int act, int tiles, hipStream_t s)
 }
 #endif
 #if AMOE_PP_PART_IS(1)
+int amoe_pp_part(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s)
+{
+    return b_kc ? launch_pp_rows<true, EPI_PART, 0>(a, tiles, s) : launch_pp_rows<false, EPI_PART, 0>(a, tiles, s);
+}
 int amoe_pp_rows(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s)
 {
     return b_kc ? launch_pp_rows<true, EPI_STORE, 0>(a, tiles, s) : launch_pp_rows<false, EPI_STORE, 0>(a, tiles, s);

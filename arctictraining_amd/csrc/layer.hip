@@ -6,6 +6,7 @@
 // (One token through 128 experts of 2048 x 768: 144 us of host time a forward stage by stage, 70 us this way.)
 #include "amoe_common.h"
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -26,6 +27,25 @@ int amoe_launch_router_bwd(const float* d_scores, const float* probs, const int3
 int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map, const int32_t* offsets, void* C, int R,
                     int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype, int lda, bool out32);
 int amoe_launch_sum_parts(const void* parts, int n_parts, void* out, int parts_dtype, int dtype, long long n, hipStream_t s);
+
+// the grouped products with room for the parts of a reduction (gemm_split.hip), none if split is null
+int amoe_run_gateup_act_fwd(const void* xp, const int32_t* a_row_map, const void* w_gate_up,
+                                                 const int32_t* offsets, const float* row_scale, void* gate_up,
+                                                 void* inter, int dtype, int R,
+                                                 int E, int H, int I, int act, void* workspace, size_t workspace_bytes,
+                                                 int tile_cfg, void* stream, float* split, size_t split_bytes);
+int amoe_run_nn(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
+                                     void* C, int dtype, int R, int E, int Kd, int N, void* workspace,
+                                     size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes);
+int amoe_run_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
+                                     void* C, int dtype, int R, int E, int Kd, int N, void* workspace,
+                                     size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes);
+int amoe_run_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down,
+                                               const int32_t* offsets, const void* gate_up, const float* row_scale,
+                                               void* d_gate_up, float* score_partials, int dtype, int R, int E, int I,
+                                               int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg,
+                                               void* stream, float* split, size_t split_bytes);
+size_t amoe_split_bytes(int R, int E, int K, int N);
 
 namespace {
 
@@ -85,9 +105,20 @@ Saved cut_saved(const Shape& c, int T, void* base, bool keep)
     return s;
 }
 
+// room for the parts of the products of `R` rows of `E` experts, K[i] x N[i]
+size_t split_room(const Shape& c, int T, int K0, int N0, int K1, int N1)
+{
+    if (c.dtype == AMOE_F32 || c.tile_cfg != 0) return 0;
+    const int R = T * c.K;
+    size_t n = std::max(amoe_split_bytes(R, c.E, K0, N0), amoe_split_bytes(R, c.E, K1, N1));
+    if (c.shared) n = std::max({n, amoe_split_bytes(T, 1, K0, N0), amoe_split_bytes(T, 1, K1, N1)});
+    return n;
+}
+
 struct FwdScratch {
     char *plan_ws, *out, *sh_out;
-    size_t plan_ws_bytes, bytes;
+    float* split;
+    size_t plan_ws_bytes, split_bytes, bytes;
 };
 
 FwdScratch cut_fwd(const Shape& c, int T, void* base)
@@ -99,6 +130,8 @@ FwdScratch cut_fwd(const Shape& c, int T, void* base)
     f.plan_ws = b.take<char>(f.plan_ws_bytes);
     f.out = b.take<char>(R * c.H * c.esz());
     if (c.shared) f.sh_out = b.take<char>((size_t)T * c.H * c.esz());
+    f.split_bytes = split_room(c, T, c.H, 2 * c.I, c.I, c.H);
+    if (f.split_bytes) f.split = (float*)b.take<char>(f.split_bytes);
     f.bytes = b.used;
     return f;
 }
@@ -106,7 +139,8 @@ FwdScratch cut_fwd(const Shape& c, int T, void* base)
 struct BwdScratch {
     float *parts, *d_scores, *sh_d_sig;
     char *d_gate_up, *d_rows /* d_inter, later d_xp */, *sh_d_gate_up, *sh_d_rows;
-    size_t bytes;
+    float* split;
+    size_t split_bytes, bytes;
 };
 
 BwdScratch cut_bwd(const Shape& c, int T, void* base)
@@ -123,6 +157,8 @@ BwdScratch cut_bwd(const Shape& c, int T, void* base)
         w.sh_d_gate_up = b.take<char>((size_t)T * 2 * c.I * c.esz());
         w.sh_d_rows = b.take<char>((size_t)T * wide * c.esz());
     }
+    w.split_bytes = split_room(c, T, c.H, c.I, 2 * c.I, c.H);
+    if (w.split_bytes) w.split = (float*)b.take<char>(w.split_bytes);
     w.bytes = b.used;
     return w;
 }
@@ -242,18 +278,18 @@ AMOE_EXPORT int amoe_layer_fwd(const int32_t* config, int T, const void* x, cons
     if (stages & AMOE_STAGE_EXPERTS) {
         // the rows x[token_of] are gathered inside the product's loads; a row's score multiplies its intermediate
         // activation (the down projection is linear), so that the combine is a plain sum
-        AMOE_TRY(amoe_grouped_gemm_gateup_act_fwd(x, s.token_of, w_gate_up, s.offsets, s.scores_perm, s.gate_up, s.inter, c.dtype, R,
-                                                  c.E, c.H, c.I, c.act, s.gemm_ws, s.gemm_ws_bytes, ready, stream));
-        AMOE_TRY(amoe_grouped_gemm_nn(s.inter, nullptr, w_down, s.offsets, f.out, c.dtype, R, c.E, c.I, c.H, s.gemm_ws,
-                                      s.gemm_ws_bytes, ready, stream));
+        AMOE_TRY(amoe_run_gateup_act_fwd(x, s.token_of, w_gate_up, s.offsets, s.scores_perm, s.gate_up, s.inter, c.dtype, R, c.E, c.H, c.I,
+                                         c.act, s.gemm_ws, s.gemm_ws_bytes, ready, stream, f.split, f.split_bytes));
+        AMOE_TRY(amoe_run_nn(s.inter, nullptr, w_down, s.offsets, f.out, c.dtype, R, c.E, c.I, c.H, s.gemm_ws, s.gemm_ws_bytes, ready, stream,
+                             f.split, f.split_bytes));
     }
     if (c.shared && (stages & AMOE_STAGE_SHARED)) {
         // the shared expert is one more expert that owns every token, sigmoid(x @ gate) in the role of the score
         AMOE_TRY(amoe_launch_shared_gate(x, sh_out_gate, s.sh_sig, c.dtype, T, c.H, (hipStream_t)stream));
-        AMOE_TRY(amoe_grouped_gemm_gateup_act_fwd(x, nullptr, sh_gate_up, all_rows, s.sh_sig, s.sh_gate_up, s.sh_inter, c.dtype, T, 1,
-                                                  c.H, c.I, c.act, s.sh_ws, s.sh_ws_bytes, c.tile_cfg, stream));
-        AMOE_TRY(amoe_grouped_gemm_nn(s.sh_inter, nullptr, sh_down, all_rows, f.sh_out, c.dtype, T, 1, c.I, c.H, s.sh_ws,
-                                      s.sh_ws_bytes, ready, stream));
+        AMOE_TRY(amoe_run_gateup_act_fwd(x, nullptr, sh_gate_up, all_rows, s.sh_sig, s.sh_gate_up, s.sh_inter, c.dtype, T, 1, c.H, c.I, c.act,
+                                         s.sh_ws, s.sh_ws_bytes, c.tile_cfg, stream, f.split, f.split_bytes));
+        AMOE_TRY(amoe_run_nn(s.sh_inter, nullptr, sh_down, all_rows, f.sh_out, c.dtype, T, 1, c.I, c.H, s.sh_ws, s.sh_ws_bytes, ready, stream,
+                             f.split, f.split_bytes));
     }
     if (stages & AMOE_STAGE_COMBINE)
         AMOE_TRY(amoe_gather_rows_bwd(f.out, s.row_of, c.shared ? f.sh_out : nullptr, y, c.dtype, T, c.K, c.H, stream));
@@ -289,8 +325,8 @@ static int layer_bwd(const int32_t* config, int T, const void* x, const void* dy
     if (c.fused_bwd()) {
         // data gradient of the down projection with the backward of the gated activation as its epilogue; the score
         // gradients come back as sums over the columns of one tile each
-        AMOE_TRY(amoe_grouped_gemm_nt_gated_bwd(dy, s.token_of, w_down, s.offsets, s.gate_up, s.scores_perm, w.d_gate_up, w.parts,
-                                                c.dtype, R, c.E, c.I, c.H, c.act, s.gemm_ws, s.gemm_ws_bytes, ready, stream));
+        AMOE_TRY(amoe_run_nt_gated_bwd(dy, s.token_of, w_down, s.offsets, s.gate_up, s.scores_perm, w.d_gate_up, w.parts, c.dtype, R, c.E, c.I,
+                                       c.H, c.act, s.gemm_ws, s.gemm_ws_bytes, ready, stream, w.split, w.split_bytes));
     } else {
         AMOE_TRY(amoe_grouped_gemm_nt(dy, s.token_of, w_down, s.offsets, w.d_rows, c.dtype, R, c.E, c.I, c.H, s.gemm_ws,
                                       s.gemm_ws_bytes, ready, stream));
@@ -378,8 +414,8 @@ AMOE_EXPORT int amoe_layer_bwd_shared(const int32_t* config, int T, const void* 
     const BwdScratch w = cut_bwd(c, T, scratch);
     const hipStream_t main = (hipStream_t)stream;
     // the chain of amoe_layer_bwd for the expert that owns every token; its score gradient goes on through the sigmoid
-    AMOE_TRY(amoe_grouped_gemm_nt(dy, nullptr, sh_down, all_rows, w.sh_d_rows, c.dtype, T, 1, c.I, c.H, s.sh_ws, s.sh_ws_bytes,
-                                  c.tile_cfg | AMOE_TILE_MAP_READY, stream));
+    AMOE_TRY(amoe_run_nt(dy, nullptr, sh_down, all_rows, w.sh_d_rows, c.dtype, T, 1, c.I, c.H, s.sh_ws, s.sh_ws_bytes,
+                         c.tile_cfg | AMOE_TILE_MAP_READY, stream, w.split, w.split_bytes));
     if (d_sh_down)
         AMOE_TRY(amoe_dense_wgrad(s.sh_inter, dy, down_chunks, down_splits, parts, d_sh_down, c.dtype, T, c.I, c.H, c.tile_cfg, stream));
     AMOE_TRY(amoe_launch_gated_act_bwd_rows(s.sh_gate_up, w.sh_d_rows, s.sh_sig, w.sh_d_gate_up, w.sh_d_sig, c.dtype, T, c.I, c.act, main));
@@ -404,11 +440,11 @@ AMOE_EXPORT int amoe_layer_bwd_input(const int32_t* config, int T, const void* w
         AMOE_REQUIRE(w_gate_up && dx_router, AMOE_ERR_BAD_ARG, "layer_bwd_input: null pointer");
         AMOE_REQUIRE(!c.shared || (sh_gate_up && sh_out_gate && all_rows && d_pre), AMOE_ERR_BAD_ARG,
                      "layer_bwd_input: null shared expert");
-        AMOE_TRY(amoe_grouped_gemm_nt(w.d_gate_up, nullptr, w_gate_up, s.offsets, w.d_rows, c.dtype, R, c.E, c.H, 2 * c.I, s.gemm_ws,
-                                      s.gemm_ws_bytes, ready, stream));
+        AMOE_TRY(amoe_run_nt(w.d_gate_up, nullptr, w_gate_up, s.offsets, w.d_rows, c.dtype, R, c.E, c.H, 2 * c.I, s.gemm_ws, s.gemm_ws_bytes,
+                             ready, stream, w.split, w.split_bytes));
         if (c.shared)
-            AMOE_TRY(amoe_grouped_gemm_nt(w.sh_d_gate_up, nullptr, sh_gate_up, all_rows, w.sh_d_rows, c.dtype, T, 1, c.H, 2 * c.I,
-                                          s.sh_ws, s.sh_ws_bytes, ready, stream));
+            AMOE_TRY(amoe_run_nt(w.sh_d_gate_up, nullptr, sh_gate_up, all_rows, w.sh_d_rows, c.dtype, T, 1, c.H, 2 * c.I, s.sh_ws,
+                                 s.sh_ws_bytes, ready, stream, w.split, w.split_bytes));
         AMOE_TRY(amoe_launch_input_grad(w.d_rows, s.row_of, dx_router, c.shared ? w.sh_d_rows : nullptr, d_pre, sh_out_gate, dx,
                                         c.dtype, T, c.K, c.H, main));
     }

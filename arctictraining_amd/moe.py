@@ -316,12 +316,14 @@ def _overlap_pays(config_key, T: int) -> bool:
     """Whether the expert weight gradients go on the second stream.  The events that order the streams cost the host 40-60 us a
     step; a step that the GPU takes less time for than the host is longer by that much (20 of 60 steps drawn over the sizes of
     this layer: 12-39 %), one that it takes longer for is mostly 3-15 % shorter with the second stream.  The line lies where
-    the products at 800 TFLOP/s (float32 100) and the weights, read twice and their gradients written, at 3 TB/s make 150 us:
-    T=556 H=1760 E=8 K=6 I=672 (129 us) 268 us with it, 228 without; T=95 H=2336 E=12 K=2 I=1536 (188) 274 and 299."""
+    the products at 800 TFLOP/s (float32 100), their columns rounded up to whole tiles, and the weights, read twice and their
+    gradients written, at 3 TB/s make 150 us: T=556 H=1760 E=8 K=6 I=672 (143 us) 268 us with it, 228 without; T=95 H=2336 E=12
+    K=2 I=1536 (193) 274 and 299, T=3065 H=320 E=19 K=5 I=1088 (243) 353 and 398."""
     E, K, H, I, dtype, shared = *config_key[:4], config_key[5], config_key[8]
     size, rate = (4, 1e8) if dtype == ops.F32 else (2, 8e8)
-    rows = T * K + (T if shared else 0)
-    return 18.0 * rows * H * I / rate + 6.0 * size * (E + (1 if shared else 0)) * H * I / 3e6 > 150.0
+    rows, weights = T * K + (T if shared else 0), (E + (1 if shared else 0)) * H * I
+    padded = -(-H // 256) * 256 * -(-I // 128) * 128
+    return 18.0 * rows * padded / rate + 6.0 * size * weights / 3e6 > 150.0
 
 
 def _check_operand(t, name, like, shape) -> None:
