@@ -8,17 +8,19 @@
 //                                                  (down_proj [E, H, I] -> expert_down [E, I, H])
 //   unpack  out_g[e][i][h] = in[e][h][G*i + g]     the inverse, for saving a checkpoint
 //
-// Pure byte movement, HBM bound: 64 x 64 tiles go through LDS so that both the reads and the
-// writes are 16-byte accesses along the contiguous dimension of their tensor.
+// Pure byte movement, HBM bound: tiles go through LDS so that both the reads and the writes are 16-byte accesses along
+// the contiguous dimension of their tensor, and every byte passes once: both sides bypass the caches' replacement order
+// (a linear copy of 1 GB takes 5.8 TB/s with ordinary accesses and 6.35 with these).
 //
 // Experts that are modules of their own are read and written where their weights lie (Listed below): at E=128, H=2048,
-// I=768 in bf16 a layer's 2 x 1.21 GB take 474 us in and 489 us out, 5.0-5.1 TB/s; stacked copies and copies into the
-// parameters beside the kernels took 1.79 and 2.15 ms.
+// I=768 in bf16 a layer's 2 x 1.21 GB take 426 us in and 427 us out, 5.7 TB/s (with 64 x 64 tiles, 2-byte LDS accesses
+// and ordinary loads and stores 474 and 489 us); stacked copies and copies into the parameters beside the kernels took
+// 1.79 and 2.15 ms.
 #include "amoe_common.h"
 
 namespace {
 
-constexpr int TILE = 64;
+constexpr int TILE = 64;   // (of 4-byte elements)
 
 // Where the per-expert matrices of the split side are: a strided tensor, or one address each.  The addresses of up to
 // kListExperts experts travel as kernel arguments (2 KB: no copy to the device, nothing to keep alive).
@@ -35,7 +37,98 @@ struct Listed {
     __device__ __forceinline__ T* at(int g, int e) const { return (T*)p[g][e]; }
 };
 
-// T is the element as raw bits (uint16_t / uint32_t); V = elements per 16-byte access
+// 2-byte elements: 256 columns h by 64 dwords of two elements that lie side by side in the joint side, (gate, up) of one
+// i, or i and i + 1 of a single projection.  A thread moves two rows' 16-byte vectors, interleaved in registers, so that
+// LDS sees dwords; 16-byte chunk c of LDS row h is kept at c ^ ((h / 8) % 16), which spreads a wavefront's dwords (8 rows
+// apart) over all banks.  Wide tiles for long pieces: with 128 or 64 columns the split side is accessed in pieces of 256
+// or 128 bytes instead of 512, and gate and up of the size above take 288 or 298 us, with 256 270.
+template <int G, bool PACK, typename SPLIT>
+__global__ void __launch_bounds__(256) remap16_kernel(SPLIT split, uint16_t* __restrict__ joint, int I, int H, long long joint_es)
+{
+    constexpr int TH = 256, W = 64, ROWS = W * 2 / G;     // columns h, dwords of a joint row, rows i
+    constexpr int NS = W * TH / 8 / 256, NJ = TH * W / 4 / 256;
+    __shared__ __attribute__((aligned(16))) uint32_t tile[TH * W];
+    typedef uint32_t vec_t __attribute__((ext_vector_type(4)));
+    const int tid = threadIdx.x;
+    const int h0 = blockIdx.x * TH, i0 = blockIdx.y * ROWS, e = blockIdx.z;
+    uint16_t* const row0 = split.template at<uint16_t>(0, e);
+    uint16_t* const row1 = G == 2 ? split.template at<uint16_t>(1, e) : row0 + H;
+    uint16_t* const j = joint + (long long)e * joint_es;
+    auto at = [](int h, int d) { return h * W + (((d >> 2) ^ (h >> 3)) & 15) * 4 + (d & 3); };
+    // vector n of this thread: split side, rows of dword d and column h; joint side, row h and column c
+    auto split_at = [&](int n, int& d, int& hh, long long& off) {
+        const int v = tid + n * 256;
+        d = v / (TH / 8);
+        hh = v % (TH / 8) * 8;
+        const int i = i0 + (G == 2 ? d : 2 * d);
+        off = (long long)i * H + h0 + hh;
+        return i < I && h0 + hh < H;
+    };
+    auto joint_at = [&](int n, int& hh, int& d, long long& off) {
+        const int v = tid + n * 256;
+        hh = v / (W / 4);
+        d = v % (W / 4) * 4;
+        const int c = G * i0 + 2 * d;
+        off = (long long)(h0 + hh) * (G * I) + c;
+        return h0 + hh < H && c < G * I;
+    };
+    int d, hh;
+    long long off;
+    if (PACK) {
+        vec_t a[NS], b[NS];
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+            if (split_at(n, d, hh, off)) {
+                a[n] = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(row0 + off));
+                b[n] = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(row1 + off));
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+            split_at(n, d, hh, off);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                tile[at(hh + 2 * k, d)] = __builtin_amdgcn_perm(b[n][k], a[n][k], 0x05040100);
+                tile[at(hh + 2 * k + 1, d)] = __builtin_amdgcn_perm(b[n][k], a[n][k], 0x07060302);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < NJ; ++n) {
+            if (joint_at(n, hh, d, off))
+                __builtin_nontemporal_store(*reinterpret_cast<const vec_t*>(&tile[at(hh, d)]), reinterpret_cast<vec_t*>(j + off));
+        }
+    } else {
+        vec_t x[NJ];
+#pragma unroll
+        for (int n = 0; n < NJ; ++n) {
+            if (joint_at(n, hh, d, off)) x[n] = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(j + off));
+        }
+#pragma unroll
+        for (int n = 0; n < NJ; ++n) {
+            joint_at(n, hh, d, off);
+            *reinterpret_cast<vec_t*>(&tile[at(hh, d)]) = x[n];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+            const bool in = split_at(n, d, hh, off);
+            vec_t a, b;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t p = tile[at(hh + 2 * k, d)], q = tile[at(hh + 2 * k + 1, d)];
+                a[k] = __builtin_amdgcn_perm(q, p, 0x05040100);
+                b[k] = __builtin_amdgcn_perm(q, p, 0x07060302);
+            }
+            if (in) {
+                __builtin_nontemporal_store(a, reinterpret_cast<vec_t*>(row0 + off));
+                __builtin_nontemporal_store(b, reinterpret_cast<vec_t*>(row1 + off));
+            }
+        }
+    }
+}
+
+// 4-byte elements, as raw bits; V = elements per 16-byte access
 template <typename T, int G, bool PACK, typename SPLIT>
 __global__ void __launch_bounds__(256)
 remap_kernel(SPLIT split /* the [E,I,H] side */, T* __restrict__ joint /* the [E,H,G*I] side */, int I, int H, long long joint_es)
@@ -57,7 +150,7 @@ remap_kernel(SPLIT split /* the [E,I,H] side */, T* __restrict__ joint /* the [E
                 const int ii = v / VPR, hv = (v % VPR) * V;
                 const int i = i0 + ii, h = h0 + hv;
                 if (i < I && h < H) {
-                    const vec_t x = *reinterpret_cast<const vec_t*>(src + (long long)i * H + h);
+                    const vec_t x = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(src + (long long)i * H + h));
 #pragma unroll
                     for (int k = 0; k < V; ++k) tile[hv + k][G * ii + g] = x[k];
                 }
@@ -71,7 +164,7 @@ remap_kernel(SPLIT split /* the [E,I,H] side */, T* __restrict__ joint /* the [E
             const int hh = v / VPJ, cv = (v % VPJ) * V;
             const int h = h0 + hh, c = G * i0 + cv;
             if (h < H && c < G * I)
-                *reinterpret_cast<vec_t*>(dst + (long long)h * (G * I) + c) = *reinterpret_cast<const vec_t*>(&tile[hh][cv]);
+                __builtin_nontemporal_store(*reinterpret_cast<const vec_t*>(&tile[hh][cv]), reinterpret_cast<vec_t*>(dst + (long long)h * (G * I) + c));
         }
     } else {
         constexpr int VPJ = G * TILE / V;
@@ -80,7 +173,7 @@ remap_kernel(SPLIT split /* the [E,I,H] side */, T* __restrict__ joint /* the [E
             const int hh = v / VPJ, cv = (v % VPJ) * V;
             const int h = h0 + hh, c = G * i0 + cv;
             if (h < H && c < G * I)
-                *reinterpret_cast<vec_t*>(&tile[hh][cv]) = *reinterpret_cast<const vec_t*>(src + (long long)h * (G * I) + c);
+                *reinterpret_cast<vec_t*>(&tile[hh][cv]) = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(src + (long long)h * (G * I) + c));
         }
         __syncthreads();
         constexpr int VPR = TILE / V;
@@ -93,30 +186,39 @@ remap_kernel(SPLIT split /* the [E,I,H] side */, T* __restrict__ joint /* the [E
                     vec_t x;
 #pragma unroll
                     for (int k = 0; k < V; ++k) x[k] = tile[hv + k][G * ii + g];
-                    *reinterpret_cast<vec_t*>(dst + (long long)i * H + h) = x;
+                    __builtin_nontemporal_store(x, reinterpret_cast<vec_t*>(dst + (long long)i * H + h));
                 }
             }
         }
     }
 }
 
-template <typename T, typename SPLIT>
-void launch(bool pack, bool two, const SPLIT& split, void* joint, int E, int I, int H, hipStream_t s)
+template <int G, bool PACK, typename SPLIT>
+void launch(bool wide, const SPLIT& split, void* joint, int E, int I, int H, hipStream_t s)
 {
-    const dim3 grid((H + TILE - 1) / TILE, (I + TILE - 1) / TILE, E), block(256);
-    const long long joint_es = (long long)H * I * (two ? 2 : 1);
-    T* j = (T*)joint;
-    if (pack && two) hipLaunchKernelGGL((remap_kernel<T, 2, true, SPLIT>), grid, block, 0, s, split, j, I, H, joint_es);
-    else if (pack) hipLaunchKernelGGL((remap_kernel<T, 1, true, SPLIT>), grid, block, 0, s, split, j, I, H, joint_es);
-    else if (two) hipLaunchKernelGGL((remap_kernel<T, 2, false, SPLIT>), grid, block, 0, s, split, j, I, H, joint_es);
-    else hipLaunchKernelGGL((remap_kernel<T, 1, false, SPLIT>), grid, block, 0, s, split, j, I, H, joint_es);
+    const long long joint_es = (long long)H * I * G;
+    if (wide) {
+        const dim3 grid((H + TILE - 1) / TILE, (I + TILE - 1) / TILE, E);
+        hipLaunchKernelGGL((remap_kernel<uint32_t, G, PACK, SPLIT>), grid, dim3(256), 0, s, split, (uint32_t*)joint, I, H, joint_es);
+    } else {
+        const dim3 grid((H + 255) / 256, (I * G + 127) / 128, E);
+        hipLaunchKernelGGL((remap16_kernel<G, PACK, SPLIT>), grid, dim3(256), 0, s, split, (uint16_t*)joint, I, H, joint_es);
+    }
+}
+
+template <typename SPLIT>
+void launch(bool pack, bool two, bool wide, const SPLIT& split, void* joint, int E, int I, int H, hipStream_t s)
+{
+    if (pack && two) launch<2, true>(wide, split, joint, E, I, H, s);
+    else if (pack) launch<1, true>(wide, split, joint, E, I, H, s);
+    else if (two) launch<2, false>(wide, split, joint, E, I, H, s);
+    else launch<1, false>(wide, split, joint, E, I, H, s);
 }
 
 int launch_strided(bool pack, const void* s0, const void* s1, void* joint, int dtype, int E, int I, int H, long long es, void* stream)
 {
     const Strided split = {{s0, s1}, es};
-    if (dtype != AMOE_F32) launch<uint16_t>(pack, s1 != nullptr, split, joint, E, I, H, (hipStream_t)stream);
-    else launch<uint32_t>(pack, s1 != nullptr, split, joint, E, I, H, (hipStream_t)stream);
+    launch(pack, s1 != nullptr, dtype == AMOE_F32, split, joint, E, I, H, (hipStream_t)stream);
     return amoe_check_launch(pack ? "remap_pack" : "remap_unpack");
 }
 
@@ -168,8 +270,7 @@ static int remap_list(const char* what, bool pack, const void* const* s0, const 
             split.p[1][e] = s1 ? s1[e0 + e] : nullptr;
         }
         char* j = (char*)joint + (size_t)e0 * H * I * (s1 ? 2 : 1) * esz;
-        if (dtype != AMOE_F32) launch<uint16_t>(pack, s1 != nullptr, split, j, n, I, H, (hipStream_t)stream);
-        else launch<uint32_t>(pack, s1 != nullptr, split, j, n, I, H, (hipStream_t)stream);
+        launch(pack, s1 != nullptr, dtype == AMOE_F32, split, j, n, I, H, (hipStream_t)stream);
     }
     return amoe_check_launch(what);
 }

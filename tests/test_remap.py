@@ -127,6 +127,24 @@ def test_hip_remap_bit_exact(ops, gpu_device, dtype, E, I, H):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,E,I,H", [
+    (torch.float16, 2, 64, 256), (torch.bfloat16, 2, 136, 264), (torch.float16, 1, 120, 520), (torch.bfloat16, 3, 264, 248),
+])
+def test_hip_remap_tile_edges(ops, gpu_device, dtype, E, I, H):
+    """Around the tiles of the 2-byte kernel: 256 columns by 64 rows of gate and up, by 128 rows of a single projection."""
+    print("remap", dtype, E, I, H, flush=True)
+    bits = torch.randint(-2**15, 2**15, (3, E, I, H), generator=torch.Generator().manual_seed(E * 1000 + I + H), dtype=torch.int16)
+    gate, up = bits[0].view(dtype).to(gpu_device), bits[1].view(dtype).to(gpu_device)
+    down = bits[2].view(E, H, I).view(dtype).to(gpu_device)
+    raw = lambda t: t.cpu().view(torch.int16).numpy().view(np.uint16)
+    gu, dn = ops.remap_pack(gate, up), ops.remap_pack(down)
+    assert np.array_equal(raw(gu), RO.pack_gate_up(raw(gate), raw(up)))
+    assert np.array_equal(raw(dn), RO.pack_down(raw(down)))
+    assert all(np.array_equal(raw(a), raw(b)) for a, b in zip(ops.remap_unpack(gu, two=True), (gate, up)))
+    assert np.array_equal(raw(ops.remap_unpack(dn, two=False)), raw(down))
+
+
+@pytest.mark.gpu
 def test_hip_remap_headline_shape_round_trip(ops, gpu_device):
     E, I, H = 128, 768, 2048
     g = torch.Generator(device=gpu_device).manual_seed(5)
