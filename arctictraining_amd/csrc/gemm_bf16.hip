@@ -1406,6 +1406,19 @@ int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, int tiles, h
 int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s);
 int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s);
 
+// Weights that a call reads once and that the last-level cache (256 MiB in front of all XCDs) cannot hold until the next call
+// are loaded past the caches: a read of 1 GB takes 6.3 TB/s with ordinary loads, 7.1 with non-temporal ones, and what lies in
+// the cache stays (of weights that fit, the ordinary loads are faster: of 8 experts of 2048 x 768 for one token 10 %).
+// Once means one tile of rows; the kernel of 256-row tiles leaves the experts with more to the caches (with 384 rows an expert
+// the products of 128 experts of 2048 x 768 were 13 % slower past them).
+// Before and after, bf16, K=8 of 128 experts of 2048 x 768: 64 tokens 245 -> 221 us, 3001 tokens 360 -> 336, a training step
+// of 509 tokens 963 -> 905; 30 other sizes of such weights 0.98 to 1.12 times faster, 1.05 on average.  Whether a single
+// product gains depends on what it finds in the cache and has to displace: only whole passes say something.
+static bool streamed_weights(int R, int E, long long strideB)
+{
+    return R <= 256ll * E && (long long)(R < E ? R : E) * strideB * 2 > 256ll << 20;
+}
+
 // rows mode driver shared by the three row-grouped entry points
 // split, split_bytes: where the parts of a reduction that is cut into parts go (null: it is not cut)
 template <bool B_KC, int EPI, int ACT>
@@ -1459,6 +1472,7 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
         const size_t fit = (workspace_bytes - 16) / sizeof(int4);
         a.max_mtiles = fit < (1u << 20) ? (int)fit : 1 << 20;
     }
+    a.stream = streamed_weights(R, E, strideB);
     if (bm < tc.bm) {
         if constexpr (EPI == EPI_GATED) return amoe_skinny_gateup_act(a, ACT, bm, s);
         else if constexpr (EPI == EPI_STORE && !B_KC) return amoe_skinny_nn(a, bm, s);
@@ -1580,7 +1594,9 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
     if (tile_cfg == 0) {
         // Below 256 rows per expert the product is bound by the gradients' stores, and a tile of the default kernel is
         // never done in less than three K tiles: the 32-wide K tiles and one-tile workgroups of shape 5 are faster there
-        // (128 experts of 2048 x 1536: 32 rows 0.19 against 0.21 ms, 188 rows equal, 375 rows 0.43 against 0.40).
+        // (128 experts of 2048 x 1536: 32 rows 0.19 against 0.21 ms, 188 rows equal, 375 rows 0.43 against 0.40), and leave
+        // compute units to the other stream's products (64 experts of 2048 x 1408, 250 rows, gate_up's gradient alone 0.37
+        // against 0.34 ms, the whole step 1.63 against 1.74).
         if (R >= 256ll * E && offsets32 && per * per * E < (1ll << 32))
             return amoe_pp_wgrad(a, s);
         tile_cfg = 5;

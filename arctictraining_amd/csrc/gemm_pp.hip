@@ -58,13 +58,20 @@ struct Mfma16<f16_t> {
 // rows past an expert's end, columns past the matrix and the K remainder need no clamping and no masking.
 // Not known to the compiler: the kernel's own vmcnt waits cover it.
 // (lds_addr = lds_base + LDS_OFF is formed in M0 itself)
-template <uint32_t LDS_OFF>
+// STREAM: non-temporal, for what is read once
+template <uint32_t LDS_OFF, bool STREAM = false>
 __device__ __forceinline__ void pp_dma16(const srd_t& d, uint32_t off, uint32_t lds_base)
 {
-    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :
-                 : "s"(lds_base), "v"(off), "s"(d), "n"(LDS_OFF)
-                 : "memory", "scc");
+    if constexpr (STREAM)
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+                     :
+                     : "s"(lds_base), "v"(off), "s"(d), "n"(LDS_OFF)
+                     : "memory", "scc");
+    else
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :
+                     : "s"(lds_base), "v"(off), "s"(d), "n"(LDS_OFF)
+                     : "memory", "scc");
 }
 __device__ __forceinline__ srd_t pp_srd(const void* base)
 {
@@ -165,7 +172,7 @@ __device__ __forceinline__ int pp_here(int v)
 // is about 5 us, of which half are its stores.  The gated epilogues cost more: the gate_up product of K = 2048 runs at
 // 0.96-1.08 (128 uneven / even experts; the library's plain product of that size at 1.0), the gated backward one at 0.87.  The kernel this one replaced (32-wide K tiles, 32x32x16 MFMAs, all
 // eight waves in step) ran at 1.0-1.1 on the same problems.
-template <bool B_KC, int EPI, int ACT, typename ET>
+template <bool B_KC, int EPI, int ACT, bool STREAM, typename ET>
 __device__ __forceinline__ void pp_rows_body()
 {
     typedef typename Elem16<ET>::frag_t frag_t;
@@ -254,7 +261,13 @@ __device__ __forceinline__ void pp_rows_body()
     const bf16_t* const A = pp_args().A;
     const bool gather = pp_args().a_row_map != nullptr;
     const uint32_t bstep = B_KC ? PP_BK * 2 : (uint32_t)ldb * (PP_BK * 2);
-    auto expert_b = [&](int e) { args_t& p = pp_args(); return p.B + (long long)e * p.strideB; };
+    // STREAM: the weights of an expert whose rows are one tile are read once, those of the others by several workgroups
+    bool stream_b = false, stream_n = false;
+    auto expert_b = [&](int e) {
+        args_t& p = pp_args();
+        if (STREAM) stream_n = scalar_load_i32(p.offsets + e + 1) - scalar_load_i32(p.offsets + e) <= PP_BM;
+        return p.B + (long long)e * p.strideB;
+    };
     // a plan without rows (m0 == mend) or columns (n0 >= N) reads nothing
     auto plan_a = [&](int m0, int mend, const int32_t* map, int k0) {     // map: the row map (first tile), else the indices are in LDS
         const int th = pp_here(tid);
@@ -279,6 +292,7 @@ __device__ __forceinline__ void pp_rows_body()
         const int k = ((th & 7) ^ ((r >> 1) & 7)) * 8;
         const int col = ((th & 15) ^ (2 * ((kr & 3) | (((kr >> 3) & 1) << 2)))) * 8;
         bd = pp_srd(B);
+        if (STREAM) stream_b = stream_n;
         if constexpr (PART) pp_advance(bd, B_KC ? (uint32_t)k0 * 2u : (uint32_t)k0 * ((uint32_t)ldb * 2u));
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -309,8 +323,13 @@ __device__ __forceinline__ void pp_rows_body()
     };
     auto dma_b = [&](auto B_) {
         constexpr int b = decltype(B_)::value;
-        pp_dma16<(2 + b) * PP_HALF>(bd, boff[b][0], fill);
-        pp_dma16<(2 + b) * PP_HALF + 8192u>(bd, boff[b][1], fill);
+        if (STREAM && stream_b) {
+            pp_dma16<(2 + b) * PP_HALF, true>(bd, boff[b][0], fill);
+            pp_dma16<(2 + b) * PP_HALF + 8192u, true>(bd, boff[b][1], fill);
+        } else {
+            pp_dma16<(2 + b) * PP_HALF>(bd, boff[b][0], fill);
+            pp_dma16<(2 + b) * PP_HALF + 8192u>(bd, boff[b][1], fill);
+        }
     };
     auto next_k = [&]() {
         fill ^= PP_STAGE;
@@ -1092,15 +1111,15 @@ __device__ __forceinline__ void pp_wgrad_body()
     pp_vmwait<0>();   // (loads past the last tile wrote zeros into LDS: landed before the workgroup leaves)
 }
 
-template <bool B_KC, int EPI, int ACT>
+template <bool B_KC, int EPI, int ACT, bool STREAM>
 __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_rows_bf16_kernel(GemmArgs)
 {
-    pp_rows_body<B_KC, EPI, ACT, bf16_t>();
+    pp_rows_body<B_KC, EPI, ACT, STREAM, bf16_t>();
 }
-template <bool B_KC, int EPI, int ACT>
+template <bool B_KC, int EPI, int ACT, bool STREAM>
 __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_rows_f16_kernel(GemmArgs)
 {
-    pp_rows_body<B_KC, EPI, ACT, f16_t>();
+    pp_rows_body<B_KC, EPI, ACT, STREAM, f16_t>();
 }
 
 template <int MAPS>
@@ -1118,6 +1137,12 @@ __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_wgrad_f16_kerne
 
 #include "gemm_launch.h"
 
+template <bool B_KC, int EPI, int ACT, bool STREAM>
+static int launch_pp_rows(const GemmArgs& a, int grid, hipStream_t s)
+{
+    if (a.f16) return launch_kernel<grouped_gemm_pp_rows_f16_kernel<B_KC, EPI, ACT, STREAM>, PP_THREADS, PP_LDS>(a, grid, s);
+    return launch_kernel<grouped_gemm_pp_rows_bf16_kernel<B_KC, EPI, ACT, STREAM>, PP_THREADS, PP_LDS>(a, grid, s);
+}
 template <bool B_KC, int EPI, int ACT>
 static int launch_pp_rows(const GemmArgs& a, int tiles, hipStream_t s)
 {
@@ -1125,8 +1150,9 @@ static int launch_pp_rows(const GemmArgs& a, int tiles, hipStream_t s)
     AMOE_REQUIRE(cus > 0, AMOE_ERR_LAUNCH, "grouped_gemm: cannot read the number of compute units");
     // (a multiple of 8: every XCD then runs the same number of workgroups)
     const int grid = ((tiles < cus ? tiles : cus) + 7) & ~7;
-    if (a.f16) return launch_kernel<grouped_gemm_pp_rows_f16_kernel<B_KC, EPI, ACT>, PP_THREADS, PP_LDS>(a, grid, s);
-    return launch_kernel<grouped_gemm_pp_rows_bf16_kernel<B_KC, EPI, ACT>, PP_THREADS, PP_LDS>(a, grid, s);
+    // (parts of a reduction are of few tiles: weights that the caches hold)
+    if (EPI != EPI_PART && a.stream) return launch_pp_rows<B_KC, EPI, ACT, EPI != EPI_PART>(a, grid, s);
+    return launch_pp_rows<B_KC, EPI, ACT, false>(a, grid, s);
 }
 
 // `tiles`: upper bound of the number of tiles

@@ -41,7 +41,7 @@ struct MfmaSkinny<f16_t> {
     }
 };
 
-template <int MT, int CPL, int NW, int EPI, int ACT, typename ET>
+template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET>
 __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[NW][CPL * 64], int e, int m0, int mend, int n0)
 {
     constexpr int W = CPL / 2, H = CPL / 4;           // dwords of a lane's row, groups of four columns
@@ -77,11 +77,11 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[N
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             if constexpr (CPL == 8) {
-                const u32x4_t v = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(bd, vb, sb + k * row_bytes, 0));
+                const u32x4_t v = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(bd, vb, sb + k * row_bytes, STREAM ? 2 : 0));
 #pragma unroll
                 for (int w = 0; w < 4; ++w) s.b[k][w] = v[w];
             } else {
-                const u32x2_t v = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(bd, vb, sb + k * row_bytes, 0));
+                const u32x2_t v = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(bd, vb, sb + k * row_bytes, STREAM ? 2 : 0));
                 s.b[k][0] = v[0];
                 s.b[k][1] = v[1];
             }
@@ -157,7 +157,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[N
 
 // A map's tile is 16 * MT rows where the launch's own rule built it; the taller tiles of a map that was built for another
 // bound of the rows are walked in parts.
-template <int MT, int CPL, int NW, int EPI, int ACT, typename ET>
+template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET>
 __device__ __forceinline__ void skinny_body(const GemmArgs& p)
 {
     __shared__ sk_f32x4 red[NW][CPL * 64];
@@ -171,24 +171,35 @@ __device__ __forceinline__ void skinny_body(const GemmArgs& p)
         m0 = scalar_load_i32(ent + 1);
         mend = scalar_load_i32(ent + 2);
     }
-    skinny_tile<MT, CPL, NW, EPI, ACT, ET>(p, red, e, m0, mend, n0);
+    skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET>(p, red, e, m0, mend, n0);
 #pragma unroll 1
     for (m0 += 16 * MT; m0 < mend; m0 += 16 * MT) {
         __syncthreads();   // (the sums are read before the next part's are written)
-        skinny_tile<MT, CPL, NW, EPI, ACT, ET>(p, red, e, m0, mend, n0);
+        skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET>(p, red, e, m0, mend, n0);
     }
 }
 
 // (at least 4 wavefronts per SIMD with 16 rows, 3 with 32)
-template <int MT, int CPL, int NW, int EPI, int ACT>
+// STREAM: B is loaded past the caches
+template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM>
 __global__ void __launch_bounds__(NW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_bf16_kernel(GemmArgs p)
 {
-    skinny_body<MT, CPL, NW, EPI, ACT, bf16_t>(p);
+    skinny_body<MT, CPL, NW, EPI, ACT, STREAM, bf16_t>(p);
 }
-template <int MT, int CPL, int NW, int EPI, int ACT>
+template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM>
 __global__ void __launch_bounds__(NW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_f16_kernel(GemmArgs p)
 {
-    skinny_body<MT, CPL, NW, EPI, ACT, f16_t>(p);
+    skinny_body<MT, CPL, NW, EPI, ACT, STREAM, f16_t>(p);
+}
+
+template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM>
+int launch_skinny(const GemmArgs& a, int grid, hipStream_t s)
+{
+    if (a.f16)
+        hipLaunchKernelGGL((grouped_gemm_skinny_f16_kernel<MT, CPL, NW, EPI, ACT, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a);
+    else
+        hipLaunchKernelGGL((grouped_gemm_skinny_bf16_kernel<MT, CPL, NW, EPI, ACT, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a);
+    return amoe_check_launch("grouped_gemm_skinny");
 }
 
 template <int MT, int CPL, int NW, int EPI, int ACT>
@@ -197,11 +208,8 @@ int launch_skinny(GemmArgs a, int m_tiles, hipStream_t s)
     a.n_ntiles = (a.N + 16 * CPL - 1) / (16 * CPL);
     const long long grid = (long long)m_tiles * a.n_ntiles;
     AMOE_REQUIRE(grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
-    if (a.f16)
-        hipLaunchKernelGGL((grouped_gemm_skinny_f16_kernel<MT, CPL, NW, EPI, ACT>), dim3((int)grid), dim3(NW * 64), 0, s, a);
-    else
-        hipLaunchKernelGGL((grouped_gemm_skinny_bf16_kernel<MT, CPL, NW, EPI, ACT>), dim3((int)grid), dim3(NW * 64), 0, s, a);
-    return amoe_check_launch("grouped_gemm_skinny");
+    if (a.stream) return launch_skinny<MT, CPL, NW, EPI, ACT, true>(a, (int)grid, s);
+    return launch_skinny<MT, CPL, NW, EPI, ACT, false>(a, (int)grid, s);
 }
 
 // bm: height of the map's tiles; R rows of a.E experts

@@ -1,0 +1,69 @@
+"""Products whose weights are more than the last-level cache holds and are loaded past the caches: 302 MB of nine experts,
+against the same products of five and four of them (168 and 134 MB, loaded through the caches), bit by bit: experts without
+rows, with one tile of 256 rows and with more.  The kernel for few rows sums in another order for fewer tiles: there
+against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+E, K, N = 9, 4128, 4064
+
+
+@pytest.fixture(scope="module")
+def ops(gpu_device):
+    from arctictraining_amd import ops as _ops
+
+    return _ops
+
+
+def _case(gpu_device, dtype, counts):
+    g = torch.Generator(device=gpu_device).manual_seed(sum(counts))
+    draw = lambda *shape: torch.empty(shape, dtype=dtype, device=gpu_device).normal_(0.0, 0.1, generator=g)
+    off = torch.tensor([0] + counts, dtype=torch.int32).cumsum(0).to(torch.int32)
+    return draw, off, int(off[-1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tall_tiles(ops, gpu_device, dtype):
+    draw, off, R = _case(gpu_device, dtype, [256, 257, 0, 255, 1, 300, 32, 90, 511])
+    wide, deep = draw(E, K, N), draw(E, N, K)
+    a, b, gate_up, scale = draw(R, K), draw(R, N), draw(R, 2 * N), torch.rand(R, device=gpu_device)
+    products = {
+        "gate_up": lambda e, r, o: ops.grouped_gemm_gateup_act_fwd(a[r], wide[e], o, row_scale=scale[r]),
+        "nn": lambda e, r, o: ops.grouped_gemm_nn(a[r], wide[e], o),
+        "nt": lambda e, r, o: ops.grouped_gemm_nt(b[r], wide[e], o),
+        "gated_bwd": lambda e, r, o: ops.grouped_gemm_nt_gated_bwd(a[r], deep[e], o, gate_up[r], row_scale=scale[r]),
+    }
+    for name, run in products.items():
+        print("streamed weights", dtype, name, flush=True)
+        whole = run(slice(0, E), slice(0, R), off.to(gpu_device))
+        whole = whole if isinstance(whole, tuple) else (whole,)
+        for lo, hi in ((0, 5), (5, E)):
+            rows = slice(int(off[lo]), int(off[hi]))
+            part = run(slice(lo, hi), rows, (off[lo:hi + 1] - off[lo]).to(gpu_device))
+            for w, p in zip(whole, part if isinstance(part, tuple) else (part,)):
+                assert torch.equal(w[:, rows] if w.dim() == 2 and w.shape[0] != R else w[rows], p), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts", [[1, 0, 16, 3, 0, 8, 5, 2, 0], [17, 8, 0, 31, 1, 2, 0, 4, 7]])   # tiles of 16 and of 32 rows
+def test_low_tiles(ops, gpu_device, dtype, counts):
+    print("streamed weights", dtype, counts, flush=True)
+    draw, off, R = _case(gpu_device, dtype, counts)
+    w, a = draw(E, K, N), draw(R, K)
+    offsets = off.to(gpu_device)
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    got = ops.grouped_gemm_nn(a, w, offsets)
+    gate_up, inter = ops.grouped_gemm_gateup_act_fwd(a, w, offsets)
+    assert torch.equal(gate_up, got)
+    gate, up = gate_up[:, 0::2].double(), gate_up[:, 1::2].double()
+    h = up * gate * torch.sigmoid(gate)
+    # rounded once, and float32's exponential and reciprocal
+    assert bool(((inter.double() - h).abs() <= (u + 2.0 ** -20) * h.abs() + 2.0 ** -24).all())
+    for e in range(E):
+        r = slice(int(off[e]), int(off[e + 1]))
+        x, y = a[r].double(), w[e].double()
+        ref, size = x @ y, x.abs() @ y.abs()
+        # rounded once, and K products summed in float32
+        assert bool(((got[r].double() - ref).abs() <= u * ref.abs() + K * 2.0 ** -24 * size).all()), e
