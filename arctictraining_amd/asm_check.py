@@ -18,7 +18,7 @@ import subprocess
 
 _REG = re.compile(r"\bv(\d+)\b|\bv\[(\d+):(\d+)\]")
 _LABEL = re.compile(r"^(\.LBB\d+_\d+):")
-_KERNEL = re.compile(r"^(_Z\w*grouped_gemm_(?:rows|wgrad|wgrad_parts|pp_rows|pp_wgrad)_(?:bf16|f16)_kernel\w*):")
+_KERNEL = re.compile(r"^(_Z\w*grouped_gemm_(?:rows|wgrad|wgrad_parts|pp_rows|pp_wgrad|short_wgrad)_(?:bf16|f16)_kernel\w*):")
 _BRANCH = re.compile(r"^\s*(s_cbranch_\w+|s_branch)\s+(\.LBB\d+_\d+)")
 
 
@@ -159,8 +159,8 @@ def check_assembly(asm_text: str, min_kernels: int = 1, require_tr: bool = True)
         raise RuntimeError(f"expected at least {min_kernels} GEMM kernels in the assembly, found {len(kernels)}")
     total_tr = 0
     for name, lines in kernels.items():
-        # (the gemm_pp kernels take the transposing read from the compiler, which places its waits itself)
-        violations, n_tr = check_kernel(lines) if "grouped_gemm_pp_" not in name else ([], 0)
+        # (the gemm_pp and gemm_short kernels take the transposing read from the compiler, which places its waits itself)
+        violations, n_tr = check_kernel(lines) if not re.search("grouped_gemm_(pp|short)_", name) else ([], 0)
         total_tr += n_tr
         if violations:
             raise RuntimeError(f"{name}: register touched while a transposing LDS read is outstanding: {violations[:5]}")
@@ -168,7 +168,7 @@ def check_assembly(asm_text: str, min_kernels: int = 1, require_tr: bool = True)
         # array the compiler could not keep in registers (a select between freshly loaded row
         # indices once became a lookup in a scratch array and cost 5 % of the weight gradients).
         # (only the kernels that write M0 in inline assembly: the compiler tracks its own uses)
-        m0 = check_m0(lines) if "grouped_gemm_rows_" in name or "grouped_gemm_pp_" in name else []
+        m0 = check_m0(lines) if re.search("grouped_gemm_(rows|pp|short)_", name) else []
         if m0:
             raise RuntimeError(f"{name}: {m0[:3]}")
         private = [l.strip() for l in lines if re.match(r"\s*scratch_(load|store)", l)]

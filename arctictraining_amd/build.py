@@ -20,7 +20,7 @@ LIB_PATH = os.path.join(LIB_DIR, "libarctic_moe_hip.so")
 
 # (source, object name, extra flags); the 16-bit grouped GEMM is compiled as four groups of entry points in parallel
 GEMM_PARTS = 4
-SOURCES = [(f, os.path.splitext(f)[0], []) for f in ("api.hip", "router.hip", "permute.hip", "rows.hip", "layer.hip", "gemm_skinny.hip", "gemm_split.hip", "gemm_f32.hip", "remap.hip")]
+SOURCES = [(f, os.path.splitext(f)[0], []) for f in ("api.hip", "router.hip", "permute.hip", "rows.hip", "layer.hip", "gemm_skinny.hip", "gemm_split.hip", "gemm_short.hip", "gemm_f32.hip", "remap.hip")]
 # the default tile shape of the same products: one group per epilogue, and the weight gradients
 PP_PARTS = 4
 SOURCES = [("gemm_pp.hip", f"gemm_pp_p{i}", [f"-DAMOE_PP_PART={i}"]) for i in range(PP_PARTS)] + SOURCES
@@ -117,7 +117,7 @@ def build(force: bool = True, jobs: int = 8) -> str:
             return LIB_PATH
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         objs_f = [ex.submit(_compile, item) for item in SOURCES]
-        checks = [ex.submit(_check_gemm_assembly, item) for item in SOURCES if item[0] in ("gemm_bf16.hip", "gemm_pp.hip")]
+        checks = [ex.submit(_check_gemm_assembly, item) for item in SOURCES if item[0] in ("gemm_bf16.hip", "gemm_pp.hip", "gemm_short.hip")]
         objs = [f.result() for f in objs_f]
         # a violation raises here: no library is linked from a source that fails the check
         counts = [c.result() for c in checks]

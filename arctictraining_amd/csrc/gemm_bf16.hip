@@ -1399,6 +1399,8 @@ int amoe_pp_gateup_act(const GemmArgs& a, int act, int tiles, hipStream_t s);
 int amoe_pp_rows(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s);
 int amoe_pp_gated_bwd(const GemmArgs& a, int act, int tiles, hipStream_t s);
 int amoe_pp_wgrad(GemmArgs a, hipStream_t s);
+// few rows to reduce over (gemm_short.hip)
+int amoe_short_wgrad(GemmArgs a, hipStream_t s);
 // few tiles of a deep reduction (gemm_split.hip)
 int amoe_split_count(int R, int E, int K, int N);
 int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, int tiles, hipStream_t s);
@@ -1592,11 +1594,13 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
     // tiles, the kernel with 64-bit addresses runs.
     const long long per = (long long)a.n_mt * a.n_ntiles;
     if (tile_cfg == 0) {
-        // Below 256 rows per expert the product is bound by the gradients' stores, and a tile of the default kernel is
-        // never done in less than three K tiles: the 32-wide K tiles and one-tile workgroups of shape 5 are faster there
-        // (128 experts of 2048 x 1536: 32 rows 0.19 against 0.21 ms, 188 rows equal, 375 rows 0.43 against 0.40), and leave
-        // compute units to the other stream's products (64 experts of 2048 x 1408, 250 rows, gate_up's gradient alone 0.37
-        // against 0.34 ms, the whole step 1.63 against 1.74).
+        // Up to 128 rows per expert the product is bound by the gradients' stores: gemm_short.hip, where its 32-bit tile
+        // numbers reach (with a fourth of these tiles' size).  It and shape 5 inside a training step: 812 against 905 us at 32
+        // rows, 545 against 572 at 111, 334 against 363 at 136 (and the same without the second stream), 764 against 710 at 250.
+        // A tile of the default kernel is never done in less than three K tiles, and its workgroups leave no compute unit to
+        // the other stream's products: below 256 rows the one-tile workgroups of shape 5 are faster (64 experts of 2048 x
+        // 1408, 250 rows, gate_up's gradient alone 0.37 against 0.34 ms, the whole step 1.63 against 1.74).
+        if (R <= 128ll * E && offsets32 && 16 * per * per * E < (1ll << 32)) return amoe_short_wgrad(a, s);
         if (R >= 256ll * E && offsets32 && per * per * E < (1ll << 32))
             return amoe_pp_wgrad(a, s);
         tile_cfg = 5;
