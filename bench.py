@@ -306,16 +306,17 @@ def main():
     tile = {1: "128, 128, 2, 2", 2: "256, 128, 2, 2", 3: "256, 256, 2, 2", 5: "256, 256, 4, 2"}.get(c, "256, 256, 2, 4")
     rows = f"grouped_gemm_rows_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_rows_bf16_kernel<"
     wgrad = f"grouped_gemm_wgrad_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_wgrad_bf16_kernel<"
+    end = ">" if c else ", false>"   # (every workload here has far more than a tile of rows per expert)
     gathered = token_of is not None
     sym = {
-        # grouped_gemm_pp_rows_bf16_kernel<B K-contiguous, epilogue, activation>; other tile shapes:
+        # grouped_gemm_pp_rows_bf16_kernel<B K-contiguous, epilogue, activation, B past the caches>; other tile shapes:
         # grouped_gemm_rows_bf16_kernel<BM, BN, waves along M, waves along N, B K-contiguous, epilogue, activation>
-        "gemm_gateup_act_fwd": f"{rows}false, 1, 0>",
-        "gemm_down_fwd": f"{rows}false, 0, 0>",
-        "gemm_dgrad_down": f"{rows}true, 0, 0>",
-        "gemm_dgrad_down_gated_bwd": f"{rows}true, 2, 0>",
-        "gemm_dgrad_gateup": f"{rows}true, 0, 0>",
-        # grouped_gemm_pp_wgrad_bf16_kernel<gathered operand>; other tile shapes, and fewer than 256 rows per expert:
+        "gemm_gateup_act_fwd": f"{rows}false, 1, 0{end}",
+        "gemm_down_fwd": f"{rows}false, 0, 0{end}",
+        "gemm_dgrad_down": f"{rows}true, 0, 0{end}",
+        "gemm_dgrad_down_gated_bwd": f"{rows}true, 2, 0{end}",
+        "gemm_dgrad_gateup": f"{rows}true, 0, 0{end}",
+        # grouped_gemm_pp_wgrad_bf16_kernel<gathered operand> (256 rows per expert or more); other tile shapes:
         # grouped_gemm_wgrad_bf16_kernel<BM, BN, waves along M, waves along N, gathered operand>
         "gemm_wgrad_down": f"{wgrad}{2 if gathered else 0}>",
         "gemm_wgrad_gateup": f"{wgrad}{1 if gathered else 0}>",
