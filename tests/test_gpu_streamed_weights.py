@@ -1,7 +1,7 @@
 """Products whose weights are more than the last-level cache holds and are loaded past the caches: 302 MB of nine experts,
 against the same products of five and four of them (168 and 134 MB, loaded through the caches), bit by bit: experts without
 rows, with one tile of 256 rows and with more.  The kernel for few rows sums in another order for fewer tiles: there
-against float64."""
+against float64.  The sums of rows over the same bound as well."""
 import pytest
 import torch
 
@@ -67,3 +67,20 @@ def test_low_tiles(ops, gpu_device, dtype, counts):
         ref, size = x @ y, x.abs() @ y.abs()
         # rounded once, and K products summed in float32
         assert bool(((got[r].double() - ref).abs() <= u * ref.abs() + K * 2.0 ** -24 * size).all()), e
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("top_k", [2, 4, 7, 9])
+def test_row_sums(ops, gpu_device, dtype, top_k):
+    """Sums of more rows than the last-level cache holds, against the same in two halves, bit by bit."""
+    size, H = torch.finfo(dtype).bits // 8, 4104
+    T = (300 << 20) // (top_k * H * size)
+    print("streamed rows", dtype, top_k, T, flush=True)
+    g = torch.Generator(device=gpu_device).manual_seed(top_k)
+    rows = torch.empty((T * top_k, H), dtype=dtype, device=gpu_device).normal_(generator=g)
+    row_of = torch.randperm(T * top_k, device=gpu_device, generator=g).view(T, top_k).to(torch.int32)
+    scores = torch.rand((T, top_k), device=gpu_device, generator=g)
+    addend = torch.empty((T, H), dtype=dtype, device=gpu_device).normal_(generator=g)
+    for run in (lambda t: ops.combine_fwd(rows, row_of[t].contiguous(), scores[t].contiguous()),
+                lambda t: ops.gather_rows_bwd(rows, row_of[t].contiguous(), addend[t].contiguous())):
+        assert torch.equal(run(slice(0, T)), torch.cat([run(slice(0, T // 2)), run(slice(T // 2, T))]))
