@@ -114,7 +114,8 @@ __device__ __forceinline__ void dma4_sbase(const void* base, uint32_t lane_offse
 // (a tile for every tenth compute unit) 72 -> 46; gate_up of the first 257 -> 230.
 __device__ __forceinline__ void gelu_parts(float g, float& phi, float& ex)
 {
-    const float d = 1.0f + 0.261629509f * fabsf(g), r = __builtin_amdgcn_rcpf(d), t = r + r * __builtin_fmaf(-d, r, 1.0f);
+    // (infinities: from 14 on ex is 0, and the bound keeps inf * 0 out of t)
+    const float d = 1.0f + 0.261629509f * fminf(fabsf(g), 16.0f), r = __builtin_amdgcn_rcpf(d), t = r + r * __builtin_fmaf(-d, r, 1.0f);
     ex = __builtin_amdgcn_exp2f(-0.72134752f * g * g);
     float h = 0.0308933929f;
     h = h * t + -0.151304632f;

@@ -658,3 +658,49 @@ def test_gelu_of_the_epilogues(gpu_device, dtype, copies):
         got = dg.cpu().double()
         assert ((got[:, 0::2] - d).abs() <= eps * d.abs() + 1e-6).all()
         assert ((got[:, 1::2] - ref).abs() <= eps * ref.abs() + tiny).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("copies,cfg", [(1, 0), (40, 0), (40, 1)])
+def test_gelu_of_gates_without_end(gpu_device, dtype, copies, cfg):
+    """Gates that are infinite (by overflow: each sum of two terms), the largest that there are, NaN, and where the
+    exponential ends: as 0.5 g (1 + erff(g / sqrt 2)) and its derivative have them."""
+    from arctictraining_amd import ops
+
+    print("gelu without end", dtype, copies, cfg, flush=True)
+    top = torch.finfo(dtype).max
+    pairs = torch.tensor([(top, top), (-top, -top), (top, 0), (-top, 0), (14, 0), (-14, 0), (40, 0), (-40, 0), (0, 0), (-0.0, 0)])
+    x = torch.zeros(len(pairs), 32, dtype=dtype)
+    x[:, 0], x[:, 1], x[:, 2] = pairs[:, 0].to(dtype), pairs[:, 1].to(dtype), 1.0
+    w = torch.zeros(1, 32, 128, dtype=dtype)
+    w[0, :2, 0::2] = 1.0
+    w[0, 2, 1::2] = 1.0
+    x = x.repeat(copies, 1).to(gpu_device)
+    off = torch.tensor([0, x.shape[0]], dtype=torch.int32, device=gpu_device)
+    gu, inter = ops.grouped_gemm_gateup_act_fwd(x, w.to(gpu_device), off, ops.ACT_GELU, tile_cfg=cfg)
+    g = gu[:, 0].cpu().float()
+    assert g.isinf().sum() == 2 * copies
+
+    def same(got, ref):
+        got, ref = got.cpu().float(), ref.to(dtype).float()
+        assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+        ok = ref.isfinite()
+        # (a tail that 1 + erff has lost is not 0 here: below 1e-40 it is in neither type)
+        assert ((got - ref)[ok].abs() <= 2.0**-7 * ref[ok].abs() + 1e-40).all() and torch.equal(got[ref.isinf()], ref[ref.isinf()])
+
+    def former(g):
+        phi = 0.5 * (1.0 + torch.erf(g * 0.7071067811865476))
+        return g * phi, phi + g * (0.3989422804014327 * torch.exp(-0.5 * g * g))
+
+    for col in (0, 63):
+        same(inter[:, col], former(g)[0])
+    gu[3, 0::2] = float("nan")
+    g = gu[:, 0].cpu().float()
+    wd = torch.zeros(1, 64, 32, dtype=dtype)
+    wd[0, :, 0] = 1.0
+    dy = torch.zeros(x.shape[0], 32, dtype=dtype, device=gpu_device)
+    dy[:, 0] = 1.0
+    dg, _ = ops.grouped_gemm_nt_gated_bwd(dy, wd.to(gpu_device), off, gu, ops.ACT_GELU, tile_cfg=cfg)
+    f, df = former(g)
+    same(dg[:, 0], df)
+    same(dg[:, 127], f)
