@@ -103,30 +103,39 @@ __device__ __forceinline__ void dma4_sbase(const void* base, uint32_t lane_offse
                  : "memory");
 }
 
-// Phi(g), the normal distribution function of the exact gelu, and exp(-g^2 / 2), which its derivative needs as well:
-// erfc(z) = exp(-z^2) P(1 / (1 + 0.37 z)) for z = |g| / sqrt 2, P of degree 9 without a constant term, fitted to the least
-// largest relative error (1.8e-8) on z < 9.6; below 0 it is half of that, above it 1 less half of it.
-// In float32 the values are off by 1.5e-8 on average and 2.3e-7 at most (erff: 1.2e-8, 6e-8), and in the lower tail by
-// 1.5e-6 of themselves (1 + erff(z) has no digit left there); the products' errors against float64 stay what they were, to
-// four digits in 16-bit results, within 3 % up and down in the float32 row sums.
-// Bound by vector instructions, of which erff takes some 60 and both sides of a branch: gated backward product of 10650 rows,
-// 21 experts, 896 x 4320 308 -> 181 us, of 7512 rows, 114 experts, 3072 x 608 199 -> 157, of 3969 rows, 6 experts, 1504 x 128
-// (a tile for every tenth compute unit) 72 -> 46; gate_up of the first 257 -> 230.
+// Phi(g), the normal distribution function of the exact gelu, and exp(-g^2 / 2), which its derivative needs as well.
+// |g| < 1.484375: 0.5 + g S(g^2), S of degree 6, off by 2.0e-9 at most.  Beyond it the tail on the far side, exp(-g^2 / 2) times
+// a polynomial of degree 7 without a constant term in t = 1 / (1 + 0.4 |g|), off by 4.9e-8 of itself (both fitted to the least
+// largest error, coefficients rounded one after the other): below 0 Phi itself, above it 1 less it.  The tail's form alone
+// will not do: 1 less a tail of nearly 0.5 keeps every rounding of the tail's chain.
+// Error of gelu(g) / g in float32 over all float16 gates up to 8, with erff / with that form alone / so: largest 1.05e-7 / 1.95e-7 /
+// 0.90e-7, root mean square 2.06e-8 / 4.73e-8 / 1.89e-8, and in the lower tail 1.5e-6 of its value, where 1 + erff(z) has no
+// digit left.  Infinities and NaN come out as with erff: gelu(inf) = inf, gelu(-inf) = -inf * 0 = NaN, the derivative of both
+// inf * 0 = NaN.  (No step from |g| to t may meet inf * 0: a Newton step on the reciprocal would.)
+// Bound by vector instructions, of which erff takes some 60 and both sides of a branch.  With erff / so, gated backward
+// product of 10650 rows, 21 experts, 896 x 4320 321 / 191 us (the tail's form alone 183), of 7512 rows, 114 experts, 3072 x 608
+// 201 / 151 (145), of 3969 rows, 6 experts, 1504 x 128 (a tile for every tenth compute unit) 71 / 49 (46); gate_up of the
+// first 254 / 232 (225).
 __device__ __forceinline__ void gelu_parts(float g, float& phi, float& ex)
 {
-    // (infinities: from 14 on ex is 0, and the bound keeps inf * 0 out of t)
-    const float d = 1.0f + 0.261629509f * fminf(fabsf(g), 16.0f), r = __builtin_amdgcn_rcpf(d), t = r + r * __builtin_fmaf(-d, r, 1.0f);
-    ex = __builtin_amdgcn_exp2f(-0.72134752f * g * g);
-    float h = 0.0308933929f;
-    h = h * t + -0.151304632f;
-    h = h * t + 0.242733046f;
-    h = h * t + -0.141864985f;
-    h = h * t + 0.154850304f;
-    h = h * t + 0.0534974113f;
-    h = h * t + 0.103065364f;
-    h = h * t + 0.103723742f;
-    h = h * t + 0.104406342f;
-    phi = g < 0.f ? h * (t * ex) : __builtin_fmaf(-h, t * ex, 1.0f);
+    const float a = fabsf(g), u = g * g, t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.4f, a, 1.0f));
+    ex = __builtin_amdgcn_exp2f(-0.72134752f * u);
+    float h = 0.0687517524f;
+    h = __builtin_fmaf(h, t, -0.18816857f);
+    h = __builtin_fmaf(h, t, 0.10725268f);
+    h = __builtin_fmaf(h, t, 0.0545073859f);
+    h = __builtin_fmaf(h, t, 0.139302209f);
+    h = __builtin_fmaf(h, t, 0.159056231f);
+    h = __builtin_fmaf(h, t, 0.159598291f);
+    float s = 3.58700191e-07f;
+    s = __builtin_fmaf(s, u, -8.34226012e-06f);
+    s = __builtin_fmaf(s, u, 0.000113329719f);
+    s = __builtin_fmaf(s, u, -0.00118514698f);
+    s = __builtin_fmaf(s, u, 0.00997239258f);
+    s = __builtin_fmaf(s, u, -0.0664901063f);
+    s = __builtin_fmaf(s, u, 0.398942262f);
+    const float q = t * ex, tail = g < 0.f ? h * q : __builtin_fmaf(-h, q, 1.0f);
+    phi = a < 1.484375f ? __builtin_fmaf(g, s, 0.5f) : tail;
 }
 
 // Activation for the bf16 epilogue: the sigmoid's division by the hardware reciprocal (1 ulp; the

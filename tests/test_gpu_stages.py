@@ -661,6 +661,30 @@ def test_gelu_of_the_epilogues(gpu_device, dtype, copies):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("cfg", [0, 1])
+def test_gelu_is_no_further_off_than_with_erff(gpu_device, dtype, cfg):
+    """Every 16-bit gate up to 8, in float32: with one column of d_inter and of up that is not zero, a score partial is
+    gelu of that column's gate.  0.5 (1 + erff(z)), of roundings of half a place of 1 + erff and of erff and of z, is off by
+    up to 6.1e-8; the product with the gate is rounded once more."""
+    from arctictraining_amd import ops
+
+    print("gelu against erff", dtype, cfg, flush=True)
+    v = torch.arange(-(1 << 15), 1 << 15, dtype=torch.int32).to(torch.int16).view(dtype)
+    v = v[v.float().abs() <= 8]
+    R, H, I = v.numel(), 32, 64
+    gu = torch.zeros(R, 2 * I, dtype=dtype)
+    gu[:, 0], gu[:, 1] = v, 1.0
+    wd = torch.zeros(1, I, H, dtype=dtype)
+    wd[0, 0, 0] = 1.0
+    dy = torch.zeros(R, H, dtype=dtype)
+    dy[:, 0] = 1.0
+    off = torch.tensor([0, R], dtype=torch.int32, device=gpu_device)
+    _, parts = ops.grouped_gemm_nt_gated_bwd(dy.to(gpu_device), wd.to(gpu_device), off, gu.to(gpu_device), ops.ACT_GELU, tile_cfg=cfg)
+    got, ref = parts.sum(0).cpu().double(), v.double() * torch.special.ndtr(v.double())
+    assert ((got - ref).abs() <= 6.1e-8 * v.double().abs() + 2.0**-24 * ref.abs() + 2.0**-126).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("copies,cfg", [(1, 0), (40, 0), (40, 1)])
 def test_gelu_of_gates_without_end(gpu_device, dtype, copies, cfg):
     """Gates that are infinite (by overflow: each sum of two terms), the largest that there are, NaN, and where the
