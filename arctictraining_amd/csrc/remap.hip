@@ -18,6 +18,8 @@
 // 1.79 and 2.15 ms.
 #include "amoe_common.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int TILE = 64;   // (of 4-byte elements)
@@ -37,15 +39,15 @@ struct Listed {
     __device__ __forceinline__ T* at(int g, int e) const { return (T*)p[g][e]; }
 };
 
-// 2-byte elements: 256 columns h by 64 dwords of two elements that lie side by side in the joint side, (gate, up) of one
+// 2-byte elements: TH = 256 (or 128) columns h by 64 dwords of two elements that lie side by side in the joint side, (gate, up) of one
 // i, or i and i + 1 of a single projection.  A thread moves two rows' 16-byte vectors, interleaved in registers, so that
 // LDS sees dwords; 16-byte chunk c of LDS row h is kept at c ^ ((h / 8) % 16), which spreads a wavefront's dwords (8 rows
 // apart) over all banks.  Wide tiles for long pieces: with 128 or 64 columns the split side is accessed in pieces of 256
 // or 128 bytes instead of 512, and gate and up of the size above take 288 or 298 us, with 256 270.
-template <int G, bool PACK, typename SPLIT>
+template <int TH, int G, bool PACK, typename SPLIT>
 __global__ void __launch_bounds__(256) remap16_kernel(SPLIT split, uint16_t* __restrict__ joint, int I, int H, long long joint_es)
 {
-    constexpr int TH = 256, W = 64, ROWS = W * 2 / G;     // columns h, dwords of a joint row, rows i
+    constexpr int W = 64, ROWS = W * 2 / G;     // dwords of a joint row, rows i
     constexpr int NS = W * TH / 8 / 256, NJ = TH * W / 4 / 256;
     __shared__ __attribute__((aligned(16))) uint32_t tile[TH * W];
     typedef uint32_t vec_t __attribute__((ext_vector_type(4)));
@@ -102,7 +104,10 @@ __global__ void __launch_bounds__(256) remap16_kernel(SPLIT split, uint16_t* __r
         vec_t x[NJ];
 #pragma unroll
         for (int n = 0; n < NJ; ++n) {
-            if (joint_at(n, hh, d, off)) x[n] = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(j + off));
+            const bool in = joint_at(n, hh, d, off);
+            // (the narrow form without a branch, what is past the end a copy of the first: around branches the compiler keeps eight
+            // vectors as one value of 232 registers)
+            if (TH < 256 || in) x[n] = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(j + (in ? off : 0)));
         }
 #pragma unroll
         for (int n = 0; n < NJ; ++n) {
@@ -201,8 +206,18 @@ void launch(bool wide, const SPLIT& split, void* joint, int E, int I, int H, hip
         const dim3 grid((H + TILE - 1) / TILE, (I + TILE - 1) / TILE, E);
         hipLaunchKernelGGL((remap_kernel<uint32_t, G, PACK, SPLIT>), grid, dim3(256), 0, s, split, (uint32_t*)joint, I, H, joint_es);
     } else {
-        const dim3 grid((H + 255) / 256, (I * G + 127) / 128, E);
-        hipLaunchKernelGGL((remap16_kernel<G, PACK, SPLIT>), grid, dim3(256), 0, s, split, (uint16_t*)joint, I, H, joint_es);
+        // Narrow tiles where wide ones would leave most of their lanes idle.  64 matrices each of gate and up, 0.6 GB in all, import /
+        // export, us, narrow / wide: H = 64 201 / 248 and 206 / 220, 96 208 / 219 and 206 / 221, 288 239 / 254 and 229 / 254, 320 211 / 233 and
+        // 208 / 245, 384 213 / 233 and 205 / 231; past the lines 160 262 / 219 and 248 / 219, 416 245 / 243, 512 223 / 215, 2048 218 / 208.
+        // (64 x 64 tiles: 244 and 239 at 288.)  Rows that are no multiple of 64 bytes are exported
+        // faster by wide tiles: 272 309 / 300, 296 346 / 308.
+        const bool narrow = H <= 96 || (H > 256 && H <= 384 && (PACK || H % 32 == 0));
+        auto run = [&](auto TH) {
+            const dim3 grid((H + TH - 1) / TH, (I * G + 127) / 128, E);
+            hipLaunchKernelGGL((remap16_kernel<decltype(TH)::value, G, PACK, SPLIT>), grid, dim3(256), 0, s, split, (uint16_t*)joint, I, H, joint_es);
+        };
+        if (narrow) run(std::integral_constant<int, 128>{});
+        else run(std::integral_constant<int, 256>{});
     }
 }
 

@@ -129,9 +129,12 @@ def test_hip_remap_bit_exact(ops, gpu_device, dtype, E, I, H):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,E,I,H", [
     (torch.float16, 2, 64, 256), (torch.bfloat16, 2, 136, 264), (torch.float16, 1, 120, 520), (torch.bfloat16, 3, 264, 248),
+    (torch.bfloat16, 2, 72, 96), (torch.float16, 1, 136, 104), (torch.bfloat16, 2, 136, 288), (torch.float16, 2, 72, 384),
+    (torch.bfloat16, 1, 288, 392), (torch.float16, 1, 96, 16),
 ])
 def test_hip_remap_tile_edges(ops, gpu_device, dtype, E, I, H):
-    """Around the tiles of the 2-byte kernel: 256 columns by 64 rows of gate and up, by 128 rows of a single projection."""
+    """Around the tiles of the 2-byte kernel, 256 or 128 columns by 64 rows of gate and up, by 128 rows of a single
+    projection, and on both sides of the rule that chooses between them."""
     print("remap", dtype, E, I, H, flush=True)
     bits = torch.randint(-2**15, 2**15, (3, E, I, H), generator=torch.Generator().manual_seed(E * 1000 + I + H), dtype=torch.int16)
     gate, up = bits[0].view(dtype).to(gpu_device), bits[1].view(dtype).to(gpu_device)
