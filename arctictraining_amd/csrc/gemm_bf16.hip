@@ -1408,17 +1408,23 @@ int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, int tiles, h
 int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s);
 int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s);
 
-// Weights that a call reads once and that the last-level cache (256 MiB in front of all XCDs) cannot hold until the next call
-// are loaded past the caches: a read of 1 GB takes 6.3 TB/s with ordinary loads, 7.1 with non-temporal ones, and what lies in
-// the cache stays (of weights that fit, the ordinary loads are faster: of 8 experts of 2048 x 768 for one token 10 %).
+// From how many tiles of rows on a product's weights are loaded past the caches (0: never).
+// Weights that are read once and that the last-level cache (256 MiB in front of all XCDs) cannot hold until the next call
+// are: a read of 1 GB takes 6.3 TB/s with ordinary loads, 7.1 with non-temporal ones, and what lies in the cache stays (of
+// weights that fit, the ordinary loads are faster: of 8 experts of 2048 x 768 for one token 10 %).
 // Once means one tile of rows; the kernel of 256-row tiles leaves the experts with more to the caches (with 384 rows an expert
-// the products of 128 experts of 2048 x 768 were 13 % slower past them).
-// Before and after, bf16, K=8 of 128 experts of 2048 x 768: 64 tokens 245 -> 221 us, 3001 tokens 360 -> 336, a training step
-// of 509 tokens 963 -> 905; 30 other sizes of such weights 0.98 to 1.12 times faster, 1.05 on average.  Whether a single
+// the products of 128 experts of 2048 x 768 were 13 % slower past them).  How many experts have rows at all only the GPU
+// knows, so that the kernel of 256-row tiles compares their number: of 154 experts of 960 x 1152 of which a skewed router uses
+// some twenty, 1679 tokens took 160 us past the caches and 154 through them.  (The kernel for few rows goes by the bound: with
+// both forms in one its registers spill.)
+// Before and after, bf16, K=8 of 128 experts of 2048 x 768: 64 tokens 242 -> 219 us, 3001 tokens 365 -> 341, a training step
+// of 509 tokens 905 -> 827; 124 other sizes of such weights 0.98 to 1.19 times faster, 1.04 on average.  Whether a single
 // product gains depends on what it finds in the cache and has to displace: only whole passes say something.
-static bool streamed_weights(int R, int E, long long strideB)
+static int stream_from(int R, int E, long long strideB)
 {
-    return R <= 256ll * E && (long long)(R < E ? R : E) * strideB * 2 > 256ll << 20;
+    const long long least = (256ll << 20) / (strideB * 2) + 1;
+    if (R > 256ll * E || (R < E ? R : E) < least) return 0;
+    return (int)least;
 }
 
 // rows mode driver shared by the three row-grouped entry points
@@ -1474,7 +1480,7 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
         const size_t fit = (workspace_bytes - 16) / sizeof(int4);
         a.max_mtiles = fit < (1u << 20) ? (int)fit : 1 << 20;
     }
-    a.stream = streamed_weights(R, E, strideB);
+    a.stream_from = stream_from(R, E, strideB);
     if (bm < tc.bm) {
         if constexpr (EPI == EPI_GATED) return amoe_skinny_gateup_act(a, ACT, bm, s);
         else if constexpr (EPI == EPI_STORE && !B_KC) return amoe_skinny_nn(a, bm, s);

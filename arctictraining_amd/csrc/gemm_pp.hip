@@ -135,11 +135,13 @@ __device__ __forceinline__ void pp_rows_body()
     const bf16_t* const A = pp_args().A;
     const bool gather = pp_args().a_row_map != nullptr;
     const uint32_t bstep = B_KC ? PP_BK * 2 : (uint32_t)ldb * (PP_BK * 2);
-    // STREAM: the weights of an expert whose rows are one tile are read once, those of the others by several workgroups
+    // STREAM: the weights of an expert whose rows are one tile are read once, those of the others by several workgroups; all
+    // the tiles' weights have to be more than the caches hold
+    const bool stream = STREAM && n_mtiles >= pp_args().stream_from;
     bool stream_b = false, stream_n = false;
     auto expert_b = [&](int e) {
         args_t& p = pp_args();
-        if (STREAM) stream_n = scalar_load_i32(p.offsets + e + 1) - scalar_load_i32(p.offsets + e) <= PP_BM;
+        if (STREAM) stream_n = stream && scalar_load_i32(p.offsets + e + 1) - scalar_load_i32(p.offsets + e) <= PP_BM;
         return p.B + (long long)e * p.strideB;
     };
     // a plan without rows (m0 == mend) or columns (n0 >= N) reads nothing
@@ -1025,7 +1027,7 @@ static int launch_pp_rows(const GemmArgs& a, int tiles, hipStream_t s)
     // (a multiple of 8: every XCD then runs the same number of workgroups)
     const int grid = ((tiles < cus ? tiles : cus) + 7) & ~7;
     // (parts of a reduction are of few tiles: weights that the caches hold)
-    if (EPI != EPI_PART && a.stream) return launch_pp_rows<B_KC, EPI, ACT, EPI != EPI_PART>(a, grid, s);
+    if (EPI != EPI_PART && a.stream_from) return launch_pp_rows<B_KC, EPI, ACT, EPI != EPI_PART>(a, grid, s);
     return launch_pp_rows<B_KC, EPI, ACT, false>(a, grid, s);
 }
 

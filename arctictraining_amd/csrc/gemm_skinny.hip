@@ -208,7 +208,7 @@ int launch_skinny(GemmArgs a, int m_tiles, hipStream_t s)
     a.n_ntiles = (a.N + 16 * CPL - 1) / (16 * CPL);
     const long long grid = (long long)m_tiles * a.n_ntiles;
     AMOE_REQUIRE(grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
-    if (a.stream) return launch_skinny<MT, CPL, NW, EPI, ACT, true>(a, (int)grid, s);
+    if (a.stream_from) return launch_skinny<MT, CPL, NW, EPI, ACT, true>(a, (int)grid, s);
     return launch_skinny<MT, CPL, NW, EPI, ACT, false>(a, (int)grid, s);
 }
 

@@ -25,8 +25,13 @@ def _case(gpu_device, dtype, counts):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_tall_tiles(ops, gpu_device, dtype):
-    draw, off, R = _case(gpu_device, dtype, [256, 257, 0, 255, 1, 300, 32, 90, 511])
+@pytest.mark.parametrize("counts", [
+    [256, 257, 0, 255, 1, 300, 32, 90, 511],
+    [33, 8, 12, 3, 1, 9, 4, 1, 256],          # nine tiles, the fewest whose weights are more than the cache holds
+    [200, 90, 0, 255, 1, 90, 14, 1, 1],       # eight: loaded through the caches
+])
+def test_tall_tiles(ops, gpu_device, dtype, counts):
+    draw, off, R = _case(gpu_device, dtype, counts)
     wide, deep = draw(E, K, N), draw(E, N, K)
     a, b, gate_up, scale = draw(R, K), draw(R, N), draw(R, 2 * N), torch.rand(R, device=gpu_device)
     products = {
