@@ -1026,8 +1026,7 @@ static int launch_pp_rows(const GemmArgs& a, int tiles, hipStream_t s)
     AMOE_REQUIRE(cus > 0, AMOE_ERR_LAUNCH, "grouped_gemm: cannot read the number of compute units");
     // (a multiple of 8: every XCD then runs the same number of workgroups)
     const int grid = ((tiles < cus ? tiles : cus) + 7) & ~7;
-    // (parts of a reduction are of few tiles: weights that the caches hold)
-    if (EPI != EPI_PART && a.stream_from) return launch_pp_rows<B_KC, EPI, ACT, EPI != EPI_PART>(a, grid, s);
+    if (a.stream_from) return launch_pp_rows<B_KC, EPI, ACT, true>(a, grid, s);
     return launch_pp_rows<B_KC, EPI, ACT, false>(a, grid, s);
 }
 

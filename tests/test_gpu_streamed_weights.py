@@ -89,3 +89,46 @@ def test_row_sums(ops, gpu_device, dtype, top_k):
     for run in (lambda t: ops.combine_fwd(rows, row_of[t].contiguous(), scores[t].contiguous()),
                 lambda t: ops.gather_rows_bwd(rows, row_of[t].contiguous(), addend[t].contiguous())):
         assert torch.equal(run(slice(0, T)), torch.cat([run(slice(0, T // 2)), run(slice(T // 2, T))]))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_parts_of_a_reduction(gpu_device, dtype):
+    """Products of few tiles that the layer cuts into parts (down projection and last data gradient, 294 and 587 MB), past the
+    caches with rows of all ten experts and through them with rows of nine: bit by bit for the tokens that both have."""
+    from arctictraining_amd import ArcticMoE, MoEConfig, moe
+
+    T, H, E, K, I = 100, 512, 10, 2, 28672
+    print("streamed weights", dtype, "parts", flush=True)
+    # (the layer's scratch has room for parts)
+    assert moe._layer_sizes((E, K, H, I, 0, 1, True, 0, False), T, False)[1] - T * K * H * 2 >= 2 * T * K * H * 4
+    cfg = MoEConfig(input_dtype=dtype, intermediate_dim=I, model_dim=H, num_experts=E, top_k=K, loss_coeff=0.0, normalize_topk_scores=True,
+                    act_fn=torch.nn.functional.silu, enable_routing_replay=True)
+    layer = ArcticMoE(cfg).to(gpu_device)
+    g = torch.Generator(device=gpu_device).manual_seed(9)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, 0.02, generator=g)
+    x, dy = (torch.empty((T, H), dtype=dtype, device=gpu_device).normal_(generator=g) for _ in range(2))
+    t = torch.arange(T, device=gpu_device)
+    some = torch.stack([t % 8, (t + 3) % 8], 1).to(torch.int32)
+    some[90:] = torch.tensor([8, 7], dtype=torch.int32, device=gpu_device)
+    every = some.clone()
+    every[90:, 1] = 9
+    got = []
+    for assign in (every, some):
+        xg = x.clone().requires_grad_(True)
+        out = layer(xg, assign)
+        y = out[0] if isinstance(out, tuple) else out
+        y.backward(dy)
+        got.append((y.detach()[:90], xg.grad[:90]))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    # token 0 goes to experts 0 and 3
+    with torch.no_grad():
+        p = torch.softmax((x[:1] @ layer.router_gate.t()).float(), -1).topk(K, -1).values
+        w = (p / p.sum()).to(dtype).double()[0]
+        ref = 0.0
+        for e, s in zip((0, 3), w):
+            h = x[:1].double() @ layer.expert_gate_up[e].double()
+            ref = ref + s * ((torch.nn.functional.silu(h[:, 0::2]) * h[:, 1::2]) @ layer.expert_down[e].double())
+        assert (got[0][0][:1].double() - ref).norm() <= 1e-2 * ref.norm()
