@@ -1417,13 +1417,17 @@ int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s);
 // knows, so that the kernel of 256-row tiles compares their number: of 154 experts of 960 x 1152 of which a skewed router uses
 // some twenty, 1679 tokens took 160 us past the caches and 154 through them.  (The kernel for few rows goes by the bound: with
 // both forms in one its registers spill.)
+// A gate_up product of a short reduction and many rows is not bound by the reading: it gains nothing, and the caches' dirty
+// lines, which ordinary loads would push out meanwhile, are then written under the next product.  K = 352, 79 rows an expert
+// 523 us with and 504 without, K = 288, 31 rows 522 / 507, K = 992, 46 rows 298 / 294; past the lines K = 768, 19 rows 227 / 232,
+// K = 672, 24 rows 143 / 147.
 // Before and after, bf16, K=8 of 128 experts of 2048 x 768: 64 tokens 242 -> 219 us, 3001 tokens 365 -> 341, a training step
 // of 509 tokens 905 -> 827; 124 other sizes of such weights 0.98 to 1.19 times faster, 1.04 on average.  Whether a single
 // product gains depends on what it finds in the cache and has to displace: only whole passes say something.
-static int stream_from(int R, int E, long long strideB)
+static int stream_from(int R, int E, long long strideB, int Kred, bool gate_up)
 {
     const long long least = (256ll << 20) / (strideB * 2) + 1;
-    if (R > 256ll * E || (R < E ? R : E) < least) return 0;
+    if (R > 256ll * E || (R < E ? R : E) < least || (gate_up && Kred < 1024 && R > 28ll * E)) return 0;
     return (int)least;
 }
 
@@ -1480,7 +1484,7 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
         const size_t fit = (workspace_bytes - 16) / sizeof(int4);
         a.max_mtiles = fit < (1u << 20) ? (int)fit : 1 << 20;
     }
-    a.stream_from = stream_from(R, E, strideB);
+    a.stream_from = stream_from(R, E, strideB, Kred, EPI == EPI_GATED);
     if (bm < tc.bm) {
         if constexpr (EPI == EPI_GATED) return amoe_skinny_gateup_act(a, ACT, bm, s);
         else if constexpr (EPI == EPI_STORE && !B_KC) return amoe_skinny_nn(a, bm, s);
