@@ -3,14 +3,14 @@
 // that can reach the last bits of a float32 sum are taken, on v_mfma_f32_16x16x32_bf16, into float32 accumulators: h h in
 // one, the five small ones in another.
 // Error against float64, 2-norm, normal inputs: 0.9 to 4e-7 where v_mfma_f32_32x32x2_f32, which adds two products at a time,
-// had 3e-7 to 1.1e-6 (K 256 to 4096; weight gradients of 5 to 700 rows 0.3 to 1.5e-7, before 0.4 to 4.8e-7).  Parts of values
-// below 2^-110 are lost to the bfloat16 range.
+// had 3e-7 to 1.1e-6 (K 256 to 4096; weight gradients of 5 to 700 rows 0.3 to 1.5e-7, before 0.4 to 4.8e-7), whatever the
+// operands' magnitude: what bfloat16's range does not hold of the parts is dealt with at split3 and redo_exact.
 //
-// What bounds it: vector instructions (11 to split two values; a SIMD does not overlap them with its matrix instructions) and
+// What bounds it: vector instructions (13 to split two values; a SIMD does not overlap them with its matrix instructions) and
 // LDS traffic (three planes of every stage), so that tiles are as wide as the number of them allows.  One MI355X, 39 experts
-// x 709 rows, 768 x 1856 and 928 x 768: A B 800 and 407 -> 530 and 270 us, A B^T 416 and 782 -> 271 and 500, weight
-// gradients 423 and 827 -> 272 and 500 (150-160 TFLOP/s; the float32 instruction's peak is 157).  8 experts x 512 rows,
-// 512 x 2048 and 1024 x 512: 106 and 68 -> 75 and 51, 61 and 131 -> 45 and 87, 61 and 100 -> 42 and 58: there are about as
+// x 709 rows, 768 x 1856 and 928 x 768: A B 800 and 407 -> 549 and 281 us, A B^T 416 and 782 -> 285 and 520, weight
+// gradients 423 and 827 -> 275 and 503 (140-157 TFLOP/s; the float32 instruction's peak is 157).  8 experts x 512 rows,
+// 512 x 2048 and 1024 x 512: 106 and 68 -> 77 and 55, 61 and 131 -> 46 and 94, 61 and 100 -> 43 and 61: there are about as
 // many tiles as compute units, the last round is half empty.  Dealing each XCD a contiguous eighth of the tiles changed none of these figures.
 #include "amoe_common.h"
 
@@ -42,13 +42,21 @@ struct GemmArgsF32 {
     int E, Kd, M, N, n_ntiles, n_mt;
 };
 
-// x = h + m + l in three bf16 (round to nearest: |m| <= 2^-8 |x|, |l| <= 2^-16 |x|, what is left 2^-24 |x| at most)
-__device__ __forceinline__ void split3(const f32x4_t& x, u32x2_t (&out)[3])
+// The parts are of 2^16 x: of x itself, those of a value below 2^-110 would reach below bfloat16's smallest, 2^-133, which is
+// float32's smallest times 2^16.  A sum of products is 2^32 times what it stands for.  (Results of 2^96 and more overflow
+// on the way, as operands of 2^112 and more do in their parts: see redo_exact.)  Without it a product of operands at 2^-118 is
+// off by 9e-6, at 2^-126 by 2e-3; it costs two of the 13 instructions, 3 to 4 % of the time.  (The remainder by a dot product of
+// two bfloat16, four instructions fewer, is slower: that one runs at half the rate.)
+constexpr float PART_SCALE = 65536.0f, SUM_SCALE = 1.0f / (65536.0f * 65536.0f);
+
+// 2^16 x = h + m + l in three bf16 (round to nearest: |m| <= 2^-8 |h|, |l| <= 2^-16 |h|, nothing is left)
+__device__ __forceinline__ void split3(const f32x4_t& v, u32x2_t (&out)[3])
 {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const uint32_t h = pack_bf16x2(x[2 * i], x[2 * i + 1]);
-        const float r0 = x[2 * i] - bf16_lo(h), r1 = x[2 * i + 1] - bf16_hi(h);
+        const float x0 = v[2 * i] * PART_SCALE, x1 = v[2 * i + 1] * PART_SCALE;
+        const uint32_t h = pack_bf16x2(x0, x1);
+        const float r0 = x0 - bf16_lo(h), r1 = x1 - bf16_hi(h);
         const uint32_t m = pack_bf16x2(r0, r1);
         out[0][i] = h;
         out[1][i] = m;
@@ -108,7 +116,7 @@ __device__ __forceinline__ bool finite4(const f32x4_t& c)
     return ok;
 }
 
-// An infinity or a NaN in an operand has no three parts (inf - inf), and a value next to the largest rounds to infinity: a
+// An infinity or a NaN in an operand has no three parts (inf - inf), and large values overflow (see split3): a
 // wavefront that met either works its rows x columns out again with the float32 instruction, straight from memory.
 // a_at(row, k), b_at(k, column): addresses of elements that exist
 template <typename FA, typename FB, typename FC>
@@ -269,7 +277,7 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const f32x4_t c = hi[i][j] + lo[i][j];
+            const f32x4_t c = (hi[i][j] + lo[i][j]) * SUM_SCALE;
             finite = finite && finite4(c);
             const int row = m0 + i * 16 + l16, col = n0 + j * 16 + 4 * lq;
             if (row < mend && col < p.N) *reinterpret_cast<f32x4_t*>(p.C + (long long)row * p.ldc + col) = c;
@@ -401,6 +409,7 @@ grouped_gemm_f32_deep_kernel(GemmArgsF32 p)
             f32x4_t c = red[0][tid];
 #pragma unroll
             for (int w = 1; w < NW_DEEP; ++w) c += red[w][tid];
+            c *= SUM_SCALE;
             finite = finite && finite4(c);
             const int l = tid & 63, u = tid >> 6;
             const int row = m0 + i * 16 + (l & 15), col = n0 + (B_KC ? u * 16 + 4 * (l >> 4) : 16 * (l >> 4) + 4 * u);
@@ -522,7 +531,7 @@ grouped_gemm_f32_wgrad_kernel(GemmArgsF32 p)
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const f32x4_t c = hi[i][j] + lo[i][j];
+            const f32x4_t c = (hi[i][j] + lo[i][j]) * SUM_SCALE;
             finite = finite && finite4(c);
             const int row = mw + i * 16 + l16, col = nw + j * 16 + 4 * lq;
             if (row < p.M && col < p.N) *reinterpret_cast<f32x4_t*>(Cb + (long long)row * p.ldc + col) = c;
@@ -590,7 +599,7 @@ int amoe_f32_rows(const void* A, const int32_t* a_row_map, const void* B, const 
     a.n_ntiles = (N + BN_ROWS - 1) / BN_ROWS;
     const long long grid = (long long)max_mtiles * a.n_ntiles;
     AMOE_REQUIRE(grid * (BM_ROWS / 32) < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm(f32): grid too large");
-    // Few tiles, which the wavefronts of a compute unit then have to share.  One MI355X, us, one group of wavefronts / two groups / the
+    // Few tiles, which the wavefronts of a compute unit then have to share.  One MI355X, us (with 11 instructions for two values), one group of wavefronts / two groups / the
     // eight-wave form:
     //   32 x 64 tiles (an expert's last one is not full) up to 400: 8 experts, 256 rows, K = 1024, N = 512 29.6 / 24.1 / 11.1; 38 experts,
     //   497 rows, K = 800, N = 288 24.1 / 20.8 / 18.0; past the line K = 288, N = 800 13.6 / 20.5 / 20.4.

@@ -89,3 +89,30 @@ def test_values_that_have_no_parts(gpu_device, counts, K, N):
         same(nn[s], a[s].double() @ b[e].double())
         same(nt[s], a[s].double() @ b[e].double())
         same(w[e], a[s].double().t() @ d[s].double())
+
+
+@pytest.mark.parametrize("counts,K,N", [([40, 3], 64, 68), ([300, 180], 1024, 132), ([700, 96, 640], 64, 1028)])
+@pytest.mark.parametrize("ea,eb", [(-118, 100), (100, -122), (-126, 110), (120, -140), (-62, -60), (60, 50)])
+def test_values_near_the_ends_of_the_range(gpu_device, counts, K, N, ea, eb):
+    """Operands around 2^ea and 2^eb, subnormal ones among them, as exact as any others; rows of zeros give zeros."""
+    from arctictraining_amd import ops
+
+    print("float32 range", counts, K, N, ea, eb, flush=True)
+    R, E = sum(counts), len(counts)
+    g = torch.Generator(gpu_device).manual_seed(R)
+
+    def rand(e, *s):
+        return (torch.randn(s, device=gpu_device, generator=g).double() * 2.0**e).float()
+
+    a, b, d = rand(ea, R, K), rand(eb, E, K, N), rand(eb, R, N)
+    a[1], a[:, 2] = 0.0, 0.0
+    off = _offsets(counts, gpu_device)
+    nn, nt = ops.grouped_gemm_nn(a, b, off), ops.grouped_gemm_nt(a, b.transpose(1, 2).contiguous(), off)
+    w = ops.grouped_gemm_wgrad(a, d, off, E)
+    assert not nn[1].any() and not nt[1].any() and not w[:, 2].any()
+    for e in range(E):
+        s = slice(sum(counts[:e]), sum(counts[: e + 1]))
+        for got, ref in ((nn[s], a[s].double() @ b[e].double()), (nt[s], a[s].double() @ b[e].double()),
+                         (w[e], a[s].double().t() @ d[s].double())):
+            # (and half of the smallest float32 for each)
+            assert (got.double() - ref).norm() <= TOL * ref.norm() + 2.0**-150 * ref.numel() ** 0.5
