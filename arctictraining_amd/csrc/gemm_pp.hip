@@ -169,6 +169,7 @@ __device__ __forceinline__ void pp_rows_body()
         const int col = ((th & 15) ^ (2 * ((kr & 3) | (((kr >> 3) & 1) << 2)))) * 8;
         bd = pp_srd(B);
         if (STREAM) stream_b = stream_n;
+        // (an expert's matrix is below 4 GiB, or the call is refused: no offset in it wraps)
         if constexpr (PART) pp_advance(bd, B_KC ? (uint32_t)k0 * 2u : (uint32_t)k0 * ((uint32_t)ldb * 2u));
 #pragma unroll
         for (int b = 0; b < 2; ++b)

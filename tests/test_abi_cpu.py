@@ -150,6 +150,21 @@ def test_workspace_of_the_largest_call_serves_smaller_ones(lib, E):
         assert f32(R, 16 * (R // 64 + E + 1)) == -3 and product(R, 16 * (R // 256 + E + 1), cfg=5) == -3
 
 
+@pytest.mark.parametrize("cfg", [0, 1, 2])
+def test_weights_of_4_gib_are_refused(lib, cfg):
+    """The kernels address one expert's matrix, and a part of its reduction, with 32-bit byte offsets: refused before any
+    launch, also where the number of elements fits 32 bits (100 rows of one expert: a reduction that would be cut)."""
+    big = 1 << 20
+    assert lib.amoe_grouped_gemm_gateup_act_fwd(P, None, P, P, None, P, P, 1, 100, 1, 196608, 8192, 0, P, big, cfg, None) == -2
+    assert b"4 GiB" in lib.amoe_last_error()
+    assert lib.amoe_grouped_gemm_nn(P, None, P, P, P, 2, 100, 1, 196608, 16384, P, big, cfg, None) == -2
+    assert b"4 GiB" in lib.amoe_last_error()
+    assert lib.amoe_grouped_gemm_nt(P, None, P, P, P, 1, 100, 1, 16384, 196608, P, big, cfg, None) == -2
+    assert b"4 GiB" in lib.amoe_last_error()
+    assert lib.amoe_grouped_gemm_nt_gated_bwd(P, None, P, P, P, None, P, None, 1, 100, 1, 16384, 196608, 0, P, big, cfg, None) == -2
+    assert b"4 GiB" in lib.amoe_last_error()
+
+
 def test_gated_bwd_gemm_argument_errors(lib):
     big = 1 << 20
     f = lib.amoe_grouped_gemm_nt_gated_bwd
