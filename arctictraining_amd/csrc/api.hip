@@ -1,6 +1,7 @@
 // Exported grouped-GEMM entry points (argument validation + dtype dispatch), the version
 // query and the per-thread error message.
 #include "amoe_common.h"
+#include "gemm_calls.h"
 
 #include <string.h>
 
@@ -27,8 +28,6 @@ int amoe_bf16_nn(const void* A, const int32_t* a_row_map, const void* B, const i
 int amoe_bf16_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int R, int E,
                  int Kd, int N, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype, float* split,
                  size_t split_bytes);
-int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map,
-                    const int32_t* offsets, void* C, int R, int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype, int lda, bool out32);
 int amoe_bf16_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down, const int32_t* offsets,
                            const void* gate_up, const float* row_scale, void* d_gate_up, float* partials, int R, int E,
                            int I, int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg, hipStream_t s, int dtype,

@@ -32,6 +32,7 @@
 // and super-tiles rotate over the XCDs, which keeps them evenly loaded whatever the routing
 // skew.
 #include "gemm_common.h"
+#include "gemm_calls.h"
 #include "gemm_launch.h"
 
 #include <algorithm>
@@ -1402,7 +1403,6 @@ int amoe_pp_wgrad(GemmArgs a, hipStream_t s);
 // few rows to reduce over (gemm_short.hip)
 int amoe_short_wgrad(GemmArgs a, hipStream_t s);
 // few tiles of a deep reduction (gemm_split.hip)
-int amoe_split_count(int R, int E, int K, int N);
 int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, int tiles, hipStream_t s);
 // few rows per expert (gemm_skinny.hip)
 int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s);

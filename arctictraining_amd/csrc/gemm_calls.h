@@ -1,0 +1,23 @@
+// Grouped products as the layer's calls and the exported entry points share them.
+#pragma once
+
+#include "amoe_common.h"
+
+// With room for the parts of a reduction (gemm_split.hip), none if split is null: amoe_split_bytes of the same rows, experts,
+// reduction length K and columns N as the product has, or the call is refused.
+int amoe_run_gateup_act_fwd(const void* xp, const int32_t* a_row_map, const void* w_gate_up, const int32_t* offsets, const float* row_scale,
+                            void* gate_up, void* inter, int dtype, int R, int E, int H, int I, int act, void* workspace,
+                            size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes);
+int amoe_run_nn(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int dtype, int R, int E, int Kd,
+                int N, void* workspace, size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes);
+int amoe_run_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int dtype, int R, int E, int Kd,
+                int N, void* workspace, size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes);
+int amoe_run_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down, const int32_t* offsets, const void* gate_up,
+                          const float* row_scale, void* d_gate_up, float* score_partials, int dtype, int R, int E, int I, int H, int act,
+                          void* workspace, size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes);
+int amoe_split_count(int R, int E, int K, int N);
+size_t amoe_split_bytes(int R, int E, int K, int N);
+
+// weight gradients in 16 bits (gemm_bf16.hip)
+int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map, const int32_t* offsets, void* C, int R,
+                    int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype, int lda, bool out32);

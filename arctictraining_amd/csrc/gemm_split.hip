@@ -7,6 +7,7 @@
 // experts, K = 3200, N = 640 40 / 17 + 4; 3165 rows of 7 experts, A B^T of K = 13568, N = 1152 268 / 120 + 9; 3390 rows of 6
 // experts, the gated product of K = 6560, N = 896 114 / 55 + 8.
 #include "gemm_common.h"
+#include "gemm_calls.h"
 #include "gemm_launch.h"
 
 int amoe_pp_part(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s);

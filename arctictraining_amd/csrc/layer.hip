@@ -5,6 +5,7 @@
 // of the router stay with the caller, between the calls.
 // (One token through 128 experts of 2048 x 768: 144 us of host time a forward stage by stage, 70 us this way.)
 #include "amoe_common.h"
+#include "gemm_calls.h"
 
 #include <algorithm>
 #include <mutex>
@@ -24,28 +25,7 @@ int amoe_launch_gated_act_bwd_rows(const void* gate_up, const void* d_inter, con
                                    int dtype, int R, int I, int act, hipStream_t s);
 int amoe_launch_router_bwd(const float* d_scores, const float* probs, const int32_t* topk_idx, const int32_t* counts, int dtype, int T,
                            int E, int K, int normalize, float lb_coeff, void* d_logits, int ld, hipStream_t s);
-int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, const int32_t* b_row_map, const int32_t* offsets, void* C, int R,
-                    int E, int Kd, int N, int tile_cfg, hipStream_t s, int dtype, int lda, bool out32);
 int amoe_launch_sum_parts(const void* parts, int n_parts, void* out, int parts_dtype, int dtype, long long n, hipStream_t s);
-
-// the grouped products with room for the parts of a reduction (gemm_split.hip), none if split is null
-int amoe_run_gateup_act_fwd(const void* xp, const int32_t* a_row_map, const void* w_gate_up,
-                                                 const int32_t* offsets, const float* row_scale, void* gate_up,
-                                                 void* inter, int dtype, int R,
-                                                 int E, int H, int I, int act, void* workspace, size_t workspace_bytes,
-                                                 int tile_cfg, void* stream, float* split, size_t split_bytes);
-int amoe_run_nn(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
-                                     void* C, int dtype, int R, int E, int Kd, int N, void* workspace,
-                                     size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes);
-int amoe_run_nt(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets,
-                                     void* C, int dtype, int R, int E, int Kd, int N, void* workspace,
-                                     size_t workspace_bytes, int tile_cfg, void* stream, float* split, size_t split_bytes);
-int amoe_run_nt_gated_bwd(const void* dy, const int32_t* a_row_map, const void* w_down,
-                                               const int32_t* offsets, const void* gate_up, const float* row_scale,
-                                               void* d_gate_up, float* score_partials, int dtype, int R, int E, int I,
-                                               int H, int act, void* workspace, size_t workspace_bytes, int tile_cfg,
-                                               void* stream, float* split, size_t split_bytes);
-size_t amoe_split_bytes(int R, int E, int K, int N);
 
 namespace {
 

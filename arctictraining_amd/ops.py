@@ -91,7 +91,7 @@ def router_input_grad(d_logits: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     rc = _lib.load().amoe_router_input_grad_rows(
         d_logits.data_ptr(), d_logits.stride(0), w.data_ptr(), out.data_ptr(), _dtype_code(w), T, E, H, _stream()
     )
-    _lib.check(rc, "amoe_router_input_grad")
+    _lib.check(rc, "amoe_router_input_grad_rows")
     return out
 
 
