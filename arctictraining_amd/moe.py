@@ -238,11 +238,10 @@ def _router_input_grad(d_logits: torch.Tensor, router_gate: torch.Tensor, padded
 
 
 def _router_weight_grad(d_logits: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """dW_router [E,H] = d_logits^T [E,T] @ x [T,H] (autograd of moe.py:233): skinny (E rows) and
-    deep (T), the library GEMM leaves most of the chip idle on it (128 experts, H = 2048: 4096 tokens 34 us
-    against 13).  With few tokens it is the host that counts, 19 us against 10: a step of 160 to 768 tokens, bound by the
-    host (16 experts, H = 1024), takes 1-2 % less, one bound by the GPU (128, 64, 256 or 8 experts) between 1.3 % less and
-    0.9 % more, at most sizes 0.2-0.5 % more."""
+    """dW_router [E,H] = d_logits^T [E,T] @ x [T,H] (autograd of moe.py:233), where the layer's native call does not form it:
+    experts without a gate, a router in another type or of fewer rows than experts, float32.  Skinny (E rows) and deep (T), so
+    that the library GEMM leaves most of the chip idle on it (128 experts, H = 2048: 4096 tokens 35 us against 17, 16384 tokens 135
+    against 21, the sum of the parts included)."""
     if x.dtype == torch.float32 or d_logits.shape[1] % 8:
         return torch.matmul(d_logits.t(), x)
     return _dense_weight_grad(d_logits, x, tile_cfg=1, tile=128)  # 128x128 tiles
@@ -318,7 +317,8 @@ def _overlap_pays(config_key, T: int) -> bool:
     this layer: 12-39 %), one that it takes longer for is mostly 3-15 % shorter with the second stream.  The line lies where
     the products at 800 TFLOP/s (float32 100), their columns rounded up to whole tiles, and the weights, read twice and their
     gradients written, at 3 TB/s make 150 us: T=556 H=1760 E=8 K=6 I=672 (143 us) 268 us with it, 228 without; T=95 H=2336 E=12
-    K=2 I=1536 (193) 274 and 299, T=3065 H=320 E=19 K=5 I=1088 (243) 353 and 398."""
+    K=2 I=1536 (193) 274 and 299, T=3065 H=320 E=19 K=5 I=1088 (243) 353 and 398.  (Not all: 509 tokens of 128 experts of
+    2048 x 768, bound by memory on both streams, take 2 % longer with it.)"""
     E, K, H, I, dtype, shared = *config_key[:4], config_key[5], config_key[8]
     size, rate = (4, 1e8) if dtype == ops.F32 else (2, 8e8)
     rows, weights = T * K + (T if shared else 0), (E + (1 if shared else 0)) * H * I
