@@ -1607,12 +1607,11 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
         // Up to 128 rows per expert the product is bound by the gradients' stores: gemm_short.hip, where its 32-bit tile
         // numbers reach (with a fourth of these tiles' size).  It and shape 5 inside a training step: 812 against 905 us at 32
         // rows, 545 against 572 at 111, 334 against 363 at 136 (and the same without the second stream), 764 against 710 at 250.
-        // A tile of the default kernel is never done in less than three K tiles, and its workgroups leave no compute unit to
-        // the other stream's products: below 256 rows the one-tile workgroups of shape 5 are faster (64 experts of 2048 x
-        // 1408, 250 rows, gate_up's gradient alone 0.37 against 0.34 ms, the whole step 1.63 against 1.74).
+        // Beyond, gemm_pp.hip, whose tiles are never done in less than three K tiles.  The line: with 102 rows an expert it and
+        // gemm_short.hip are within 1.5 % of each other, either way (steps of 27 experts of 1024 x 9184, 1.34 against 1.36 ms, 97 of
+        // 1856 x 1920, 1.88 against 1.86).
         if (R <= 128ll * E && offsets32 && 16 * per * per * E < (1ll << 32)) return amoe_short_wgrad(a, s);
-        if (R >= 256ll * E && offsets32 && per * per * E < (1ll << 32))
-            return amoe_pp_wgrad(a, s);
+        if (offsets32 && per * per * E < (1ll << 32)) return amoe_pp_wgrad(a, s);
         tile_cfg = 5;
     }
     long long grid = 0;

@@ -81,6 +81,13 @@ __device__ __forceinline__ void pp_barrier()
     __builtin_amdgcn_s_barrier();
     pp_fence();
 }
+// Between a wavefront's writes to LDS and its reads of what other lanes wrote, and back: the LDS serves a wavefront in order,
+// so that only the compiler has to keep the order
+__device__ __forceinline__ void pp_lds_turn()
+{
+    pp_fence();
+    asm volatile("" ::: "memory");
+}
 template <typename T>
 __device__ __forceinline__ T pp_lds(uint32_t addr)
 {

@@ -24,6 +24,7 @@ constexpr uint32_t PP_IDX = 2 * PP_STAGE;            // row indices of the next 
 constexpr uint32_t PP_SCALE = PP_IDX + 8 * 64 * 4;   // row scales of two tiles
 constexpr uint32_t PP_PART = PP_SCALE + 2 * PP_BM * 4;   // row-sum partials, one row of 256 per wave column
 constexpr uint32_t PP_LDS = PP_PART + 4 * PP_BM * 4;
+constexpr uint32_t PP_WGRAD_LDS = 2 * PP_STAGE + 8 * 2048;   // and 2 KB a wavefront for its epilogue
 
 // ------------------------------------------------------------------ row-grouped products
 // C[rows_e,:] = A[rows_e,:] @ B[e] (B_KC false: B [Kd,N]) or @ B[e]^T (B_KC: B [N,Kd]).
@@ -639,13 +640,19 @@ __device__ __forceinline__ void pp_rows_body()
 
 // ------------------------------------------------------------------ weight gradients
 // C[e] = A[rows_e,:]^T @ B[rows_e,:]: the reduction runs over the expert's rows, both operands are K-strided.  The same
-// phases and the same persistent stream of K tiles as the row-grouped kernel; a tile is 256 x 256 of one expert's
-// gradient, its number of K tiles that of the expert's rows (three at least, the missing ones empty).
+// phases and the same stream of K tiles from tile to tile as the row-grouped kernel; a tile is 256 x 256 of one expert's
+// gradient, its number of K tiles that of the expert's rows (three at least, the missing ones empty).  Half a is 128 columns of A,
+// 64 k deep; half s of B is 32 k deep and all 256 columns wide, so that a phase is one k step of 64 x 64 a wavefront: its
+// columns then are 64 in a row, and the epilogue stores whole lines.
 // MAPS: 1 = the rows of A, 2 = the rows of B are gathered through a row map: the indices of a K tile are fetched by
 // scalar loads a phase before its offsets are worked out beside the MFMAs.
+// What bounds it: up to a few hundred rows an expert the stores of the gradients, behind which, in order, no load of their
+// wavefront completes; beyond, the MFMAs.  Alone, bf16, 64 experts of 2048 x 1408, the rows of one operand gathered,
+// gate_up's / down's gradient, us, with 64-byte pieces of rows by lanes 16 apart, ordinary stores / as now: 125 rows 286 / 148 -> 207 / 94,
+// 250 rows 328 / 173 -> 280 / 147, 375 rows 385 / 203 -> 340 / 180; 128 of 2048 x 768, 1024 rows 743 / 388 -> 730 / 354.
 // Rows past the expert's end read as zeros: an operand that is not gathered has a descriptor that ends with them, a
 // gathered one gets PP_NOWHERE for them.
-template <int MAPS, typename ET>
+template <int MAPS, bool STREAM, typename ET>
 __device__ __forceinline__ void pp_wgrad_body()
 {
     typedef typename Elem16<ET>::frag_t frag_t;
@@ -657,6 +664,7 @@ __device__ __forceinline__ void pp_wgrad_body()
     const int grp = wave >> 2, wc = wave & 3;
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
     using I4 = std::integral_constant<int, 4>;
     constexpr bool A_MAP = MAPS == 1, B_MAP = MAPS == 2;
 
@@ -664,6 +672,7 @@ __device__ __forceinline__ void pp_wgrad_body()
     // Tiles are numbered expert by expert, inside an expert in strips of gn columns; XCD x (workgroups with
     // blockIdx % 8 == x) works through chunks x, x + 8, ... of 32 consecutive tiles, so that the workgroups of an XCD
     // share operand panels in its L2; the tiles left over from the last whole group of chunks are dealt one by one.
+    // A workgroup takes gm tiles, one from each of gm chunks in a row.
     auto divide = [](int n, uint32_t inv) -> int { return inv ? (int)(((uint64_t)(uint32_t)n * inv) >> 32) : n; };
     struct Tile { int e, m0, n0, r0, r1; };
     auto decode = [&](int q, Tile& t) -> bool {       // q-th tile of this XCD
@@ -689,33 +698,44 @@ __device__ __forceinline__ void pp_wgrad_body()
     };
 
     // ------------------------------------------------------------ loads
-    // Thread tid fills k rows tid / 16 and tid / 16 + 32 of every half tile.
+    // Thread tid fills k rows tid / 16 and tid / 16 + 32 of either half (128 columns) of A, and k rows tid / 32 and tid / 32 + 16 of
+    // either half (32 k) of B.
     uint32_t aoff[2][2], boff[2][2];
-    uint32_t acol[2], bcol[2];        // byte offsets of its columns in the two halves (PP_NOWHERE outside the matrix)
+    uint32_t acol[2], bcol;           // byte offsets of its columns (PP_NOWHERE outside the matrix)
     srd_t ad, bd;
     const uint32_t lda2 = (uint32_t)pp_args().lda * 2u, ldb2 = (uint32_t)pp_args().ldb * 2u;
     int left = 0;                     // rows of the expert from the K tile loaded next
-    int row_n = 0, left_n = 0;        // gathered: map position of the K tile whose indices are fetched next
-    int idx[2][4];
+    int row_n = 0;                    // gathered: map position of the K tile whose indices are fetched next
+    int idx[8];
     auto add_sat = [](uint32_t a, uint32_t b) { return __builtin_elementwise_add_sat(a, b); };
     auto fetch_idx = [&]() {
         if constexpr (MAPS != 0) {
             args_t& p = pp_args();
             const int32_t* map = A_MAP ? p.a_row_map : p.b_row_map;
             typedef int i32x4_t __attribute__((ext_vector_type(4), aligned(4)));
-            const int row = row_n + wave * 4;
+            typedef int i32x2_t __attribute__((ext_vector_type(2), aligned(4)));
+            // A: rows 4 wave ..+3 and those 32 on; B: rows 2 wave, 2 wave + 1 and those 16, 32 and 48 on
+            constexpr int G = A_MAP ? 4 : 2, STEP = A_MAP ? 32 : 16;
+            const int row = row_n + wave * G;
             if (row_n + 64 <= p.rows_total) {
+                if constexpr (A_MAP) {
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const i32x4_t v = *(const __attribute__((address_space(4))) i32x4_t*)(map + row + 32 * j);
+                    for (int j = 0; j < 2; ++j) {
+                        const i32x4_t v = *(const __attribute__((address_space(4))) i32x4_t*)(map + row + 32 * j);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) idx[j][q] = v[q];
+                        for (int q = 0; q < 4; ++q) idx[4 * j + q] = v[q];
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const i32x2_t v = *(const __attribute__((address_space(4))) i32x2_t*)(map + row + 16 * j);
+                        idx[2 * j] = v[0];
+                        idx[2 * j + 1] = v[1];
+                    }
                 }
             } else {
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) idx[j][q] = scalar_load_i32(map + min(row + 32 * j + q, p.rows_total - 1));
+                for (int k = 0; k < 8; ++k) idx[k] = scalar_load_i32(map + min(row + STEP * (k / G) + k % G, p.rows_total - 1));
             }
         }
     };
@@ -723,14 +743,22 @@ __device__ __forceinline__ void pp_wgrad_body()
     auto gather_offsets = [&](int rows) {
         if constexpr (MAPS != 0) {
             const int th = pp_here(tid);
-            const int q = (th >> 4) & 3, kr = th >> 4;
+            if constexpr (A_MAP) {
+                const int q = (th >> 4) & 3, kr = th >> 4;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int i01 = q & 1 ? idx[j][1] : idx[j][0], i23 = q & 1 ? idx[j][3] : idx[j][2];
-                const uint32_t o = kr + 32 * j < rows ? (uint32_t)(q & 2 ? i23 : i01) * (A_MAP ? lda2 : ldb2) : PP_NOWHERE;
+                for (int j = 0; j < 2; ++j) {
+                    const int i01 = q & 1 ? idx[4 * j + 1] : idx[4 * j], i23 = q & 1 ? idx[4 * j + 3] : idx[4 * j + 2];
+                    const uint32_t o = kr + 32 * j < rows ? (uint32_t)(q & 2 ? i23 : i01) * lda2 : PP_NOWHERE;
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    if (A_MAP) aoff[h][j] = add_sat(o, acol[h]); else boff[h][j] = add_sat(o, bcol[h]);
+                    for (int h = 0; h < 2; ++h) aoff[h][j] = add_sat(o, acol[h]);
+                }
+            } else {
+                const int kr = th >> 5;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t r = (uint32_t)(kr & 1 ? idx[2 * k + 1] : idx[2 * k]);
+                    boff[k >> 1][k & 1] = kr + 16 * k < rows ? add_sat(r * ldb2, bcol) : PP_NOWHERE;
+                }
             }
         }
     };
@@ -750,15 +778,17 @@ __device__ __forceinline__ void pp_wgrad_body()
         bd = pp_srd(B_MAP ? p.B : p.B + (long long)t.r0 * p.ldb);
         left = t.r1 - t.r0;
         limit();
+        const int krb = th >> 5;
+        const int n = t.n0 + ((th & 31) ^ (2 * ((krb & 3) | (((krb >> 3) & 1) << 2)))) * 8;
+        bcol = n < p.N ? (uint32_t)n * 2u : PP_NOWHERE;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int m = t.m0 + h * 128 + col, n = t.n0 + h * 128 + col;
+            const int m = t.m0 + h * 128 + col;
             acol[h] = m < p.M ? (uint32_t)m * 2u : PP_NOWHERE;
-            bcol[h] = n < p.N ? (uint32_t)n * 2u : PP_NOWHERE;
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 if (!A_MAP) aoff[h][j] = add_sat((uint32_t)(kr + 32 * j) * lda2, acol[h]);
-                if (!B_MAP) boff[h][j] = add_sat((uint32_t)(kr + 32 * j) * ldb2, bcol[h]);
+                if (!B_MAP) boff[h][j] = add_sat((uint32_t)(krb + 32 * h + 16 * j) * ldb2, bcol);
             }
         }
         gather_offsets(left);
@@ -783,8 +813,8 @@ __device__ __forceinline__ void pp_wgrad_body()
     };
 
     // ------------------------------------------------------------ fragments
-    frag_t fa[4][2], fb0[2][2], fb1[2][2];
-    uint32_t ra[4], rb[2];            // LDS read addresses per 16-column tile
+    frag_t fa[4][2], fb0[4], fb1[4];
+    uint32_t ra[4], rb[4];            // LDS read addresses per 16-column tile
     {
         const int l16 = lane & 15, lq = lane >> 4;
         const int k = 8 * lq + (l16 >> 2), key = 2 * ((l16 >> 2) | ((lq & 1) << 2));
@@ -792,49 +822,53 @@ __device__ __forceinline__ void pp_wgrad_body()
 #pragma unroll
         for (int i = 0; i < 4; ++i) ra[i] = base + (uint32_t)((grp * 8 + 2 * i + ((l16 & 3) >> 1)) ^ key) * 16u;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) rb[j] = base + 2 * PP_HALF + (uint32_t)((wc * 4 + 2 * j + ((l16 & 3) >> 1)) ^ key) * 16u;
+        for (int j = 0; j < 4; ++j) rb[j] = base + 2 * PP_HALF + (uint32_t)(k * 256) + (uint32_t)((wc * 8 + 2 * j + ((l16 & 3) >> 1)) ^ key) * 16u;
     }
     auto flip = [&]() {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ra[i] ^= PP_STAGE;
-        rb[0] ^= PP_STAGE;
-        rb[1] ^= PP_STAGE;
+        for (int i = 0; i < 4; ++i) {
+            ra[i] ^= PP_STAGE;
+            rb[i] ^= PP_STAGE;
+        }
     };
-    auto read_tr = [&](uint32_t ad) -> frag_t {
+    auto read_tr = [&](uint32_t ad, uint32_t four_rows) -> frag_t {
         typedef __attribute__((address_space(3))) i16x4_t* tr_ptr;
         const u32x2_t lo = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)ad));
-        const u32x2_t hi = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)(ad + 1024u)));
+        const u32x2_t hi = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)(ad + four_rows)));
         return __builtin_bit_cast(frag_t, u32x4_t{lo[0], lo[1], hi[0], hi[1]});
     };
     auto read_a = [&](auto A_, auto N_) {
 #pragma unroll
         for (int i = 0; i < decltype(N_)::value; ++i)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) fa[i][s] = read_tr(ra[i] + decltype(A_)::value * PP_HALF + s * 8192u);
+            for (int s = 0; s < 2; ++s) fa[i][s] = read_tr(ra[i] + decltype(A_)::value * PP_HALF + s * 8192u, 1024u);
     };
-    auto read_b = [&](auto B_, frag_t (&fb)[2][2]) {
+    auto read_b = [&](auto S_, frag_t (&fb)[4]) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) fb[j][s] = read_tr(rb[j] + decltype(B_)::value * PP_HALF + s * 8192u);
+        for (int j = 0; j < 4; ++j) fb[j] = read_tr(rb[j] + decltype(S_)::value * PP_HALF, 2048u);
     };
-    auto mma = [&](auto FIRST, auto N_, mfma_f32x4 (&c)[4][2], const frag_t (&fb)[2][2]) {
+    // step S_ of the K tile; FIRST: the half's first one, nothing to add to
+    auto mma = [&](auto FIRST, auto S_, auto N_, mfma_f32x4 (&c)[4][4], const frag_t (&fb)[4]) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+        for (int i = 0; i < decltype(N_)::value; ++i)
 #pragma unroll
-            for (int i = 0; i < decltype(N_)::value; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    c[i][j] = Mfma16<ET>::run(fb[j][s], fa[i][s], decltype(FIRST)::value && s == 0 ? mfma_f32x4{0.f, 0.f, 0.f, 0.f} : c[i][j]);
+            for (int j = 0; j < 4; ++j)
+                c[i][j] = Mfma16<ET>::run(fb[j], fa[i][decltype(S_)::value], decltype(FIRST)::value ? mfma_f32x4{0.f, 0.f, 0.f, 0.f} : c[i][j]);
     };
 
     // ------------------------------------------------------------ tile state
     Tile cur, nxt = {0, 0, 0, 0, 0}, far = {0, 0, 0, 0, 0};
-    int q = blockIdx.x >> 3;                       // position of the last tile taken in this XCD's queue
-    const int gq = gridDim.x >> 3;
+    // position of the last tile taken in this XCD's queue, and the end of what this workgroup takes
+    int q = (int)(blockIdx.x >> 8) * 32 * pp_args().gm + (int)((blockIdx.x >> 3) & 31);
+    const int q_end = q + 32 * pp_args().gm;
     if (!decode(q, cur)) return;
-    bool have_n = decode(q += gq, nxt), have_nn = false;
+    bool have_n = (q += 32) < q_end && decode(q, nxt), have_nn = false;
 
+    // Epilogue: a wavefront's columns of the tile are 64, 128 bytes of a row.  Lane (lq, l16) holds columns 16 j + 4 lq ..+3 of row
+    // l16 of every 16-row block; through 2 KB of LDS of the wavefront's own (chunk c of row r at c ^ (r & 7), its halves the other way
+    // round from row 8 on: no bank conflicts) eight lanes come to hold a row's 128 bytes, and a store writes whole lines.
+    // (Adjacent lanes in adjacent rows, as the accumulators have them, are a request each: 128 such stores take 3.5 us on a compute
+    // unit and 0.9 so.)
     bf16_t* e_c;
     int e_ldc2 = 0, e_cols = 0, e_rows = 0;
     uint32_t e_off = 0;
@@ -842,34 +876,42 @@ __device__ __forceinline__ void pp_wgrad_body()
         args_t& p = pp_args();
         const int le = pp_here(lane);
         e_ldc2 = p.ldc * 2;
-        e_c = p.C + (long long)cur.e * p.strideC + (long long)(cur.m0 + grp * 64) * p.ldc + cur.n0 + wc * 32;
-        e_cols = p.N - cur.n0 - wc * 32;
+        e_c = p.C + (long long)cur.e * p.strideC + (long long)(cur.m0 + grp * 64) * p.ldc + cur.n0 + wc * 64;
+        e_cols = p.N - cur.n0 - wc * 64;
         e_rows = p.M - cur.m0 - grp * 64;
-        e_off = (uint32_t)((le & 15) * e_ldc2 + 16 * (le >> 4));
+        e_off = (uint32_t)((le >> 3) * e_ldc2 + 16 * (le & 7));
     };
-    auto epilogue = [&](auto A_, auto B_, const mfma_f32x4 (&acc)[4][2]) {
-        constexpr int a = decltype(A_)::value, b = decltype(B_)::value;
+    auto epilogue = [&](auto A_, auto FROM, const mfma_f32x4 (&acc)[4][4]) {      // two 16-row blocks
+        constexpr int a = decltype(A_)::value, from = decltype(FROM)::value;
         const int le = pp_here(lane);
-        const int eq = le >> 4, rl = le & 15;
+        const int r16 = le & 15, r8 = le >> 3;
+        const uint32_t at = lds + 2 * PP_STAGE + (uint32_t)wave * 2048u;
+        const uint32_t wr = at + (uint32_t)(r16 * 128 + (((le >> 5) ^ (r16 & 7)) * 16) + (((le >> 4) ^ (r16 >> 3)) & 1) * 8);
+        const uint32_t rd = at + (uint32_t)(r8 * 128 + ((le & 7) ^ r8) * 16);
         const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc(e_c, (short)0, (int)PP_DROP, 0x00020000);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = from; i < from + 2; ++i) {
             pp_fence();
-            const bool ok = b * 128 + 8 * eq < e_cols && a * 128 + i * 16 + rl < e_rows;
-            uint32_t x[2], y[2];
 #pragma unroll
-            for (int v = 0; v < 2; ++v) {
-                x[v] = Elem16<ET>::pack2(acc[i][0][2 * v], acc[i][0][2 * v + 1]);
-                y[v] = Elem16<ET>::pack2(acc[i][1][2 * v], acc[i][1][2 * v + 1]);
+            for (int j = 0; j < 4; ++j)
+                *(__attribute__((address_space(3))) u32x2_t*)(uintptr_t)(wr ^ (32u * j)) =
+                    u32x2_t{Elem16<ET>::pack2(acc[i][j][0], acc[i][j][1]), Elem16<ET>::pack2(acc[i][j][2], acc[i][j][3])};
+            pp_lds_turn();
+            u32x4_t v[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) v[t] = pp_lds<u32x4_t>(rd + t * 1024u);
+            pp_lds_turn();
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const bool ok = 8 * (le & 7) < e_cols && a * 128 + i * 16 + t * 8 + r8 < e_rows;
+                pp_store16<STREAM>(d, t == 0 ? v[0] : u32x4_t{v[1][2], v[1][3], v[1][0], v[1][1]}, ok ? e_off : PP_DROP,
+                                   (uint32_t)((a * 128 + i * 16 + t * 8) * e_ldc2));
             }
-            pp_join(x[0], y[0]);
-            pp_join(x[1], y[1]);
-            pp_store16(d, u32x4_t{x[0], x[1], y[0], y[1]}, ok ? e_off : PP_DROP, (uint32_t)((a * 128 + i * 16) * e_ldc2 + b * 256));
         }
     };
 
     auto run_tile = [&]() {
-        mfma_f32x4 acc[2][2][4][2];
+        mfma_f32x4 acc[2][4][4];
         const int KT = max(3, (cur.r1 - cur.r0 + PP_BK - 1) >> 6);
         // ---- phase 0 of the first K tile
         read_a(I0{}, I4{});
@@ -877,9 +919,9 @@ __device__ __forceinline__ void pp_wgrad_body()
         fill ^= PP_STAGE;
         pp_vmwait<10>();
         pp_barrier();
-        mma(T_{}, I4{}, acc[0][0], fb0);
+        mma(T_{}, I0{}, I4{}, acc[0], fb0);
         next_k();
-        have_nn = have_n && decode(q += gq, far);
+        have_nn = have_n && (q += 32) < q_end && decode(q, far);
         if (!have_nn) far = Tile{0, 0, 0, 0, 0};
         pp_barrier();
         auto k_tile = [&](auto FIRST, auto TURN, auto N_, bool turn_next) {
@@ -889,14 +931,14 @@ __device__ __forceinline__ void pp_wgrad_body()
             dma_b(I0{});
             pp_vmwait<10>();
             pp_barrier();
-            mma(FIRST, I4{}, acc[0][1], fb1);
+            mma(F_{}, I1{}, I4{}, acc[0], fb1);
             pp_barrier();
             // phase 2
             read_a(I1{}, N_);
             dma_a(I0{});
             pp_vmwait<10>();
             pp_barrier();
-            mma(FIRST, N_, acc[1][0], fb0);
+            mma(FIRST, I0{}, N_, acc[1], fb0);
             pp_barrier();
             // phase 3
             flip();
@@ -904,7 +946,7 @@ __device__ __forceinline__ void pp_wgrad_body()
             dma_b(I1{});
             pp_vmwait<10>();
             pp_barrier();
-            mma(FIRST, N_, acc[1][1], fb1);
+            mma(F_{}, I1{}, N_, acc[1], fb1);
             row_n = turn_next ? nxt.r0 : row_n + PP_BK;
             fetch_idx();
             pp_barrier();
@@ -914,7 +956,7 @@ __device__ __forceinline__ void pp_wgrad_body()
             fill ^= PP_STAGE;
             pp_vmwait<10>();
             pp_barrier();
-            mma(F_{}, I4{}, acc[0][0], fb0);
+            mma(F_{}, I0{}, I4{}, acc[0], fb0);
             if (decltype(TURN)::value) prepare_epilogue();
             next_k();
             pp_barrier();
@@ -930,32 +972,32 @@ __device__ __forceinline__ void pp_wgrad_body()
         if constexpr (MAPS != 0)
             for (; t < KT - 2; ++t) k_tile(F_{}, F_{}, I0{}, t == KT - 3);
         k_tile(F_{}, T_{}, I4{}, false);
-        // ---- last K tile: the epilogue of each finished quadrant in the memory part of the phase after it
+        // ---- last K tile: the epilogue of each finished half in the memory parts of the phases after it
         read_b(I1{}, fb1);
         dma_b(I0{});
-        epilogue(I0{}, I0{}, acc[0][0]);
         pp_vmwait<10>();
         pp_barrier();
-        mma(F_{}, I4{}, acc[0][1], fb1);
+        mma(F_{}, I1{}, I4{}, acc[0], fb1);
         pp_barrier();
         read_a(I1{}, I4{});
         dma_a(I0{});
-        epilogue(I0{}, I1{}, acc[0][1]);
+        epilogue(I0{}, I0{}, acc[0]);
         pp_vmwait<10>();
         pp_barrier();
-        mma(F_{}, I4{}, acc[1][0], fb0);
+        mma(F_{}, I0{}, I4{}, acc[1], fb0);
         pp_barrier();
         flip();
         read_b(I0{}, fb0);
         dma_b(I1{});
-        epilogue(I1{}, I0{}, acc[1][0]);
+        epilogue(I0{}, I2{}, acc[0]);
         pp_vmwait<10>();
         pp_barrier();
-        mma(F_{}, I4{}, acc[1][1], fb1);
+        mma(F_{}, I1{}, I4{}, acc[1], fb1);
         row_n += PP_BK;
         fetch_idx();
         pp_barrier();
-        epilogue(I1{}, I1{}, acc[1][1]);
+        epilogue(I1{}, I0{}, acc[1]);
+        epilogue(I1{}, I2{}, acc[1]);
     };
 
     // ------------------------------------------------------------ the workgroup's tiles
@@ -999,15 +1041,15 @@ __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_rows_f16_kernel
     pp_rows_body<B_KC, EPI, ACT, STREAM, f16_t>();
 }
 
-template <int MAPS>
+template <int MAPS, bool STREAM>
 __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_wgrad_bf16_kernel(GemmArgs)
 {
-    pp_wgrad_body<MAPS, bf16_t>();
+    pp_wgrad_body<MAPS, STREAM, bf16_t>();
 }
-template <int MAPS>
+template <int MAPS, bool STREAM>
 __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_wgrad_f16_kernel(GemmArgs)
 {
-    pp_wgrad_body<MAPS, f16_t>();
+    pp_wgrad_body<MAPS, STREAM, f16_t>();
 }
 
 }  // namespace
@@ -1057,17 +1099,21 @@ int amoe_pp_gated_bwd(const GemmArgs& a, int act, int tiles, hipStream_t s)
 }
 #endif
 #if AMOE_PP_PART_IS(3)
+template <int MAPS, bool STREAM>
+static int launch_pp_wgrad(const GemmArgs& a, int grid, hipStream_t s)
+{
+    if (a.f16) return launch_kernel<grouped_gemm_pp_wgrad_f16_kernel<MAPS, STREAM>, PP_THREADS, PP_WGRAD_LDS>(a, grid, s);
+    return launch_kernel<grouped_gemm_pp_wgrad_bf16_kernel<MAPS, STREAM>, PP_THREADS, PP_WGRAD_LDS>(a, grid, s);
+}
 template <int MAPS>
 static int launch_pp_wgrad(const GemmArgs& a, int grid, hipStream_t s)
 {
-    if (a.f16) return launch_kernel<grouped_gemm_pp_wgrad_f16_kernel<MAPS>, PP_THREADS, 2 * PP_STAGE>(a, grid, s);
-    return launch_kernel<grouped_gemm_pp_wgrad_bf16_kernel<MAPS>, PP_THREADS, 2 * PP_STAGE>(a, grid, s);
+    if (a.stream_from) return launch_pp_wgrad<MAPS, true>(a, grid, s);
+    return launch_pp_wgrad<MAPS, false>(a, grid, s);
 }
 
 int amoe_pp_wgrad(GemmArgs a, hipStream_t s)
 {
-    const int cus = device_cu_count();
-    AMOE_REQUIRE(cus > 0, AMOE_ERR_LAUNCH, "grouped_gemm: cannot read the number of compute units");
     const int strips = (a.n_ntiles + 7) / 8;
     a.gn = (a.n_ntiles + strips - 1) / strips;
     a.sn = (a.n_ntiles + a.gn - 1) / a.gn;
@@ -1078,7 +1124,20 @@ int amoe_pp_wgrad(GemmArgs a, hipStream_t s)
     a.inv_sn = inverse(a.n_mt * a.gn);
     a.inv_gn = inverse(a.gn);
     a.inv_gm = inverse(a.n_ntiles - (a.sn - 1) * a.gn);
-    const int grid = (int)(((total < cus ? total : cus) + 7) & ~7);
+    // Tiles a workgroup: all that fall to it from 11 K tiles an expert on (fewer workgroups then only fill their pipelines again: 1024
+    // rows of 128 experts of 2048 x 768, a training step 3.80 ms, with two tiles each 3.92), below that two, so that the other stream's
+    // workgroups get compute units between them.  Steps with one / two / four / all, ms, against shape 5 (to 256 rows) or all:
+    //   64 experts of 2048 x 1408, 250 rows, shared expert  1.59 / 1.62 / 1.64 / 1.67, 1.67
+    //   37 experts of 5568 x 1600, 221 rows                 2.08 / 2.02 / 1.99 / 1.94, 2.17
+    //   24 experts of  480 x 7360, 230 rows                 0.73 / 0.73 / 0.75 / 0.76, 0.79
+    //   22 experts of  832 x 11840, 615 rows                3.18 / 3.17 / 3.19 / 3.38, 3.40
+    //   16 experts of 1728 x 2208, 742 rows                 0.99 / 1.01 / 1.00 / 0.98, 1.00
+    const long long rounds = (total + 255) / 256;
+    a.gm = (int)(a.rows_total < 11ll * PP_BK * a.E && rounds > 2 ? 2 : rounds);
+    const int grid = rounds == 1 ? (int)((total + 7) & ~7ll) : (int)((rounds + a.gm - 1) / a.gm * 256);
+    // Gradients that the L2s (8 x 4 MB) do not hold are stored past the caches: with ordinary stores a tile's 128 KB wait for dirty
+    // lines of older ones to be written out, behind which no load of the next tile completes.
+    a.stream_from = 2ll * a.E * a.M * a.N > (32ll << 20);
     if (a.a_row_map) return launch_pp_wgrad<1>(a, grid, s);
     if (a.b_row_map) return launch_pp_wgrad<2>(a, grid, s);
     return launch_pp_wgrad<0>(a, grid, s);

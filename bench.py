@@ -307,6 +307,7 @@ def main():
     rows = f"grouped_gemm_rows_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_rows_bf16_kernel<"
     wgrad = f"grouped_gemm_wgrad_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_wgrad_bf16_kernel<"
     end = ">" if c else ", false>"   # (every workload here has far more than a tile of rows per expert)
+    wend = ">" if c else ", true>"   # (and gradients that the L2s do not hold)
     gathered = token_of is not None
     sym = {
         # grouped_gemm_pp_rows_bf16_kernel<B K-contiguous, epilogue, activation, B past the caches>; other tile shapes:
@@ -316,10 +317,10 @@ def main():
         "gemm_dgrad_down": f"{rows}true, 0, 0{end}",
         "gemm_dgrad_down_gated_bwd": f"{rows}true, 2, 0{end}",
         "gemm_dgrad_gateup": f"{rows}true, 0, 0{end}",
-        # grouped_gemm_pp_wgrad_bf16_kernel<gathered operand> (256 rows per expert or more); other tile shapes:
+        # grouped_gemm_pp_wgrad_bf16_kernel<gathered operand, stored past the caches>; other tile shapes:
         # grouped_gemm_wgrad_bf16_kernel<BM, BN, waves along M, waves along N, gathered operand>
-        "gemm_wgrad_down": f"{wgrad}{2 if gathered else 0}>",
-        "gemm_wgrad_gateup": f"{wgrad}{1 if gathered else 0}>",
+        "gemm_wgrad_down": f"{wgrad}{2 if gathered else 0}{wend}",
+        "gemm_wgrad_gateup": f"{wgrad}{1 if gathered else 0}{wend}",
     }
     if dtype != torch.bfloat16:
         sym = {k: "grouped_gemm_f32_kernel" for k in sym}
