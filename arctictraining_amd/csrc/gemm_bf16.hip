@@ -1407,6 +1407,8 @@ int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, int tiles, h
 // few rows per expert (gemm_skinny.hip)
 int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s);
 int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s);
+int amoe_skinny_gateup_routed(const GemmArgs& a, int act, const AmoeRoute& r, hipStream_t s);
+int amoe_skinny_nn_combined(const GemmArgs& a, const AmoeCombine& c, hipStream_t s);
 
 // From how many tiles of rows on a product's weights are loaded past the caches (0: never).
 // Weights that are read once and that the last-level cache (256 MiB in front of all XCDs) cannot hold until the next call
@@ -1524,6 +1526,68 @@ int amoe_bf16_gateup_act(const void* xp, const int32_t* a_row_map, const void* w
     return AMOE_ERR_BAD_ARG;
 }
 
+#endif
+
+#if AMOE_PART(0)
+// Up to 8 tokens: each of the product's workgroups selects for itself, and with many of them that takes longer than a launch.  bf16, one
+// forward pass, us, logits / routing / gate_up / down / sums as five launches and as three: 8 of 128 experts of 2048 x 768, 1 token
+// 35.3 / 29.9, 2 53.8 / 49.2, 4 76.2 / 75.8, 8 111.5 / 111.0, 12 135.2 / 143.1; 2 of 243 experts of 288 x 3712, 1 token 29.7 / 26.0,
+// 8 45.5 / 41.8, 12 56.9 / 59.5; 4 of 32 experts of 4096 x 2048, 1 token 59.5 / 52.3, 8 200.6 / 191.7, 16 261 / 260 (sizes that are bound by
+// the host 29.8 / 26.2).
+bool amoe_routed_fits(int dtype, int T, int K, int E, int H, int I, int tile_cfg)
+{
+    return (dtype == AMOE_BF16 || dtype == AMOE_F16) && tile_cfg == 0 && T <= 8 && T * K <= 128 && E <= 256 && K <= E && K <= AMOE_MAX_TOPK &&
+           rows_tile_height(T * K, E, 0) == 16 && H % 32 == 0 && I % 32 == 0 && (unsigned long long)H * 2 * I * 2 < (1ull << 32);
+}
+
+int amoe_run_gateup_routed(const void* x, const void* w_gate_up, void* gate_up, void* inter, const AmoeRoute& r, int dtype, int E, int H, int I,
+                           int act, void* workspace, size_t workspace_bytes, hipStream_t s)
+{
+    AMOE_REQUIRE(x && w_gate_up && inter && r.logits && act >= AMOE_ACT_SILU && act <= AMOE_ACT_GPT_OSS, AMOE_ERR_BAD_ARG,
+                 "gateup_routed: bad argument");
+    const int R = r.T * r.K;
+    GemmArgs a = {};
+    AmoeRoute route = r;
+    const int4* map = nullptr;
+    const int32_t* count = nullptr;
+    int rc = amoe_build_tile_map(nullptr, R, E, 16, workspace, workspace_bytes, &map, &count, &a.max_mtiles, s, true);
+    if (rc) return rc;
+    route.tile_map = const_cast<int4*>(map);
+    route.n_mtiles = const_cast<int32_t*>(count);
+    a.A = (const bf16_t*)x;
+    a.B = (const bf16_t*)w_gate_up;
+    a.C = (bf16_t*)gate_up;
+    a.C2 = (bf16_t*)inter;
+    a.f16 = dtype == AMOE_F16;
+    a.lda = a.Kd = H;
+    a.ldb = a.ldc = a.N = 2 * I;
+    a.ldc2 = I;
+    a.strideB = (long long)H * 2 * I;
+    a.E = E;
+    a.M = R;
+    a.stream_from = stream_from(R, E, a.strideB, H, true);
+    return amoe_skinny_gateup_routed(a, act, route, s);
+}
+
+int amoe_run_down_combined(const void* inter, const void* w_down, void* out, const AmoeCombine& c, int dtype, int E, int H, int I, void* workspace,
+                           size_t workspace_bytes, hipStream_t s)
+{
+    AMOE_REQUIRE(inter && w_down && out && c.arrived && c.row_of && c.y, AMOE_ERR_BAD_ARG, "down_combined: null pointer");
+    GemmArgs a = {};
+    a.M = c.T * c.K;
+    int rc = amoe_build_tile_map(nullptr, a.M, E, 16, workspace, workspace_bytes, &a.tile_map, &a.n_mtiles, &a.max_mtiles, s, true);
+    if (rc) return rc;
+    a.A = (const bf16_t*)inter;
+    a.B = (const bf16_t*)w_down;
+    a.C = (bf16_t*)out;
+    a.f16 = dtype == AMOE_F16;
+    a.lda = a.Kd = I;
+    a.ldb = a.ldc = a.N = H;
+    a.strideB = (long long)I * H;
+    a.E = E;
+    a.stream_from = stream_from(a.M, E, a.strideB, I, false);
+    return amoe_skinny_nn_combined(a, c, s);
+}
 #endif
 
 #if AMOE_PART(1)

@@ -15,8 +15,10 @@
 // 4096 x 14336, 1 row 292 and 184 -> 256 and 129, 4 rows 334 and 195 -> 330 and 149; 16 experts of 512 x 512, 4 rows 17
 // and 12 -> 11 and 9.  A 64-row form at 32 rows an expert of the first took 222 and 90 us (one-tile workgroups of 256 rows
 // 204 and 83) and is not kept.
+#include "gemm_calls.h"
 #include "gemm_common.h"
 #include "gemm_launch.h"
+#include "router_topk.h"
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float sk_f32x4;
 
@@ -41,8 +43,11 @@ struct MfmaSkinny<f16_t> {
     }
 };
 
-template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET>
-__device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[NW][CPL * 64], int e, int m0, int mend, int n0)
+// source_of(row): the row of A that stands for a row; scale_of(row): its factor in the gated epilogue
+// SHARED: C is stored where workgroups of other XCDs see it (agent scope: through the L2s)
+template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET, bool SHARED = false, typename SourceOf, typename ScaleOf>
+__device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[NW][CPL * 64], int e, int m0, int mend, int n0,
+                                            SourceOf source_of, ScaleOf scale_of)
 {
     constexpr int W = CPL / 2, H = CPL / 4;           // dwords of a lane's row, groups of four columns
     const int tid = threadIdx.x, lane = tid & 63;
@@ -61,8 +66,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[N
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const int row = m0 + i * 16 + l16;
-        const int src = row < mend && p.a_row_map ? p.a_row_map[row] : row;
-        aoff[i] = row < mend ? ((uint32_t)src * (uint32_t)p.lda + lq * 8) * 2u : SK_NOWHERE;
+        aoff[i] = row < mend ? ((uint32_t)source_of(row) * (uint32_t)p.lda + lq * 8) * 2u : SK_NOWHERE;
     }
 
     struct Step {
@@ -143,9 +147,12 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[N
             const int col = n0 + ((l >> 4) * 4 + q / H) * CPL + (q % H) * 4;
             if (row < mend && col < p.N) {
                 const uint32_t x = Elem16<ET>::pack2(c[0], c[1]), y = Elem16<ET>::pack2(c[2], c[3]);
-                if (EPI != EPI_GATED || p.C) *reinterpret_cast<u32x2_t*>(p.C + (long long)row * p.ldc + col) = u32x2_t{x, y};
+                bf16_t* const at = p.C + (long long)row * p.ldc + col;
+                if constexpr (SHARED)
+                    __hip_atomic_store(reinterpret_cast<uint64_t*>(at), (uint64_t)y << 32 | x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else if (EPI != EPI_GATED || p.C) *reinterpret_cast<u32x2_t*>(at) = u32x2_t{x, y};
                 if constexpr (EPI == EPI_GATED) {
-                    const float s = p.row_scale ? p.row_scale[row] : 1.0f;
+                    const float s = scale_of(row);
                     *reinterpret_cast<uint32_t*>(p.C2 + (long long)row * p.ldc2 + (col >> 1)) =
                         Elem16<ET>::pack2(s * Elem16<ET>::hi(x) * act_fwd_fast<ACT>(Elem16<ET>::lo(x)),
                                           s * Elem16<ET>::hi(y) * act_fwd_fast<ACT>(Elem16<ET>::lo(y)));
@@ -171,11 +178,13 @@ __device__ __forceinline__ void skinny_body(const GemmArgs& p)
         m0 = scalar_load_i32(ent + 1);
         mend = scalar_load_i32(ent + 2);
     }
-    skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET>(p, red, e, m0, mend, n0);
+    const auto source_of = [&](int row) { return p.a_row_map ? p.a_row_map[row] : row; };
+    const auto scale_of = [&](int row) { return p.row_scale ? p.row_scale[row] : 1.0f; };
+    skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET>(p, red, e, m0, mend, n0, source_of, scale_of);
 #pragma unroll 1
     for (m0 += 16 * MT; m0 < mend; m0 += 16 * MT) {
         __syncthreads();   // (the sums are read before the next part's are written)
-        skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET>(p, red, e, m0, mend, n0);
+        skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET>(p, red, e, m0, mend, n0, source_of, scale_of);
     }
 }
 
@@ -227,6 +236,219 @@ int launch_height(const GemmArgs& a, int bm, hipStream_t s)
     const int cus = device_cu_count();
     if ((long long)m_tiles * ((a.N + 127) / 128) < cus) return launch_skinny<1, 4, 8, EPI, ACT>(a, m_tiles, s);
     return launch_skinny<1, 8, 4, EPI, ACT>(a, m_tiles, s);
+}
+
+// ------------------------------------------------------------------ gate_up product with the routing of a few tokens
+// Softmax, top-k and the plan of a few tokens (one wavefront a token, then a walk over the at most kRoutedRows selected slots in
+// LDS) cost a launch of one workgroup 6 us, most of it the launch and memory round trips that the product then waits for.
+// Here every workgroup of the product selects for itself and finds its own expert and rows; what the other products and backward
+// read of the routing is written by one more workgroup, which multiplies nothing.
+// (At amoe_routed_fits: where this pays, and what it measured.)
+constexpr int kRoutedRows = 128, kRoutedExperts = 256;
+
+template <int CPL, int NW, int ACT, bool STREAM, typename ET>
+__device__ __forceinline__ void skinny_routed_body(const GemmArgs& p, const AmoeRoute& r)
+{
+    constexpr int VPT = kRoutedExperts / 64, WORDS = kRoutedExperts / 32;
+    __shared__ sk_f32x4 red[NW][CPL * 64];
+    __shared__ __attribute__((aligned(16))) int sel[kRoutedRows];      // expert of flat slot k * T + t
+    __shared__ float score[kRoutedRows], row_score[kRoutedRows];
+    __shared__ int row_token[kRoutedRows];
+    __shared__ uint32_t met[WORDS];                                    // experts that have a row
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int T = r.T, K = r.K, E = p.E, R = T * K;
+    const bool writer = blockIdx.x == 0;
+    if (tid < WORDS) met[tid] = 0;
+    if (tid < kRoutedRows) sel[tid] = kRoutedExperts;                  // (past the last slot: of no expert)
+    __syncthreads();
+    for (int t = wave; t < T; t += NW) {
+        int e;
+        float s;
+        router_topk_token<ET, VPT>((const ET*)r.logits + (size_t)t * E, E, K, r.normalize, lane, writer ? r.probs + (size_t)t * E : nullptr, e, s);
+        if (lane < K) {
+            e = min(max(e, 0), E - 1);
+            sel[lane * T + t] = e;
+            score[lane * T + t] = s;
+            atomicOr(&met[e >> 5], 1u << (e & 31));
+            if (writer) {
+                r.topk_idx[t * K + lane] = e;
+                r.scores[t * K + lane] = s;
+            }
+        }
+    }
+    __syncthreads();
+    // slots of smaller experts, and of this one before slot f
+    auto walk = [&](int e, int f, int& smaller, int& before) {
+        smaller = before = 0;
+        for (int g = 0; g < R; g += 4) {
+            const int4 v = *reinterpret_cast<const int4*>(sel + g);
+            const int x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                smaller += x[i] < e;
+                before += x[i] == e && g + i < f;
+            }
+        }
+    };
+    auto experts_below = [&](int e) {
+        int n = 0;
+#pragma unroll
+        for (int w = 0; w < WORDS; ++w) {
+            const int left = e - 32 * w;
+            n += __popc(left >= 32 ? met[w] : left > 0 ? met[w] & ((1u << left) - 1u) : 0u);
+        }
+        return n;
+    };
+    if (writer) {
+        if (tid < R) {
+            const int e = sel[tid], k = tid / T, t = tid - k * T;
+            int smaller, before;
+            walk(e, tid, smaller, before);
+            const int row = smaller + before;
+            r.token_of[row] = t;
+            r.slot_of[row] = tid;
+            r.row_of[t * K + k] = row;
+            r.scores_perm[row] = score[tid];
+        }
+        for (int e = tid; e < E; e += NW * 64) {
+            int smaller, rows;
+            walk(e, R, smaller, rows);
+            r.counts[e] = rows;
+            r.offsets[e + 1] = smaller + rows;
+            // (an expert's rows are at most the T tokens: one tile)
+            if (rows) r.tile_map[experts_below(e)] = make_int4(e, smaller, smaller + rows, 0);
+        }
+        const int tiles = experts_below(E);
+        for (int i = tiles + tid; i < p.max_mtiles; i += NW * 64) r.tile_map[i] = make_int4(-1, 0, 0, 0);
+        if (tid == 0) r.offsets[0] = 0;
+        if (tid < 4) r.n_mtiles[tid] = tid ? 0 : tiles;
+        for (int i = tid; i < r.n_arrived; i += NW * 64) r.arrived[i] = 0;
+        return;
+    }
+    const int pm = (int)(blockIdx.x - 1) / p.n_ntiles;
+    const int n0 = ((int)(blockIdx.x - 1) - pm * p.n_ntiles) * 16 * CPL;
+    if (pm >= experts_below(E)) return;
+    int e = 0, skip = pm;                // the pm-th expert that has a row
+#pragma unroll
+    for (int w = 0; w < WORDS; ++w) {
+        const int n = __popc(met[w]);
+        if (skip >= 0 && skip < n) {
+            uint32_t m = met[w];
+            for (; skip; --skip) m &= m - 1;
+            e = 32 * w + __builtin_ctz(m);
+            skip = -1;
+        } else if (skip >= 0) skip -= n;
+    }
+    e = __builtin_amdgcn_readfirstlane(e);
+    int m0, rows, rank;
+    walk(e, R, m0, rows);
+    if (tid < R && sel[tid] == e) {
+        walk(e, tid, m0, rank);
+        row_token[rank] = tid % T;
+        row_score[rank] = score[tid];
+    }
+    m0 = __builtin_amdgcn_readfirstlane(m0);
+    rows = __builtin_amdgcn_readfirstlane(rows);
+    __syncthreads();
+    skinny_tile<1, CPL, NW, EPI_GATED, ACT, STREAM, ET>(p, red, e, m0, m0 + rows, n0, [&](int row) { return row_token[row - m0]; },
+                                                        [&](int row) { return row_score[row - m0]; });
+}
+
+template <int CPL, int NW, int ACT, bool STREAM>
+__global__ void __launch_bounds__(NW * 64, 4) grouped_gemm_skinny_routed_bf16_kernel(GemmArgs p, AmoeRoute r)
+{
+    skinny_routed_body<CPL, NW, ACT, STREAM, bf16_t>(p, r);
+}
+template <int CPL, int NW, int ACT, bool STREAM>
+__global__ void __launch_bounds__(NW * 64, 4) grouped_gemm_skinny_routed_f16_kernel(GemmArgs p, AmoeRoute r)
+{
+    skinny_routed_body<CPL, NW, ACT, STREAM, f16_t>(p, r);
+}
+
+template <int CPL, int NW, int ACT, bool STREAM>
+int launch_routed(const GemmArgs& a, const AmoeRoute& r, int grid, hipStream_t s)
+{
+    if (a.f16) hipLaunchKernelGGL((grouped_gemm_skinny_routed_f16_kernel<CPL, NW, ACT, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a, r);
+    else hipLaunchKernelGGL((grouped_gemm_skinny_routed_bf16_kernel<CPL, NW, ACT, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a, r);
+    return amoe_check_launch("grouped_gemm_skinny_routed");
+}
+template <int CPL, int NW, int ACT>
+int launch_routed(GemmArgs a, const AmoeRoute& r, int m_tiles, hipStream_t s)
+{
+    a.n_ntiles = (a.N + 16 * CPL - 1) / (16 * CPL);
+    const long long grid = (long long)m_tiles * a.n_ntiles + 1;
+    AMOE_REQUIRE(grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
+    if (a.stream_from) return launch_routed<CPL, NW, ACT, true>(a, r, (int)grid, s);
+    return launch_routed<CPL, NW, ACT, false>(a, r, (int)grid, s);
+}
+
+// ------------------------------------------------------------------ down product with the sums over a token's rows
+// As grouped_gemm_skinny with a map of 16-row tiles; the last of a column tile's workgroups to arrive adds up the tokens' rows
+// there, as stored and in the order of k (gather_reduce_kernel's sum, bit for bit), instead of a launch of its own that waits for all of them.
+template <int CPL, int NW, bool STREAM, typename ET>
+__device__ __forceinline__ void skinny_combine_body(const GemmArgs& p, const AmoeCombine& c)
+{
+    __shared__ sk_f32x4 red[NW][CPL * 64];
+    __shared__ int before;
+    const int pm = blockIdx.x / p.n_ntiles, nt = blockIdx.x - pm * p.n_ntiles, n0 = nt * 16 * CPL;
+    const int tiles = min(scalar_load_i32(p.n_mtiles), p.max_mtiles);
+    if (pm >= tiles) return;
+    const int32_t* ent = reinterpret_cast<const int32_t*>(p.tile_map + pm);
+    skinny_tile<1, CPL, NW, EPI_STORE, 0, STREAM, ET, true>(p, red, scalar_load_i32(ent), scalar_load_i32(ent + 1), scalar_load_i32(ent + 2), n0,
+                                                            [](int row) { return row; }, [](int) { return 1.0f; });
+    // Rows are stored and read past the L2s, and every wavefront awaits its stores before the workgroup arrives: a release would
+    // write out all of the XCD's L2 besides, a microsecond or more in every workgroup (4 tokens of 8 of 128 experts of 2048 x
+    // 768, the whole pass 75 us with a launch of its own for the sums, 89 with a release, 75 so; 1 token 30.8, 32.3, 29.9).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) before = __hip_atomic_fetch_add(c.arrived + nt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (before != tiles - 1) return;
+    constexpr int PIECES = 4 * CPL;                     // of four columns
+    for (int i = threadIdx.x; i < c.T * PIECES; i += NW * 64) {
+        const int t = i / PIECES, col = n0 + (i - t * PIECES) * 4;
+        if (col >= p.N) continue;
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < c.K; ++k) {
+            const u32x2_t v = __builtin_bit_cast(u32x2_t, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p.C + (long long)c.row_of[t * c.K + k] * p.ldc + col),
+                                                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                sum[2 * j] += Elem16<ET>::lo(v[j]);
+                sum[2 * j + 1] += Elem16<ET>::hi(v[j]);
+            }
+        }
+        *reinterpret_cast<u32x2_t*>((bf16_t*)c.y + (long long)t * p.ldc + col) =
+            u32x2_t{Elem16<ET>::pack2(sum[0], sum[1]), Elem16<ET>::pack2(sum[2], sum[3])};
+    }
+}
+
+template <int CPL, int NW, bool STREAM>
+__global__ void __launch_bounds__(NW * 64, 4) grouped_gemm_skinny_combine_bf16_kernel(GemmArgs p, AmoeCombine c)
+{
+    skinny_combine_body<CPL, NW, STREAM, bf16_t>(p, c);
+}
+template <int CPL, int NW, bool STREAM>
+__global__ void __launch_bounds__(NW * 64, 4) grouped_gemm_skinny_combine_f16_kernel(GemmArgs p, AmoeCombine c)
+{
+    skinny_combine_body<CPL, NW, STREAM, f16_t>(p, c);
+}
+
+template <int CPL, int NW, bool STREAM>
+int launch_combine(const GemmArgs& a, const AmoeCombine& c, int grid, hipStream_t s)
+{
+    if (a.f16) hipLaunchKernelGGL((grouped_gemm_skinny_combine_f16_kernel<CPL, NW, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a, c);
+    else hipLaunchKernelGGL((grouped_gemm_skinny_combine_bf16_kernel<CPL, NW, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a, c);
+    return amoe_check_launch("grouped_gemm_skinny_combine");
+}
+template <int CPL, int NW>
+int launch_combine(GemmArgs a, const AmoeCombine& c, int m_tiles, hipStream_t s)
+{
+    a.n_ntiles = (a.N + 16 * CPL - 1) / (16 * CPL);
+    const long long grid = (long long)m_tiles * a.n_ntiles;
+    AMOE_REQUIRE(grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
+    if (a.stream_from) return launch_combine<CPL, NW, true>(a, c, (int)grid, s);
+    return launch_combine<CPL, NW, false>(a, c, (int)grid, s);
 }
 
 // ------------------------------------------------------------------ the router's linear map for few tokens
@@ -289,6 +511,25 @@ int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s)
 {
     AMOE_DISPATCH_ACT(act, return (launch_height<EPI_GATED, ACT>(a, bm, s)))
     return AMOE_ERR_BAD_ARG;
+}
+
+// a: as for amoe_skinny_gateup_act, without the maps and scales that the routing gives
+int amoe_skinny_gateup_routed(const GemmArgs& a, int act, const AmoeRoute& r, hipStream_t s)
+{
+    const int R = r.T * r.K, m_tiles = a.E < R ? a.E : R;
+    AMOE_REQUIRE(r.T <= 16 && R <= kRoutedRows && a.E <= kRoutedExperts, AMOE_ERR_UNSUPPORTED,   // (a tile holds 16 rows)
+                 "grouped_gemm: routing of %d rows of %d experts", R, a.E);
+    const bool narrow = (long long)m_tiles * ((a.N + 127) / 128) < device_cu_count();   // (as in launch_height)
+    AMOE_DISPATCH_ACT(act, return narrow ? (launch_routed<4, 8, ACT>(a, r, m_tiles, s)) : (launch_routed<8, 4, ACT>(a, r, m_tiles, s)))
+    return AMOE_ERR_BAD_ARG;
+}
+
+// c.arrived holds a count for every 64 columns
+int amoe_skinny_nn_combined(const GemmArgs& a, const AmoeCombine& c, hipStream_t s)
+{
+    const int m_tiles = a.E < a.M ? a.E : a.M;
+    const bool narrow = (long long)m_tiles * ((a.N + 127) / 128) < device_cu_count();
+    return narrow ? launch_combine<4, 8>(a, c, m_tiles, s) : launch_combine<8, 4>(a, c, m_tiles, s);
 }
 
 int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s) { return launch_height<EPI_STORE, 0>(a, bm, s); }

@@ -90,7 +90,7 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long k)
 __device__ __forceinline__ unsigned long long wave_max_key(unsigned long long k) { return wave_max_u64(k); }
 
 // One token on one wavefront: its K experts and scores (lane k holds the k-th), and the softmax of its row of E logits
-// into prow.
+// into prow (none if null).
 template <typename T, int VPT>
 __device__ __forceinline__ void router_topk_token(const T* row, int E, int K, int normalize, int lane, float* prow, int& top_e_out,
                                                   float& score_out)
@@ -145,7 +145,7 @@ __device__ __forceinline__ void router_topk_token(const T* row, int E, int K, in
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         int e = lane + 64 * j;
-        if (e < E) prow[e] = ex[j] / z;
+        if (prow && e < E) prow[e] = ex[j] / z;
     }
     // (the division stays an IEEE division: the probabilities are compared with the library softmax)
 
