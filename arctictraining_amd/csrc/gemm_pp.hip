@@ -82,49 +82,70 @@ __device__ __forceinline__ void pp_rows_body()
     };
 
     // ------------------------------------------------------------ this workgroup's tiles
-    // Virtual blocks b, b + grid, b + 2 grid, ...; virtual block v belongs to XCD v % 8 (the hardware deals
-    // workgroups to the XCDs round-robin) and is slot (v / 8) % (gm gn) of super-tile ((v / 8) / (gm gn)) * 8
-    // + v % 8: the workgroups resident on one XCD work on one super-tile of gm x gn tiles at a time (its gm A
-    // panels and gn B panels are shared in that XCD's L2) and the super-tiles rotate over the XCDs.  Only whole
-    // groups of 8 super-tiles are dealt that way; the up to 7 left over go to the XCDs tile by tile.
-    // (divisions by multiplication with the host's rounded-up reciprocals: exact for the numerators that occur)
-    int vb_next = blockIdx.x;
-    const int n_mtiles = min(scalar_load_i32(pp_args().n_mtiles), pp_args().max_mtiles);
-    auto advance = [&](int& pm, int& nt) -> bool {
-        args_t& p = pp_args();
-        const int per_super = p.gm * p.gn;
-        const int supers = (divide(n_mtiles + p.gm - 1, p.inv_gm)) * p.sn;
-        const int vb_rot = (supers >> 3) * 8 * per_super;
-        const int vb_total = supers * per_super;
-        while (vb_next < vb_total) {
-            const int vb = vb_next;
-            vb_next += gridDim.x;
-            int sid, w;
-            if (vb < vb_rot) {
-                const int xcd = vb & 7, q = vb >> 3;
-                sid = divide(q, p.inv_super);
-                w = q - sid * per_super;
-                sid = sid * 8 + xcd;
-            } else {
-                sid = divide(vb, p.inv_super);
-                w = vb - sid * per_super;
-            }
-            const int sm = divide(sid, p.inv_sn), sn_i = sid - sm * p.sn;
-            const int wm = divide(w, p.inv_gn);
-            pm = sm * p.gm + wm;
-            nt = sn_i * p.gn + w - wm * p.gn;
-            if (nt < p.n_ntiles && pm < n_mtiles) return true;
-        }
-        return false;
+    // The tiles that there are stand in one row: groups of gm tile rows, in a group super-columns of gn tiles (the last one
+    // narrower), tile row by tile row inside them.  XCD x (the hardware deals workgroups to the XCDs round-robin) takes the x-th
+    // eighth of each gridDim.x of them, so that its workgroups share the gm A panels and gn B panels of a super-tile in its L2.
+    // The last, partial round's tiles of more than 6 blocks of 32 rows are cut into 2 or 4 pieces of whole blocks where there are
+    // workgroups for them: a round lasts as long as its tallest tile.  (Lower ones are bound by reading the weights, and each piece
+    // reads them: 188 rows an expert, gated backward of 1.5 rounds of tiles 181 us whole, 182 in halves.  A piece's weights are
+    // not read past the caches.)
+    // Before, blocks of a padded grid were dealt, super-tile by super-tile, whether there was a tile or not: of 968 tiles, 88 x 11,
+    // some workgroups got five and others three.  Steps, before / now, ms: 4001 tokens of 64 experts of 2048 x 1408 and a shared
+    // one 1.653 / 1.616, 8192 tokens of 8 experts of 4096 x 14336 (4.25 rounds in two products) 13.88 / 13.80, 32768 uneven
+    // ones 6.607 / 6.537; alone, us, one expert of 4001 rows: gate_up 60 / 56, down 37 / 33, gated backward 63 / 57.
+    // (a product with 2^32 / d rounded up gives n / d or, past n d = 2^32, one more)
+    auto divide_any = [](int n, int d, uint32_t inv) -> int {
+        const int q = inv ? (int)(((uint64_t)(uint32_t)n * inv) >> 32) : n;
+        return q - (int)((uint32_t)q * (uint32_t)d > (uint32_t)n);
     };
-    auto load_entry = [&](int pm) -> int4 {
-        const int32_t* ent = reinterpret_cast<const int32_t*>(pp_args().tile_map + pm);
-        int4 v;
-        v.x = scalar_load_i32(ent);
-        v.y = scalar_load_i32(ent + 1);
-        v.z = scalar_load_i32(ent + 2);
-        v.w = 0;
-        return v;
+    const int n_mtiles = min(scalar_load_i32(pp_args().n_mtiles), pp_args().max_mtiles);
+    int round_first = 0;                 // first tile of the round dealt next
+    // the next tile: its entry of the tile map (a piece's rows in it, and in w whether it is a piece) and N tile
+    auto next_tile = [&](int4& tm, int& nt) -> bool {
+        args_t& p = pp_args();
+        const int total = n_mtiles * p.n_ntiles, left = total - round_first, grid = gridDim.x;
+        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+        int i, piece = 0, cut = 0;
+        if (left >= grid) {
+            i = round_first + xcd * (grid >> 3) + slot;
+        } else {
+            const int share = (max(left, 0) + 7) >> 3;        // an XCD's tiles; the first pieces of all, then the second ones ..
+            cut = (share * 16 <= grid) + (share * 32 <= grid);
+            piece = (slot >= share) + (slot >= 2 * share) + (slot >= 3 * share);
+            const int q = xcd * share + slot - piece * share;
+            if (slot >= share << cut || q >= left) return false;
+            i = round_first + q;
+        }
+        round_first += grid;
+        const int per_group = p.gm * p.n_ntiles;
+        const int g = divide_any(i, per_group, p.inv_group);
+        int r = i - g * per_group, pm = g * p.gm;
+        if (pm + p.gm <= n_mtiles) {
+            const int c = divide(r, p.inv_super);
+            r -= c * p.gm * p.gn;
+            const bool last = c == p.sn - 1;
+            const int m = divide(r, last ? p.inv_last : p.inv_gn);
+            pm += m;
+            nt = c * p.gn + r - m * (last ? p.n_ntiles - c * p.gn : p.gn);
+        } else {
+            const int m = divide(r, p.inv_n);
+            pm += m;
+            nt = r - m * p.n_ntiles;
+        }
+        const int32_t* ent = reinterpret_cast<const int32_t*>(p.tile_map + pm);
+        tm.x = scalar_load_i32(ent);
+        tm.y = scalar_load_i32(ent + 1);
+        tm.z = scalar_load_i32(ent + 2);
+        tm.w = 0;
+        if (cut) {
+            const int blocks = (tm.z - tm.y + 31) >> 5;
+            const int rows = blocks > 6 ? ((blocks + (1 << cut) - 1) >> cut) * 32 : PP_BM;
+            tm.w = blocks > 6;
+            tm.y += piece * rows;
+            if (tm.y >= tm.z) return false;           // (the last round: this workgroup is done)
+            tm.z = min(tm.z, tm.y + rows);
+        }
+        return true;
     };
 
     // ------------------------------------------------------------ loads
@@ -140,10 +161,10 @@ __device__ __forceinline__ void pp_rows_body()
     // the tiles' weights have to be more than the caches hold
     const bool stream = STREAM && n_mtiles >= pp_args().stream_from;
     bool stream_b = false, stream_n = false;
-    auto expert_b = [&](int e) {
+    auto expert_b = [&](const int4& tm) {
         args_t& p = pp_args();
-        if (STREAM) stream_n = stream && scalar_load_i32(p.offsets + e + 1) - scalar_load_i32(p.offsets + e) <= PP_BM;
-        return p.B + (long long)e * p.strideB;
+        if (STREAM) stream_n = stream && tm.w == 0 && scalar_load_i32(p.offsets + tm.x + 1) - scalar_load_i32(p.offsets + tm.x) <= PP_BM;
+        return p.B + (long long)tm.x * p.strideB;
     };
     // a plan without rows (m0 == mend) or columns (n0 >= N) reads nothing
     auto plan_a = [&](int m0, int mend, const int32_t* map, int k0) {     // map: the row map (first tile), else the indices are in LDS
@@ -272,25 +293,23 @@ __device__ __forceinline__ void pp_rows_body()
     };
 
     // ------------------------------------------------------------ tile state
-    int m0, mend, nt, n0;
+    int m0, mend, nt = 0, n0;
     Part part, part_n;                   // this tile's part of the reduction, the next one's
     bool have_n, have_nn = false;        // is there a next tile, and one after it
     int nt_n = 0, nt_nn = 0;
     int4 tm_n, tm_nn = make_int4(0, 0, 0, 0);
     const bf16_t* b_n = nullptr;
     {
-        int pm = 0;
-        nt = 0;
-        if (!advance(pm, nt)) return;
-        const int4 tm = load_entry(pm);
+        int4 tm;
+        if (!next_tile(tm, nt)) return;
         m0 = tm.y;
         mend = tm.z;
-        have_n = advance(pm, nt_n);
-        tm_n = have_n ? load_entry(pm) : make_int4(0, 0, 0, 0);
+        have_n = next_tile(tm_n, nt_n);
+        if (!have_n) tm_n = make_int4(0, 0, 0, 0);
         part = part_of(nt);
         n0 = nt * PP_BN;
         plan_a(m0, mend, pp_args().a_row_map, part.k0);
-        plan_b(expert_b(tm.x), n0, part.k0);
+        plan_b(expert_b(tm), n0, part.k0);
     }
     int par = 0;            // row scales: which of the two LDS rows is this tile's
     bool sums_due = false;  // row-sum partials of the previous tile are complete in LDS and not yet written
@@ -477,11 +496,10 @@ __device__ __forceinline__ void pp_rows_body()
         mma(T_{}, I4{}, acc[0][0], fb0);
         {
             // the next tile's weights; which tile follows it, and its entry of the tile map
-            b_n = expert_b(tm_n.x);
+            b_n = expert_b(tm_n);
             part_n = part_of(nt_n);
-            int pm = 0;
-            have_nn = have_n && advance(pm, nt_nn);
-            tm_nn = have_nn ? load_entry(pm) : make_int4(0, 0, 0, 0);
+            have_nn = have_n && next_tile(tm_nn, nt_nn);
+            if (!have_nn) tm_nn = make_int4(0, 0, 0, 0);
         }
         pp_barrier();
         write_sums();
@@ -1056,6 +1074,9 @@ __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_wgrad_f16_kerne
 
 #include "gemm_launch.h"
 
+// ceil(2^32 / d), 0 for a divisor of 1
+static inline uint32_t tile_inverse(int d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; }
+
 template <bool B_KC, int EPI, int ACT, bool STREAM>
 static int launch_pp_rows(const GemmArgs& a, int grid, hipStream_t s)
 {
@@ -1067,10 +1088,14 @@ static int launch_pp_rows(const GemmArgs& a, int tiles, hipStream_t s)
 {
     const int cus = device_cu_count();
     AMOE_REQUIRE(cus > 0, AMOE_ERR_LAUNCH, "grouped_gemm: cannot read the number of compute units");
-    // (a multiple of 8: every XCD then runs the same number of workgroups)
-    const int grid = ((tiles < cus ? tiles : cus) + 7) & ~7;
-    if (a.stream_from) return launch_pp_rows<B_KC, EPI, ACT, true>(a, grid, s);
-    return launch_pp_rows<B_KC, EPI, ACT, false>(a, grid, s);
+    // (a multiple of 8: every XCD then runs the same number of workgroups; a tile can become four pieces)
+    const int grid = ((tiles < (cus + 3) / 4 ? 4 * tiles : cus) + 7) & ~7;
+    GemmArgs b = a;
+    b.inv_group = tile_inverse(a.gm * a.n_ntiles);
+    b.inv_n = tile_inverse(a.n_ntiles);
+    b.inv_last = tile_inverse(a.n_ntiles - (a.sn - 1) * a.gn);
+    if (a.stream_from) return launch_pp_rows<B_KC, EPI, ACT, true>(b, grid, s);
+    return launch_pp_rows<B_KC, EPI, ACT, false>(b, grid, s);
 }
 
 // `tiles`: upper bound of the number of tiles
@@ -1117,13 +1142,12 @@ int amoe_pp_wgrad(GemmArgs a, hipStream_t s)
     const int strips = (a.n_ntiles + 7) / 8;
     a.gn = (a.n_ntiles + strips - 1) / strips;
     a.sn = (a.n_ntiles + a.gn - 1) / a.gn;
-    auto inverse = [](int d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; };
     const long long per = (long long)a.n_mt * a.n_ntiles, total = per * a.E;
     AMOE_REQUIRE(total * per < (1ll << 32), AMOE_ERR_UNSUPPORTED, "grouped_gemm_wgrad: too many tiles");
-    a.inv_super = inverse((int)per);
-    a.inv_sn = inverse(a.n_mt * a.gn);
-    a.inv_gn = inverse(a.gn);
-    a.inv_gm = inverse(a.n_ntiles - (a.sn - 1) * a.gn);
+    a.inv_super = tile_inverse((int)per);
+    a.inv_sn = tile_inverse(a.n_mt * a.gn);
+    a.inv_gn = tile_inverse(a.gn);
+    a.inv_gm = tile_inverse(a.n_ntiles - (a.sn - 1) * a.gn);
     // Tiles a workgroup: all that fall to it from 11 K tiles an expert on (fewer workgroups then only fill their pipelines again: 1024
     // rows of 128 experts of 2048 x 768, a training step 3.80 ms, with two tiles each 3.92), below that two, so that the other stream's
     // workgroups get compute units between them.  Steps with one / two / four / all, ms, against shape 5 (to 256 rows) or all:
