@@ -74,7 +74,7 @@ struct GemmArgs {
     int f16;         // host side only: the operands are float16 (launch the f16 instance), else bf16
 };
 
-enum { EPI_STORE = 0, EPI_GATED = 1, EPI_GATED_BWD = 2, EPI_PART = 3 };
+enum { EPI_STORE = 0, EPI_GATED = 1, EPI_GATED_BWD = 2, EPI_PART = 3, EPI_STORE_PAST = 4 /* gemm_pp.hip: past the caches */ };
 
 namespace {
 

@@ -307,16 +307,17 @@ def main():
     rows = f"grouped_gemm_rows_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_rows_bf16_kernel<"
     wgrad = f"grouped_gemm_wgrad_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_wgrad_bf16_kernel<"
     end = ">" if c else ", false>"   # (every workload here has far more than a tile of rows per expert)
+    plain = lambda n: 4 if c == 0 and 2 * R * n >= 128 << 20 else 0   # epilogue: plain, or plain and past the caches
     wend = ">" if c else ", true>"   # (and gradients that the L2s do not hold)
     gathered = token_of is not None
     sym = {
         # grouped_gemm_pp_rows_bf16_kernel<B K-contiguous, epilogue, activation, B past the caches>; other tile shapes:
         # grouped_gemm_rows_bf16_kernel<BM, BN, waves along M, waves along N, B K-contiguous, epilogue, activation>
         "gemm_gateup_act_fwd": f"{rows}false, 1, 0{end}",
-        "gemm_down_fwd": f"{rows}false, 0, 0{end}",
-        "gemm_dgrad_down": f"{rows}true, 0, 0{end}",
+        "gemm_down_fwd": f"{rows}false, {plain(H)}, 0{end}",
+        "gemm_dgrad_down": f"{rows}true, {plain(I)}, 0{end}",
         "gemm_dgrad_down_gated_bwd": f"{rows}true, 2, 0{end}",
-        "gemm_dgrad_gateup": f"{rows}true, 0, 0{end}",
+        "gemm_dgrad_gateup": f"{rows}true, {plain(H)}, 0{end}",
         # grouped_gemm_pp_wgrad_bf16_kernel<gathered operand, stored past the caches>; other tile shapes:
         # grouped_gemm_wgrad_bf16_kernel<BM, BN, waves along M, waves along N, gathered operand>
         "gemm_wgrad_down": f"{wgrad}{2 if gathered else 0}{wend}",

@@ -13,6 +13,7 @@ CASES = {
     "one_round": ([256] * 16, 96, 4096),                         # 16 x 16 = 256
     "few_left": ([257, 250, 255] * 8, 64, 2200),                 # 32 x 9, super-columns of 5 and 4, 32 left, in quarters
     "many_left": ([200, 256, 0, 7] * 13, 64, 2816),              # 39 x 11, super-columns of 6 and 5, 173 left
+    "past_the_caches": ([1000, 31, 2000, 0, 5200], 64, 8200),    # an output of 128 MiB and more is stored past the caches
     "short_group": ([256, 31] * 19 + [250], 64, 1904),           # 39 x 8, groups of 4
 }
 
