@@ -1,5 +1,5 @@
 // Deterministic token-to-expert permutation plan: a stable counting sort of the k-major
-// flattened assignment vector, in one launch of one block for few rows and otherwise in three launches
+// flattened assignment vector, in one launch up to 65536 rows and otherwise in three launches
 //   1. per-chunk expert histograms (LDS counters),
 //   2. a one-block scan over chunks and experts (counts, offsets, per-chunk bases),
 //   3. per-chunk ranking in ascending slot order (ballot match inside a wavefront, LDS
@@ -13,14 +13,20 @@
 namespace {
 
 constexpr int kChunk = 512;         // flat slots per wavefront
-constexpr int kWavesPerBlock = 4;   // independent chunks per block
+constexpr int kWavesPerBlock = 1;   // independent chunks per block (a compute unit takes a cycle for every scattered element it stores)
 
-__device__ __forceinline__ int load_expert(const int32_t* assign, int f, int T, int K, int E)
+constexpr int kSteps = kChunk / AMOE_WAVE;
+
+// place of flat slot f in the [T,K] arrays; the token is `t`
+__device__ __forceinline__ int place_of(int f, int T, int K, int& t)
 {
-    int k = f / T;
-    int t = f - k * T;
-    int e = assign[(size_t)t * K + k];
-    return min(max(e, 0), E - 1);  // memory safety for caller-supplied assignments
+    const int k = f / T;
+    t = f - k * T;
+    return t * K + k;
+}
+__device__ __forceinline__ int load_expert(const int32_t* assign, int place, int E)
+{
+    return min(max(assign[place], 0), E - 1);  // memory safety for caller-supplied assignments
 }
 
 __global__ void __launch_bounds__(kWavesPerBlock * AMOE_WAVE)
@@ -33,9 +39,16 @@ permute_hist_kernel(const int32_t* __restrict__ assign, int T, int K, int E, int
     for (int e = lane; e < E; e += 64) cnt[w][e] = 0;
     __syncthreads();
     if (c < n_chunks) {
-        const int f0 = c * kChunk;
-        const int f1 = min(f0 + kChunk, R);
-        for (int f = f0 + lane; f < f1; f += 64) atomicAdd(&cnt[w][load_expert(assign, f, T, K, E)], 1);
+        int e[kSteps];
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i) {
+            const int f = c * kChunk + i * 64 + lane;
+            int t;
+            e[i] = f < R ? load_expert(assign, place_of(f, T, K, t), E) : -1;
+        }
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i)
+            if (e[i] >= 0) atomicAdd(&cnt[w][e[i]], 1);
     }
     __syncthreads();
     if (c < n_chunks)
@@ -84,13 +97,13 @@ __device__ __forceinline__ int rank_of(int e, bool valid, int lane, bool* last)
 // One block of 1024 threads: with EP = E rounded up to a power of two, thread t works for
 // expert t % EP on the (t / EP)-th slice of the chunks, so that the walk over chunks (the only
 // sequential part) is 1024 / EP ways parallel and every load is coalesced over experts.  A
-// thread holds its slice of counts in registers between the two passes (kScanBatch at a time):
+// thread holds its slice of counts in registers (kScanBatch at a time; one batch from pass to pass):
 // the exclusive bases overwrite the counts in place, and loads issued after such a store cannot
 // be moved ahead of it, which would turn the second pass into a chain of dependent round trips.
 // When tile_map is non-null the block also writes the row-grouped GEMMs' tile map (one int4
 // {expert, first row, end row, 0} per `bm`-row tile, {-1,0,0,0} past the last) and its tile count.
 constexpr int kScanThreads = 1024;
-constexpr int kScanBatch = 16;
+constexpr int kScanBatch = 32;
 
 __global__ void __launch_bounds__(kScanThreads)
 permute_scan_kernel(int32_t* __restrict__ chunk_counts /* in: counts, out: exclusive base inside expert */,
@@ -106,10 +119,9 @@ permute_scan_kernel(int32_t* __restrict__ chunk_counts /* in: counts, out: exclu
     const int G = kScanThreads / EP;
     const int per = (n_chunks + G - 1) / G;
     const int c0 = min(g * per, n_chunks), c1 = min(c0 + per, n_chunks);
-    int sum = 0;
+    int sum = 0, v[kScanBatch];
     if (e < E)
         for (int cb = c0; cb < c1; cb += kScanBatch) {
-            int v[kScanBatch];
 #pragma unroll
             for (int i = 0; i < kScanBatch; ++i) v[i] = cb + i < c1 ? chunk_counts[(size_t)(cb + i) * E + e] : 0;
 #pragma unroll
@@ -125,9 +137,10 @@ permute_scan_kernel(int32_t* __restrict__ chunk_counts /* in: counts, out: exclu
     }
     if (e < E)
         for (int cb = c0; cb < c1; cb += kScanBatch) {
-            int v[kScanBatch];
+            if (per > kScanBatch) {
 #pragma unroll
-            for (int i = 0; i < kScanBatch; ++i) v[i] = cb + i < c1 ? chunk_counts[(size_t)(cb + i) * E + e] : 0;
+                for (int i = 0; i < kScanBatch; ++i) v[i] = cb + i < c1 ? chunk_counts[(size_t)(cb + i) * E + e] : 0;
+            }
 #pragma unroll
             for (int i = 0; i < kScanBatch; ++i) {
                 if (cb + i < c1) chunk_counts[(size_t)(cb + i) * E + e] = run;
@@ -155,14 +168,26 @@ permute_scatter_kernel(const int32_t* __restrict__ assign, int T, int K, int E, 
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int c = blockIdx.x * kWavesPerBlock + w;
     if (c >= n_chunks) return;  // no block-wide barrier below: every wavefront is independent
+    // (all that a chunk reads is requested before the chain of its steps, and a block is one wavefront: 131072 rows 13.6 -> 9.8 us)
+    int ex[kSteps], tok[kSteps], at[kSteps];
+    float sc[kSteps];
+#pragma unroll
+    for (int i = 0; i < kSteps; ++i) {
+        const int f = c * kChunk + i * 64 + lane;
+        ex[i] = -1;
+        sc[i] = 0.f;
+        if (f < R) {
+            at[i] = place_of(f, T, K, tok[i]);
+            ex[i] = load_expert(assign, at[i], E);
+            if (scores_perm) sc[i] = scores[at[i]];
+        }
+    }
     for (int e = lane; e < E; e += 64) run[w][e] = offsets[e] + chunk_base[(size_t)c * E + e];
     __builtin_amdgcn_wave_barrier();
-    const int f0 = c * kChunk;
-    const int f1 = min(f0 + kChunk, R);
-    for (int fb = f0; fb < f1; fb += 64) {
-        const int f = fb + lane;
-        const bool valid = f < f1;
-        const int e = valid ? load_expert(assign, f, T, K, E) : 0;
+#pragma unroll
+    for (int i = 0; i < kSteps; ++i) {
+        const bool valid = ex[i] >= 0;
+        const int e = valid ? ex[i] : 0;
         bool last;
         const int rank = rank_of(e, valid, lane, &last);
         int row = 0;
@@ -172,23 +197,28 @@ permute_scatter_kernel(const int32_t* __restrict__ assign, int T, int K, int E, 
         if (last) run[w][e] = row + 1;
         __builtin_amdgcn_wave_barrier();
         if (valid) {
-            int k = f / T;
-            int t = f - k * T;
-            token_of[row] = t;
-            slot_of[row] = f;
-            row_of[(size_t)t * K + k] = row;
-            if (scores_perm) scores_perm[row] = scores[(size_t)t * K + k];
+            token_of[row] = tok[i];
+            slot_of[row] = c * kChunk + i * 64 + lane;
+            row_of[at[i]] = row;
+            if (scores_perm) scores_perm[row] = sc[i];
         }
     }
 }
 
-// The whole plan in one block, for up to kSmallRows routed rows: the three kernels above are 2-8 us each there, most
-// of it their launches and the chain of memory round trips between them (one token 8.7 us, 512 rows 17 us).  Sixteen
-// wavefronts take consecutive chunks of the slots, so an expert's rows come in ascending slot order as above; the
-// chunk counts stay in LDS and the experts of a wavefront's slots in its registers.  One MI355X:
-// one token of 8 experts 8.7 -> 4.8 us, 4096 rows 20 -> 11 us, and two launches fewer for the host.
-constexpr int kSmallWaves = 16, kSmallSteps = 8;
-constexpr int kSmallRows = kSmallWaves * kSmallSteps * AMOE_WAVE;
+// The whole plan in one launch, for up to kOneLaunchRows routed rows: the three kernels above are 5-8 us each there, most
+// of it their launches and the chain of memory round trips between them.  A block of sixteen wavefronts owns 1024 consecutive
+// slots, one to a thread, and counts ALL slots by itself, told apart as before its own, its own by wavefront, and after them:
+// that gives every wavefront the bases of its rows without a word between blocks.  (The slots are counted in the order in which
+// they are stored, 16 bytes a lane.)  Up to 8192 rows one block did all of it before, a store of a scattered element a cycle.
+// Launches back to back, us, before / so: 512 rows of 128 experts 5.1 / 4.3, 4072 14.5 / 7.3, 8000 24.9 / 7.7, 24008 18.6 / 10.3,
+// 65536 20.0 / 16.3, all of them to 8 experts 18.9 / 15.6, 4096 rows of 8 experts 9.5 / 6.3; with 131072 rows, which each of 128
+// blocks would count, 27 / 30.
+constexpr int kSmallWaves = 16;
+constexpr int kSmallRows = kSmallWaves * AMOE_WAVE;
+constexpr int kOneLaunchRows = 1 << 16;
+// Lanes add to one of 8 copies of the counters, in banks of their own: where all slots go to one expert they would else wait for
+// each other (65536 slots 59 us, so 15).
+constexpr int kCopies = 8, kCopyStride = AMOE_MAX_EXPERTS + 1;
 
 struct PlanOut {
     int32_t *counts, *offsets, *token_of, *slot_of, *row_of;
@@ -198,77 +228,110 @@ struct PlanOut {
     int bm, max_mtiles;
 };
 
-// expert_of(flat slot), score_of(token, k)
-template <typename ExpertOf, typename ScoreOf>
-__device__ __forceinline__ void plan_in_block(ExpertOf expert_of, ScoreOf score_of, int T, int K, int E, int R,
-                                              int steps /* of 64 slots per wavefront */, const PlanOut& o)
+// count_others(before, after): adds the slots that are not this block's.  e, tok, at, score: this thread's slot, its expert
+// (-1: none), token, place t K + k and score
+template <typename CountOthers>
+__device__ __forceinline__ void plan_in_block(CountOthers count_others, int e, int slot, int tok, int at, float score, int E, const PlanOut& o)
 {
     __shared__ int32_t run[kSmallWaves][AMOE_MAX_EXPERTS];
+    __shared__ int32_t before[kCopies * kCopyStride], after[kCopies * kCopyStride];
     __shared__ int32_t tot[AMOE_MAX_EXPERTS + 1];
     __shared__ int32_t tstart[AMOE_MAX_EXPERTS + 1];
     const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-    const int f0 = w * steps * AMOE_WAVE + lane;
-    int ex[kSmallSteps];
-#pragma unroll
-    for (int i = 0; i < kSmallSteps; ++i) {
-        const int f = f0 + i * AMOE_WAVE;
-        ex[i] = i < steps && f < R ? expert_of(f) : -1;
-    }
-    for (int e = lane; e < E; e += AMOE_WAVE) run[w][e] = 0;
+    const bool valid = e >= 0, first = blockIdx.x == 0, alone = gridDim.x == 1;
+    for (int i = lane; i < E; i += AMOE_WAVE) run[w][i] = 0;
+    if (!alone)
+        for (int i = t; i < kCopies * kCopyStride; i += kSmallRows) before[i] = after[i] = 0;
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kSmallSteps; ++i)
-        if (ex[i] >= 0) atomicAdd(&run[w][ex[i]], 1);
+    if (valid) atomicAdd(&run[w][e], 1);
+    if (!alone) count_others(before, after);
     __syncthreads();
     if (t < AMOE_MAX_EXPERTS) {
         int sum = 0;
         if (t < E) {
-            // counts of the chunks -> exclusive bases inside the expert
+            // counts of the wavefronts -> exclusive bases inside the expert
+            int rest = 0;
+            if (!alone) {
+#pragma unroll
+                for (int c = 0; c < kCopies; ++c) {
+                    sum += before[c * kCopyStride + t];
+                    rest += after[c * kCopyStride + t];
+                }
+            }
 #pragma unroll
             for (int c = 0; c < kSmallWaves; ++c) {
                 const int v = run[c][t];
                 run[c][t] = sum;
                 sum += v;
             }
-            o.counts[t] = sum;
+            sum += rest;
+            if (first) o.counts[t] = sum;
         }
         tot[t] = sum;
     }
     __syncthreads();
     if (t < AMOE_WAVE) scan_row_counts(tot, t);
     __syncthreads();
-    if (t < E) o.offsets[t + 1] = tot[t];
-    if (t == 0) o.offsets[0] = 0;
-#pragma unroll
-    for (int i = 0; i < kSmallSteps; ++i) {
-        if (i >= steps) break;
-        const bool valid = ex[i] >= 0;
-        const int e = valid ? ex[i] : 0;
-        bool last;
-        const int rank = rank_of(e, valid, lane, &last);
-        int in_expert = 0;
-        if (valid) in_expert = run[w][e] + rank;
-        __builtin_amdgcn_wave_barrier();
-        if (last) run[w][e] = in_expert + 1;
-        __builtin_amdgcn_wave_barrier();
-        if (valid) {
-            const int f = f0 + i * AMOE_WAVE;
-            const int k = f / T, tok = f - k * T;
-            const int row = in_expert + (e ? tot[e - 1] : 0);
-            o.token_of[row] = tok;
-            o.slot_of[row] = f;
-            o.row_of[(size_t)tok * K + k] = row;
-            if (o.scores_perm) o.scores_perm[row] = score_of(tok, k);
-        }
+    if (first) {
+        if (t < E) o.offsets[t + 1] = tot[t];
+        if (t == 0) o.offsets[0] = 0;
     }
-    if (o.tile_map) amoe_emit_tile_map<kSmallWaves * AMOE_WAVE>(tot, 0, E, o.bm, o.tile_map, o.n_mtiles, o.max_mtiles, tstart);
+    bool last;
+    const int rank = rank_of(valid ? e : 0, valid, lane, &last);
+    if (valid) {
+        const int row = run[w][e] + rank + (e ? tot[e - 1] : 0);
+        o.token_of[row] = tok;
+        o.slot_of[row] = slot;
+        o.row_of[at] = row;
+        if (o.scores_perm) o.scores_perm[row] = score;
+    }
+    if (first && o.tile_map) amoe_emit_tile_map<kSmallWaves * AMOE_WAVE>(tot, 0, E, o.bm, o.tile_map, o.n_mtiles, o.max_mtiles, tstart);
 }
 
+// inv_k: 2^32 / K rounded up (0 for K = 1); VEC: assign lies on 16 bytes
+template <bool VEC>
 __global__ void __launch_bounds__(kSmallWaves * AMOE_WAVE)
-permute_small_kernel(const int32_t* __restrict__ assign, int T, int K, int E, int R, int steps, const float* __restrict__ scores, PlanOut o)
+permute_small_kernel(const int32_t* __restrict__ assign, int T, int K, uint32_t inv_k, int E, int R, const float* __restrict__ scores, PlanOut o)
 {
-    plan_in_block([&](int f) { return load_expert(assign, f, T, K, E); }, [&](int t, int k) { return scores[(size_t)t * K + k]; }, T, K, E, R,
-                  steps, o);
+    const int lo = blockIdx.x * kSmallRows, hi = lo + kSmallRows, slot = lo + threadIdx.x;
+    int e = -1, tok = 0, at = 0;
+    float score = 0.f;
+    if (slot < R) {
+        at = place_of(slot, T, K, tok);
+        e = load_expert(assign, at, E);
+        if (o.scores_perm) score = scores[at];
+    }
+    auto count_others = [&](int32_t* before, int32_t* after) {
+        const int copy = threadIdx.x % kCopies * kCopyStride;
+        auto count = [&](int place, int expert) {
+            const int token = inv_k ? (int)(((uint64_t)(uint32_t)place * inv_k) >> 32) : place;
+            const int f = (place - token * K) * T + token;
+            if (f < lo || f >= hi) atomicAdd((f < lo ? before : after) + copy + min(max(expert, 0), E - 1), 1);
+        };
+        constexpr int W = VEC ? 4 : 1, BATCH = VEC ? 4 : 8;
+        typedef int32_t vec_t __attribute__((ext_vector_type(W)));
+        for (int p0 = threadIdx.x * W; p0 < R; p0 += kSmallRows * W * BATCH) {
+            int32_t v[BATCH][W];
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i) {
+                const int p = p0 + i * kSmallRows * W;
+                if (p + W <= R) {
+                    const vec_t q = *reinterpret_cast<const vec_t*>(assign + p);
+#pragma unroll
+                    for (int j = 0; j < W; ++j) v[i][j] = q[j];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < W; ++j) v[i][j] = p + j < R ? assign[p + j] : 0;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i)
+#pragma unroll
+                for (int j = 0; j < W; ++j)
+                    if (p0 + i * kSmallRows * W + j < R) count(p0 + i * kSmallRows * W + j, v[i][j]);
+        }
+    };
+    plan_in_block(count_others, e, slot, tok, at, score, E, o);
 }
 
 // Softmax, top-k and the plan of at most one token per wavefront of the block: the selection reaches the plan through LDS.
@@ -278,8 +341,8 @@ __global__ void __launch_bounds__(kSmallWaves * AMOE_WAVE)
 route_small_kernel(const T* __restrict__ logits, int n_tokens, int E, int K, int normalize, float* __restrict__ probs,
                    int32_t* __restrict__ topk_idx, float* __restrict__ scores, PlanOut o)
 {
-    __shared__ int32_t sel[kSmallWaves][AMOE_MAX_TOPK];
-    __shared__ float sc[kSmallWaves][AMOE_MAX_TOPK];
+    __shared__ int32_t sel[kSmallWaves * AMOE_MAX_TOPK];    // [token][K]
+    __shared__ float sc[kSmallWaves * AMOE_MAX_TOPK];
     const int lane = threadIdx.x & 63, t = threadIdx.x >> 6;
     if (t < n_tokens) {
         int e;
@@ -288,18 +351,16 @@ route_small_kernel(const T* __restrict__ logits, int n_tokens, int E, int K, int
         if (lane < K) {
             topk_idx[(size_t)t * K + lane] = e;
             scores[(size_t)t * K + lane] = s;
-            sel[t][lane] = min(max(e, 0), E - 1);
-            sc[t][lane] = s;
+            sel[t * K + lane] = min(max(e, 0), E - 1);
+            sc[t * K + lane] = s;
         }
     }
     __syncthreads();
-    const int R = n_tokens * K;
-    auto expert_of = [&](int f) {
-        const int k = f / n_tokens;
-        return sel[f - k * n_tokens][k];
-    };
-    plan_in_block(expert_of, [&](int tok, int k) { return sc[tok][k]; }, n_tokens, K, E, R,
-                  (R + kSmallWaves * AMOE_WAVE - 1) / (kSmallWaves * AMOE_WAVE), o);
+    const int slot = threadIdx.x;
+    int tok = 0, at = 0;
+    const bool valid = slot < n_tokens * K;        // (16 tokens of 16 at most)
+    if (valid) at = place_of(slot, n_tokens, K, tok);
+    plan_in_block([](int32_t*, int32_t*) {}, valid ? sel[at] : -1, slot, tok, at, valid ? sc[at] : 0.f, E, o);
 }
 
 }  // namespace
@@ -333,10 +394,12 @@ static int launch_plan(const int32_t* assign, const float* scores, int T, int K,
                        int max_mtiles = 0)
 {
     const int R = T * K;
-    if (R <= kSmallRows) {
-        const int steps = (R + kSmallWaves * AMOE_WAVE - 1) / (kSmallWaves * AMOE_WAVE);
-        hipLaunchKernelGGL(permute_small_kernel, dim3(1), dim3(kSmallWaves * AMOE_WAVE), 0, s, assign, T, K, E, R, steps, scores,
-                           PlanOut{counts, offsets, token_of, slot_of, row_of, scores_perm, tile_map, n_mtiles, bm, max_mtiles});
+    if (R <= kOneLaunchRows) {
+        const dim3 grid((R + kSmallRows - 1) / kSmallRows), block(kSmallRows);
+        const uint32_t inv_k = K > 1 ? (uint32_t)(((1ull << 32) + K - 1) / K) : 0u;      // (exact: R K < 2^32)
+        const PlanOut o{counts, offsets, token_of, slot_of, row_of, scores_perm, tile_map, n_mtiles, bm, max_mtiles};
+        if (((uintptr_t)assign & 15) == 0) hipLaunchKernelGGL(permute_small_kernel<true>, grid, block, 0, s, assign, T, K, inv_k, E, R, scores, o);
+        else hipLaunchKernelGGL(permute_small_kernel<false>, grid, block, 0, s, assign, T, K, inv_k, E, R, scores, o);
         return amoe_check_launch("permute_plan");
     }
     const int n_chunks = permute_chunks(R);
