@@ -68,6 +68,13 @@ __device__ __forceinline__ void pp_advance(srd_t& d, uint32_t bytes)
     d[1] = (uint32_t)(b >> 32);
 }
 
+__device__ __forceinline__ void pp_go_back(srd_t& d, uint32_t bytes)
+{
+    const uint64_t b = (((uint64_t)d[1] << 32) | d[0]) - bytes;
+    d[0] = (uint32_t)b;
+    d[1] = (uint32_t)(b >> 32);
+}
+
 template <int N>
 __device__ __forceinline__ void pp_vmwait()
 {

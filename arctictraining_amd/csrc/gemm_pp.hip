@@ -73,6 +73,11 @@ __device__ __forceinline__ void pp_rows_body()
     // fewer in some (the launch sees to it that there are four at least)
     const int KT = PART ? divide(KT_all + pp_args().splits - 1, pp_args().inv_splits) : max(4, KT_all);
     const bool ragged_k = PART || Kd < KT * PP_BK;
+    // B^T whose rows lie 4, 8 or 12 KB apart (launch_pp_rows): the 128 bytes of a K tile of all rows are in a few of the memory's
+    // channels, and all workgroups ask for the same K tile at about the same time.  Expert e's reduction starts at K tile 5 e and goes
+    // around, so that those in flight together are spread; one expert's tiles start together and share what they load.
+    constexpr bool TURNED = B_KC && !PART;
+    const int first_step = TURNED ? pp_args().first_step : 0;
     struct Part { int i, k0, kd; };                                // number, first k and length
     auto part_of = [&](int& nt) -> Part {                          // N tile of all parts -> of its part
         if constexpr (PART) {
@@ -83,6 +88,10 @@ __device__ __forceinline__ void pp_rows_body()
             return {i, t0 * PP_BK, min(t1 * PP_BK, Kd) - t0 * PP_BK};
         }
         return {0, 0, Kd};
+    };
+    auto first_k_of = [&](int e) -> int {                          // (K tile)
+        const int k = first_step * e;
+        return k - divide(k, pp_args().inv_kt) * KT;
     };
 
     // ------------------------------------------------------------ this workgroup's tiles
@@ -186,7 +195,7 @@ __device__ __forceinline__ void pp_rows_body()
                 aoff[a][j] = row < mend && k < Kd ? ((uint32_t)gr * (uint32_t)lda + k) * 2u : PP_NOWHERE;
             }
         ad = pp_srd(A);
-        if constexpr (PART) pp_advance(ad, (uint32_t)k0 * 2u);
+        if constexpr (PART || TURNED) pp_advance(ad, (uint32_t)k0 * 2u);
     };
     auto plan_b = [&](const bf16_t* B, int n0, int k0) {
         const int th = pp_here(tid);
@@ -196,7 +205,7 @@ __device__ __forceinline__ void pp_rows_body()
         bd = pp_srd(B);
         if (STREAM) stream_b = stream_n;
         // (an expert's matrix is below 4 GiB, or the call is refused: no offset in it wraps)
-        if constexpr (PART) pp_advance(bd, B_KC ? (uint32_t)k0 * 2u : (uint32_t)k0 * ((uint32_t)ldb * 2u));
+        if constexpr (PART || TURNED) pp_advance(bd, B_KC ? (uint32_t)k0 * 2u : (uint32_t)k0 * ((uint32_t)ldb * 2u));
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
@@ -236,10 +245,16 @@ __device__ __forceinline__ void pp_rows_body()
             pp_dma16<(2 + b) * PP_HALF + 8192u>(bd, boff[b][1], fill);
         }
     };
+    int to_wrap = 0;                     // K tiles of the tile being loaded until its last one
     auto next_k = [&]() {
         fill ^= PP_STAGE;
         pp_advance(ad, PP_BK * 2);
         pp_advance(bd, bstep);
+        if constexpr (TURNED) {
+            const bool wrap = --to_wrap == 0;
+            pp_go_back(ad, wrap ? (uint32_t)Kd * 2u : 0u);
+            pp_go_back(bd, wrap ? (uint32_t)KT * bstep : 0u);
+        }
     };
 
     // ------------------------------------------------------------ fragments
@@ -324,6 +339,10 @@ __device__ __forceinline__ void pp_rows_body()
         have_n = next_tile(tm_n, nt_n);
         if (!have_n) tm_n = make_int4(0, 0, 0, 0);
         part = part_of(nt);
+        if constexpr (TURNED) {
+            to_wrap = KT - first_k_of(tm.x);
+            part.k0 = (KT - to_wrap) * PP_BK;
+        }
         n0 = nt * PP_BN;
         plan_a(m0, mend, pp_args().a_row_map, part.k0);
         plan_b(expert_b(tm), n0, part.k0);
@@ -545,6 +564,7 @@ __device__ __forceinline__ void pp_rows_body()
             // the next tile's weights; which tile follows it, and its entry of the tile map
             b_n = expert_b(tm_n);
             part_n = part_of(nt_n);
+            if constexpr (TURNED) part_n.k0 = first_k_of(tm_n.x) * PP_BK;
             have_nn = have_n && next_tile(tm_nn, nt_nn);
             if (!have_nn) tm_nn = make_int4(0, 0, 0, 0);
         }
@@ -566,6 +586,7 @@ __device__ __forceinline__ void pp_rows_body()
             read_a(I1{}, N_);
             if (turn) {
                 plan_a(tm_n.y, tm_n.z, nullptr, have_n ? part_n.k0 : 0);
+                if constexpr (TURNED) to_wrap = KT - part_n.k0 / PP_BK;
             }
             dma_a(I0{});
             pp_vmwait<10>();
@@ -1132,6 +1153,13 @@ static int launch_pp_rows(const GemmArgs& a, int tiles, hipStream_t s)
     GemmArgs b = a;
     b.inv_group = tile_inverse(a.gm * a.n_ntiles);
     b.inv_n = tile_inverse(a.n_ntiles);
+    // Where expert e's reduction starts (see first_step in the kernel), 128 experts of N = 2048, 32 rows each, us, at 0 / at 5 e: K = 2048
+    // 240 / 188, 4096 433 / 355; 16 of N = 4096, 24 rows: K = 4096 123 / 92, 6144 153 / 135; 64 of N = 2048, 300 rows: K = 2048 199 / 179.
+    // Other strides have no such channels, and lose what neighbours read of one memory page: K = 1984 182 / 187, 4160 351 / 366, 8192 170 /
+    // 180, 3072 276 / 280.  From 512 rows an expert on the products are not bound by the reading (600 rows 219 / 222).  With B not
+    // transposed, read in rows of 512 bytes, K = 2048 180 / 183.
+    b.first_step = B_KC && a.Kd % 2048 == 0 && a.Kd <= 6144 && a.M <= 512ll * a.E ? 5 : 0;
+    b.inv_kt = tile_inverse(a.Kd / PP_BK);
     b.inv_last = tile_inverse(a.n_ntiles - (a.sn - 1) * a.gn);
     if (a.stream_from) return launch_pp_rows<B_KC, EPI, ACT, true>(b, grid, s);
     return launch_pp_rows<B_KC, EPI, ACT, false>(b, grid, s);

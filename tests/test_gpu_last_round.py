@@ -14,6 +14,8 @@ CASES = {
     "few_left": ([257, 250, 255] * 8, 64, 2200),                 # 32 x 9, super-columns of 5 and 4, 32 left, in quarters
     "many_left": ([200, 256, 0, 7] * 13, 64, 2816),              # 39 x 11, super-columns of 6 and 5, 173 left
     "past_the_caches": ([1000, 31, 2000, 0, 5200], 64, 8200),    # an output of 128 MiB and more is stored past the caches
+    "turned_2048": ([200, 31, 0, 256, 257, 90], 2048, 264),      # reductions that start at another K tile for every expert (B^T)
+    "turned_6144": ([40, 300] * 4, 6144, 72),
     "short_group": ([256, 31] * 19 + [250], 64, 1904),           # 39 x 8, groups of 4
 }
 
