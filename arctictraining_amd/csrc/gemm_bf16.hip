@@ -1668,13 +1668,13 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
     // tiles, the kernel with 64-bit addresses runs.
     const long long per = (long long)a.n_mt * a.n_ntiles;
     if (tile_cfg == 0) {
-        // Up to 128 rows per expert the product is bound by the gradients' stores: gemm_short.hip, where its 32-bit tile
-        // numbers reach (with a fourth of these tiles' size).  It and shape 5 inside a training step: 812 against 905 us at 32
-        // rows, 545 against 572 at 111, 334 against 363 at 136 (and the same without the second stream), 764 against 710 at 250.
-        // Beyond, gemm_pp.hip, whose tiles are never done in less than three K tiles.  The line: with 102 rows an expert it and
-        // gemm_short.hip are within 1.5 % of each other, either way (steps of 27 experts of 1024 x 9184, 1.34 against 1.36 ms, 97 of
-        // 1856 x 1920, 1.88 against 1.86).
-        if (R <= 128ll * E && offsets32 && 16 * per * per * E < (1ll << 32)) return amoe_short_wgrad(a, s);
+        // Up to 104 rows per expert the product is bound by the gradients' stores: gemm_short.hip, where its 32-bit tile
+        // numbers reach (with a fourth of these tiles' size).  Beyond, gemm_pp.hip, whose tiles are never done in less than three
+        // K tiles.  Alone they meet at 80 rows; inside a step, where the short kernel's workgroups leave more to the other stream's, at
+        // 105 (short / pp, us): 64 experts of 2048 x 1408, 81 rows 802 / 823, 100 819 / 843, 128 900 / 893; 128 of 2048 x 768, 88 rows
+        // 867 / 902, 112 977 / 934, 128 1036 / 963; 8 of 4096 x 7168, 100 rows 948 / 966; 97 of 1856 x 960, 105 rows 913 / 914; 27 of
+        // 1024 x 4608, 100 rows 669 / 641.
+        if (R <= 104ll * E && offsets32 && 16 * per * per * E < (1ll << 32)) return amoe_short_wgrad(a, s);
         if (offsets32 && per * per * E < (1ll << 32)) return amoe_pp_wgrad(a, s);
         tile_cfg = 5;
     }

@@ -9,15 +9,14 @@
 // the weights that the kernels beside and behind this one read.  With ordinary stores 32 rows of 128 experts of 2048 x 768 took
 // 112 us for down's gradient, with these 75.
 //
-// bf16, inside a backward pass, gate_up's and down's gradient, us, against 256 x 256 tiles with ordinary 4-byte stores, and
-// the whole training step:
-//   128 experts of 2048 x  768,  32 rows  198 -> 161,  95 -> 82,   905 -> 812
-//   146 experts of  384 x 3104,   2 rows  201 -> 130,  97 -> 68,   866 -> 773
-//    51 experts of 2848 x 1472,  23 rows  215 -> 158, 107 -> 80,   978 -> 912
-//   173 experts of 1952 x 1056,  15 rows  373 -> 292, 181 -> 169, 1488 -> 1316   (a sixteenth of the experts with most rows)
-//   114 experts of 3072 x  608,  66 rows  244 -> 217, 131 -> 132, 1117 -> 1031   (the same)
-//    29 experts of 4288 x  672, 111 rows  120 -> 127,  65 -> 70,   572 -> 545
-//    64 experts of 2048 x 1408, 250 rows  369 -> 476, 186 -> 266, 1677 -> 1962   (float16; not taken)
+// Lines are whole: eight lanes store a row's 128 bytes, which the accumulators reach through 1 KB of LDS a wavefront.  Out of a cold
+// cache, bf16, the rows of one operand gathered, us, with 16 bytes of 16 rows an instruction (a request a lane) / so:
+//   128 experts,  32 rows, 2048 x 1536  285 / 173 (4.7 TB/s),  768 x 2048  132 /  90
+//   146 experts,   2 rows,  384 x 6208  142 / 139,            3104 x  384   97 /  70
+//    51 experts,  23 rows, 2848 x 2944  237 / 162 (5.3 TB/s)
+//    64 experts,  60 rows, 1408 x 2048  147 / 105;   8 experts, 100 rows, 4096 x 4096  117 / 93
+// and a training step of 509 tokens of 128 experts of 2048 x 768 751 / 735.  The same step with 256 x 256 tiles and ordinary 4-byte
+// stores took 93 us longer than with the former, 64 experts of 2048 x 1408 with 250 rows (not taken) 285 us less.
 #include "gemm_dma.h"
 #include "gemm_launch.h"
 
@@ -26,17 +25,18 @@ namespace {
 constexpr int SH_THREADS = 320, SH_WGS = 3;      // (workgroups on a compute unit)
 constexpr int SH_BM = 128, SH_BN = 128, SH_BK = 32, SH_NS = 3;
 constexpr uint32_t SH_OPERAND = SH_BM * SH_BK * 2, SH_STAGE = 2 * SH_OPERAND;
+constexpr uint32_t SH_TURN = 1024;               // a wavefront's for its epilogue
 
 // MAPS: 1 = the rows of A, 2 = the rows of B are gathered through a row map
 template <int MAPS, typename ET>
 __device__ __forceinline__ void short_wgrad_body(const GemmArgs& p)
 {
     typedef typename Elem16<ET>::frag_t frag_t;
-    __shared__ __attribute__((aligned(1024))) char smem[SH_NS * SH_STAGE + 64];
+    __shared__ __attribute__((aligned(1024))) char smem[SH_NS * SH_STAGE + 4 * SH_TURN + 64];
     const uint32_t lds = (uint32_t)(uintptr_t)(lptr_t)smem;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr bool A_MAP = MAPS == 1, B_MAP = MAPS == 2;
-    constexpr uint32_t END = SH_NS * SH_STAGE, FLAGS = END;      // per stage: whether it is its tile's last
+    constexpr uint32_t END = SH_NS * SH_STAGE, FLAGS = END + 4 * SH_TURN;      // per stage: whether it is its tile's last
 
     // ------------------------------------------------------------ this workgroup's tiles
     // Tiles are numbered expert by expert, row by row inside one; XCD x (workgroups with blockIdx % 8 == x) works through chunks
@@ -203,25 +203,36 @@ __device__ __forceinline__ void short_wgrad_body(const GemmArgs& p)
             pp_fence();
             at = at + SH_STAGE == END ? 0 : at + SH_STAGE;
         } while (!__builtin_amdgcn_readfirstlane(last));
-        // Lane (lq, l16) holds columns 4 lq .. + 3 of row l16 of each 16 x 16 tile, after the exchange 8 lq .. + 7 of two of them.
+        // Lane (lq, l16) holds columns 4 lq .. + 3 of row l16 of each 16 x 16 tile.  Eight rows of 128 bytes at a time go through LDS
+        // (chunk c of row r at c ^ r), after which eight lanes hold a row's and a store writes whole lines.
         bf16_t* const c = p.C + (long long)t.e * p.strideC + (long long)(t.m0 + wm * 64) * p.ldc + t.n0 + wn * 64;
         const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc(c, (short)0, (int)PP_DROP, 0x00020000);
-        const uint32_t ldc2 = (uint32_t)p.ldc * 2u, off = (uint32_t)l16 * ldc2 + 16u * lq;
-        const int rows = p.M - t.m0 - wm * 64 - l16, cols = p.N - t.n0 - wn * 64 - 8 * lq;
+        const uint32_t ldc2 = (uint32_t)p.ldc * 2u;
+        const int r8 = lane >> 3, c8 = lane & 7;
+        const uint32_t off = 8 * c8 < p.N - t.n0 - wn * 64 ? (uint32_t)r8 * ldc2 + 16u * c8 : PP_DROP;
+        const int rows = p.M - t.m0 - wm * 64 - r8;
+        const uint32_t turn = lds + END + (uint32_t)wave * SH_TURN;
+        const uint32_t wr = turn + (uint32_t)((l16 & 7) * 128 + ((lq >> 1) ^ (l16 & 7)) * 16 + (lq & 1) * 8);
+        const uint32_t rd = turn + (uint32_t)(r8 * 128 + (c8 ^ r8) * 16);
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < 4; ++a) {
+            u32x2_t x[4];
 #pragma unroll
-            for (int b = 0; b < 4; b += 2) {
-                uint32_t x[2], y[2];
+            for (int b = 0; b < 4; ++b) x[b] = u32x2_t{Elem16<ET>::pack2(acc[a][b][0], acc[a][b][1]), Elem16<ET>::pack2(acc[a][b][2], acc[a][b][3])};
+            u32x4_t y[2];
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    x[u] = Elem16<ET>::pack2(acc[a][b][2 * u], acc[a][b][2 * u + 1]);
-                    y[u] = Elem16<ET>::pack2(acc[a][b + 1][2 * u], acc[a][b + 1][2 * u + 1]);
+            for (int h = 0; h < 2; ++h) {
+                if (l16 >> 3 == h) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) *(__attribute__((address_space(3))) u32x2_t*)(uintptr_t)(wr ^ (32u * b)) = x[b];
                 }
-                pp_join(x[0], y[0]);
-                pp_join(x[1], y[1]);
-                pp_store16<true>(d, u32x4_t{x[0], x[1], y[0], y[1]}, a * 16 < rows && b * 16 < cols ? off : PP_DROP, (uint32_t)(a * 16) * ldc2 + b * 32u);
+                pp_lds_turn();
+                y[h] = pp_lds<u32x4_t>(rd);
+                pp_lds_turn();
             }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) pp_store16<true>(d, y[h], a * 16 + h * 8 < rows ? off : PP_DROP, (uint32_t)(a * 16 + h * 8) * ldc2);
+        }
         v = number(q += gq);
     } while (v < total);
 }
