@@ -1304,9 +1304,7 @@ static int set_supertiles(GemmArgs& a, long long m_tiles, long long* grid)
     const long long supers = sm * a.sn;
     *grid = 8 * ((supers + 7) / 8) * a.gm * a.gn;
     auto inverse = [](int d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; };
-    a.inv_gm = inverse(a.gm);
     a.inv_gn = inverse(a.gn);
-    a.inv_sn = inverse(a.sn);
     a.inv_super = inverse(a.gm * a.gn);
     // (n / d by multiplication with these is exact while n d < 2^32; every n here is a tile index)
     AMOE_REQUIRE(*grid < (1ll << 31) / 32 && *grid * a.sn < (1ll << 32), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");

@@ -64,7 +64,8 @@ struct GemmArgs {
     int rows_total;  // weight gradient: length of the row maps; gemm_skinny.hip: rows of B (0: Kd)
     int gm, gn;   // blocks of one XCD work on super-tiles of gm x gn tiles
     int sn;       // super-tiles along N
-    uint32_t inv_gm, inv_gn, inv_sn, inv_super;   // ceil(2^32 / gm), .. gn, sn, gm gn (0 for a divisor of 1)
+    uint32_t inv_gn, inv_super;                   // ceil(2^32 / gn), .. gm gn (0 for a divisor of 1; weight gradients: see their launches)
+    uint32_t inv_gm, inv_sn;                      // weight gradients only
     uint32_t inv_group, inv_n, inv_last, inv_kt;  // gemm_pp.hip, .. gm n_ntiles, n_ntiles, width of the last super-column, Kd / 64
     int first_step;  // gemm_pp.hip: K tile at which the reduction of expert 1 starts, of e times that, modulo Kd / 64 (0: all at the first)
     int max_mtiles;  // rows mode: entries of tile_map (those past the last tile hold expert -1)
