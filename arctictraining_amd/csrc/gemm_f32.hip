@@ -40,7 +40,42 @@ struct GemmArgsF32 {
     int lda, ldb, ldc;
     long long strideB, strideC;
     int E, Kd, M, N, n_ntiles, n_mt;
+    float* inter;              // gated products: [R, N / 2]
+    const float* row_scale;    // null: 1
+    int act;
 };
+
+// Gated products: a vector of C is (gate, up) of two intermediate columns, which leave the epilogue as row_scale up act(gate).
+// With a kernel of its own that read C again and wrote them / so, a forward pass, us: 2048 tokens x 2 of 8 experts of 512 x 1024
+// 147 / 143, 4096 x 2 of 8 of 1024 x 2048 729 / 713, 650 x 6 of 20 of 384 x 160 and a shared one 80 / 75, one token 57 / 54; a
+// training step of the first 388 / 383.
+__device__ __forceinline__ float activate(int act, float g)
+{
+    switch (act) {
+        case AMOE_ACT_SILU: return act_fwd<AMOE_ACT_SILU>(g);
+        case AMOE_ACT_GELU: return act_fwd<AMOE_ACT_GELU>(g);
+        case AMOE_ACT_RELU: return act_fwd<AMOE_ACT_RELU>(g);
+        default: return act_fwd<AMOE_ACT_GPT_OSS>(g);
+    }
+}
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ f32x2_t gated(const GemmArgsF32& p, float s, const f32x4_t& c)
+{
+    return f32x2_t{s * c[1] * activate(p.act, c[0]), s * c[3] * activate(p.act, c[2])};
+}
+__device__ __forceinline__ void store_gated(const GemmArgsF32& p, int row, int col, const f32x4_t& c)
+{
+    *reinterpret_cast<f32x2_t*>(p.inter + (long long)row * (p.N / 2) + col / 2) = gated(p, p.row_scale ? p.row_scale[row] : 1.0f, c);
+}
+// the same of `rows` x `cols` elements of C that this wavefront has written one by one (redo_exact)
+__device__ __forceinline__ void store_gated_again(const GemmArgsF32& p, int m0, int mend, int n0, int rows, int cols)
+{
+    __threadfence();
+    for (int v = threadIdx.x & 63; v < rows * cols / 4; v += 64) {
+        const int row = m0 + v / (cols / 4), col = n0 + v % (cols / 4) * 4;
+        if (row < mend && col < p.N) store_gated(p, row, col, *reinterpret_cast<const f32x4_t*>(p.C + (long long)row * p.ldc + col));
+    }
+}
 
 // The parts are of 2^16 x: of x itself, those of a value below 2^-110 would reach below bfloat16's smallest, 2^-133, which is
 // float32's smallest times 2^16.  A sum of products is 2^32 times what it stands for.  (Results of 2^96 and more overflow
@@ -144,7 +179,7 @@ __device__ __forceinline__ void redo_exact(int rows, int cols, int k_len, FA a_a
 // ------------------------------------------------------------------ row-grouped products
 // Four wavefronts of 32 rows x 64 columns.  Each loads its rows of A straight into registers and splits them there; B is
 // split once for all four and goes through LDS.
-template <bool B_KC, int KG>
+template <bool B_KC, int KG, bool GATED>
 __global__ void __launch_bounds__(NT * KG, 2)
 grouped_gemm_f32_kernel(GemmArgsF32 p)
 {
@@ -274,14 +309,34 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
     // Lane (lq, l16) holds columns 4 lq .. + 3 of row l16 of each 16 x 16 tile.
     bool finite = true;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) {
+        const int row = m0 + i * 16 + l16;
+        const float scale = GATED && p.row_scale ? p.row_scale[min(row, mend - 1)] : 1.0f;
+        f32x2_t h[TN];
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const f32x4_t c = (hi[i][j] + lo[i][j]) * SUM_SCALE;
             finite = finite && finite4(c);
-            const int row = m0 + i * 16 + l16, col = n0 + j * 16 + 4 * lq;
+            const int col = n0 + j * 16 + 4 * lq;
             if (row < mend && col < p.N) *reinterpret_cast<f32x4_t*>(p.C + (long long)row * p.ldc + col) = c;
+            if constexpr (GATED) h[j] = gated(p, scale, c);
         }
+        if constexpr (GATED) {
+            // of tiles j and j + 1 lane quarters 0 and 2 take j's columns, 1 and 3 the other's: 16 bytes a lane, 64 of a row together
+#pragma unroll
+            for (int j = 0; j < TN; j += 2) {
+                f32x4_t x;
+#pragma unroll
+                for (int v = 0; v < 2; ++v) {
+                    const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[j][v]), __float_as_uint(h[j + 1][v]), false, false);
+                    x[v] = __uint_as_float(t[0]);
+                    x[2 + v] = __uint_as_float(t[1]);
+                }
+                const int col = n0 / 2 + (j + (lq & 1)) * 8 + (lq >> 1) * 4;
+                if (row < mend && 2 * col < p.N) *reinterpret_cast<f32x4_t*>(p.inter + (long long)row * (p.N / 2) + col) = x;
+            }
+        }
+    }
     if (!live || !__any(!finite)) return;
     redo_exact(32, BN_ROWS, k_len,
                [&](int i, int k) {
@@ -292,6 +347,7 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
                [&](int i, int j, float c) {
                    if (m0 + i < mend && n0 + j < p.N) p.C[(long long)(m0 + i) * p.ldc + n0 + j] = c;
                });
+    if constexpr (GATED) store_gated_again(p, m0, mend, n0, 32, BN_ROWS);
 }
 
 // The same products where 128 x 64 tiles do not give every compute unit two workgroups: a wavefront on its own issues a
@@ -300,7 +356,7 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
 // sums meet in LDS, in a fixed order.
 constexpr int NW_DEEP = 8;
 
-template <bool B_KC>
+template <bool B_KC, bool GATED>
 __global__ void __launch_bounds__(NW_DEEP * 64, 2)
 grouped_gemm_f32_deep_kernel(GemmArgsF32 p)
 {
@@ -413,7 +469,10 @@ grouped_gemm_f32_deep_kernel(GemmArgsF32 p)
             finite = finite && finite4(c);
             const int l = tid & 63, u = tid >> 6;
             const int row = m0 + i * 16 + (l & 15), col = n0 + (B_KC ? u * 16 + 4 * (l >> 4) : 16 * (l >> 4) + 4 * u);
-            if (row < mend && col < p.N) *reinterpret_cast<f32x4_t*>(p.C + (long long)row * p.ldc + col) = c;
+            if (row < mend && col < p.N) {
+                *reinterpret_cast<f32x4_t*>(p.C + (long long)row * p.ldc + col) = c;
+                if constexpr (GATED) store_gated(p, row, col, c);
+            }
         }
     }
     if (!__syncthreads_or(!finite) || wave) return;
@@ -426,6 +485,7 @@ grouped_gemm_f32_deep_kernel(GemmArgsF32 p)
                [&](int i, int j, float c) {
                    if (m0 + i < mend && n0 + j < p.N) p.C[(long long)(m0 + i) * p.ldc + n0 + j] = c;
                });
+    if constexpr (GATED) store_gated_again(p, m0, mend, n0, 32, 64);
 }
 
 // ------------------------------------------------------------------ weight gradients
@@ -562,22 +622,25 @@ int launch_wgrad(const GemmArgsF32& a, hipStream_t s)
     return a.b_row_map ? launch_wgrad<BM, BN, 2>(a, s) : launch_wgrad<BM, BN, 0>(a, s);
 }
 
-template <bool B_KC>
+template <bool B_KC, bool GATED = false>
 void launch_rows(const GemmArgsF32& a, int grid, int form, hipStream_t s)
 {
-    if (form == 2) hipLaunchKernelGGL((grouped_gemm_f32_deep_kernel<B_KC>), dim3(grid * (BM_ROWS / 32)), dim3(NW_DEEP * 64), 0, s, a);
-    else if (form == 1) hipLaunchKernelGGL((grouped_gemm_f32_kernel<B_KC, 2>), dim3(grid), dim3(NT * 2), 0, s, a);
-    else hipLaunchKernelGGL((grouped_gemm_f32_kernel<B_KC, 1>), dim3(grid), dim3(NT), 0, s, a);
+    if (form == 2) hipLaunchKernelGGL((grouped_gemm_f32_deep_kernel<B_KC, GATED>), dim3(grid * (BM_ROWS / 32)), dim3(NW_DEEP * 64), 0, s, a);
+    else if (form == 1) hipLaunchKernelGGL((grouped_gemm_f32_kernel<B_KC, 2, GATED>), dim3(grid), dim3(NT * 2), 0, s, a);
+    else hipLaunchKernelGGL((grouped_gemm_f32_kernel<B_KC, 1, GATED>), dim3(grid), dim3(NT), 0, s, a);
 }
 
 }  // namespace
 
-// rows mode: C[rows_e, :N] = A[rows_e, :Kred] @ op(B[e]);  b_kc selects B stored [N,Kred]
+// rows mode: C[rows_e, :N] = A[rows_e, :Kred] @ op(B[e]);  b_kc selects B stored [N,Kred]; inter (B as it is only): the gated activation too
 int amoe_f32_rows(const void* A, const int32_t* a_row_map, const void* B, const int32_t* offsets, void* C, int R, int E,
                   int Kred, int N, int ldb, long long strideB, bool b_kc, void* workspace, size_t workspace_bytes,
-                  bool map_ready, hipStream_t s)
+                  bool map_ready, hipStream_t s, float* inter, const float* row_scale, int act)
 {
     GemmArgsF32 a = {};
+    a.inter = inter;
+    a.row_scale = row_scale;
+    a.act = act;
     int max_mtiles = 0;
     // map_ready (AMOE_TILE_MAP_READY): the workspace already holds the map for these offsets, nothing is launched
     int rc = amoe_build_tile_map(offsets, R, E, BM_ROWS, workspace, workspace_bytes, &a.tile_map, &a.n_mtiles, &max_mtiles, s,
@@ -609,7 +672,8 @@ int amoe_f32_rows(const void* A, const int32_t* a_row_map, const void* B, const 
     int form = 0;
     if ((R / 32 + met) * a.n_ntiles <= 400) form = 2;
     else if ((R / 128 + met / 2 + 1) * a.n_ntiles <= 256 && Kred >= 512) form = 1;
-    if (b_kc) launch_rows<true>(a, (int)grid, form, s);
+    if (inter) launch_rows<false, true>(a, (int)grid, form, s);
+    else if (b_kc) launch_rows<true>(a, (int)grid, form, s);
     else launch_rows<false>(a, (int)grid, form, s);
     return amoe_check_launch("grouped_gemm_f32");
 }

@@ -1,6 +1,6 @@
 // HBM-bound row kernels: gather, weighted gather-reduce (combine / gather backward),
-// combine backward, and the elementwise gated activation (forward for the f32 path,
-// backward for both).  All move 16-byte vectors per lane; a row of H elements is walked by
+// combine backward, and the backward of the gated activation
+// (float32, and the shared expert).  All move 16-byte vectors per lane; a row of H elements is walked by
 // the 256 lanes of a block in steps of 256 vectors so every access is fully coalesced.
 #include "amoe_common.h"
 #include <type_traits>
@@ -116,32 +116,6 @@ combine_bwd_kernel(const T* __restrict__ dy, const T* __restrict__ out, const in
                 for (int i = 0; i < kBlock / AMOE_WAVE; ++i) tot += red[i];
                 d_scores[(size_t)t * K + k] = tot;
             }
-        }
-    }
-}
-
-// inter[r,i] = scale[r] * gu[r,2i+1] * act(gu[r,2i])     (one wavefront per row; scale == null -> 1)
-template <typename T, int ACT>
-__global__ void __launch_bounds__(kBlock)
-gated_act_fwd_kernel(const T* __restrict__ gu, const float* __restrict__ scale, T* __restrict__ inter, int R, int I)
-{
-    constexpr int V = ElemTraits<T>::kVec;
-    const int lane = threadIdx.x & 63;
-    const int nvec = I / V;
-    for (int r = blockIdx.x * (kBlock / AMOE_WAVE) + (threadIdx.x >> 6); r < R; r += gridDim.x * (kBlock / AMOE_WAVE)) {
-        const float sc = scale ? scale[r] : 1.0f;
-        const u32x4_t* g = reinterpret_cast<const u32x4_t*>(gu + (size_t)r * 2 * I);
-        u32x4_t* o = reinterpret_cast<u32x4_t*>(inter + (size_t)r * I);
-        for (int i = lane; i < nvec; i += AMOE_WAVE) {
-            float a[V], b[V], out[V];
-            ElemTraits<T>::unpack(g[2 * i], a);
-            ElemTraits<T>::unpack(g[2 * i + 1], b);
-#pragma unroll
-            for (int j = 0; j < V / 2; ++j) {
-                out[j] = sc * a[2 * j + 1] * act_fwd<ACT>(a[2 * j]);
-                out[V / 2 + j] = sc * b[2 * j + 1] * act_fwd<ACT>(b[2 * j]);
-            }
-            o[i] = ElemTraits<T>::pack(out);
         }
     }
 }
@@ -402,18 +376,6 @@ AMOE_EXPORT int amoe_combine_bwd(const void* dy, const void* moe_out, const int3
 }
 
 // used by the f32 gate_up path, which does not fuse the activation into its GEMM
-int amoe_launch_gated_act_fwd(const void* gu, const float* row_scale, void* inter, int dtype, int R, int I, int act,
-                              hipStream_t s)
-{
-    const int rows_per_block = kBlock / AMOE_WAVE;
-    const int grid = (R + rows_per_block - 1) / rows_per_block < 65536 ? (R + rows_per_block - 1) / rows_per_block : 65536;
-    AMOE_DISPATCH_ACT(act, {
-        AMOE_DISPATCH_ELEM(dtype, hipLaunchKernelGGL((gated_act_fwd_kernel<ELEM, ACT>), dim3(grid), dim3(kBlock), 0, s,
-                                                     (const ELEM*)gu, row_scale, (ELEM*)inter, R, I))
-    })
-    return amoe_check_launch("gated_act_fwd");
-}
-
 static void launch_act_bwd(const void* gate_up, const void* d_inter, const float* row_scale, const int32_t* slot_of, void* d_gate_up,
                            float* d_row_scale, int dtype, int R, int I, int T, int K, int act, hipStream_t s)
 {
