@@ -1666,13 +1666,15 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
     // tiles, the kernel with 64-bit addresses runs.
     const long long per = (long long)a.n_mt * a.n_ntiles;
     if (tile_cfg == 0) {
-        // Up to 104 rows per expert the product is bound by the gradients' stores: gemm_short.hip, where its 32-bit tile
+        // Up to 128 rows per expert the product is bound by the gradients' stores: gemm_short.hip, where its 32-bit tile
         // numbers reach (with a fourth of these tiles' size).  Beyond, gemm_pp.hip, whose tiles are never done in less than three
-        // K tiles.  Alone they meet at 80 rows; inside a step, where the short kernel's workgroups leave more to the other stream's, at
-        // 105 (short / pp, us): 64 experts of 2048 x 1408, 81 rows 802 / 823, 100 819 / 843, 128 900 / 893; 128 of 2048 x 768, 88 rows
-        // 867 / 902, 112 977 / 934, 128 1036 / 963; 8 of 4096 x 7168, 100 rows 948 / 966; 97 of 1856 x 960, 105 rows 913 / 914; 27 of
-        // 1024 x 4608, 100 rows 669 / 641.
-        if (R <= 104ll * E && offsets32 && 16 * per * per * E < (1ll << 32)) return amoe_short_wgrad(a, s);
+        // K tiles and that deals tiles by number: with uneven loads the deep ones fall to a few compute units, four times as large as the
+        // short kernel's.  Steps, us, short / pp: 128 experts of 2048 x 768, even loads, 105 rows 957 / 923, 128 rows 1013 / 949, Zipf loads
+        // 1127 / 1216; 64 of 2048 x 1408, even, 105 rows 822 / 846, 128 rows 891 / 871; 97 of 1856 x 960, 128 rows, even 1058 / 1065,
+        // a sixteenth of the experts with half of the rows 1041 / 1117; 32 of 1024 x 2048, 128 rows, even 403 / 381, a sixteenth
+        // 436 / 463; 27 of 1024 x 4608, 128 rows, even 719 / 670.  The two gradients alone, 64 of 1024 x 2048, 106 rows, all on one expert
+        // 217 / 411, on a quarter of them 201 / 302, even 199 / 218.
+        if (R <= 128ll * E && offsets32 && 16 * per * per * E < (1ll << 32)) return amoe_short_wgrad(a, s);
         if (offsets32 && per * per * E < (1ll << 32)) return amoe_pp_wgrad(a, s);
         tile_cfg = 5;
     }

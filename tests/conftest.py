@@ -19,3 +19,20 @@ def gpu_device():
     if not torch.cuda.is_available():
         pytest.skip("no GPU visible")
     return torch.device("cuda:0")
+
+
+@pytest.fixture(scope="session")
+def launched(gpu_device):
+    """launched(f): the names of the kernels that f() launches"""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+
+    def names(f):
+        f()
+        torch.cuda.synchronize()
+        with profile(activities=[ProfilerActivity.CUDA]) as p:
+            f()
+            torch.cuda.synchronize()
+        return [e.key for e in p.key_averages()]
+
+    return names
