@@ -1527,15 +1527,30 @@ int amoe_bf16_gateup_act(const void* xp, const int32_t* a_row_map, const void* w
 #endif
 
 #if AMOE_PART(0)
-// Up to 8 tokens: each of the product's workgroups selects for itself, and with many of them that takes longer than a launch.  bf16, one
-// forward pass, us, logits / routing / gate_up / down / sums as five launches and as three: 8 of 128 experts of 2048 x 768, 1 token
-// 35.3 / 29.9, 2 53.8 / 49.2, 4 76.2 / 75.8, 8 111.5 / 111.0, 12 135.2 / 143.1; 2 of 243 experts of 288 x 3712, 1 token 29.7 / 26.0,
-// 8 45.5 / 41.8, 12 56.9 / 59.5; 4 of 32 experts of 4096 x 2048, 1 token 59.5 / 52.3, 8 200.6 / 191.7, 16 261 / 260 (sizes that are bound by
-// the host 29.8 / 26.2).
-bool amoe_routed_fits(int dtype, int T, int K, int E, int H, int I, int tile_cfg)
+// Up to 8 tokens: each of the product's workgroups selects for itself and walks over the rows, which pays while that takes less
+// than the two launches that it saves, 7 us.  `steps`: how many experts are selected one after the other on a compute unit, which
+// holds two workgroups of eight wavefronts or four of four; a wavefront takes the tokens in turn.  One forward pass, us, logits /
+// routing / gate_up / down / sums as five launches and as three (T tokens, K of E experts of H x I):
+//   more workgroups than are held: 243 experts of 288 x 3712, T=4 K=8 (steps 16) 58 / 58, K=16 (64) 103 / 121, T=8 K=16 (192) 157 / 268
+//   two tokens in turn: 64 of 1024 x 512, T=6 K=6 (12) 34 / 35, T=8 K=8 (16) 42 / 45; 128 of 2048 x 768, T=8 K=4 (8) 66 / 67; 243 of
+//     288 x 3712, T=8 K=2 (4) 39 / 36
+//   R + 3 K: 256 of 512 x 256, T=5 K=10 (80) 32 / 31, T=6 (90) 32 / 33, T=8 K=16 (176) 39 / 48; 64 of 1024 x 512, K=16, T=2 (80)
+//     39 / 36, T=3 (96) 44 / 45
+//   long rows, whose reading hides it: 32 of 4096 x 1408, T=1 K=8 72 / 66, T=8 K=16 (steps 32) 201 / 199; 32 of 2880 x 2880, T=5 K=8
+//     (32) 221 / 216, T=8 K=16 (64) 265 / 268
+// One token of 8 of 128 experts of 2048 x 768 34 / 29; passes that are bound by the host 33 / 26.
+int amoe_routed_fits(int dtype, int T, int K, int E, int H, int I, int tile_cfg)
 {
-    return (dtype == AMOE_BF16 || dtype == AMOE_F16) && tile_cfg == 0 && T <= 8 && T * K <= 128 && E <= 256 && K <= E && K <= AMOE_MAX_TOPK &&
-           rows_tile_height(T * K, E, 0) == 16 && H % 32 == 0 && I % 32 == 0 && (unsigned long long)H * 2 * I * 2 < (1ull << 32);
+    if ((dtype != AMOE_BF16 && dtype != AMOE_F16) || tile_cfg != 0 || T > 8 || T * K > 128 || E > 256 || K > E || K > AMOE_MAX_TOPK ||
+        rows_tile_height(T * K, E, 0) != 16 || H % 32 || I % 32 || (unsigned long long)H * 2 * I * 2 >= (1ull << 32))
+        return 0;
+    const int R = T * K, m_tiles = E < R ? E : R, cus = device_cu_count();
+    if (cus <= 0) return 0;
+    const bool narrow = skinny_narrow(m_tiles, 2 * I, cus);
+    const int in_turn = (T + (narrow ? 7 : 3)) / (narrow ? 8 : 4), held = cus * (narrow ? 2 : 4), cols = narrow ? 64 : 128;
+    const long long steps = in_turn * K * (((long long)m_tiles * ((2 * I + cols - 1) / cols) + held - 1) / held);
+    const bool pays = H >= 2560 ? steps <= 32 : steps <= (in_turn > 1 ? 6 : 16) && R + 3 * K <= 80;
+    return pays ? cus : 0;
 }
 
 int amoe_run_gateup_routed(const void* x, const void* w_gate_up, void* gate_up, void* inter, const AmoeRoute& r, int dtype, int E, int H, int I,

@@ -33,16 +33,18 @@ struct AmoeRoute {
     int32_t* n_mtiles;
     int32_t* arrived;        // AmoeCombine's, which it sets to zero
     int n_arrived;
+    int cus;                 // compute units of the device
 };
 // The sums over a token's K rows inside the down product: the workgroup of a column tile that is the last to arrive adds them up.
 struct AmoeCombine {
     int32_t* arrived;        // workgroups of a column tile that have stored their rows, zero before
     const int32_t* row_of;   // [T,K]
     void* y;                 // [T,N]
-    int T, K;
+    int T, K, cus;
 };
-// whether it takes them (and then the product does, with every check of amoe_run_gateup_act_fwd on its sizes made)
-bool amoe_routed_fits(int dtype, int T, int K, int E, int H, int I, int tile_cfg);
+// compute units of the device if it takes them (and then the product does, with every check of amoe_run_gateup_act_fwd on its sizes
+// made), else 0
+int amoe_routed_fits(int dtype, int T, int K, int E, int H, int I, int tile_cfg);
 int amoe_run_gateup_routed(const void* x, const void* w_gate_up, void* gate_up, void* inter, const AmoeRoute& r, int dtype, int E, int H, int I,
                            int act, void* workspace, size_t workspace_bytes, hipStream_t s);
 // out [T*K,H] = inter @ w_down[e] by the map that amoe_run_gateup_routed left, and y as above

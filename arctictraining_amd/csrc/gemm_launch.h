@@ -19,6 +19,10 @@ static int device_cu_count()
     return n;
 }
 
+// The few-row kernel's 16-row tiles: 64 columns and eight wavefronts each where 128 columns and four do not give every compute unit
+// one (one token), 128 and four otherwise
+static bool skinny_narrow(int m_tiles, int N, int cus) { return (long long)m_tiles * ((N + 127) / 128) < cus; }
+
 template <auto KERN, int THREADS, int LDS_BYTES>
 int launch_kernel(const GemmArgs& a, int grid, hipStream_t s)
 {

@@ -232,9 +232,7 @@ int launch_height(const GemmArgs& a, int bm, hipStream_t s)
     if (m_tiles > a.max_mtiles) m_tiles = a.max_mtiles;
     AMOE_REQUIRE(bm == 16 || bm == 32, AMOE_ERR_UNSUPPORTED, "grouped_gemm: no kernel for tiles of %d rows", bm);
     if (bm == 32) return launch_skinny<2, 8, 4, EPI, ACT>(a, m_tiles, s);
-    // too few tiles of 128 columns for the compute units (one token): half as wide, twice as many wavefronts each
-    const int cus = device_cu_count();
-    if ((long long)m_tiles * ((a.N + 127) / 128) < cus) return launch_skinny<1, 4, 8, EPI, ACT>(a, m_tiles, s);
+    if (skinny_narrow(m_tiles, a.N, device_cu_count())) return launch_skinny<1, 4, 8, EPI, ACT>(a, m_tiles, s);
     return launch_skinny<1, 8, 4, EPI, ACT>(a, m_tiles, s);
 }
 
@@ -519,8 +517,7 @@ int amoe_skinny_gateup_routed(const GemmArgs& a, int act, const AmoeRoute& r, hi
     const int R = r.T * r.K, m_tiles = a.E < R ? a.E : R;
     AMOE_REQUIRE(r.T <= 16 && R <= kRoutedRows && a.E <= kRoutedExperts, AMOE_ERR_UNSUPPORTED,   // (a tile holds 16 rows)
                  "grouped_gemm: routing of %d rows of %d experts", R, a.E);
-    const bool narrow = (long long)m_tiles * ((a.N + 127) / 128) < device_cu_count();   // (as in launch_height)
-    AMOE_DISPATCH_ACT(act, return narrow ? (launch_routed<4, 8, ACT>(a, r, m_tiles, s)) : (launch_routed<8, 4, ACT>(a, r, m_tiles, s)))
+    AMOE_DISPATCH_ACT(act, return skinny_narrow(m_tiles, a.N, r.cus) ? (launch_routed<4, 8, ACT>(a, r, m_tiles, s)) : (launch_routed<8, 4, ACT>(a, r, m_tiles, s)))
     return AMOE_ERR_BAD_ARG;
 }
 
@@ -528,8 +525,7 @@ int amoe_skinny_gateup_routed(const GemmArgs& a, int act, const AmoeRoute& r, hi
 int amoe_skinny_nn_combined(const GemmArgs& a, const AmoeCombine& c, hipStream_t s)
 {
     const int m_tiles = a.E < a.M ? a.E : a.M;
-    const bool narrow = (long long)m_tiles * ((a.N + 127) / 128) < device_cu_count();
-    return narrow ? launch_combine<4, 8>(a, c, m_tiles, s) : launch_combine<8, 4>(a, c, m_tiles, s);
+    return skinny_narrow(m_tiles, a.N, c.cus) ? launch_combine<4, 8>(a, c, m_tiles, s) : launch_combine<8, 4>(a, c, m_tiles, s);
 }
 
 int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s) { return launch_height<EPI_STORE, 0>(a, bm, s); }

@@ -288,18 +288,19 @@ AMOE_EXPORT int amoe_layer_fwd_router(const int32_t* config, int T, const void* 
     AMOE_TRY(read_shape("layer_fwd_router", config, T, &c));
     if (stages & AMOE_STAGE_ROUTE) AMOE_TRY(amoe_router_logits(x, router_gate, logits, c.dtype, T, c.E, c.H, stream));
     const int fused = AMOE_STAGE_ROUTE | AMOE_STAGE_EXPERTS;
-    if (!assign && (stages & fused) == fused && amoe_routed_fits(c.dtype, T, c.K, c.E, c.H, c.I, c.tile_cfg)) {
+    const int cus = !assign && (stages & fused) == fused ? amoe_routed_fits(c.dtype, T, c.K, c.E, c.H, c.I, c.tile_cfg) : 0;
+    if (cus) {
         AMOE_REQUIRE(x && w_gate_up && w_down && saved && scratch && y, AMOE_ERR_BAD_ARG, "layer_fwd_router: null pointer");
         // (a few tokens: their routing inside the gate_up product)
         const Saved s = cut_saved(c, T, saved, keep != 0);
         const FwdScratch f = cut_fwd(c, T, scratch);
         const AmoeRoute route = {logits, T, c.K, c.normalize, s.probs, s.scores, s.scores_perm, s.topk_idx, s.counts, s.offsets, s.token_of,
-                                 s.slot_of, s.row_of, nullptr, nullptr, f.arrived, (c.H + 63) / 64};
+                                 s.slot_of, s.row_of, nullptr, nullptr, f.arrived, (c.H + 63) / 64, cus};
         AMOE_TRY(amoe_run_gateup_routed(x, w_gate_up, s.gate_up, s.inter, route, c.dtype, c.E, c.H, c.I, c.act, s.gemm_ws, s.gemm_ws_bytes,
                                         (hipStream_t)stream));
         stages &= ~fused;
         if (!c.shared && (stages & AMOE_STAGE_COMBINE)) {
-            const AmoeCombine combine = {f.arrived, s.row_of, y, T, c.K};
+            const AmoeCombine combine = {f.arrived, s.row_of, y, T, c.K, cus};
             return amoe_run_down_combined(s.inter, w_down, f.out, combine, c.dtype, c.E, c.H, c.I, s.gemm_ws, s.gemm_ws_bytes, (hipStream_t)stream);
         }
         AMOE_TRY(amoe_run_nn(s.inter, nullptr, w_down, s.offsets, f.out, c.dtype, T * c.K, c.E, c.I, c.H, s.gemm_ws, s.gemm_ws_bytes,
