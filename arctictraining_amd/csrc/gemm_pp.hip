@@ -141,7 +141,7 @@ __device__ __forceinline__ void pp_rows_body()
             pm += m;
             nt = c * p.gn + r - m * (last ? p.n_ntiles - c * p.gn : p.gn);
         } else {
-            const int m = divide(r, p.inv_n);
+            const int m = divide_any(r, p.n_ntiles, p.inv_n);
             pm += m;
             nt = r - m * p.n_ntiles;
         }

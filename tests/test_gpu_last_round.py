@@ -49,3 +49,20 @@ def test_every_tile_once(gpu_device, name, dtype):
     want = torch.stack((ref * up * (gate > 0), ref * gate.relu()), -1).flatten(1).to(dtype)
     assert torch.equal(d_gu, want)
     assert torch.equal(parts.sum(0), (ref * up * gate.relu()).sum(1))
+
+
+def test_more_columns_than_the_reciprocal_divides(gpu_device):
+    """Tile numbers of a short group are divided by the number of column tiles with its reciprocal rounded up, which is one too many
+    for the last one of the third row of 37927: that tile would lie in a row that does not exist.  Three rows, 1.9 GB of weights."""
+    from arctictraining_amd import ops
+
+    n_tiles = 37927
+    last, inv = 3 * n_tiles - 1, -(-2 ** 32 // n_tiles)
+    assert last * inv >> 32 == last // n_tiles + 1
+    print("many columns", n_tiles, flush=True)
+    g = torch.Generator(device=gpu_device).manual_seed(1)
+    draw = lambda *shape: torch.randint(-2, 3, shape, device=gpu_device, generator=g, dtype=torch.int8).to(torch.bfloat16)
+    a, w = draw(3, 32), draw(3, 256 * n_tiles, 32)
+    got = ops.grouped_gemm_nt(a, w, torch.arange(4, dtype=torch.int32, device=gpu_device))
+    for e in range(3):
+        assert torch.equal(got[e], (w[e].float() @ a[e].float()).to(torch.bfloat16)), e
