@@ -1394,14 +1394,14 @@ int amoe_tile_map_layout(int R, int E, int dtype, int tile_cfg, void* workspace,
 #endif
 
 // the default tile shape (gemm_pp.hip)
-int amoe_pp_gateup_act(const GemmArgs& a, int act, int tiles, hipStream_t s);
-int amoe_pp_rows(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s);
-int amoe_pp_gated_bwd(const GemmArgs& a, int act, int tiles, hipStream_t s);
+int amoe_pp_gateup_act(const GemmArgs& a, int act, hipStream_t s);
+int amoe_pp_rows(const GemmArgs& a, bool b_kc, hipStream_t s);
+int amoe_pp_gated_bwd(const GemmArgs& a, int act, hipStream_t s);
 int amoe_pp_wgrad(GemmArgs a, hipStream_t s);
 // few rows to reduce over (gemm_short.hip)
 int amoe_short_wgrad(GemmArgs a, hipStream_t s);
 // few tiles of a deep reduction (gemm_split.hip)
-int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, int tiles, hipStream_t s);
+int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, hipStream_t s);
 // few rows per expert (gemm_skinny.hip)
 int amoe_skinny_gateup_act(const GemmArgs& a, int act, int bm, hipStream_t s);
 int amoe_skinny_nn(const GemmArgs& a, int bm, hipStream_t s);
@@ -1504,11 +1504,11 @@ static int run_rows_bf16(const void* A, const int32_t* a_row_map, const void* B,
     }
     rc = set_supertiles(a, max_mtiles, &grid);
     if (rc) return rc;
-    if (splits > 1) return amoe_split_rows(a, B_KC, EPI, ACT, (int)grid, s);
+    if (splits > 1) return amoe_split_rows(a, B_KC, EPI, ACT, s);
     if (tile_cfg == 0) {
-        if constexpr (EPI == EPI_GATED) return amoe_pp_gateup_act(a, ACT, (int)grid, s);
-        else if constexpr (EPI == EPI_GATED_BWD) return amoe_pp_gated_bwd(a, ACT, (int)grid, s);
-        else return amoe_pp_rows(a, B_KC, (int)grid, s);
+        if constexpr (EPI == EPI_GATED) return amoe_pp_gateup_act(a, ACT, s);
+        else if constexpr (EPI == EPI_GATED_BWD) return amoe_pp_gated_bwd(a, ACT, s);
+        else return amoe_pp_rows(a, B_KC, s);
     }
     return launch_any<true, B_KC, EPI, ACT>(a, tile_cfg, (int)grid, s);
 }

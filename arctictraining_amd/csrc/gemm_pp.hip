@@ -1144,12 +1144,12 @@ static int launch_pp_rows(const GemmArgs& a, int grid, hipStream_t s)
     return launch_kernel<grouped_gemm_pp_rows_bf16_kernel<B_KC, EPI, ACT, STREAM>, PP_THREADS, PP_LDS>(a, grid, s);
 }
 template <bool B_KC, int EPI, int ACT>
-static int launch_pp_rows(const GemmArgs& a, int tiles, hipStream_t s)
+static int launch_pp_rows(const GemmArgs& a, hipStream_t s)
 {
     const int cus = device_cu_count();
     AMOE_REQUIRE(cus > 0, AMOE_ERR_LAUNCH, "grouped_gemm: cannot read the number of compute units");
-    // (a multiple of 8: every XCD then runs the same number of workgroups; a tile can become four pieces)
-    const int grid = ((tiles < (cus + 3) / 4 ? 4 * tiles : cus) + 7) & ~7;
+    // (a multiple of 8: every XCD then runs the same number of workgroups; how many tiles there are, only the device knows)
+    const int grid = (cus + 7) & ~7;
     GemmArgs b = a;
     b.inv_group = tile_inverse(a.gm * a.n_ntiles);
     b.inv_n = tile_inverse(a.n_ntiles);
@@ -1165,32 +1165,31 @@ static int launch_pp_rows(const GemmArgs& a, int tiles, hipStream_t s)
     return launch_pp_rows<B_KC, EPI, ACT, false>(b, grid, s);
 }
 
-// `tiles`: upper bound of the number of tiles
 #if AMOE_PP_PART_IS(0)
-int amoe_pp_gateup_act(const GemmArgs& a, int act, int tiles, hipStream_t s)
+int amoe_pp_gateup_act(const GemmArgs& a, int act, hipStream_t s)
 {
-    AMOE_DISPATCH_ACT(act, return (launch_pp_rows<false, EPI_GATED, ACT>(a, tiles, s)))
+    AMOE_DISPATCH_ACT(act, return (launch_pp_rows<false, EPI_GATED, ACT>(a, s)))
     return AMOE_ERR_BAD_ARG;
 }
 #endif
 #if AMOE_PP_PART_IS(1)
-int amoe_pp_part(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s)
+int amoe_pp_part(const GemmArgs& a, bool b_kc, hipStream_t s)
 {
-    return b_kc ? launch_pp_rows<true, EPI_PART, 0>(a, tiles, s) : launch_pp_rows<false, EPI_PART, 0>(a, tiles, s);
+    return b_kc ? launch_pp_rows<true, EPI_PART, 0>(a, s) : launch_pp_rows<false, EPI_PART, 0>(a, s);
 }
-int amoe_pp_rows(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s)
+int amoe_pp_rows(const GemmArgs& a, bool b_kc, hipStream_t s)
 {
     // An output of half the last-level cache or more is stored past the caches (218 MB: 0.828 ms a step with ordinary stores, 0.801
     // so; 1 GB 5.00 / 4.94; 45 MB 0.136 / 0.141).
     const bool past = 2ll * a.M * a.N >= 128ll << 20;
-    if (past) return b_kc ? launch_pp_rows<true, EPI_STORE_PAST, 0>(a, tiles, s) : launch_pp_rows<false, EPI_STORE_PAST, 0>(a, tiles, s);
-    return b_kc ? launch_pp_rows<true, EPI_STORE, 0>(a, tiles, s) : launch_pp_rows<false, EPI_STORE, 0>(a, tiles, s);
+    if (past) return b_kc ? launch_pp_rows<true, EPI_STORE_PAST, 0>(a, s) : launch_pp_rows<false, EPI_STORE_PAST, 0>(a, s);
+    return b_kc ? launch_pp_rows<true, EPI_STORE, 0>(a, s) : launch_pp_rows<false, EPI_STORE, 0>(a, s);
 }
 #endif
 #if AMOE_PP_PART_IS(2)
-int amoe_pp_gated_bwd(const GemmArgs& a, int act, int tiles, hipStream_t s)
+int amoe_pp_gated_bwd(const GemmArgs& a, int act, hipStream_t s)
 {
-    AMOE_DISPATCH_ACT(act, return (launch_pp_rows<true, EPI_GATED_BWD, ACT>(a, tiles, s)))
+    AMOE_DISPATCH_ACT(act, return (launch_pp_rows<true, EPI_GATED_BWD, ACT>(a, s)))
     return AMOE_ERR_BAD_ARG;
 }
 #endif

@@ -10,7 +10,7 @@
 #include "gemm_calls.h"
 #include "gemm_launch.h"
 
-int amoe_pp_part(const GemmArgs& a, bool b_kc, int tiles, hipStream_t s);
+int amoe_pp_part(const GemmArgs& a, bool b_kc, hipStream_t s);
 
 namespace {
 
@@ -133,9 +133,9 @@ size_t amoe_split_bytes(int R, int E, int K, int N)
 }
 
 // a: the product as for the default kernel, super-tiles set for n_ntiles = n_real * splits
-int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, int tiles, hipStream_t s)
+int amoe_split_rows(const GemmArgs& a, bool b_kc, int epi, int act, hipStream_t s)
 {
-    int rc = amoe_pp_part(a, b_kc, tiles, s);
+    int rc = amoe_pp_part(a, b_kc, s);
     if (rc) return rc;
     const long long n = (long long)a.M * a.N, n8 = n / 8;
     const dim3 grid((unsigned)((n8 + kBlock - 1) / kBlock)), block(kBlock);

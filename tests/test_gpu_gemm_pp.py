@@ -83,14 +83,14 @@ def test_many_tiles_per_workgroup(ops, gpu_device, E, Kd, N):
 @pytest.mark.parametrize("M,N,counts", [
     (256, 256, [0, 1, 700, 513, 0, 400]),            # empty and one-row experts, remainders of a K tile
     (136, 1032, [1100, 64, 65, 0, 200, 900]),        # edges in both extents
-    (1408, 520, [257] * 9 + [0, 600]),               # a last row tile of half height; several tiles per workgroup
+    (1408, 520, [257] * 9 + [0, 600]),               # a last row tile of half height; 198 tiles, one a workgroup
 ])
 def test_weight_gradient(ops, gpu_device, dtype, tol, M, N, counts):
     print("pp wgrad", dtype, M, N, flush=True)
     g = torch.Generator(device=gpu_device).manual_seed(M + N)
     offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(gpu_device)
     R, E = sum(counts), len(counts)
-    assert R >= 256 * E   # (below that the default is another tile shape)
+    assert R >= 256 * E   # (test_gpu_wgrad_lines.py has fewer rows)
     T = R // 3
     rows = torch.randint(0, T, (R,), device=gpu_device, generator=g, dtype=torch.int32)
     rnd = lambda *s: torch.randn(*s, device=gpu_device, generator=g).to(dtype)

@@ -7,6 +7,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 CASES = {
+    "one": ([250], 128, 256),                                    # a single tile, in quarters
+    "five": ([256, 200, 256, 31, 225], 64, 256),
     "quarters": ([256, 250, 193, 225], 128, 320),                # 4 x 2 tiles
     "halves": ([300, 225, 512, 768], 64, 2560),                  # 8 x 10, two super-columns of 5
     "whole": ([192, 190, 64, 1], 96, 4608),                      # 4 x 18, none of them tall

@@ -1,5 +1,5 @@
 """Weight gradients of 129 rows per expert and more, whose epilogue takes a wavefront's 64 columns through LDS and stores whole
-lines: edges of the 8-column pieces and 16-row blocks it writes, half tiles, one and two tiles a workgroup, gradients
+lines: edges of the 8-column pieces and 16-row blocks it writes, half tiles, one, two and all tiles a workgroup, uneven loads, gradients
 that the caches hold and that they do not (stored past them), either operand gathered, against float64."""
 import pytest
 import torch
@@ -10,7 +10,10 @@ CASES = {
     "pieces": ([130, 0, 257, 300, 1], 264, 328),             # 8 rows and 8 columns past a tile, an expert without rows
     "blocks": ([129, 200, 140], 8, 72),                      # less than one 16-row block, 8 columns past 64
     "half": ([192, 193, 64, 300], 392, 1416),                # a lower half of 8 rows; columns end inside a wavefront's
-    "past_the_caches": ([150] * 30, 520, 1096),              # 34 MB, more tiles than two a workgroup of one round
+    "past_the_caches": ([150] * 30, 520, 1096),              # 34 MB, 450 tiles: two a workgroup, of 256
+    "two_of_four": ([130] * 40, 776, 1096),                  # 800 tiles: two a workgroup, the second 256 workgroups not all filled
+    "uneven": ([0, 3000, 1, 0, 64, 1500, 7] * 6, 776, 1032), # 840 tiles of 3 to 47 K tiles, two a workgroup
+    "all_of_three": ([720] * 8, 2056, 2056),                 # 648 tiles of 11 K tiles and more: three a workgroup
     "all_to_one": ([0, 900, 0], 136, 520),
 }
 
