@@ -1153,7 +1153,9 @@ static int launch_pp_rows(const GemmArgs& a, hipStream_t s)
     GemmArgs b = a;
     b.inv_group = tile_inverse(a.gm * a.n_ntiles);
     b.inv_n = tile_inverse(a.n_ntiles);
-    // Where expert e's reduction starts (see first_step in the kernel), 128 experts of N = 2048, 32 rows each, us, at 0 / at 5 e: K = 2048
+    // Where expert e's reduction starts (see first_step in the kernel).  The three lengths are what was measured to gain, no more:
+    // few channels alone would speak for rows 16 KB apart too, which lose, and lengths of 10240 and more were not tried.  The order in
+    // which a row's products are summed depends on its expert's number there.  128 experts of N = 2048, 32 rows each, us, at 0 / at 5 e: K = 2048
     // 240 / 188, 4096 433 / 355; 16 of N = 4096, 24 rows: K = 4096 123 / 92, 6144 153 / 135; 64 of N = 2048, 300 rows: K = 2048 199 / 179.
     // Other strides have no such channels, and lose what neighbours read of one memory page: K = 1984 182 / 187, 4160 351 / 366, 8192 170 /
     // 180, 3072 276 / 280.  From 512 rows an expert on the products are not bound by the reading (600 rows 219 / 222).  With B not
@@ -1226,6 +1228,9 @@ int amoe_pp_wgrad(GemmArgs a, hipStream_t s)
     //   24 experts of  480 x 7360, 230 rows                 0.73 / 0.73 / 0.75 / 0.76, 0.79
     //   22 experts of  832 x 11840, 615 rows                3.18 / 3.17 / 3.19 / 3.38, 3.40
     //   16 experts of 1728 x 2208, 742 rows                 0.99 / 1.01 / 1.00 / 0.98, 1.00
+    // Uneven loads, both gradients alone, us, shape 5 / two tiles a workgroup: 128 experts of 2048 x 768, 175 rows, all on one expert
+    // 1049 / 1057, half on the first and the last each 749 / 760 (200 rows 813 / 835), 150 rows on a quarter of the experts 522 / 356, a
+    // sixteenth with half of them 440 / 367; 64 of 1024 x 2048, 150 rows, on one 581 / 502, a quarter 535 / 373, a sixteenth 319 / 245.
     const long long rounds = (total + 255) / 256;
     a.gm = (int)(a.rows_total < 11ll * PP_BK * a.E && rounds > 2 ? 2 : rounds);
     const int grid = rounds == 1 ? (int)((total + 7) & ~7ll) : (int)((rounds + a.gm - 1) / a.gm * 256);

@@ -72,7 +72,7 @@ Saved cut_saved(const Shape& c, int T, void* base, bool keep)
     s.gemm_ws_bytes = amoe_grouped_gemm_workspace_bytes((int)R, c.E);
     s.gemm_ws = b.take<char>(s.gemm_ws_bytes);
     s.inter = b.take<char>(R * c.I * c.esz());
-    // the float32 gate_up product reads what it stored to apply the activation
+    // float32 gate_up products store it whether backward reads it or not: rows that are worked out again are activated from it
     if (keep || c.dtype == AMOE_F32) s.gate_up = b.take<char>(R * 2 * c.I * c.esz());
     if (c.shared) {
         s.sh_sig = b.take<float>(T);
@@ -335,12 +335,12 @@ static int layer_bwd(const int32_t* config, int T, const void* x, const void* dy
                                     c.act, stream));
     }
     // The expert weight gradients feed nothing else here.  On the second stream, and queued ahead of the rest, they start as the
-    // gated backward's workgroups end; the kernels of this stream then run on what the weight gradients leave, which
-    // is little before persistent ones end (from 256 rows an expert on): with 16384 tokens of 128 experts of 2048 x 768 the router's
-    // weight gradient and the sum of its parts last 422 and 751 us, of which 24 and 5 are their own.  A step with the second
-    // stream / without, us: those 3851 / 3853, 8192 tokens of 8 experts of 4096 x 14336 14033 / 14137, 4001 tokens of 64 experts and a
-    // shared one, float16, 1701 / 1835, 2048 tokens in float32 400 / 423, 509 tokens of the first, whose weight
-    // gradients are bound by memory as the data gradients are, 825 / 808.
+    // gated backward's workgroups end; the kernels of this stream then run on what the weight gradients leave, which is little
+    // before their workgroups end (from 129 rows an expert on these take two tiles each, from 704 on all that fall to them): with
+    // 16384 tokens of 128 experts of 2048 x 768 the router's weight gradient and the sum of its parts last 422 and 759 us, of which
+    // 24 and 5 are their own.  A step with the second stream / without, us: those 3700 / 3706, 8192 tokens of 8 experts of 4096 x 14336
+    // 13560 / 13575, 4001 tokens of 64 experts and a shared one, float16, 1542 / 1581, 2048 tokens in float32 373 / 399, 128, 509, 1024,
+    // 1600, 2000 and 2400 tokens of the first 690 / 697, 735 / 740, 798 / 799, 934 / 905, 1002 / 970, 984 / 990.
     OrderEvent event;
     if (overlap) AMOE_REQUIRE(event.order(main, side), AMOE_ERR_LAUNCH, "layer_bwd: cannot order the second stream after the first");
     void* const wstream = overlap ? side_stream : stream;

@@ -375,7 +375,6 @@ AMOE_EXPORT int amoe_combine_bwd(const void* dy, const void* moe_out, const int3
     return amoe_check_launch("combine_bwd");
 }
 
-// used by the f32 gate_up path, which does not fuse the activation into its GEMM
 static void launch_act_bwd(const void* gate_up, const void* d_inter, const float* row_scale, const int32_t* slot_of, void* d_gate_up,
                            float* d_row_scale, int dtype, int R, int I, int T, int K, int act, hipStream_t s)
 {

@@ -316,9 +316,9 @@ def _overlap_pays(config_key, T: int) -> bool:
     step; a step that the GPU takes less time for than the host is longer by that much (20 of 60 steps drawn over the sizes of
     this layer: 12-39 %), one that it takes longer for is mostly 3-15 % shorter with the second stream.  The line lies where
     the products at 800 TFLOP/s (float32 100), their columns rounded up to whole tiles, and the weights, read twice and their
-    gradients written, at 3 TB/s make 150 us: T=556 H=1760 E=8 K=6 I=672 (143 us) 268 us with it, 228 without; T=95 H=2336 E=12
-    K=2 I=1536 (193) 274 and 299, T=3065 H=320 E=19 K=5 I=1088 (243) 353 and 398.  (Not all: 509 tokens of 128 experts of
-    2048 x 768, bound by memory on both streams, take 2 % longer with it.)"""
+    gradients written, at 3 TB/s make 150 us: T=556 H=1760 E=8 K=6 I=672 (143 us) 250 us with it, 220 without; T=3065 H=320 E=19
+    K=5 I=1088 (243) 268 and 283.  (Not all: T=95 H=2336 E=12 K=2 I=1536 (193), whose kernels have become faster than the host,
+    takes 261 and 228; about 110 rows an expert of 128 experts of 2048 x 768, bound by memory on both streams, 3 % longer with it.)"""
     E, K, H, I, dtype, shared = *config_key[:4], config_key[5], config_key[8]
     size, rate = (4, 1e8) if dtype == ops.F32 else (2, 8e8)
     rows, weights = T * K + (T if shared else 0), (E + (1 if shared else 0)) * H * I
