@@ -48,7 +48,9 @@ struct GemmArgsF32 {
 // Gated products: a vector of C is (gate, up) of two intermediate columns, which leave the epilogue as row_scale up act(gate).
 // With a kernel of its own that read C again and wrote them / so, a forward pass, us: 2048 tokens x 2 of 8 experts of 512 x 1024
 // 147 / 143, 4096 x 2 of 8 of 1024 x 2048 729 / 713, 650 x 6 of 20 of 384 x 160 and a shared one 80 / 75, one token 57 / 54; a
-// training step of the first 388 / 383.
+// training step of the first 388 / 383.  Few rows an expert, where a tile's epilogue counts most, with that kernel / with row scales read in
+// the epilogue and dead blocks of 16 rows activated / as now: 167 x 3 of 242 of 288 x 352 166.5 / 173.9 / 165.6, 40 x 4 of 128 of 512 x
+// 768 162.9 / 167.1 / 162.0, 300 x 4 of 64 of 1024 x 512 136.5 / 137.3 / 135.2.
 __device__ __forceinline__ float activate(int act, float g)
 {
     switch (act) {
@@ -202,10 +204,13 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
     // Rows, columns and k past the end are copies of the last ones: the products of the first two are not stored, the last
     // are set to zero before they are split.  (No load is behind a branch: its result would pass through a copy, and the
     // copy awaits it.)
+    // (Row scales as well: behind the stores of an epilogue a load waits for them too.)
     const float* a_ptr[2];
+    float scale[2] = {1.0f, 1.0f};
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         int gr = min(m0 + i * 16 + l16, mend - 1);
+        if (GATED && p.row_scale) scale[i] = p.row_scale[gr];
         if (p.a_row_map) gr = p.a_row_map[gr];
         a_ptr[i] = p.A + (long long)gr * p.lda;
     }
@@ -310,8 +315,8 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
     bool finite = true;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
+        if (m0 + i * 16 >= mend) break;
         const int row = m0 + i * 16 + l16;
-        const float scale = GATED && p.row_scale ? p.row_scale[min(row, mend - 1)] : 1.0f;
         f32x2_t h[TN];
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
@@ -319,7 +324,7 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
             finite = finite && finite4(c);
             const int col = n0 + j * 16 + 4 * lq;
             if (row < mend && col < p.N) *reinterpret_cast<f32x4_t*>(p.C + (long long)row * p.ldc + col) = c;
-            if constexpr (GATED) h[j] = gated(p, scale, c);
+            if constexpr (GATED) h[j] = gated(p, scale[i], c);
         }
         if constexpr (GATED) {
             // of tiles j and j + 1 lane quarters 0 and 2 take j's columns, 1 and 3 the other's: 16 bytes a lane, 64 of a row together

@@ -10,6 +10,7 @@ CASES = {
     "few_tiles": ([40, 0, 33, 1], 64, 36),          # eight wavefronts share a reduction
     "two_groups": ([700, 0, 129, 671], 512, 320),   # two groups of wavefronts
     "many_tiles": ([500, 513, 0, 987], 128, 1012),
+    "few_rows": ([1, 2, 16, 17, 33, 0] * 10, 64, 320),   # tiles of a row on, blocks of 16 without a live row
 }
 
 
