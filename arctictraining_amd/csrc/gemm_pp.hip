@@ -1182,8 +1182,9 @@ int amoe_pp_part(const GemmArgs& a, bool b_kc, hipStream_t s)
 int amoe_pp_rows(const GemmArgs& a, bool b_kc, hipStream_t s)
 {
     // An output of half the last-level cache or more is stored past the caches (218 MB: 0.828 ms a step with ordinary stores, 0.801
-    // so; 1 GB 5.00 / 4.94; 45 MB 0.136 / 0.141).
-    const bool past = 2ll * a.M * a.N >= 128ll << 20;
+    // so; 1 GB 5.00 / 4.94; 45 MB 0.136 / 0.141), if its rows are whole lines of 128 bytes: parts of lines meet in the L2 and not
+    // past it (alone, us, ordinary / past: 120000 rows, 896 x 608 140 / 150, 80000, 544 x 1504 160 / 166).
+    const bool past = a.N % 64 == 0 && 2ll * a.M * a.N >= 128ll << 20;
     if (past) return b_kc ? launch_pp_rows<true, EPI_STORE_PAST, 0>(a, s) : launch_pp_rows<false, EPI_STORE_PAST, 0>(a, s);
     return b_kc ? launch_pp_rows<true, EPI_STORE, 0>(a, s) : launch_pp_rows<false, EPI_STORE, 0>(a, s);
 }

@@ -15,7 +15,8 @@ CASES = {
     "one_round": ([256] * 16, 96, 4096),                         # 16 x 16 = 256
     "few_left": ([257, 250, 255] * 8, 64, 2200),                 # 32 x 9, super-columns of 5 and 4, 32 left, in quarters
     "many_left": ([200, 256, 0, 7] * 13, 64, 2816),              # 39 x 11, super-columns of 6 and 5, 173 left
-    "past_the_caches": ([1000, 31, 2000, 0, 5200], 64, 8200),    # an output of 128 MiB and more is stored past the caches
+    "past_the_caches": ([1000, 31, 2000, 0, 5200], 64, 8200),    # 128 MiB and more, which are stored past the caches, but not
+    "whole_lines": ([1000, 31, 2000, 0, 5200], 64, 8192),        # .. in rows of 16400 bytes: these are
     "turned_2048": ([200, 31, 0, 256, 257, 90], 2048, 264),      # reductions that start at another K tile for every expert (B^T)
     "turned_6144": ([40, 300] * 4, 6144, 72),
     "short_group": ([256, 31] * 19 + [250], 64, 1904),           # 39 x 8, groups of 4
@@ -68,3 +69,17 @@ def test_more_columns_than_the_reciprocal_divides(gpu_device):
     got = ops.grouped_gemm_nt(a, w, torch.arange(4, dtype=torch.int32, device=gpu_device))
     for e in range(3):
         assert torch.equal(got[e], (w[e].float() @ a[e].float()).to(torch.bfloat16)), e
+
+
+@pytest.mark.parametrize("name,epilogue", [("whole_lines", 4), ("past_the_caches", 0), ("whole", 0)])
+def test_which_go_past_the_caches(gpu_device, launched, name, epilogue):
+    """Large outputs, if their rows are whole lines: stores of parts of lines past the caches take longer than ordinary ones."""
+    from arctictraining_amd import ops
+
+    counts, K, N = CASES[name]
+    print("past the caches", name, flush=True)
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(gpu_device)
+    a, w = (torch.zeros(*shape, dtype=torch.bfloat16, device=gpu_device) for shape in ((sum(counts), K), (len(counts), K, N)))
+    names = launched(lambda: (ops.grouped_gemm_nn(a, w, off), ops.grouped_gemm_nt(a, w.view(len(counts), N, K), off)))
+    for b_kc in ("false", "true"):
+        assert any(f"pp_rows_bf16_kernel<{b_kc}, {epilogue}, 0," in n for n in names), names
