@@ -357,6 +357,8 @@ __device__ __forceinline__ void pp_rows_body()
     // Blocks of 32 rows without a live row are left out: the arithmetic of the gated epilogues is 4 us (gate_up) and 13 us (gated backward)
     // of a whole tile, beside which no MFMA runs.  32 rows an expert, 128 experts of 2048 x 768, us: gate_up 165 / 156, gated backward
     // 134 / 119, down 90 / 86, with B^T 170 / 165; a training step of 509 tokens 835 / 798, a forward pass of 3001 342 / 338.
+    // The gate_up epilogue asks once whether any block is (WHOLE): asked at each of its 16, a short reduction of large tiles pays for it
+    // (K = 512, 180000 rows, N = 2048 398 us before, 402-405 with a test each, 396 so; K = 608, 120000 rows, N = 1792 265 / 272 / 267).
     // LINES: a wavefront's columns of the tile are 64 in a row (else 32 of either half), 128 bytes of the output.  Through 2 KB of LDS
     // of its own (chunk c of row r at c ^ (r & 7), its halves the other way round from row 8 on: no bank conflicts) eight lanes
     // come to hold a row's, and a store writes whole lines.  Adjacent lanes in adjacent rows, as the accumulators have them, are a
@@ -414,8 +416,9 @@ __device__ __forceinline__ void pp_rows_body()
         }
     };
     float dots[4] = {0.f, 0.f, 0.f, 0.f};
-    auto epilogue = [&](auto A_, auto B_, const mfma_f32x4 (&acc)[4][4]) {
+    auto epilogue = [&](auto A_, auto B_, const mfma_f32x4 (&acc)[4][4], auto WHOLE) {
         constexpr int a = decltype(A_)::value, b = decltype(B_)::value;
+        constexpr bool whole = decltype(WHOLE)::value;      // every block has a live row
         const int le = pp_here(lane);
         const int eq = le >> 4, rl = grp * 16 + (le & 15);
         const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc(e_c, (short)0, (int)PP_DROP, 0x00020000);
@@ -490,7 +493,7 @@ __device__ __forceinline__ void pp_rows_body()
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 pp_fence();
-                if ((a * 4 + i) * 32 >= e_rows) break;
+                if (!whole && (a * 4 + i) * 32 >= e_rows) break;
                 const bool ok = b * 128 + 8 * eq < e_cols && (a * 4 + i) * 32 + rl < e_rows;
                 uint32_t x[2], y[2];
 #pragma unroll
@@ -639,7 +642,7 @@ __device__ __forceinline__ void pp_rows_body()
         dma_a(I0{});
         if constexpr (LINES) {
             // the epilogue of a finished half in the memory parts of the phases after it
-            epilogue(I0{}, I0{}, acc[0]);
+            epilogue(I0{}, I0{}, acc[0], F_{});
             pp_vmwait<10>();
             pp_barrier();
             mma(F_{}, I0{}, I4{}, acc[1], fb0);
@@ -647,13 +650,13 @@ __device__ __forceinline__ void pp_rows_body()
             flip();
             read_b(I0{}, fb0);
             dma_b(I1{});
-            epilogue(I0{}, I1{}, acc[0]);
+            epilogue(I0{}, I1{}, acc[0], F_{});
             pp_vmwait<10>();
             pp_barrier();
             mma(F_{}, I1{}, I4{}, acc[1], fb1);
             pp_barrier();
-            epilogue(I1{}, I0{}, acc[1]);
-            epilogue(I1{}, I1{}, acc[1]);
+            epilogue(I1{}, I0{}, acc[1], F_{});
+            epilogue(I1{}, I1{}, acc[1], F_{});
         } else {
             // activations are far more vector work than one arithmetic part hides: all four quadrants together, so
             // that the two wavefronts of a SIMD share its vector unit instead of taking turns at it
@@ -669,12 +672,16 @@ __device__ __forceinline__ void pp_rows_body()
             fetch_gate_up(I0{}, I0{});
             fetch_gate_up(I0{}, I1{});
             pp_barrier();
-            epilogue(I0{}, I0{}, acc[0]);
-            fetch_gate_up(I1{}, I0{});
-            epilogue(I0{}, I1{}, acc[0]);
-            fetch_gate_up(I1{}, I1{});
-            epilogue(I1{}, I0{}, acc[1]);
-            epilogue(I1{}, I1{}, acc[1]);
+            auto quadrants = [&](auto WHOLE) {
+                epilogue(I0{}, I0{}, acc[0], WHOLE);
+                fetch_gate_up(I1{}, I0{});
+                epilogue(I0{}, I1{}, acc[0], WHOLE);
+                fetch_gate_up(I1{}, I1{});
+                epilogue(I1{}, I0{}, acc[1], WHOLE);
+                epilogue(I1{}, I1{}, acc[1], WHOLE);
+            };
+            if (EPI == EPI_GATED && e_rows > PP_BM - 32) quadrants(T_{});
+            else quadrants(F_{});
             read_b(I0{}, fb0);
         }
     };

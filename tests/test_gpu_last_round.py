@@ -19,6 +19,7 @@ CASES = {
     "whole_lines": ([1000, 31, 2000, 0, 5200], 64, 8192),        # .. in rows of 16400 bytes: these are
     "turned_2048": ([200, 31, 0, 256, 257, 90], 2048, 264),      # reductions that start at another K tile for every expert (B^T)
     "turned_6144": ([40, 300] * 4, 6144, 72),
+    "tall": ([224, 225, 256, 255], 64, 10240),                   # 4 x 40, not cut: the last 32 rows of a tile dead, begun and full
     "short_group": ([256, 31] * 19 + [250], 64, 1904),           # 39 x 8, groups of 4
 }
 
