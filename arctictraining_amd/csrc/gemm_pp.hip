@@ -25,7 +25,8 @@ constexpr uint32_t PP_SCALE = PP_IDX + 8 * 64 * 4;   // row scales of two tiles
 constexpr uint32_t PP_PART = PP_SCALE + 2 * PP_BM * 4;   // row-sum partials, one row of 256 per wave column
 constexpr uint32_t PP_TURN = PP_PART + 4 * PP_BM * 4;    // 2 KB a wavefront for its epilogue
 constexpr uint32_t PP_LDS = PP_TURN + 8 * 2048;
-constexpr uint32_t PP_WGRAD_LDS = 2 * PP_STAGE + 8 * 2048;   // and 2 KB a wavefront for its epilogue
+constexpr uint32_t PP_WIDX = 2 * PP_STAGE + 8 * 2048;         // weight gradients: behind 2 KB a wavefront for its epilogue the indices of gathered rows
+constexpr uint32_t PP_WGRAD_LDS = PP_WIDX + 8 * 512;
 
 // ------------------------------------------------------------------ row-grouped products
 // C[rows_e,:] = A[rows_e,:] @ B[e] (B_KC false: B [Kd,N]) or @ B[e]^T (B_KC: B [N,Kd]).
@@ -729,12 +730,17 @@ __device__ __forceinline__ void pp_rows_body()
 // gradient, its number of K tiles that of the expert's rows (three at least, the missing ones empty).  Half a is 128 columns of A,
 // 64 k deep; half s of B is 32 k deep and all 256 columns wide, so that a phase is one k step of 64 x 64 a wavefront: its
 // columns then are 64 in a row, and the epilogue stores whole lines.
-// MAPS: 1 = the rows of A, 2 = the rows of B are gathered through a row map: the indices of a K tile are fetched by
-// scalar loads a phase before its offsets are worked out beside the MFMAs.
-// What bounds it: up to a few hundred rows an expert the stores of the gradients, behind which, in order, no load of their
-// wavefront completes; beyond, the MFMAs.  Alone, bf16, 64 experts of 2048 x 1408, the rows of one operand gathered,
-// gate_up's / down's gradient, us, with 64-byte pieces of rows by lanes 16 apart, ordinary stores / as now: 125 rows 286 / 148 -> 207 / 94,
-// 250 rows 328 / 173 -> 280 / 147, 375 rows 385 / 203 -> 340 / 180; 128 of 2048 x 768, 1024 rows 743 / 388 -> 730 / 354.
+// MAPS: 1 = the rows of A, 2 = the rows of B are gathered through a row map: the indices of a K tile are requested three K tiles ahead, by
+// direct-to-LDS loads among the others, and its offsets worked out beside the MFMAs.  (By scalar loads they came back out of order with
+// the LDS reads, so that every wait for those was one for all: the two parts behind the request took 420 and 460 cycles.)
+// What bounds it: per tile the stores of the gradients, behind which, in order, no load of their wavefront completes, and then the MFMAs.
+// With the loads between the first MFMAs and the indices out of the scalar unit's way the eight parts of a K tile take 2260 cycles
+// in all, of 2048 that the MFMAs take (in the memory parts, and scalar: 2990).  Alone, us, the rows of one operand gathered, gate_up's /
+// down's gradient, before / so: 64 experts of 2048 x 1408, 250 rows 277 / 143 -> 235 / 125, uneven 2048 rows 1472 / 767 -> 1316 / 749; 128 of 2048 x 768,
+// 188 rows 253 / 131 -> 218 / 119, 1024 rows 769 / 439 -> 713 / 426; 8 of 4096 x 14336, 2048 rows 3024 / 1495 -> 2886 / 1457; one of 2048 x 1408, 4001
+// rows 96 / 85 -> 81 / 79.  Stored as lanes 16 apart in pieces of 64 bytes, past no caches, 250 rows were 328 / 173, now 235 / 125.
+// Tried and not kept: loads by one group of wavefronts and stores by the other (250 rows 257 / 147: the loading group's 16 loads a part and
+// SIMD do not fit into it).
 // Rows past the expert's end read as zeros: an operand that is not gathered has a descriptor that ends with them, a
 // gathered one gets PP_NOWHERE for them.
 template <int MAPS, bool STREAM, typename ET>
@@ -750,6 +756,7 @@ __device__ __forceinline__ void pp_wgrad_body()
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
     using I4 = std::integral_constant<int, 4>;
     constexpr bool A_MAP = MAPS == 1, B_MAP = MAPS == 2;
 
@@ -785,65 +792,49 @@ __device__ __forceinline__ void pp_wgrad_body()
     // ------------------------------------------------------------ loads
     // Thread tid fills k rows tid / 16 and tid / 16 + 32 of either half (128 columns) of A, and k rows tid / 32 and tid / 32 + 16 of
     // either half (32 k) of B.
-    uint32_t aoff[2][2], boff[2][2];
-    uint32_t acol[2], bcol;           // byte offsets of its columns (PP_NOWHERE outside the matrix)
+    uint32_t arow[2], brow[4];        // gathered operand: byte offsets of its rows of the K tile (B: and columns; PP_NOWHERE past the last row)
+    uint32_t acol[2], bcol;           // byte offsets of its columns (PP_NOWHERE outside the matrix); not gathered: of its first row's
     srd_t ad, bd;
     const uint32_t lda2 = (uint32_t)pp_args().lda * 2u, ldb2 = (uint32_t)pp_args().ldb * 2u;
     int left = 0;                     // rows of the expert from the K tile loaded next
-    int row_n = 0;                    // gathered: map position of the K tile whose indices are fetched next
-    int idx[8];
+    int row_n = 0;                    // gathered: map position of the K tile whose indices are requested next
+    uint64_t map = (uint64_t)(uintptr_t)(A_MAP ? pp_args().a_row_map : pp_args().b_row_map);
+    map = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)map) |
+          ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(map >> 32)) << 32);
+    const int last_row = pp_args().rows_total - 1;
+    uint32_t slot = lds + PP_WIDX + (uint32_t)wave * 512u;        // this wavefront's indices of that K tile (two K tiles', by turns)
     auto add_sat = [](uint32_t a, uint32_t b) { return __builtin_elementwise_add_sat(a, b); };
+    // A: rows 4 wave ..+3 and those 32 on; B: rows 2 wave, 2 wave + 1 and those 16, 32 and 48 on
+    const int lane_row = A_MAP ? 4 * wave + (lane & 3) + 8 * (lane & 4) : 2 * wave + (lane & 1) + 8 * (lane & 6);
+    // the eight indices that this wavefront's loads of a K tile need, in the order in which gather_offsets reads them
     auto fetch_idx = [&]() {
         if constexpr (MAPS != 0) {
-            args_t& p = pp_args();
-            const int32_t* map = A_MAP ? p.a_row_map : p.b_row_map;
-            typedef int i32x4_t __attribute__((ext_vector_type(4), aligned(4)));
-            typedef int i32x2_t __attribute__((ext_vector_type(2), aligned(4)));
-            // A: rows 4 wave ..+3 and those 32 on; B: rows 2 wave, 2 wave + 1 and those 16, 32 and 48 on
-            constexpr int G = A_MAP ? 4 : 2, STEP = A_MAP ? 32 : 16;
-            const int row = row_n + wave * G;
-            if (row_n + 64 <= p.rows_total) {
-                if constexpr (A_MAP) {
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const i32x4_t v = *(const __attribute__((address_space(4))) i32x4_t*)(map + row + 32 * j);
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) idx[4 * j + q] = v[q];
-                    }
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const i32x2_t v = *(const __attribute__((address_space(4))) i32x2_t*)(map + row + 16 * j);
-                        idx[2 * j] = v[0];
-                        idx[2 * j + 1] = v[1];
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < 8; ++k) idx[k] = scalar_load_i32(map + min(row + STEP * (k / G) + k % G, p.rows_total - 1));
-            }
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                         :
+                         : "s"(slot), "v"((uint32_t)min(row_n + lane_row, last_row) * 4u), "s"(map)
+                         : "memory");
+            slot ^= 256u;
         }
     };
-    // offsets of the gathered operand for the K tile whose indices were fetched, of which `rows` rows exist
+    // the indices of the request before the last one, this thread's: read a part before its offsets are worked out beside the MFMAs
+    uint32_t idx[4];
+    auto read_idx = [&](uint32_t from) {
+        if constexpr (MAPS != 0) {
+            const int th = pp_here(tid);
+            const uint32_t at = from + (uint32_t)(A_MAP ? (th >> 2) & 12 : (th >> 3) & 4);
+#pragma unroll
+            for (int k = 0; k < (A_MAP ? 2 : 4); ++k) idx[k] = pp_lds<uint32_t>(at + (A_MAP ? 16u : 8u) * k);
+        }
+    };
+    // row offsets of the gathered operand for the K tile of these indices, of which `rows` rows exist
     auto gather_offsets = [&](int rows) {
         if constexpr (MAPS != 0) {
             const int th = pp_here(tid);
-            if constexpr (A_MAP) {
-                const int q = (th >> 4) & 3, kr = th >> 4;
+            const int kr = A_MAP ? th >> 4 : th >> 5;
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int i01 = q & 1 ? idx[4 * j + 1] : idx[4 * j], i23 = q & 1 ? idx[4 * j + 3] : idx[4 * j + 2];
-                    const uint32_t o = kr + 32 * j < rows ? (uint32_t)(q & 2 ? i23 : i01) * lda2 : PP_NOWHERE;
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) aoff[h][j] = add_sat(o, acol[h]);
-                }
-            } else {
-                const int kr = th >> 5;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const uint32_t r = (uint32_t)(kr & 1 ? idx[2 * k + 1] : idx[2 * k]);
-                    boff[k >> 1][k & 1] = kr + 16 * k < rows ? add_sat(r * ldb2, bcol) : PP_NOWHERE;
-                }
+            for (int k = 0; k < (A_MAP ? 2 : 4); ++k) {
+                const uint32_t o = A_MAP ? idx[k] * lda2 : add_sat(idx[k] * ldb2, bcol);
+                (A_MAP ? arow : brow)[k] = kr + (A_MAP ? 32 : 16) * k < rows ? o : PP_NOWHERE;
             }
         }
     };
@@ -870,32 +861,27 @@ __device__ __forceinline__ void pp_wgrad_body()
         for (int h = 0; h < 2; ++h) {
             const int m = t.m0 + h * 128 + col;
             acol[h] = m < p.M ? (uint32_t)m * 2u : PP_NOWHERE;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                if (!A_MAP) aoff[h][j] = add_sat((uint32_t)(kr + 32 * j) * lda2, acol[h]);
-                if (!B_MAP) boff[h][j] = add_sat((uint32_t)(krb + 32 * h + 16 * j) * ldb2, bcol);
-            }
+            if (!A_MAP) acol[h] = add_sat((uint32_t)kr * lda2, acol[h]);
         }
-        gather_offsets(left);
+        if (!B_MAP) bcol = add_sat((uint32_t)krb * ldb2, bcol);
     };
     auto next_k = [&]() {             // on to the next K tile of the same tile
         left -= PP_BK;
         if (!A_MAP) pp_advance(ad, PP_BK * lda2);
         if (!B_MAP) pp_advance(bd, PP_BK * ldb2);
         limit();
-        gather_offsets(left);
     };
     uint32_t fill = lds + (uint32_t)wave * 1024u;
-    auto dma_a = [&](auto A_) {
-        constexpr int a = decltype(A_)::value;
-        pp_dma16<a * PP_HALF>(ad, aoff[a][0], fill);
-        pp_dma16<a * PP_HALF + 8192u>(ad, aoff[a][1], fill);
+    // load J_ of the two of half H_ of A (Op_ 0) or B (1)
+    auto dma = [&](auto Op_, auto H_, auto J_) {
+        constexpr int h = decltype(H_)::value, j = decltype(J_)::value;
+        if constexpr (decltype(Op_)::value == 0)
+            pp_dma16<h * PP_HALF + j * 8192u>(ad, add_sat(A_MAP ? arow[j] : 32u * j * lda2, acol[h]), fill);
+        else
+            pp_dma16<(2 + h) * PP_HALF + j * 8192u>(bd, B_MAP ? brow[2 * h + j] : add_sat((32u * h + 16u * j) * ldb2, bcol), fill);
     };
-    auto dma_b = [&](auto B_) {
-        constexpr int b = decltype(B_)::value;
-        pp_dma16<(2 + b) * PP_HALF>(bd, boff[b][0], fill);
-        pp_dma16<(2 + b) * PP_HALF + 8192u>(bd, boff[b][1], fill);
-    };
+    auto dma_a = [&](auto H_) { dma(I0{}, H_, I0{}); dma(I0{}, H_, I1{}); };
+    auto dma_b = [&](auto H_) { dma(I1{}, H_, I0{}); dma(I1{}, H_, I1{}); };
 
     // ------------------------------------------------------------ fragments
     frag_t fa[4][2], fb0[4], fb1[4];
@@ -932,13 +918,29 @@ __device__ __forceinline__ void pp_wgrad_body()
 #pragma unroll
         for (int j = 0; j < 4; ++j) fb[j] = read_tr(rb[j] + decltype(S_)::value * PP_HALF, 2048u);
     };
-    // step S_ of the K tile; FIRST: the half's first one, nothing to add to
-    auto mma = [&](auto FIRST, auto S_, auto N_, mfma_f32x4 (&c)[4][4], const frag_t (&fb)[4]) {
+    // step S_ of the K tile; FIRST: the half's first one, nothing to add to.  The phase's two loads (of half H_ of operand Op_) are issued
+    // behind the first two MFMAs: a load takes the address unit, which four wavefronts share, 16 cycles.  dead: the half lies past the
+    // matrix (asked once, and behind the first MFMAs: a branch around all of a phase is two, taken ones)
+    auto mma = [&](auto FIRST, auto S_, bool dead, mfma_f32x4 (&c)[4][4], const frag_t (&fb)[4], auto Op_, auto H_) {
+        auto one = [&](int i, int j) {
+            c[i][j] = Mfma16<ET>::run(fb[j], fa[i][decltype(S_)::value], decltype(FIRST)::value ? mfma_f32x4{0.f, 0.f, 0.f, 0.f} : c[i][j]);
+        };
+        one(0, 0);
+        pp_fence();
+        dma(Op_, H_, I0{});
+        pp_fence();
+        one(0, 1);
+        pp_fence();
+        dma(Op_, H_, I1{});
+        pp_fence();
+        one(0, 2);
+        one(0, 3);
+        if (!dead) {
 #pragma unroll
-        for (int i = 0; i < decltype(N_)::value; ++i)
+            for (int i = 1; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                c[i][j] = Mfma16<ET>::run(fb[j], fa[i][decltype(S_)::value], decltype(FIRST)::value ? mfma_f32x4{0.f, 0.f, 0.f, 0.f} : c[i][j]);
+                for (int j = 0; j < 4; ++j) one(i, j);
+        }
     };
 
     // ------------------------------------------------------------ tile state
@@ -995,91 +997,103 @@ __device__ __forceinline__ void pp_wgrad_body()
         }
     };
 
+    // The waits: phase n awaits the loads issued in phase n - 5, which the next phase reads after the barrier; those of the four phases
+    // since stay in flight, and a request for indices, which one of the four phases of a K tile issues behind its wait.
+    // Indices of K tile t + 3 are requested in K tile t, and their offsets worked out in the next one: for A, loaded from phase 2 on, in phase 1,
+    // whose memory part is the shorter one; for B, loaded from phase 1 on, in phase 0.
+    constexpr int IDX = A_MAP ? 1 : B_MAP ? 0 : -1;
+    auto landed = [&](auto PHASE) { pp_vmwait<8 + (MAPS != 0 && decltype(PHASE)::value != IDX)>(); };
     auto run_tile = [&]() {
         mfma_f32x4 acc[2][4][4];
         const int KT = max(3, (cur.r1 - cur.r0 + PP_BK - 1) >> 6);
+        auto indices = [&](auto PHASE, int t) {
+            if constexpr (decltype(PHASE)::value == IDX) {
+                read_idx(slot ^ 256u);
+                row_n = t == KT - 3 ? nxt.r0 : row_n + PP_BK;
+                fetch_idx();
+            }
+        };
+        auto offsets = [&](auto PHASE) {
+            if constexpr (decltype(PHASE)::value == IDX) gather_offsets(left);
+        };
         // ---- phase 0 of the first K tile
         read_a(I0{}, I4{});
-        dma_a(I1{});
-        fill ^= PP_STAGE;
-        pp_vmwait<10>();
+        landed(I0{});
+        indices(I0{}, 0);
         pp_barrier();
-        mma(T_{}, I0{}, I4{}, acc[0], fb0);
+        mma(T_{}, I0{}, false, acc[0], fb0, I0{}, I1{});
+        fill ^= PP_STAGE;
         next_k();
+        offsets(I0{});
         have_nn = have_n && (q += 32) < q_end && decode(q, far);
         if (!have_nn) far = Tile{0, 0, 0, 0, 0};
         pp_barrier();
-        auto k_tile = [&](auto FIRST, auto TURN, auto N_, bool turn_next) {
+        // the lower half of the tile lies past the matrix
+        const bool half = cur.m0 + 128 >= pp_args().M;
+        auto k_tile = [&](auto FIRST, auto TURN, int t) {
             // phase 1
             read_b(I1{}, fb1);
-            if (decltype(TURN)::value) plan(nxt);
-            dma_b(I0{});
-            pp_vmwait<10>();
+            if (decltype(TURN)::value) {
+                plan(nxt);
+                if constexpr (B_MAP) {
+                    read_idx(slot);
+                    gather_offsets(left);
+                }
+            }
+            landed(I1{});
+            indices(I1{}, t);
             pp_barrier();
-            mma(F_{}, I1{}, I4{}, acc[0], fb1);
+            mma(F_{}, I1{}, false, acc[0], fb1, I1{}, I0{});
+            offsets(I1{});
             pp_barrier();
             // phase 2
-            read_a(I1{}, N_);
-            dma_a(I0{});
-            pp_vmwait<10>();
+            read_a(I1{}, I4{});
+            landed(I2{});
             pp_barrier();
-            mma(FIRST, I0{}, N_, acc[1], fb0);
+            mma(FIRST, I0{}, half, acc[1], fb0, I0{}, I0{});
             pp_barrier();
             // phase 3
             flip();
             read_b(I0{}, fb0);
-            dma_b(I1{});
-            pp_vmwait<10>();
+            landed(I3{});
             pp_barrier();
-            mma(F_{}, I1{}, N_, acc[1], fb1);
-            row_n = turn_next ? nxt.r0 : row_n + PP_BK;
-            fetch_idx();
+            mma(F_{}, I1{}, half, acc[1], fb1, I1{}, I1{});
             pp_barrier();
             // phase 0 of the next K tile
             read_a(I0{}, I4{});
-            dma_a(I1{});
-            fill ^= PP_STAGE;
-            pp_vmwait<10>();
+            landed(I0{});
+            indices(I0{}, t + 1);
             pp_barrier();
-            mma(F_{}, I0{}, I4{}, acc[0], fb0);
+            mma(F_{}, I0{}, false, acc[0], fb0, I0{}, I1{});
+            fill ^= PP_STAGE;
             if (decltype(TURN)::value) prepare_epilogue();
             next_k();
+            offsets(I0{});
             pp_barrier();
         };
-        // the lower half of the tile lies past the matrix (not told apart without a gathered operand: there the second
-        // copy of the loop spills)
-        const bool half = MAPS != 0 && cur.m0 + 128 >= pp_args().M;
-        k_tile(T_{}, F_{}, I4{}, KT == 3);
-        int t = 1;
-        int full = half ? 0 : KT - 2;
-        asm("" : "+s"(full));       // (left to see that one of the two loops is empty, the compiler branches between them)
-        for (; t < full; ++t) k_tile(F_{}, F_{}, I4{}, t == KT - 3);
-        if constexpr (MAPS != 0)
-            for (; t < KT - 2; ++t) k_tile(F_{}, F_{}, I0{}, t == KT - 3);
-        k_tile(F_{}, T_{}, I4{}, false);
+        k_tile(T_{}, F_{}, 0);
+        for (int t = 1; t < KT - 2; ++t) k_tile(F_{}, F_{}, t);
+        k_tile(F_{}, T_{}, KT - 2);
         // ---- last K tile: the epilogue of each finished half in the memory parts of the phases after it
         read_b(I1{}, fb1);
-        dma_b(I0{});
-        pp_vmwait<10>();
+        landed(I1{});
+        indices(I1{}, KT - 1);
         pp_barrier();
-        mma(F_{}, I1{}, I4{}, acc[0], fb1);
+        mma(F_{}, I1{}, false, acc[0], fb1, I1{}, I0{});
+        offsets(I1{});
         pp_barrier();
         read_a(I1{}, I4{});
-        dma_a(I0{});
         epilogue(I0{}, I0{}, acc[0]);
-        pp_vmwait<10>();
+        landed(I2{});
         pp_barrier();
-        mma(F_{}, I0{}, I4{}, acc[1], fb0);
+        mma(F_{}, I0{}, false, acc[1], fb0, I0{}, I0{});
         pp_barrier();
         flip();
         read_b(I0{}, fb0);
-        dma_b(I1{});
         epilogue(I0{}, I2{}, acc[0]);
-        pp_vmwait<10>();
+        landed(I3{});
         pp_barrier();
-        mma(F_{}, I1{}, I4{}, acc[1], fb1);
-        row_n += PP_BK;
-        fetch_idx();
+        mma(F_{}, I1{}, false, acc[1], fb1, I1{}, I1{});
         pp_barrier();
         epilogue(I1{}, I0{}, acc[1]);
         epilogue(I1{}, I2{}, acc[1]);
@@ -1088,20 +1102,26 @@ __device__ __forceinline__ void pp_wgrad_body()
     // ------------------------------------------------------------ the workgroup's tiles
     row_n = cur.r0;
     fetch_idx();
+    row_n += PP_BK;
+    fetch_idx();
+    if constexpr (MAPS != 0) pp_vmwait<0>();
     plan(cur);
+    read_idx(slot);
+    gather_offsets(left);
+    row_n += PP_BK;
+    if constexpr (MAPS != 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the next request takes the place of those just read)
+    fetch_idx();
     dma_b(I0{}); dma_a(I0{}); dma_b(I1{}); dma_a(I1{});
     fill ^= PP_STAGE;
-    row_n += PP_BK;
-    fetch_idx();
     next_k();
+    read_idx(slot);
+    gather_offsets(left);
     dma_b(I0{}); dma_a(I0{}); dma_b(I1{});
-    row_n += PP_BK;
-    fetch_idx();
     pp_vmwait<12>();
     pp_barrier();
     if (grp == 1) pp_barrier();
     read_b(I0{}, fb0);
-    pp_vmwait<10>();
+    pp_vmwait<8>();   // (no request for indices is among the loads since: phase 0 would await one too few)
     pp_barrier();
     pp_barrier();
     for (;;) {
