@@ -5,7 +5,8 @@
 // streams its part of the weights straight into registers: no LDS and no barrier before the last sum, so every wavefront
 // on a compute unit has its own two 8 KB steps in flight.
 //
-// A workgroup owns MT x 16 rows of an expert and 16 * CPL columns, its NW wavefronts take every NW-th step of 32 k.
+// A workgroup owns MT x 16 rows of an expert and 16 * CPL columns, its NW wavefronts take every NW-th step of 32 k; or CW such
+// groups of wavefronts stand side by side in the columns.
 // Lane (lq, l16) loads, for each of the 8 k of its quarter lq, the CPL columns l16 * CPL .. of the row of B (256 or 128
 // contiguous bytes per row and quarter); byte permutes of two such rows give the MFMA operands: fragment j holds column
 // l16 * CPL + j.  The wavefronts' partial sums meet in LDS, in a fixed order.
@@ -45,14 +46,18 @@ struct MfmaSkinny<f16_t> {
 
 // source_of(row): the row of A that stands for a row; scale_of(row): its factor in the gated epilogue
 // SHARED: C is stored where workgroups of other XCDs see it (agent scope: through the L2s)
-template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET, bool SHARED = false, typename SourceOf, typename ScaleOf>
-__device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[NW][CPL * 64], int e, int m0, int mend, int n0,
+// CW groups of NW wavefronts stand side by side in the columns, n0 is the first one's
+template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET, bool SHARED = false, int CW = 1, typename SourceOf, typename ScaleOf>
+__device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_all)[CW * NW][CPL * 64], int e, int m0, int mend, int n0,
                                             SourceOf source_of, ScaleOf scale_of)
 {
     constexpr int W = CPL / 2, H = CPL / 4;           // dwords of a lane's row, groups of four columns
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x % (NW * 64), lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = CW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (NW * 64));
     const int l16 = lane & 15, lq = lane >> 4;
+    sk_f32x4 (*const red)[CPL * 64] = red_all + group * NW;
+    n0 += group * 16 * CPL;
 
     const int steps = p.Kd / 32;                      // (the reduction length is a multiple of 32)
     const uint32_t row_bytes = (uint32_t)p.ldb * 2u;
@@ -138,7 +143,9 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[N
                 red[wave][(v * H + h) * 64 + lane] =
                     sk_f32x4{acc[i][4 * h][v], acc[i][4 * h + 1][v], acc[i][4 * h + 2][v], acc[i][4 * h + 3][v]};
         __syncthreads();
-        for (int u = tid; u < 4 * H * 64; u += NW * 64) {
+        int first = threadIdx.x;   // (worked out here: held across the reduction it spills)
+        asm volatile("" : "+v"(first));
+        for (int u = first % (NW * 64); u < 4 * H * 64; u += NW * 64) {
             sk_f32x4 c = red[0][u];
 #pragma unroll
             for (int w = 1; w < NW; ++w) c += red[w][u];
@@ -164,12 +171,12 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red)[N
 
 // A map's tile is 16 * MT rows where the launch's own rule built it; the taller tiles of a map that was built for another
 // bound of the rows are walked in parts.
-template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET>
+template <int MT, int CPL, int NW, int CW, int EPI, int ACT, bool STREAM, typename ET>
 __device__ __forceinline__ void skinny_body(const GemmArgs& p)
 {
-    __shared__ sk_f32x4 red[NW][CPL * 64];
+    __shared__ sk_f32x4 red[CW * NW][CPL * 64];
     const int pm = blockIdx.x / p.n_ntiles;
-    const int n0 = (blockIdx.x - pm * p.n_ntiles) * 16 * CPL;
+    const int n0 = (blockIdx.x - pm * p.n_ntiles) * 16 * CPL * CW;
     int e = 0, m0 = pm * 16 * MT, mend = min(m0 + 16 * MT, p.M);   // without a map: one expert that has all p.M rows
     if (p.tile_map) {
         if (pm >= min(scalar_load_i32(p.n_mtiles), p.max_mtiles)) return;
@@ -180,45 +187,60 @@ __device__ __forceinline__ void skinny_body(const GemmArgs& p)
     }
     const auto source_of = [&](int row) { return p.a_row_map ? p.a_row_map[row] : row; };
     const auto scale_of = [&](int row) { return p.row_scale ? p.row_scale[row] : 1.0f; };
-    skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET>(p, red, e, m0, mend, n0, source_of, scale_of);
+    skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET, false, CW>(p, red, e, m0, mend, n0, source_of, scale_of);
 #pragma unroll 1
     for (m0 += 16 * MT; m0 < mend; m0 += 16 * MT) {
         __syncthreads();   // (the sums are read before the next part's are written)
-        skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET>(p, red, e, m0, mend, n0, source_of, scale_of);
+        skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET, false, CW>(p, red, e, m0, mend, n0, source_of, scale_of);
     }
 }
 
 // (at least 4 wavefronts per SIMD with 16 rows, 3 with 32)
 // STREAM: B is loaded past the caches
-template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM>
-__global__ void __launch_bounds__(NW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_bf16_kernel(GemmArgs p)
+template <int MT, int CPL, int NW, int CW, int EPI, int ACT, bool STREAM>
+__global__ void __launch_bounds__(NW * CW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_bf16_kernel(GemmArgs p)
 {
-    skinny_body<MT, CPL, NW, EPI, ACT, STREAM, bf16_t>(p);
+    skinny_body<MT, CPL, NW, CW, EPI, ACT, STREAM, bf16_t>(p);
 }
-template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM>
-__global__ void __launch_bounds__(NW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_f16_kernel(GemmArgs p)
+template <int MT, int CPL, int NW, int CW, int EPI, int ACT, bool STREAM>
+__global__ void __launch_bounds__(NW * CW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_f16_kernel(GemmArgs p)
 {
-    skinny_body<MT, CPL, NW, EPI, ACT, STREAM, f16_t>(p);
+    skinny_body<MT, CPL, NW, CW, EPI, ACT, STREAM, f16_t>(p);
 }
 
-template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM>
+template <int MT, int CPL, int NW, int CW, int EPI, int ACT, bool STREAM>
 int launch_skinny(const GemmArgs& a, int grid, hipStream_t s)
 {
     if (a.f16)
-        hipLaunchKernelGGL((grouped_gemm_skinny_f16_kernel<MT, CPL, NW, EPI, ACT, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a);
+        hipLaunchKernelGGL((grouped_gemm_skinny_f16_kernel<MT, CPL, NW, CW, EPI, ACT, STREAM>), dim3(grid), dim3(NW * CW * 64), 0, s, a);
     else
-        hipLaunchKernelGGL((grouped_gemm_skinny_bf16_kernel<MT, CPL, NW, EPI, ACT, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a);
+        hipLaunchKernelGGL((grouped_gemm_skinny_bf16_kernel<MT, CPL, NW, CW, EPI, ACT, STREAM>), dim3(grid), dim3(NW * CW * 64), 0, s, a);
     return amoe_check_launch("grouped_gemm_skinny");
 }
 
-template <int MT, int CPL, int NW, int EPI, int ACT>
+template <int MT, int CPL, int NW, int CW, int EPI, int ACT>
 int launch_skinny(GemmArgs a, int m_tiles, hipStream_t s)
 {
-    a.n_ntiles = (a.N + 16 * CPL - 1) / (16 * CPL);
+    a.n_ntiles = (a.N + 16 * CPL * CW - 1) / (16 * CPL * CW);
     const long long grid = (long long)m_tiles * a.n_ntiles;
     AMOE_REQUIRE(grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
-    if (a.stream_from) return launch_skinny<MT, CPL, NW, EPI, ACT, true>(a, (int)grid, s);
-    return launch_skinny<MT, CPL, NW, EPI, ACT, false>(a, (int)grid, s);
+    if (a.stream_from) return launch_skinny<MT, CPL, NW, CW, EPI, ACT, true>(a, (int)grid, s);
+    return launch_skinny<MT, CPL, NW, CW, EPI, ACT, false>(a, (int)grid, s);
+}
+
+// Two column groups of two wavefronts instead of four wavefronts on one: a workgroup reads 512 bytes of each row together, not
+// 256 (reads alone, 128 matrices of 2048 rows of 3072 bytes: 7.0 TB/s instead of 6.5; 1024 bytes 6.5, neighbouring workgroups on
+// one XCD 6.3), and takes twice as long, so that there have to be enough of them, and their last round not nearly empty (fits:
+// workgroups that run at a time).  Gate_up and down product, us, one group / two: 128 experts of 2048 x 768, 4 rows an expert 128 / 119 and 66 /
+// 63, 6 rows 131 / 121 and 70 / 69; 64 of 2048 x 1408, 2.5 rows 111 / 108 and 58 / 53, 6 rows 117 / 113 and 64 / 57; 160 of 2048 x 768, 2.5
+// rows 161 / 149 and 80 / 78; 128 of 1024 x 3072, 3 rows 241 / 230 and 126 / 113.  Workgroups for a compute unit, of two groups: 0.5 (8 experts of
+// 4096 columns) 142 / 231, 1.0 101 / 145, 1.3 37.4 / 37.3, 1.6 44 / 39; where three run at a time, 3.1 140 / 143, 3.5 117 / 116, 5.5 183 / 180.
+// Rows that are no multiple of 512 bytes lose: 3968 bytes 131 / 143, 22272 191 / 202.  Up to 128 rows, which may be in as few
+// experts and for which the routed form below sums in the same order: 8 tokens, 8 of 256 experts of 2560 x 768 84 / 93 and 41 / 47.
+static bool skinny_pairs(const GemmArgs& a, long long fits, int cus)
+{
+    const long long workgroups = (long long)(a.E < a.M ? a.E : a.M) * (a.N / 256);
+    return a.N % 256 == 0 && a.M > 128 && 2 * workgroups >= 3ll * cus && (workgroups <= fits || 5 * workgroups >= 6 * fits);
 }
 
 // bm: height of the map's tiles; R rows of a.E experts
@@ -231,9 +253,14 @@ int launch_height(const GemmArgs& a, int bm, hipStream_t s)
     if (m_tiles > R) m_tiles = R;
     if (m_tiles > a.max_mtiles) m_tiles = a.max_mtiles;
     AMOE_REQUIRE(bm == 16 || bm == 32, AMOE_ERR_UNSUPPORTED, "grouped_gemm: no kernel for tiles of %d rows", bm);
-    if (bm == 32) return launch_skinny<2, 8, 4, EPI, ACT>(a, m_tiles, s);
-    if (skinny_narrow(m_tiles, a.N, device_cu_count())) return launch_skinny<1, 4, 8, EPI, ACT>(a, m_tiles, s);
-    return launch_skinny<1, 8, 4, EPI, ACT>(a, m_tiles, s);
+    const int cus = device_cu_count();
+    if (bm == 32) {
+        if (skinny_pairs(a, 3 * cus, cus)) return launch_skinny<2, 8, 2, 2, EPI, ACT>(a, m_tiles, s);
+        return launch_skinny<2, 8, 4, 1, EPI, ACT>(a, m_tiles, s);
+    }
+    if (skinny_narrow(m_tiles, a.N, cus)) return launch_skinny<1, 4, 8, 1, EPI, ACT>(a, m_tiles, s);
+    if (skinny_pairs(a, 4 * cus, cus)) return launch_skinny<1, 8, 2, 2, EPI, ACT>(a, m_tiles, s);
+    return launch_skinny<1, 8, 4, 1, EPI, ACT>(a, m_tiles, s);
 }
 
 // ------------------------------------------------------------------ gate_up product with the routing of a few tokens
@@ -554,8 +581,8 @@ AMOE_EXPORT int amoe_router_input_grad_rows(const void* d_logits, int ld, const 
     a.ldb = a.ldc = a.N = H;
     a.E = 1;
     a.M = T;
-    if (T <= 16) return launch_skinny<1, 4, 8, EPI_STORE, 0>(a, 1, (hipStream_t)stream);
-    return launch_skinny<2, 8, 4, EPI_STORE, 0>(a, (T + 31) / 32, (hipStream_t)stream);
+    if (T <= 16) return launch_skinny<1, 4, 8, 1, EPI_STORE, 0>(a, 1, (hipStream_t)stream);
+    return launch_skinny<2, 8, 4, 1, EPI_STORE, 0>(a, (T + 31) / 32, (hipStream_t)stream);
 }
 
 AMOE_EXPORT int amoe_router_input_grad(const void* d_logits, const void* w, void* out, int dtype, int T, int E, int H, void* stream)
