@@ -44,11 +44,16 @@ struct Listed {
 // LDS sees dwords; 16-byte chunk c of LDS row h is kept at c ^ ((h / 8) % 16), which spreads a wavefront's dwords (8 rows
 // apart) over all banks.  Wide tiles for long pieces: with 128 or 64 columns the split side is accessed in pieces of 256
 // or 128 bytes instead of 512, and gate and up of the size above take 288 or 298 us, with 256 270.
-template <int TH, int G, bool PACK, typename SPLIT>
-__global__ void __launch_bounds__(256) remap16_kernel(SPLIT split, uint16_t* __restrict__ joint, int I, int H, long long joint_es)
+// NT: threads.  Export of more than a few tiles takes 512, each with half of the vectors: twice the wavefronts stand on a compute
+// unit, which holds two tiles either way.  A launch (32 experts) of gate and up / of down, us, 256 / 512: 2048 x 768 70.1 / 68.0 and 37.1 /
+// 35.9, 2048 x 1408 123 / 121 and 66 / 65, 4096 x 14336 (8 experts) 638 / 626 and 356 / 343, 608 x 864 (1344 and 640 tiles) 26.0 /
+// 25.4 and 16.4 / 16.6, 512 x 160 (192 and 128) 5.6 / 6.2 and 5.0 / 4.8, 1024 x 512 (9 experts, 288 and 144) 9.1 / 8.9 and 5.4 / 6.0.  Import so
+// 70 / 71 and 36 / 37.
+template <int TH, int G, bool PACK, int NT, typename SPLIT>
+__global__ void __launch_bounds__(NT) remap16_kernel(SPLIT split, uint16_t* __restrict__ joint, int I, int H, long long joint_es)
 {
     constexpr int W = 64, ROWS = W * 2 / G;     // dwords of a joint row, rows i
-    constexpr int NS = W * TH / 8 / 256, NJ = TH * W / 4 / 256;
+    constexpr int NS = W * TH / 8 / NT, NJ = TH * W / 4 / NT;
     __shared__ __attribute__((aligned(16))) uint32_t tile[TH * W];
     typedef uint32_t vec_t __attribute__((ext_vector_type(4)));
     const int tid = threadIdx.x;
@@ -59,7 +64,7 @@ __global__ void __launch_bounds__(256) remap16_kernel(SPLIT split, uint16_t* __r
     auto at = [](int h, int d) { return h * W + (((d >> 2) ^ (h >> 3)) & 15) * 4 + (d & 3); };
     // vector n of this thread: split side, rows of dword d and column h; joint side, row h and column c
     auto split_at = [&](int n, int& d, int& hh, long long& off) {
-        const int v = tid + n * 256;
+        const int v = tid + n * NT;
         d = v / (TH / 8);
         hh = v % (TH / 8) * 8;
         const int i = i0 + (G == 2 ? d : 2 * d);
@@ -67,7 +72,7 @@ __global__ void __launch_bounds__(256) remap16_kernel(SPLIT split, uint16_t* __r
         return i < I && h0 + hh < H;
     };
     auto joint_at = [&](int n, int& hh, int& d, long long& off) {
-        const int v = tid + n * 256;
+        const int v = tid + n * NT;
         hh = v / (W / 4);
         d = v % (W / 4) * 4;
         const int c = G * i0 + 2 * d;
@@ -105,9 +110,9 @@ __global__ void __launch_bounds__(256) remap16_kernel(SPLIT split, uint16_t* __r
 #pragma unroll
         for (int n = 0; n < NJ; ++n) {
             const bool in = joint_at(n, hh, d, off);
-            // (the narrow form without a branch, what is past the end a copy of the first: around branches the compiler keeps eight
-            // vectors as one value of 232 registers)
-            if (TH < 256 || in) x[n] = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(j + (in ? off : 0)));
+            // (eight vectors without a branch, what is past the end a copy of the first: around branches the compiler keeps them as
+            // one value of 232 registers)
+            if (NJ <= 8 || in) x[n] = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(j + (in ? off : 0)));
         }
 #pragma unroll
         for (int n = 0; n < NJ; ++n) {
@@ -212,12 +217,16 @@ void launch(bool wide, const SPLIT& split, void* joint, int E, int I, int H, hip
         // (64 x 64 tiles: 244 and 239 at 288.)  Rows that are no multiple of 64 bytes are exported
         // faster by wide tiles: 272 309 / 300, 296 346 / 308.
         const bool narrow = H <= 96 || (H > 256 && H <= 384 && (PACK || H % 32 == 0));
-        auto run = [&](auto TH) {
+        auto run = [&](auto TH, auto NT) {
             const dim3 grid((H + TH - 1) / TH, (I * G + 127) / 128, E);
-            hipLaunchKernelGGL((remap16_kernel<decltype(TH)::value, G, PACK, SPLIT>), grid, dim3(256), 0, s, split, (uint16_t*)joint, I, H, joint_es);
+            hipLaunchKernelGGL((remap16_kernel<decltype(TH)::value, G, PACK, decltype(NT)::value, SPLIT>), grid, dim3(NT), 0, s, split, (uint16_t*)joint, I, H, joint_es);
         };
-        if (narrow) run(std::integral_constant<int, 128>{});
-        else run(std::integral_constant<int, 256>{});
+        typedef std::integral_constant<int, 128> N128;
+        typedef std::integral_constant<int, 256> N256;
+        const long long tiles = (long long)((H + 255) / 256) * ((I * G + 127) / 128) * E;
+        if (narrow) run(N128{}, N256{});
+        else if (PACK || tiles < 1024) run(N256{}, N256{});
+        else run(N256{}, std::integral_constant<int, PACK ? 256 : 512>{});
     }
 }
 
