@@ -6,13 +6,15 @@
 // had 3e-7 to 1.1e-6 (K 256 to 4096; weight gradients of 5 to 700 rows 0.3 to 1.5e-7, before 0.4 to 4.8e-7), whatever the
 // operands' magnitude: what bfloat16's range does not hold of the parts is dealt with at split3 and redo_exact.
 //
-// What bounds it: vector instructions (13 to split two values; a SIMD does not overlap them with its matrix instructions) and
+// What bounds it: vector instructions, 13 to split two values (of the 16 cycles of a matrix instruction 8 are free for those of either
+// wavefront, two of them; there are four and a half to one, so that putting them between the MFMAs of the step before gained nothing) and
 // LDS traffic (three planes of every stage), so that tiles are as wide as the number of them allows.  One MI355X, 39 experts
 // x 709 rows, 768 x 1856 and 928 x 768: A B 800 and 407 -> 549 and 281 us, A B^T 416 and 782 -> 285 and 520, weight
 // gradients 423 and 827 -> 275 and 503 (140-157 TFLOP/s; the float32 instruction's peak is 157).  8 experts x 512 rows,
-// 512 x 2048 and 1024 x 512: 106 and 68 -> 77 and 55, 61 and 131 -> 46 and 94, 61 and 100 -> 43 and 61: there are about as
-// many tiles as compute units, the last round is half empty.  Dealing each XCD a contiguous eighth of the tiles changed none of these figures.
+// 512 x 2048 and 1024 x 512: 106 and 68 -> 77 and 44, 61 and 131 -> 46 and 81, 61 and 100 -> 43 and 61: there are about as
+// many tiles as compute units, and the last round's few are worked off in parts (most_in_parts).  Dealing each XCD a contiguous eighth of the tiles changed none of these figures.
 #include "amoe_common.h"
+#include "gemm_launch.h"
 
 #include <type_traits>
 
@@ -43,6 +45,8 @@ struct GemmArgsF32 {
     float* inter;              // gated products: [R, N / 2]
     const float* row_scale;    // null: 1
     int act;
+    int max_mtiles;            // entries of tile_map
+    int cus;                   // compute units; 0: every tile is whole
 };
 
 // Gated products: a vector of C is (gate, up) of two intermediate columns, which leave the epilogue as row_scale up act(gate).
@@ -178,6 +182,138 @@ __device__ __forceinline__ void redo_exact(int rows, int cols, int k_len, FA a_a
         }
 }
 
+// A tile of 32 rows x 64 columns whose NW wavefronts take every NW-th step of 32 k: both operands go straight into registers, and
+// the partial sums meet in LDS, in a fixed order.  (The two halves of 16 rows in turn, a row of red for each wavefront.)
+template <bool B_KC, bool GATED, int NW>
+__device__ __forceinline__ void deep_tile(const GemmArgsF32& p, const int4& tm, int m0, int n0, f32x4_t (*red)[4 * 64])
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lq = lane >> 4;
+    const int mend = tm.z, k_len = p.Kd;
+    const float* const Bb = p.B + (long long)tm.x * p.strideB;
+
+    // (copies past the ends as above)
+    const float* a_ptr[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        int gr = min(m0 + i * 16 + l16, mend - 1);
+        if (p.a_row_map) gr = p.a_row_map[gr];
+        a_ptr[i] = p.A + (long long)gr * p.lda;
+    }
+    // Fragment j: K-contiguous, column j * 16 + l16, two vectors of four k; K-strided, column 4 l16 + j, of the eight k rows' vectors
+    // of four columns each.
+    const float* b_ptr[B_KC ? 4 : 1];
+#pragma unroll
+    for (int j = 0; j < (B_KC ? 4 : 1); ++j)
+        b_ptr[j] = B_KC ? Bb + (long long)min(n0 + j * 16 + l16, p.N - 1) * p.ldb : Bb + min(n0 + 4 * l16, p.N - 4);
+
+    f32x4_t xa[2][2], xb[8];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int k = min(k0 + 16 * h + 4 * lq, k_len - 4);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) xa[i][h] = *reinterpret_cast<const f32x4_t*>(a_ptr[i] + k);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                xb[h * 4 + j] = *reinterpret_cast<const f32x4_t*>(B_KC ? b_ptr[B_KC ? j : 0] + k : b_ptr[0] + (long long)(k + j) * p.ldb);
+        }
+    };
+    mfma_f32x4 hi[2][4], lo[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) hi[i][j] = lo[i][j] = mfma_f32x4{0.f, 0.f, 0.f, 0.f};
+    const int stride = NW * BK;
+    fetch(wave * BK);
+    for (int k0 = wave * BK; k0 < k_len; k0 += stride) {
+        if (k0 + BK > k_len) {
+            const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (k0 + 16 * h + 4 * lq >= k_len) {   // (zeros in one operand would do but for infinities in the other's copies)
+                    xa[0][h] = xa[1][h] = zero4;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) xb[h * 4 + j] = zero4;
+                }
+        }
+        auto join = [&](const f32x4_t& x0, const f32x4_t& x1, mfma_bf16x8 (&f)[3]) {
+            u32x2_t s0[3], s1[3];
+            split3(x0, s0);
+            split3(x1, s1);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) f[q] = __builtin_bit_cast(mfma_bf16x8, u32x4_t{s0[q][0], s0[q][1], s1[q][0], s1[q][1]});
+        };
+        mfma_bf16x8 fa[2][3], fb[4][3];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) join(xa[i][0], xa[i][1], fa[i]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (B_KC) join(xb[j], xb[4 + j], fb[j]);
+            else join(f32x4_t{xb[0][j], xb[1][j], xb[2][j], xb[3][j]}, f32x4_t{xb[4][j], xb[5][j], xb[6][j], xb[7][j]}, fb[j]);
+        }
+        fetch(k0 + stride);
+        auto mma = [&](int qa, int qb, mfma_f32x4 (&c)[2][4]) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) c[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j][qb], fa[i][qa], c[i][j], 0, 0, 0);
+        };
+        mma(0, 0, hi);
+        mma(1, 0, lo);
+        mma(2, 0, lo);
+        mma(0, 1, lo);
+        mma(1, 1, lo);
+        mma(0, 2, lo);
+    }
+
+    // the wavefronts' sums, 16 rows at a time.  Lane (lq, l16) holds row l16 and, for j and v, column j * 16 + 4 lq + v (K-contiguous) or
+    // 16 lq + 4 v + j (K-strided): four neighbouring columns are one vector.
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if (i) __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            f32x4_t c;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) c[w] = B_KC ? hi[i][u][w] + lo[i][u][w] : hi[i][w][u] + lo[i][w][u];
+            red[wave][u * 64 + lane] = c;
+        }
+        __syncthreads();
+        if (tid < 256) {
+            f32x4_t c = red[0][tid];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) c += red[w][tid];
+            c *= SUM_SCALE;
+            finite = finite && finite4(c);
+            const int l = tid & 63, u = tid >> 6;
+            const int row = m0 + i * 16 + (l & 15), col = n0 + (B_KC ? u * 16 + 4 * (l >> 4) : 16 * (l >> 4) + 4 * u);
+            if (row < mend && col < p.N) {
+                *reinterpret_cast<f32x4_t*>(p.C + (long long)row * p.ldc + col) = c;
+                if constexpr (GATED) store_gated(p, row, col, c);
+            }
+        }
+    }
+    if (!__syncthreads_or(!finite) || wave) return;
+    redo_exact(32, 64, k_len,
+               [&](int i, int k) {
+                   const int gr = min(m0 + i, mend - 1);
+                   return p.A + (long long)(p.a_row_map ? p.a_row_map[gr] : gr) * p.lda + k;
+               },
+               [&](int k, int j) { return B_KC ? Bb + (long long)min(n0 + j, p.N - 1) * p.ldb + k : Bb + (long long)k * p.ldb + min(n0 + j, p.N - 1); },
+               [&](int i, int j, float c) {
+                   if (m0 + i < mend && n0 + j < p.N) p.C[(long long)(m0 + i) * p.ldc + n0 + j] = c;
+               });
+    if constexpr (GATED) store_gated_again(p, m0, mend, n0, 32, 64);
+}
+
+// Up to how many tiles of the last round are worked off in parts, behind `full` others.  8 experts of 512 x 1024 to 1440 x 1024, 4096 rows, down
+// product and data gradient of gate_up (twice as deep, B^T), tiles on a compute unit, us, whole / in parts: 1.12 55 / 44 and 94 / 81, 1.27 56 / 45 and 99 /
+// 81, 1.41 56 / 50 and 97 / 98, 1.55 59 / 61 and 107 / 121; 2.53 101 / 86 and 181 / 180, 2.81 95 / 95 and 176 / 197, 3.2 112 / 103 and 204 /
+// 188; 4.5 (1024 x 2048, K = 2048 and 4096) 271 / 233 and 514 / 453; gate_up (512 x 2048) 4.5 80 / 77, 5.1 89 / 81.
+__host__ __device__ __forceinline__ int most_in_parts(int cus, int full) { return cus * (full > cus ? 10 : 7) / 16; }
+
 // ------------------------------------------------------------------ row-grouped products
 // Four wavefronts of 32 rows x 64 columns.  Each loads its rows of A straight into registers and splits them there; B is
 // split once for all four and goes through LDS.
@@ -194,8 +330,24 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
     const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem + (uint32_t)group * 2 * stage_bytes;
     const int tid = KG == 1 ? threadIdx.x : threadIdx.x % NT, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, lq = lane >> 4;
-    const int pm = blockIdx.x / p.n_ntiles, nt = blockIdx.x - pm * p.n_ntiles;
-    if (pm >= *p.n_mtiles) return;
+    const int total = min(*p.n_mtiles, p.max_mtiles) * p.n_ntiles;
+    int tile = blockIdx.x;
+    if (KG == 1 && p.cus) {
+        // The last round's tiles, if they are few, as four workgroups of 32 rows each: a round lasts as long as a tile.
+        const int full = total - total % p.cus;
+        if (full && total - full <= most_in_parts(p.cus, full) && tile >= full) {
+            const int sub = (tile - full) & 3;
+            tile = full + ((tile - full) >> 2);
+            if (tile >= total) return;
+            const int pm = tile / p.n_ntiles;
+            const int4 tm = p.tile_map[pm];
+            if (tm.y + sub * 32 >= tm.z) return;
+            deep_tile<B_KC, GATED, NT / 64>(p, tm, tm.y + sub * 32, (tile - pm * p.n_ntiles) * BN_ROWS, reinterpret_cast<f32x4_t(*)[4 * 64]>(smem));
+            return;
+        }
+    }
+    if (tile >= total) return;
+    const int pm = tile / p.n_ntiles, nt = tile - pm * p.n_ntiles;
     const int4 tm = p.tile_map[pm];
     const int m0 = tm.y + wave * 32, mend = tm.z, n0 = nt * BN_ROWS, k_len = p.Kd;
     const bool live = m0 < mend;
@@ -356,9 +508,7 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
 }
 
 // The same products where 128 x 64 tiles do not give every compute unit two workgroups: a wavefront on its own issues a
-// vector instruction in twice the time that two take in turn.  A workgroup is 32 rows (a part of a map's tile) x 64
-// columns, its eight wavefronts take every eighth step of 32 k, both operands go straight into registers, and the partial
-// sums meet in LDS, in a fixed order.
+// vector instruction in twice the time that two take in turn.  A workgroup is 32 rows (a part of a map's tile) x 64 columns.
 constexpr int NW_DEEP = 8;
 
 template <bool B_KC, bool GATED>
@@ -366,131 +516,14 @@ __global__ void __launch_bounds__(NW_DEEP * 64, 2)
 grouped_gemm_f32_deep_kernel(GemmArgsF32 p)
 {
     __shared__ f32x4_t red[NW_DEEP][4 * 64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l16 = lane & 15, lq = lane >> 4;
     const int sub = blockIdx.x / p.n_ntiles;
     const int n0 = (blockIdx.x - sub * p.n_ntiles) * 64;
     const int pm = sub / (BM_ROWS / 32);
     if (pm >= *p.n_mtiles) return;
     const int4 tm = p.tile_map[pm];
-    const int m0 = tm.y + (sub % (BM_ROWS / 32)) * 32, mend = tm.z, k_len = p.Kd;
-    if (m0 >= mend) return;
-    const float* const Bb = p.B + (long long)tm.x * p.strideB;
-
-    // (copies past the ends as above)
-    const float* a_ptr[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        int gr = min(m0 + i * 16 + l16, mend - 1);
-        if (p.a_row_map) gr = p.a_row_map[gr];
-        a_ptr[i] = p.A + (long long)gr * p.lda;
-    }
-    // Fragment j: K-contiguous, column j * 16 + l16, two vectors of four k; K-strided, column 4 l16 + j, of the eight k rows' vectors
-    // of four columns each.
-    const float* b_ptr[B_KC ? 4 : 1];
-#pragma unroll
-    for (int j = 0; j < (B_KC ? 4 : 1); ++j)
-        b_ptr[j] = B_KC ? Bb + (long long)min(n0 + j * 16 + l16, p.N - 1) * p.ldb : Bb + min(n0 + 4 * l16, p.N - 4);
-
-    f32x4_t xa[2][2], xb[8];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int k = min(k0 + 16 * h + 4 * lq, k_len - 4);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) xa[i][h] = *reinterpret_cast<const f32x4_t*>(a_ptr[i] + k);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                xb[h * 4 + j] = *reinterpret_cast<const f32x4_t*>(B_KC ? b_ptr[B_KC ? j : 0] + k : b_ptr[0] + (long long)(k + j) * p.ldb);
-        }
-    };
-    mfma_f32x4 hi[2][4], lo[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) hi[i][j] = lo[i][j] = mfma_f32x4{0.f, 0.f, 0.f, 0.f};
-    const int stride = NW_DEEP * BK;
-    fetch(wave * BK);
-    for (int k0 = wave * BK; k0 < k_len; k0 += stride) {
-        if (k0 + BK > k_len) {
-            const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                if (k0 + 16 * h + 4 * lq >= k_len) {   // (zeros in one operand would do but for infinities in the other's copies)
-                    xa[0][h] = xa[1][h] = zero4;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) xb[h * 4 + j] = zero4;
-                }
-        }
-        auto join = [&](const f32x4_t& x0, const f32x4_t& x1, mfma_bf16x8 (&f)[3]) {
-            u32x2_t s0[3], s1[3];
-            split3(x0, s0);
-            split3(x1, s1);
-#pragma unroll
-            for (int q = 0; q < 3; ++q) f[q] = __builtin_bit_cast(mfma_bf16x8, u32x4_t{s0[q][0], s0[q][1], s1[q][0], s1[q][1]});
-        };
-        mfma_bf16x8 fa[2][3], fb[4][3];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) join(xa[i][0], xa[i][1], fa[i]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (B_KC) join(xb[j], xb[4 + j], fb[j]);
-            else join(f32x4_t{xb[0][j], xb[1][j], xb[2][j], xb[3][j]}, f32x4_t{xb[4][j], xb[5][j], xb[6][j], xb[7][j]}, fb[j]);
-        }
-        fetch(k0 + stride);
-        auto mma = [&](int qa, int qb, mfma_f32x4 (&c)[2][4]) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int i = 0; i < 2; ++i) c[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j][qb], fa[i][qa], c[i][j], 0, 0, 0);
-        };
-        mma(0, 0, hi);
-        mma(1, 0, lo);
-        mma(2, 0, lo);
-        mma(0, 1, lo);
-        mma(1, 1, lo);
-        mma(0, 2, lo);
-    }
-
-    // the wavefronts' sums, 16 rows at a time.  Lane (lq, l16) holds row l16 and, for j and v, column j * 16 + 4 lq + v (K-contiguous) or
-    // 16 lq + 4 v + j (K-strided): four neighbouring columns are one vector.
-    bool finite = true;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        if (i) __syncthreads();
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            f32x4_t c;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) c[w] = B_KC ? hi[i][u][w] + lo[i][u][w] : hi[i][w][u] + lo[i][w][u];
-            red[wave][u * 64 + lane] = c;
-        }
-        __syncthreads();
-        if (tid < 256) {
-            f32x4_t c = red[0][tid];
-#pragma unroll
-            for (int w = 1; w < NW_DEEP; ++w) c += red[w][tid];
-            c *= SUM_SCALE;
-            finite = finite && finite4(c);
-            const int l = tid & 63, u = tid >> 6;
-            const int row = m0 + i * 16 + (l & 15), col = n0 + (B_KC ? u * 16 + 4 * (l >> 4) : 16 * (l >> 4) + 4 * u);
-            if (row < mend && col < p.N) {
-                *reinterpret_cast<f32x4_t*>(p.C + (long long)row * p.ldc + col) = c;
-                if constexpr (GATED) store_gated(p, row, col, c);
-            }
-        }
-    }
-    if (!__syncthreads_or(!finite) || wave) return;
-    redo_exact(32, 64, k_len,
-               [&](int i, int k) {
-                   const int gr = min(m0 + i, mend - 1);
-                   return p.A + (long long)(p.a_row_map ? p.a_row_map[gr] : gr) * p.lda + k;
-               },
-               [&](int k, int j) { return B_KC ? Bb + (long long)min(n0 + j, p.N - 1) * p.ldb + k : Bb + (long long)k * p.ldb + min(n0 + j, p.N - 1); },
-               [&](int i, int j, float c) {
-                   if (m0 + i < mend && n0 + j < p.N) p.C[(long long)(m0 + i) * p.ldc + n0 + j] = c;
-               });
-    if constexpr (GATED) store_gated_again(p, m0, mend, n0, 32, 64);
+    const int m0 = tm.y + (sub % (BM_ROWS / 32)) * 32;
+    if (m0 >= tm.z) return;
+    deep_tile<B_KC, GATED, NW_DEEP>(p, tm, m0, n0, red);
 }
 
 // ------------------------------------------------------------------ weight gradients
@@ -665,7 +698,8 @@ int amoe_f32_rows(const void* A, const int32_t* a_row_map, const void* B, const 
     a.M = R;
     a.N = N;
     a.n_ntiles = (N + BN_ROWS - 1) / BN_ROWS;
-    const long long grid = (long long)max_mtiles * a.n_ntiles;
+    a.max_mtiles = max_mtiles;
+    long long grid = (long long)max_mtiles * a.n_ntiles;
     AMOE_REQUIRE(grid * (BM_ROWS / 32) < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm(f32): grid too large");
     // Few tiles, which the wavefronts of a compute unit then have to share.  One MI355X, us (with 11 instructions for two values), one group of wavefronts / two groups / the
     // eight-wave form:
@@ -677,6 +711,11 @@ int amoe_f32_rows(const void* A, const int32_t* a_row_map, const void* B, const 
     int form = 0;
     if ((R / 32 + met) * a.n_ntiles <= 400) form = 2;
     else if ((R / 128 + met / 2 + 1) * a.n_ntiles <= 256 && Kred >= 512) form = 1;
+    const int cus = device_cu_count();
+    if (form == 0 && cus > 0 && grid > cus) {
+        a.cus = cus;
+        grid += 3 * most_in_parts(cus, 2 * cus);
+    }
     if (inter) launch_rows<false, true>(a, (int)grid, form, s);
     else if (b_kc) launch_rows<true>(a, (int)grid, form, s);
     else launch_rows<false>(a, (int)grid, form, s);
