@@ -26,7 +26,9 @@ constexpr uint32_t PP_PART = PP_SCALE + 2 * PP_BM * 4;   // row-sum partials, on
 constexpr uint32_t PP_TURN = PP_PART + 4 * PP_BM * 4;    // 2 KB a wavefront for its epilogue
 constexpr uint32_t PP_LDS = PP_TURN + 8 * 2048;
 constexpr uint32_t PP_WIDX = 2 * PP_STAGE + 8 * 2048;         // weight gradients: behind 2 KB a wavefront for its epilogue the indices of gathered rows
-constexpr uint32_t PP_WGRAD_LDS = PP_WIDX + 8 * 512;
+constexpr uint32_t PP_WDEPTH = PP_WIDX + 8 * 512;            // the experts' depths, and how their tiles are dealt
+constexpr uint32_t PP_WDEAL = PP_WDEPTH + AMOE_MAX_EXPERTS * 4;
+constexpr uint32_t PP_WGRAD_LDS = PP_WDEPTH, PP_WGRAD_DEAL_LDS = PP_WDEAL + AMOE_MAX_EXPERTS * 16;
 
 // ------------------------------------------------------------------ row-grouped products
 // C[rows_e,:] = A[rows_e,:] @ B[e] (B_KC false: B [Kd,N]) or @ B[e]^T (B_KC: B [N,Kd]).
@@ -743,7 +745,8 @@ __device__ __forceinline__ void pp_rows_body()
 // SIMD do not fit into it).
 // Rows past the expert's end read as zeros: an operand that is not gathered has a descriptor that ends with them, a
 // gathered one gets PP_NOWHERE for them.
-template <int MAPS, bool STREAM, typename ET>
+// DEAL: uneven loads may be dealt by depth
+template <int MAPS, bool STREAM, bool DEAL, typename ET>
 __device__ __forceinline__ void pp_wgrad_body()
 {
     typedef typename Elem16<ET>::frag_t frag_t;
@@ -767,16 +770,9 @@ __device__ __forceinline__ void pp_wgrad_body()
     // A workgroup takes gm tiles, one from each of gm chunks in a row.
     auto divide = [](int n, uint32_t inv) -> int { return inv ? (int)(((uint64_t)(uint32_t)n * inv) >> 32) : n; };
     struct Tile { int e, m0, n0, r0, r1; };
-    auto decode = [&](int q, Tile& t) -> bool {       // q-th tile of this XCD
+    auto locate = [&](int e, int i, Tile& t) {        // tile i of expert e
         args_t& p = pp_args();
-        const int xcd = blockIdx.x & 7;
-        const int per = p.n_mt * p.n_ntiles, total = p.E * per;
-        const int whole = total & ~255;
-        int v = ((q >> 5) << 8) + (xcd << 5) + (q & 31);
-        if (v >= whole) v = whole + ((q - (whole >> 3)) << 3) + xcd;
-        if (v >= total) return false;
-        t.e = divide(v, p.inv_super);
-        const int i = v - t.e * per;
+        t.e = e;
         const int strip = divide(i, p.inv_sn);
         const int r = i - strip * p.n_mt * p.gn;
         const bool last = strip == p.sn - 1;
@@ -786,6 +782,126 @@ __device__ __forceinline__ void pp_wgrad_body()
         t.n0 = (strip * p.gn + r - mt * w) * PP_BN;
         t.r0 = __builtin_amdgcn_readfirstlane(scalar_load_i32(p.offsets + t.e));
         t.r1 = __builtin_amdgcn_readfirstlane(scalar_load_i32(p.offsets + t.e + 1));
+    };
+    // Uneven loads: by number, the deep tiles' share of the workgroups differs by a whole one (a sixteenth of 64 experts with half of the
+    // rows: the most loaded workgroup has 1.22 times the mean of K tiles).  There the experts are taken in the order of their depth, and where
+    // the next one's tiles are lower by a fifth or more, the workgroups that the last turn did not reach are first filled up with
+    // those (1.01 times).  Alone, us, by number / by depth: 131072 such rows, 2048 x 1408, gate_up's gradient 1301 / 1160, down's 716 / 666; 65536
+    // rows of 32 experts of 7168 x 2048, Zipf loads (1.06 and 1.08 times the mean / 1.04 and 1.05) 2900 / 2860 and 1550 / 1540.  Every workgroup works
+    // the dealing out for itself, some 6 us for 64 experts: only where the deepest expert has twice the mean, and the work is fifty
+    // times that; in a kernel of its own, as the shallow tiles of two a workgroup took 1 % longer with it.
+    // A record per expert, in that order: tiles [0, fill) go in turns to the `behind` workgroups from `from` on, the first to the one
+    // `skip` further, the others to all from `from2` on.
+    const int my = (int)((blockIdx.x & 7) * 32 + (blockIdx.x >> 3));
+    const int per = pp_args().n_mt * pp_args().n_ntiles;
+    bool by_depth = false;
+    if constexpr (DEAL) {
+        args_t& p = pp_args();
+        const int E = p.E;
+        typedef __attribute__((address_space(3))) uint32_t* word_t;
+        int mine = 0;
+        if (tid < E) mine = min(max(3, (p.offsets[tid + 1] - p.offsets[tid] + PP_BK - 1) >> 6), 1 << 20) + 3;   // (a tile's stores: three K tiles)
+        *(word_t)(uintptr_t)(lds + PP_WDEPTH + tid * 4u) = (uint32_t)mine;
+        __syncthreads();
+        int sum = 0, most = 0;
+#pragma unroll
+        for (int k = 0; k < AMOE_MAX_EXPERTS / 64; ++k) {
+            const int d = pp_lds<int>(lds + PP_WDEPTH + (lane + 64 * k) * 4u);
+            sum += d;
+            most = max(most, d);
+        }
+#pragma unroll
+        for (int o = 32; o; o >>= 1) {
+            sum += __shfl_xor(sum, o, 64);
+            most = max(most, __shfl_xor(most, o, 64));
+        }
+        sum = __builtin_amdgcn_readfirstlane(sum);
+        most = __builtin_amdgcn_readfirstlane(most);
+        by_depth = (float)most * E > 2.f * sum && (float)sum * per >= 1024.f * E;
+        if (by_depth) {
+            int rank = 0;
+            for (int e = 0; e < E; e += 4) {
+                const u32x4_t d = pp_lds<u32x4_t>(lds + PP_WDEPTH + e * 4u);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) rank += (int)d[k] > mine || ((int)d[k] == mine && e + k < tid);
+            }
+            if (tid < E) *(__attribute__((address_space(3))) u32x4_t*)(uintptr_t)(lds + PP_WDEAL + rank * 16u) = u32x4_t{0, 0, (uint32_t)mine, (uint32_t)tid};
+            __syncthreads();
+            if (wave == 0) {
+                // left: K tiles that those behind lack; last: depth of the tiles dealt to all
+                int from = 0, behind = 256, skip = 0, left = 0, last = 0;
+                for (int k = 0; k < E; ++k) {
+                    const u32x4_t x = pp_lds<u32x4_t>(lds + PP_WDEAL + k * 16u);
+                    const int d = __builtin_amdgcn_readfirstlane(x[2]), e = __builtin_amdgcn_readfirstlane(x[3]);
+                    if (behind == 256 && 5 * d < 4 * last && skip) {
+                        from = (from + skip) & 255;
+                        behind = 256 - skip;
+                        left = behind * last;
+                        skip = 0;
+                    }
+                    const uint32_t w0 = (uint32_t)(from | skip << 8), w1 = (uint32_t)behind;
+                    int fill = 0;
+                    if (behind < 256) {
+                        const int want = (2 * left + d) / (2 * d);
+                        fill = min(per, want);
+                        skip = (skip + fill) % behind;
+                        left -= fill * d;
+                        if (fill == want) {
+                            from = (from + skip) & 255;
+                            behind = 256;
+                            skip = 0;
+                        }
+                    }
+                    const uint32_t w2 = (uint32_t)((from + skip) & 255) << 16;
+                    if (fill < per) {
+                        skip = (skip + per - fill) & 255;
+                        last = d;
+                    }
+                    if (lane == 0) *(__attribute__((address_space(3))) u32x4_t*)(uintptr_t)(lds + PP_WDEAL + k * 16u) = u32x4_t{w0 | w2, w1, (uint32_t)fill, (uint32_t)e};
+                }
+            }
+            __syncthreads();
+        }
+    }
+    // this workgroup's place in the dealing: expert (and its position), next tile, and the record's numbers
+    struct { int at, e, i, fill, behind, second; } deal = {-1, 0, 0, 0, 256, 0};
+    // position of the last tile taken in this XCD's queue, and the end of what this workgroup takes
+    int q = (int)(blockIdx.x >> 8) * 32 * pp_args().gm + (int)((blockIdx.x >> 3) & 31);
+    const int q_end = q + 32 * pp_args().gm;
+    q -= 32;
+    auto take = [&](Tile& t) -> bool {                // this workgroup's next tile
+        if (DEAL && by_depth) {
+            if (deal.i < deal.fill) {
+                deal.i += deal.behind;
+                if (deal.i >= deal.fill) deal.i = deal.second;
+            } else {
+                deal.i += 256;
+            }
+            while (deal.at < 0 || deal.i >= per) {
+                if (++deal.at >= pp_args().E) return false;
+                const u32x4_t x = pp_lds<u32x4_t>(lds + PP_WDEAL + deal.at * 16u);
+                const int w = __builtin_amdgcn_readfirstlane(x[0]);
+                deal.behind = __builtin_amdgcn_readfirstlane(x[1]);
+                deal.fill = __builtin_amdgcn_readfirstlane(x[2]);
+                deal.e = __builtin_amdgcn_readfirstlane(x[3]);
+                deal.second = deal.fill + ((my - (w >> 16)) & 255);
+                const int place = (my - w) & 255, turn = place - ((w >> 8) & 255);
+                const int first = turn < 0 ? turn + deal.behind : turn;
+                deal.i = place < deal.behind && first < deal.fill ? first : deal.second;
+            }
+            locate(deal.e, deal.i, t);
+            return true;
+        }
+        args_t& p = pp_args();
+        const int xcd = blockIdx.x & 7;
+        const int total = p.E * per;
+        const int whole = total & ~255;
+        if ((q += 32) >= q_end) return false;
+        int v = ((q >> 5) << 8) + (xcd << 5) + (q & 31);
+        if (v >= whole) v = whole + ((q - (whole >> 3)) << 3) + xcd;
+        if (v >= total) return false;
+        const int e = divide(v, p.inv_super);
+        locate(e, v - e * per, t);
         return true;
     };
 
@@ -945,11 +1061,8 @@ __device__ __forceinline__ void pp_wgrad_body()
 
     // ------------------------------------------------------------ tile state
     Tile cur, nxt = {0, 0, 0, 0, 0}, far = {0, 0, 0, 0, 0};
-    // position of the last tile taken in this XCD's queue, and the end of what this workgroup takes
-    int q = (int)(blockIdx.x >> 8) * 32 * pp_args().gm + (int)((blockIdx.x >> 3) & 31);
-    const int q_end = q + 32 * pp_args().gm;
-    if (!decode(q, cur)) return;
-    bool have_n = (q += 32) < q_end && decode(q, nxt), have_nn = false;
+    if (!take(cur)) return;
+    bool have_n = take(nxt), have_nn = false;
 
     // Epilogue: a wavefront's columns of the tile are 64, 128 bytes of a row.  Lane (lq, l16) holds columns 16 j + 4 lq ..+3 of row
     // l16 of every 16-row block; through 2 KB of LDS of the wavefront's own (chunk c of row r at c ^ (r & 7), its halves the other way
@@ -1025,7 +1138,7 @@ __device__ __forceinline__ void pp_wgrad_body()
         fill ^= PP_STAGE;
         next_k();
         offsets(I0{});
-        have_nn = have_n && (q += 32) < q_end && decode(q, far);
+        have_nn = have_n && take(far);
         if (!have_nn) far = Tile{0, 0, 0, 0, 0};
         pp_barrier();
         // the lower half of the tile lies past the matrix
@@ -1146,15 +1259,15 @@ __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_rows_f16_kernel
     pp_rows_body<B_KC, EPI, ACT, STREAM, f16_t>();
 }
 
-template <int MAPS, bool STREAM>
+template <int MAPS, bool STREAM, bool DEAL>
 __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_wgrad_bf16_kernel(GemmArgs)
 {
-    pp_wgrad_body<MAPS, STREAM, bf16_t>();
+    pp_wgrad_body<MAPS, STREAM, DEAL, bf16_t>();
 }
-template <int MAPS, bool STREAM>
+template <int MAPS, bool STREAM, bool DEAL>
 __global__ void __launch_bounds__(PP_THREADS, 2) grouped_gemm_pp_wgrad_f16_kernel(GemmArgs)
 {
-    pp_wgrad_body<MAPS, STREAM, f16_t>();
+    pp_wgrad_body<MAPS, STREAM, DEAL, f16_t>();
 }
 
 }  // namespace
@@ -1224,17 +1337,18 @@ int amoe_pp_gated_bwd(const GemmArgs& a, int act, hipStream_t s)
 }
 #endif
 #if AMOE_PP_PART_IS(3)
-template <int MAPS, bool STREAM>
+template <int MAPS, bool STREAM, bool DEAL>
 static int launch_pp_wgrad(const GemmArgs& a, int grid, hipStream_t s)
 {
-    if (a.f16) return launch_kernel<grouped_gemm_pp_wgrad_f16_kernel<MAPS, STREAM>, PP_THREADS, PP_WGRAD_LDS>(a, grid, s);
-    return launch_kernel<grouped_gemm_pp_wgrad_bf16_kernel<MAPS, STREAM>, PP_THREADS, PP_WGRAD_LDS>(a, grid, s);
+    constexpr int lds = DEAL ? PP_WGRAD_DEAL_LDS : PP_WGRAD_LDS;
+    if (a.f16) return launch_kernel<grouped_gemm_pp_wgrad_f16_kernel<MAPS, STREAM, DEAL>, PP_THREADS, lds>(a, grid, s);
+    return launch_kernel<grouped_gemm_pp_wgrad_bf16_kernel<MAPS, STREAM, DEAL>, PP_THREADS, lds>(a, grid, s);
 }
 template <int MAPS>
-static int launch_pp_wgrad(const GemmArgs& a, int grid, hipStream_t s)
+static int launch_pp_wgrad(const GemmArgs& a, bool deal, int grid, hipStream_t s)
 {
-    if (a.stream_from) return launch_pp_wgrad<MAPS, true>(a, grid, s);
-    return launch_pp_wgrad<MAPS, false>(a, grid, s);
+    if (a.stream_from) return deal ? launch_pp_wgrad<MAPS, true, true>(a, grid, s) : launch_pp_wgrad<MAPS, true, false>(a, grid, s);
+    return deal ? launch_pp_wgrad<MAPS, false, true>(a, grid, s) : launch_pp_wgrad<MAPS, false, false>(a, grid, s);
 }
 
 int amoe_pp_wgrad(GemmArgs a, hipStream_t s)
@@ -1261,12 +1375,14 @@ int amoe_pp_wgrad(GemmArgs a, hipStream_t s)
     // sixteenth with half of them 440 / 367; 64 of 1024 x 2048, 150 rows, on one 581 / 502, a quarter 535 / 373, a sixteenth 319 / 245.
     const long long rounds = (total + 255) / 256;
     a.gm = (int)(a.rows_total < 11ll * PP_BK * a.E && rounds > 2 ? 2 : rounds);
+    // Where a workgroup takes all that falls to it, that may be by depth (whether loads are uneven, only the device knows).
+    const bool deal = a.gm == rounds && rounds > 1 && a.E > 1 && a.E <= AMOE_MAX_EXPERTS;
     const int grid = rounds == 1 ? (int)((total + 7) & ~7ll) : (int)((rounds + a.gm - 1) / a.gm * 256);
     // Gradients that the L2s (8 x 4 MB) do not hold are stored past the caches: with ordinary stores a tile's 128 KB wait for dirty
     // lines of older ones to be written out, behind which no load of the next tile completes.
     a.stream_from = 2ll * a.E * a.M * a.N > (32ll << 20);
-    if (a.a_row_map) return launch_pp_wgrad<1>(a, grid, s);
-    if (a.b_row_map) return launch_pp_wgrad<2>(a, grid, s);
-    return launch_pp_wgrad<0>(a, grid, s);
+    if (a.a_row_map) return launch_pp_wgrad<1>(a, deal, grid, s);
+    if (a.b_row_map) return launch_pp_wgrad<2>(a, deal, grid, s);
+    return launch_pp_wgrad<0>(a, deal, grid, s);
 }
 #endif

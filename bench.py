@@ -308,7 +308,7 @@ def main():
     wgrad = f"grouped_gemm_wgrad_bf16_kernel<{tile}, " if c else "grouped_gemm_pp_wgrad_bf16_kernel<"
     end = ">" if c else ", false>"   # (every workload here has far more than a tile of rows per expert)
     plain = lambda n: 4 if c == 0 and 2 * R * n >= 128 << 20 else 0   # epilogue: plain, or plain and past the caches
-    wend = ">" if c else ", true>"   # (and gradients that the L2s do not hold)
+    wend = ">" if c else ", true, true>"   # (and gradients that the L2s do not hold)
     gathered = token_of is not None
     sym = {
         # grouped_gemm_pp_rows_bf16_kernel<B K-contiguous, epilogue, activation, B past the caches>; other tile shapes:
@@ -318,7 +318,7 @@ def main():
         "gemm_dgrad_down": f"{rows}true, {plain(I)}, 0{end}",
         "gemm_dgrad_down_gated_bwd": f"{rows}true, 2, 0{end}",
         "gemm_dgrad_gateup": f"{rows}true, {plain(H)}, 0{end}",
-        # grouped_gemm_pp_wgrad_bf16_kernel<gathered operand, stored past the caches>; other tile shapes:
+        # grouped_gemm_pp_wgrad_bf16_kernel<gathered operand, stored past the caches, may be dealt by depth>; other tile shapes:
         # grouped_gemm_wgrad_bf16_kernel<BM, BN, waves along M, waves along N, gathered operand>
         "gemm_wgrad_down": f"{wgrad}{2 if gathered else 0}{wend}",
         "gemm_wgrad_gateup": f"{wgrad}{1 if gathered else 0}{wend}",
