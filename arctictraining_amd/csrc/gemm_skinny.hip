@@ -5,11 +5,11 @@
 // streams its part of the weights straight into registers: no LDS and no barrier before the last sum, so every wavefront
 // on a compute unit has its own two 8 KB steps in flight.
 //
-// A workgroup owns MT x 16 rows of an expert and 16 * CPL columns, its NW wavefronts take every NW-th step of 32 k; or CW such
-// groups of wavefronts stand side by side in the columns.
+// A workgroup owns MT x 16 rows of an expert and 16 * CPL columns, its NW wavefronts take every NW-th step of 32 k; or two groups of
+// NW / 2 wavefronts stand side by side in the columns, and a wavefront takes two such parts of the reduction, one after the other.
 // Lane (lq, l16) loads, for each of the 8 k of its quarter lq, the CPL columns l16 * CPL .. of the row of B (256 or 128
 // contiguous bytes per row and quarter); byte permutes of two such rows give the MFMA operands: fragment j holds column
-// l16 * CPL + j.  The wavefronts' partial sums meet in LDS, in a fixed order.
+// l16 * CPL + j.  The NW parts' sums meet in LDS, in the order of the parts: the two forms give the same bits.
 //
 // One MI355X, bf16, gate_up and down product, against 256-row tiles: 128 experts of 2048 x 768, 1 row an expert 105 and
 // 55 -> 99 and 43 us, 4 rows 152 and 78 -> 145 and 74 (5.5 TB/s, what a read of that size reaches); 8 experts of
@@ -46,17 +46,19 @@ struct MfmaSkinny<f16_t> {
 
 // source_of(row): the row of A that stands for a row; scale_of(row): its factor in the gated epilogue
 // SHARED: C is stored where workgroups of other XCDs see it (agent scope: through the L2s)
-// CW groups of NW wavefronts stand side by side in the columns, n0 is the first one's
-template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET, bool SHARED = false, int CW = 1, typename SourceOf, typename ScaleOf>
-__device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_all)[CW * NW][CPL * 64], int e, int m0, int mend, int n0,
+// PAIRS: two groups of wavefronts stand side by side in the columns, n0 is the first one's
+template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET, bool SHARED = false, bool PAIRS = false, typename SourceOf, typename ScaleOf>
+__device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_all)[NW][CPL * 64], int e, int m0, int mend, int n0,
                                             SourceOf source_of, ScaleOf scale_of)
 {
     constexpr int W = CPL / 2, H = CPL / 4;           // dwords of a lane's row, groups of four columns
-    const int tid = threadIdx.x % (NW * 64), lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int group = CW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (NW * 64));
-    const int l16 = lane & 15, lq = lane >> 4;
-    sk_f32x4 (*const red)[CPL * 64] = red_all + group * NW;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+    constexpr int GW = PAIRS ? NW / 2 : NW;           // wavefronts of a group
+    int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int group = wave / GW;
+    wave %= GW;
+    static_assert(!PAIRS || (GW == 2 && MT <= GW), "a row of red for every 16 rows");
+    sk_f32x4 (*const red)[CPL * 64] = red_all + group * GW;
     n0 += group * 16 * CPL;
 
     const int steps = p.Kd / 32;                      // (the reduction length is a multiple of 32)
@@ -100,10 +102,13 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_al
             s.a[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ad, live ? aoff[i] : SK_NOWHERE, sa, 0));
     };
     sk_f32x4 acc[MT][CPL];
+    auto clear = [&]() {
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < CPL; ++j) acc[i][j] = sk_f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < CPL; ++j) acc[i][j] = sk_f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    clear();
     auto multiply = [&](const Step& s) {
 #pragma unroll
         for (int w = 0; w < W; ++w) {
@@ -121,34 +126,83 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_al
         }
     };
 
-    const int rounds = (steps + NW - 1) / NW;
-    Step s0, s1;
-    load(s0, wave);
-    for (int r = 0; r < rounds; r += 2) {
-        load(s1, (r + 1) * NW + wave);
-        multiply(s0);
-        load(s0, (r + 2) * NW + wave);
-        multiply(s1);
-    }
-
-    // the wavefronts' sums, 16 rows at a time.  Lane (lq, l16) holds columns (4 lq + v) * CPL + j of row l16.
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        if (m0 + i * 16 >= mend) break;
-        if (i) __syncthreads();
+    // Lane (lq, l16) holds columns (4 lq + v) * CPL + j of row l16.
+    auto sums = [&](int i, auto use) {
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
             for (int h = 0; h < H; ++h)
-                red[wave][(v * H + h) * 64 + lane] =
-                    sk_f32x4{acc[i][4 * h][v], acc[i][4 * h + 1][v], acc[i][4 * h + 2][v], acc[i][4 * h + 3][v]};
+                use((v * H + h) * 64 + lane, sk_f32x4{acc[i][4 * h][v], acc[i][4 * h + 1][v], acc[i][4 * h + 2][v], acc[i][4 * h + 3][v]});
+    };
+    // Part p of the reduction is the steps p, p + NW, .. (those past the last are zeros).
+    const int rounds = (steps + NW - 1) / NW;
+    Step s0, s1;
+    load(s0, wave);
+    if constexpr (!PAIRS) {
+        for (int r = 0; r < rounds; r += 2) {
+            load(s1, (r + 1) * NW + wave);
+            multiply(s0);
+            load(s0, (r + 2) * NW + wave);
+            multiply(s1);
+        }
+    } else {
+        // Row i of red takes ((part 0 + part 1) + part 2) + part 3 of rows 16 i ..+15, in two halves, of which the two
+        // wavefronts add to one each.
+        auto half = [&](int which, auto use) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                if (MT == 1 || i == which) sums(i, [&](int u, sk_f32x4 c) {
+                    if (MT > 1 || u / (2 * H * 64) == which) use(red[i][u], c);
+                });
+        };
+        const auto put = [](sk_f32x4& at, sk_f32x4 c) { at = c; };
+        const auto add = [](sk_f32x4& at, sk_f32x4 c) { at += c; };
+#pragma unroll 1
+        for (int part = wave;; part += GW) {
+            const bool last = part >= GW;
+            for (int r = 0; r + 1 < rounds; r += 2) {
+                load(s1, (r + 1) * NW + part);
+                multiply(s0);
+                load(s0, r + 2 < rounds || last ? (r + 2) * NW + part : part + GW);
+                multiply(s1);
+            }
+            if (rounds & 1) {
+                multiply(s0);
+                if (!last) load(s0, part + GW);
+            }
+            if (last) break;
+            if (wave == 0) half(1, put);
+            else half(0, put);
+            __syncthreads();
+            if (wave == 0) half(0, add);
+            else half(1, add);
+            clear();
+        }
+        if (wave == 0) half(0, add);
         __syncthreads();
+        if (wave == 0) half(1, add);
+        else half(0, add);
+        __syncthreads();
+        if (wave == 1) half(1, add);
+        __syncthreads();
+    }
+    // 16 rows at a time
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        if (m0 + i * 16 >= mend) break;
+        if constexpr (!PAIRS) {
+            if (i) __syncthreads();
+            sums(i, [&](int u, sk_f32x4 c) { red[wave][u] = c; });
+            __syncthreads();
+        }
         int first = threadIdx.x;   // (worked out here: held across the reduction it spills)
         asm volatile("" : "+v"(first));
-        for (int u = first % (NW * 64); u < 4 * H * 64; u += NW * 64) {
-            sk_f32x4 c = red[0][u];
+        for (int u = first % (GW * 64); u < 4 * H * 64; u += GW * 64) {
+            sk_f32x4 c = red[PAIRS ? i : 0][u];
+            if constexpr (!PAIRS) {
 #pragma unroll
-            for (int w = 1; w < NW; ++w) c += red[w][u];
+                for (int w = 1; w < NW; ++w) c += red[w][u];
+            }
             const int l = u & 63, q = u >> 6;
             const int row = m0 + i * 16 + (l & 15);
             const int col = n0 + ((l >> 4) * 4 + q / H) * CPL + (q % H) * 4;
@@ -171,12 +225,12 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_al
 
 // A map's tile is 16 * MT rows where the launch's own rule built it; the taller tiles of a map that was built for another
 // bound of the rows are walked in parts.
-template <int MT, int CPL, int NW, int CW, int EPI, int ACT, bool STREAM, typename ET>
+template <int MT, int CPL, int NW, bool PAIRS, int EPI, int ACT, bool STREAM, typename ET>
 __device__ __forceinline__ void skinny_body(const GemmArgs& p)
 {
-    __shared__ sk_f32x4 red[CW * NW][CPL * 64];
+    __shared__ sk_f32x4 red[NW][CPL * 64];
     const int pm = blockIdx.x / p.n_ntiles;
-    const int n0 = (blockIdx.x - pm * p.n_ntiles) * 16 * CPL * CW;
+    const int n0 = (blockIdx.x - pm * p.n_ntiles) * 16 * CPL * (PAIRS ? 2 : 1);
     int e = 0, m0 = pm * 16 * MT, mend = min(m0 + 16 * MT, p.M);   // without a map: one expert that has all p.M rows
     if (p.tile_map) {
         if (pm >= min(scalar_load_i32(p.n_mtiles), p.max_mtiles)) return;
@@ -187,45 +241,46 @@ __device__ __forceinline__ void skinny_body(const GemmArgs& p)
     }
     const auto source_of = [&](int row) { return p.a_row_map ? p.a_row_map[row] : row; };
     const auto scale_of = [&](int row) { return p.row_scale ? p.row_scale[row] : 1.0f; };
-    skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET, false, CW>(p, red, e, m0, mend, n0, source_of, scale_of);
 #pragma unroll 1
-    for (m0 += 16 * MT; m0 < mend; m0 += 16 * MT) {
+    for (;;) {
+        skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET, false, PAIRS>(p, red, e, m0, mend, n0, source_of, scale_of);
+        if ((m0 += 16 * MT) >= mend) break;
         __syncthreads();   // (the sums are read before the next part's are written)
-        skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET, false, CW>(p, red, e, m0, mend, n0, source_of, scale_of);
     }
 }
 
 // (at least 4 wavefronts per SIMD with 16 rows, 3 with 32)
 // STREAM: B is loaded past the caches
-template <int MT, int CPL, int NW, int CW, int EPI, int ACT, bool STREAM>
-__global__ void __launch_bounds__(NW * CW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_bf16_kernel(GemmArgs p)
+template <int MT, int CPL, int NW, bool PAIRS, int EPI, int ACT, bool STREAM>
+__global__ void __launch_bounds__(NW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_bf16_kernel(GemmArgs p)
 {
-    skinny_body<MT, CPL, NW, CW, EPI, ACT, STREAM, bf16_t>(p);
+    skinny_body<MT, CPL, NW, PAIRS, EPI, ACT, STREAM, bf16_t>(p);
 }
-template <int MT, int CPL, int NW, int CW, int EPI, int ACT, bool STREAM>
-__global__ void __launch_bounds__(NW * CW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_f16_kernel(GemmArgs p)
+template <int MT, int CPL, int NW, bool PAIRS, int EPI, int ACT, bool STREAM>
+__global__ void __launch_bounds__(NW * 64, MT == 1 ? 4 : 3) grouped_gemm_skinny_f16_kernel(GemmArgs p)
 {
-    skinny_body<MT, CPL, NW, CW, EPI, ACT, STREAM, f16_t>(p);
+    skinny_body<MT, CPL, NW, PAIRS, EPI, ACT, STREAM, f16_t>(p);
 }
 
-template <int MT, int CPL, int NW, int CW, int EPI, int ACT, bool STREAM>
+template <int MT, int CPL, int NW, bool PAIRS, int EPI, int ACT, bool STREAM>
 int launch_skinny(const GemmArgs& a, int grid, hipStream_t s)
 {
     if (a.f16)
-        hipLaunchKernelGGL((grouped_gemm_skinny_f16_kernel<MT, CPL, NW, CW, EPI, ACT, STREAM>), dim3(grid), dim3(NW * CW * 64), 0, s, a);
+        hipLaunchKernelGGL((grouped_gemm_skinny_f16_kernel<MT, CPL, NW, PAIRS, EPI, ACT, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a);
     else
-        hipLaunchKernelGGL((grouped_gemm_skinny_bf16_kernel<MT, CPL, NW, CW, EPI, ACT, STREAM>), dim3(grid), dim3(NW * CW * 64), 0, s, a);
+        hipLaunchKernelGGL((grouped_gemm_skinny_bf16_kernel<MT, CPL, NW, PAIRS, EPI, ACT, STREAM>), dim3(grid), dim3(NW * 64), 0, s, a);
     return amoe_check_launch("grouped_gemm_skinny");
 }
 
-template <int MT, int CPL, int NW, int CW, int EPI, int ACT>
+template <int MT, int CPL, int NW, bool PAIRS, int EPI, int ACT>
 int launch_skinny(GemmArgs a, int m_tiles, hipStream_t s)
 {
-    a.n_ntiles = (a.N + 16 * CPL * CW - 1) / (16 * CPL * CW);
+    a.n_ntiles = (a.N + 16 * CPL - 1) / (16 * CPL);
+    if (PAIRS) a.n_ntiles /= 2;   // (skinny_pairs: whole pairs)
     const long long grid = (long long)m_tiles * a.n_ntiles;
     AMOE_REQUIRE(grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
-    if (a.stream_from) return launch_skinny<MT, CPL, NW, CW, EPI, ACT, true>(a, (int)grid, s);
-    return launch_skinny<MT, CPL, NW, CW, EPI, ACT, false>(a, (int)grid, s);
+    if (a.stream_from) return launch_skinny<MT, CPL, NW, PAIRS, EPI, ACT, true>(a, (int)grid, s);
+    return launch_skinny<MT, CPL, NW, PAIRS, EPI, ACT, false>(a, (int)grid, s);
 }
 
 // Two column groups of two wavefronts instead of four wavefronts on one: a workgroup reads 512 bytes of each row together, not
@@ -255,12 +310,12 @@ int launch_height(const GemmArgs& a, int bm, hipStream_t s)
     AMOE_REQUIRE(bm == 16 || bm == 32, AMOE_ERR_UNSUPPORTED, "grouped_gemm: no kernel for tiles of %d rows", bm);
     const int cus = device_cu_count();
     if (bm == 32) {
-        if (skinny_pairs(a, 3 * cus, cus)) return launch_skinny<2, 8, 2, 2, EPI, ACT>(a, m_tiles, s);
-        return launch_skinny<2, 8, 4, 1, EPI, ACT>(a, m_tiles, s);
+        if (skinny_pairs(a, 3 * cus, cus)) return launch_skinny<2, 8, 4, true, EPI, ACT>(a, m_tiles, s);
+        return launch_skinny<2, 8, 4, false, EPI, ACT>(a, m_tiles, s);
     }
-    if (skinny_narrow(m_tiles, a.N, cus)) return launch_skinny<1, 4, 8, 1, EPI, ACT>(a, m_tiles, s);
-    if (skinny_pairs(a, 4 * cus, cus)) return launch_skinny<1, 8, 2, 2, EPI, ACT>(a, m_tiles, s);
-    return launch_skinny<1, 8, 4, 1, EPI, ACT>(a, m_tiles, s);
+    if (skinny_narrow(m_tiles, a.N, cus)) return launch_skinny<1, 4, 8, false, EPI, ACT>(a, m_tiles, s);
+    if (skinny_pairs(a, 4 * cus, cus)) return launch_skinny<1, 8, 4, true, EPI, ACT>(a, m_tiles, s);
+    return launch_skinny<1, 8, 4, false, EPI, ACT>(a, m_tiles, s);
 }
 
 // ------------------------------------------------------------------ gate_up product with the routing of a few tokens
@@ -581,8 +636,8 @@ AMOE_EXPORT int amoe_router_input_grad_rows(const void* d_logits, int ld, const 
     a.ldb = a.ldc = a.N = H;
     a.E = 1;
     a.M = T;
-    if (T <= 16) return launch_skinny<1, 4, 8, 1, EPI_STORE, 0>(a, 1, (hipStream_t)stream);
-    return launch_skinny<2, 8, 4, 1, EPI_STORE, 0>(a, (T + 31) / 32, (hipStream_t)stream);
+    if (T <= 16) return launch_skinny<1, 4, 8, false, EPI_STORE, 0>(a, 1, (hipStream_t)stream);
+    return launch_skinny<2, 8, 4, false, EPI_STORE, 0>(a, (T + 31) / 32, (hipStream_t)stream);
 }
 
 AMOE_EXPORT int amoe_router_input_grad(const void* d_logits, const void* w, void* out, int dtype, int T, int E, int H, void* stream)
