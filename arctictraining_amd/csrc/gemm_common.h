@@ -73,6 +73,7 @@ struct GemmArgs {
     int splits, n_real;  // EPI_PART: parts of the reduction, N tiles of one part (n_ntiles counts the tiles of all)
     uint32_t inv_splits, inv_real;   // ceil(2^32 / splits), .. n_real (0 for a divisor of 1)
     int stream_from;  // rows mode: from this number of tiles on B is loaded past the caches (0: never; gemm_skinny.hip: always otherwise)
+    int pairs_cus, pairs_always;  // gemm_skinny.hip: compute units; workgroups of two column groups from which on there are always such
     int f16;         // host side only: the operands are float16 (launch the f16 instance), else bf16
 };
 

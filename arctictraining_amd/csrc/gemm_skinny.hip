@@ -52,9 +52,11 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_al
                                             SourceOf source_of, ScaleOf scale_of)
 {
     constexpr int W = CPL / 2, H = CPL / 4;           // dwords of a lane's row, groups of four columns
-    const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+    int tid = threadIdx.x;            // (of its own in either form: what both work out ahead of the branch between them is held across the reduction and spills)
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, l16 = lane & 15, lq = lane >> 4;
     constexpr int GW = PAIRS ? NW / 2 : NW;           // wavefronts of a group
-    int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int group = wave / GW;
     wave %= GW;
     static_assert(!PAIRS || (GW == 2 && MT <= GW), "a row of red for every 16 rows");
@@ -223,30 +225,64 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_al
     }
 }
 
+// Two column groups of two wavefronts instead of four wavefronts on one: a workgroup reads 512 bytes of each row together, not
+// 256 (reads alone, 128 matrices of 2048 rows of 3072 bytes: 7.0 TB/s instead of 6.5; 1024 bytes 6.5, neighbouring workgroups on
+// one XCD 6.3), and takes twice as long.  By the tiles that the map holds, which only the device knows: with all rows on a few experts there are
+// few, whatever the host's bound says.  w: workgroups of two groups for a compute unit.  Where whole ones of them and halves of one
+// round up to the same, two groups are faster, otherwise the most loaded compute unit has half a workgroup more: products of
+// K x N = 256 x 1024 to 4096 x 2048, 2.5 and 6 rows an expert, times as fast: w 0.5 to 1.3 0.72 .. 1.06; 1.56 1.05 .. 1.24; 1.7 to 2 1.00 .. 1.21;
+// 2.02 to 2.5 0.91 .. 1.12 (median 0.99); 2.6 to 3 1.02 .. 1.13; 3.1 to 3.5 0.96 .. 1.05 (1.00); 3.52 to 4 0.98 .. 1.12 (1.05).  With several rounds of
+// them that no longer counts: 4.1 to 4.5 0.98 .. 1.05, 4.6 to 8 1.00 .. 1.20 (1.05).
+__device__ __forceinline__ bool skinny_pairs(const GemmArgs& p, int tiles, int n_pairs)
+{
+    const int workgroups = tiles * n_pairs, cus = p.pairs_cus;
+    return 2 * workgroups >= 3 * cus && (workgroups > p.pairs_always || (2 * workgroups + cus - 1) / cus % 2 == 0);
+}
+
 // A map's tile is 16 * MT rows where the launch's own rule built it; the taller tiles of a map that was built for another
 // bound of the rows are walked in parts.
 template <int MT, int CPL, int NW, bool PAIRS, int EPI, int ACT, bool STREAM, typename ET>
 __device__ __forceinline__ void skinny_body(const GemmArgs& p)
 {
     __shared__ sk_f32x4 red[NW][CPL * 64];
-    const int pm = blockIdx.x / p.n_ntiles;
-    const int n0 = (blockIdx.x - pm * p.n_ntiles) * 16 * CPL * (PAIRS ? 2 : 1);
+    int pm = blockIdx.x / p.n_ntiles, nt = blockIdx.x - pm * p.n_ntiles;
     int e = 0, m0 = pm * 16 * MT, mend = min(m0 + 16 * MT, p.M);   // without a map: one expert that has all p.M rows
+    bool two = false;
     if (p.tile_map) {
-        if (pm >= min(scalar_load_i32(p.n_mtiles), p.max_mtiles)) return;
+        const int tiles = min(scalar_load_i32(p.n_mtiles), p.max_mtiles);
         const int32_t* ent = reinterpret_cast<const int32_t*>(p.tile_map + pm);
         e = scalar_load_i32(ent);
         m0 = scalar_load_i32(ent + 1);
         mend = scalar_load_i32(ent + 2);
+        if constexpr (PAIRS) {
+            // (the entries of both forms are read beside the number of tiles, not after it)
+            const int n_pairs = p.n_ntiles / 2, pm2 = blockIdx.x / n_pairs;
+            const int32_t* ent2 = reinterpret_cast<const int32_t*>(p.tile_map + min(pm2, p.max_mtiles - 1));
+            const int e2 = scalar_load_i32(ent2), from2 = scalar_load_i32(ent2 + 1), to2 = scalar_load_i32(ent2 + 2);
+            two = skinny_pairs(p, tiles, n_pairs);
+            if (two) {
+                pm = pm2;
+                nt = 2 * ((int)blockIdx.x - pm2 * n_pairs);
+                e = e2;
+                m0 = from2;
+                mend = to2;
+            }
+        }
+        if (pm >= tiles) return;
     }
+    const int n0 = nt * 16 * CPL;
     const auto source_of = [&](int row) { return p.a_row_map ? p.a_row_map[row] : row; };
     const auto scale_of = [&](int row) { return p.row_scale ? p.row_scale[row] : 1.0f; };
+    auto walk = [&](auto TWO) {
 #pragma unroll 1
-    for (;;) {
-        skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET, false, PAIRS>(p, red, e, m0, mend, n0, source_of, scale_of);
-        if ((m0 += 16 * MT) >= mend) break;
-        __syncthreads();   // (the sums are read before the next part's are written)
-    }
+        for (;;) {
+            skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET, false, decltype(TWO)::value>(p, red, e, m0, mend, n0, source_of, scale_of);
+            if ((m0 += 16 * MT) >= mend) break;
+            __syncthreads();   // (the sums are read before the next part's are written)
+        }
+    };
+    if (two) walk(std::integral_constant<bool, PAIRS>{});
+    else walk(std::integral_constant<bool, false>{});
 }
 
 // (at least 4 wavefronts per SIMD with 16 rows, 3 with 32)
@@ -276,31 +312,27 @@ template <int MT, int CPL, int NW, bool PAIRS, int EPI, int ACT>
 int launch_skinny(GemmArgs a, int m_tiles, hipStream_t s)
 {
     a.n_ntiles = (a.N + 16 * CPL - 1) / (16 * CPL);
-    if (PAIRS) a.n_ntiles /= 2;   // (skinny_pairs: whole pairs)
-    const long long grid = (long long)m_tiles * a.n_ntiles;
+    long long grid = (long long)m_tiles * a.n_ntiles;
+    if (PAIRS && grid / 2 > a.pairs_always)   // (of one column group there are at most as many as skinny_pairs lets be)
+        grid = grid / 2 > 2ll * a.pairs_always ? grid / 2 : 2ll * a.pairs_always;
     AMOE_REQUIRE(grid < (1ll << 31), AMOE_ERR_UNSUPPORTED, "grouped_gemm: grid too large");
     if (a.stream_from) return launch_skinny<MT, CPL, NW, PAIRS, EPI, ACT, true>(a, (int)grid, s);
     return launch_skinny<MT, CPL, NW, PAIRS, EPI, ACT, false>(a, (int)grid, s);
 }
 
-// Two column groups of two wavefronts instead of four wavefronts on one: a workgroup reads 512 bytes of each row together, not
-// 256 (reads alone, 128 matrices of 2048 rows of 3072 bytes: 7.0 TB/s instead of 6.5; 1024 bytes 6.5, neighbouring workgroups on
-// one XCD 6.3), and takes twice as long, so that there have to be enough of them, and their last round not nearly empty (fits:
-// workgroups that run at a time).  Gate_up and down product, us, one group / two: 128 experts of 2048 x 768, 4 rows an expert 128 / 119 and 66 /
-// 63, 6 rows 131 / 121 and 70 / 69; 64 of 2048 x 1408, 2.5 rows 111 / 108 and 58 / 53, 6 rows 117 / 113 and 64 / 57; 160 of 2048 x 768, 2.5
-// rows 161 / 149 and 80 / 78; 128 of 1024 x 3072, 3 rows 241 / 230 and 126 / 113.  Workgroups for a compute unit, of two groups: 0.5 (8 experts of
-// 4096 columns) 142 / 231, 1.0 101 / 145, 1.3 37.4 / 37.3, 1.6 44 / 39; where three run at a time, 3.1 140 / 143, 3.5 117 / 116, 5.5 183 / 180.
-// Rows that are no multiple of 512 bytes lose: 3968 bytes 131 / 143, 22272 191 / 202.  Up to 128 rows, which may be in as few
-// experts and for which the routed form below sums in the same order: 8 tokens, 8 of 256 experts of 2560 x 768 84 / 93 and 41 / 47.
-static bool skinny_pairs(const GemmArgs& a, long long fits, int cus)
+// Whether there can be workgroups of two column groups (skinny_pairs).  Rows that are no multiple of 512 bytes lose: 3968 bytes 131 / 143 us,
+// 22272 191 / 202.  Up to 128 rows, which may be in as few experts: 8 tokens, 8 of 256 experts of 2560 x 768 84 / 93 and 41 / 47.
+static bool skinny_may_pair(GemmArgs& a, int m_tiles, int fit, int cus)
 {
-    const long long workgroups = (long long)(a.E < a.M ? a.E : a.M) * (a.N / 256);
-    return a.N % 256 == 0 && a.M > 128 && 2 * workgroups >= 3ll * cus && (workgroups <= fits || 5 * workgroups >= 6 * fits);
+    a.pairs_cus = cus;
+    a.pairs_always = (fit + 1) * cus;
+    const long long workgroups = (long long)m_tiles * (a.N / 256);
+    return cus && a.tile_map && a.N % 256 == 0 && a.M > 128 && 2 * workgroups >= 3ll * cus && workgroups < (1 << 29);
 }
 
 // bm: height of the map's tiles; R rows of a.E experts
 template <int EPI, int ACT>
-int launch_height(const GemmArgs& a, int bm, hipStream_t s)
+int launch_height(GemmArgs a, int bm, hipStream_t s)
 {
     const int R = a.M;
     // every expert with a row has at most rows / 16 + 1 tiles, whatever rule built the map
@@ -310,11 +342,11 @@ int launch_height(const GemmArgs& a, int bm, hipStream_t s)
     AMOE_REQUIRE(bm == 16 || bm == 32, AMOE_ERR_UNSUPPORTED, "grouped_gemm: no kernel for tiles of %d rows", bm);
     const int cus = device_cu_count();
     if (bm == 32) {
-        if (skinny_pairs(a, 3 * cus, cus)) return launch_skinny<2, 8, 4, true, EPI, ACT>(a, m_tiles, s);
+        if (skinny_may_pair(a, m_tiles, 3, cus)) return launch_skinny<2, 8, 4, true, EPI, ACT>(a, m_tiles, s);
         return launch_skinny<2, 8, 4, false, EPI, ACT>(a, m_tiles, s);
     }
     if (skinny_narrow(m_tiles, a.N, cus)) return launch_skinny<1, 4, 8, false, EPI, ACT>(a, m_tiles, s);
-    if (skinny_pairs(a, 4 * cus, cus)) return launch_skinny<1, 8, 4, true, EPI, ACT>(a, m_tiles, s);
+    if (skinny_may_pair(a, m_tiles, 4, cus)) return launch_skinny<1, 8, 4, true, EPI, ACT>(a, m_tiles, s);
     return launch_skinny<1, 8, 4, false, EPI, ACT>(a, m_tiles, s);
 }
 

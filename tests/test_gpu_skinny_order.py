@@ -79,3 +79,29 @@ def test_map_of_another_bound(gpu_device, plan_rows, call_rows):
         assert torch.equal(got, want)
     else:   # (the default tiles' order of sums)
         assert (got.double() - want.double()).norm() <= 2.0 ** -7 * want.double().norm()
+
+
+@pytest.mark.parametrize("rows", [1000, 1900])   # tiles of 16 and of 32 rows
+@pytest.mark.parametrize("on", [1, 7, 64, 100, 130, 180, 205, 230, 260, 275, 300])
+def test_rows_on_some_of_the_experts(gpu_device, rows, on):
+    """one or two column groups by the tiles that there are (256 compute units: from 96 of these on), and every tile by some workgroup:
+    the memory of the output holds NaN before"""
+    from arctictraining_amd import ops
+
+    print("few rows on some of the experts", rows, on, flush=True)
+    E, Kd, N = 300, 64, 1024
+    counts = [0] * E
+    for r in range(rows):
+        counts[(r % on) * E // on] += 1
+    assert sum(c > 0 for c in counts) == on and (rows <= 4 * E) == (rows == 1000) and rows <= 8 * E
+    g = torch.Generator(device=gpu_device).manual_seed(on)
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(gpu_device)
+    a = torch.randn(rows, Kd, device=gpu_device, generator=g).bfloat16()
+    w = (torch.randn(E, Kd, N, device=gpu_device, generator=g) * 0.05).bfloat16()
+    ref = torch.cat([p.double() @ w[e].double() for e, p in enumerate(a.split(counts)) if counts[e]])
+    size = torch.cat([p.double().abs() @ w[e].double().abs() for e, p in enumerate(a.split(counts)) if counts[e]])
+    torch.cuda.empty_cache()
+    torch.full((rows, N), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    got = ops.grouped_gemm_nn(a, w, offs)
+    # (rounded once, the products summed in float32)
+    assert bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + Kd * 2.0 ** -24 * size).all())
