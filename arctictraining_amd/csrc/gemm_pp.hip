@@ -8,6 +8,7 @@
 // MFMAs, the other does everything else, so reads, loads and the epilogue's conversions and stores sit under
 // the matrix pipe instead of between its bursts.
 #include "gemm_dma.h"
+#include "wgrad_deal.h"
 
 #ifndef AMOE_PP_PART
 #define AMOE_PP_PART -1
@@ -28,6 +29,7 @@ constexpr uint32_t PP_LDS = PP_TURN + 8 * 2048;
 constexpr uint32_t PP_WIDX = 2 * PP_STAGE + 8 * 2048;         // weight gradients: behind 2 KB a wavefront for its epilogue the indices of gathered rows
 constexpr uint32_t PP_WDEPTH = PP_WIDX + 8 * 512;            // the experts' depths, and how their tiles are dealt
 constexpr uint32_t PP_WDEAL = PP_WDEPTH + AMOE_MAX_EXPERTS * 4;
+constexpr uint32_t PP_WLOAD = 2 * PP_STAGE;                  // (while they are worked out) the workgroups' loads by number and by depth
 constexpr uint32_t PP_WGRAD_LDS = PP_WDEPTH, PP_WGRAD_DEAL_LDS = PP_WDEAL + AMOE_MAX_EXPERTS * 16;
 
 // ------------------------------------------------------------------ row-grouped products
@@ -784,14 +786,14 @@ __device__ __forceinline__ void pp_wgrad_body()
         t.r1 = __builtin_amdgcn_readfirstlane(scalar_load_i32(p.offsets + t.e + 1));
     };
     // Uneven loads: by number, the deep tiles' share of the workgroups differs by a whole one (a sixteenth of 64 experts with half of the
-    // rows: the most loaded workgroup has 1.22 times the mean of K tiles).  There the experts are taken in the order of their depth, and where
-    // the next one's tiles are lower by a fifth or more, the workgroups that the last turn did not reach are first filled up with
-    // those (1.01 times).  Alone, us, by number / by depth: 131072 such rows, 2048 x 1408, gate_up's gradient 1301 / 1160, down's 716 / 666; 65536
-    // rows of 32 experts of 7168 x 2048, Zipf loads (1.06 and 1.08 times the mean / 1.04 and 1.05) 2900 / 2860 and 1550 / 1540.  Every workgroup works
-    // the dealing out for itself, some 6 us for 64 experts: only where the deepest expert has twice the mean, and the work is fifty
-    // times that; in a kernel of its own, as the shallow tiles of two a workgroup took 1 % longer with it.
-    // A record per expert, in that order: tiles [0, fill) go in turns to the `behind` workgroups from `from` on, the first to the one
-    // `skip` further, the others to all from `from2` on.
+    // rows: the most loaded workgroup has 1.22 times the mean of K tiles).  By depth (wgrad_deal.h) it has 1.01 times.  Where an expert's tiles just miss
+    // whole rounds, by depth can be the worse one (8 experts, Zipf loads, 253 tiles each 1.01 / 1.08): the largest loads of both orders are
+    // worked out, and the smaller one decides.  Alone, us, by number / by depth: 131072 rows as above, 2048 x 1408, gate_up's gradient 1264 / 1164,
+    // down's 671 / 644; 65536 rows of 32 experts of 7168 x 2048, Zipf loads (1.06 and 1.08 times the mean / 1.04 and 1.05) 2880 / 2830 and 1478 / 1448 (within
+    // the noise of a whole pass of 13 ms); the 253 tiles 774 / 793 (768 now), 250 765 / 795 (765).  Every workgroup works the dealing out for itself,
+    // some 10 us for 64 experts: only where the deepest expert has twice the mean, and the work is fifty times that.  To find that it has not takes
+    // 0 to 2 us (even loads, without / with it: 64 experts of 2048 x 1408, 800 rows 264.0 / 264.4, 128 of 2048 x 768, 1024 rows 689 / 690 and 337 / 338);
+    // in a kernel of its own, as the shallow tiles of two a workgroup took 1 % longer with it.
     const int my = (int)((blockIdx.x & 7) * 32 + (blockIdx.x >> 3));
     const int per = pp_args().n_mt * pp_args().n_ntiles;
     bool by_depth = false;
@@ -802,6 +804,7 @@ __device__ __forceinline__ void pp_wgrad_body()
         int mine = 0;
         if (tid < E) mine = min(max(3, (p.offsets[tid + 1] - p.offsets[tid] + PP_BK - 1) >> 6), 1 << 20) + 3;   // (a tile's stores: three K tiles)
         *(word_t)(uintptr_t)(lds + PP_WDEPTH + tid * 4u) = (uint32_t)mine;
+        *(word_t)(uintptr_t)(lds + PP_WLOAD + tid * 4u) = 0u;
         __syncthreads();
         int sum = 0, most = 0;
 #pragma unroll
@@ -825,71 +828,71 @@ __device__ __forceinline__ void pp_wgrad_body()
 #pragma unroll
                 for (int k = 0; k < 4; ++k) rank += (int)d[k] > mine || ((int)d[k] == mine && e + k < tid);
             }
-            if (tid < E) *(__attribute__((address_space(3))) u32x4_t*)(uintptr_t)(lds + PP_WDEAL + rank * 16u) = u32x4_t{0, 0, (uint32_t)mine, (uint32_t)tid};
+            // the workgroups' loads by number and, behind them, by depth
+            auto more = [&](uint32_t at) {
+                return [at](int w, int d) { __hip_atomic_fetch_add((__attribute__((address_space(3))) int*)(uintptr_t)(at + w * 4u), d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+            };
+            const auto by_number = more(lds + PP_WLOAD), of_depth = more(lds + PP_WLOAD + 1024u);
+            if (tid < E) {
+                *(__attribute__((address_space(3))) u32x4_t*)(uintptr_t)(lds + PP_WDEAL + rank * 16u) = u32x4_t{0, 0, (uint32_t)mine, (uint32_t)tid};
+                amoe_deal::add_by_number(tid, mine, per, by_number);
+            }
+            const int whole = E * per & ~255;
+            if (tid < E * per - whole) {
+                const int d = pp_lds<int>(lds + PP_WDEPTH + divide(whole + tid, p.inv_super) * 4u);
+                amoe_deal::add_arc(tid, 1, -d, by_number);
+                amoe_deal::add_arc(amoe_deal::last_of(tid), 1, d, by_number);
+            }
             __syncthreads();
             if (wave == 0) {
-                // left: K tiles that those behind lack; last: depth of the tiles dealt to all
-                int from = 0, behind = 256, skip = 0, left = 0, last = 0;
+                amoe_deal::Walk walk;
                 for (int k = 0; k < E; ++k) {
                     const u32x4_t x = pp_lds<u32x4_t>(lds + PP_WDEAL + k * 16u);
-                    const int d = __builtin_amdgcn_readfirstlane(x[2]), e = __builtin_amdgcn_readfirstlane(x[3]);
-                    if (behind == 256 && 5 * d < 4 * last && skip) {
-                        from = (from + skip) & 255;
-                        behind = 256 - skip;
-                        left = behind * last;
-                        skip = 0;
-                    }
-                    const uint32_t w0 = (uint32_t)(from | skip << 8), w1 = (uint32_t)behind;
-                    int fill = 0;
-                    if (behind < 256) {
-                        const int want = (2 * left + d) / (2 * d);
-                        fill = min(per, want);
-                        skip = (skip + fill) % behind;
-                        left -= fill * d;
-                        if (fill == want) {
-                            from = (from + skip) & 255;
-                            behind = 256;
-                            skip = 0;
-                        }
-                    }
-                    const uint32_t w2 = (uint32_t)((from + skip) & 255) << 16;
-                    if (fill < per) {
-                        skip = (skip + per - fill) & 255;
-                        last = d;
-                    }
-                    if (lane == 0) *(__attribute__((address_space(3))) u32x4_t*)(uintptr_t)(lds + PP_WDEAL + k * 16u) = u32x4_t{w0 | w2, w1, (uint32_t)fill, (uint32_t)e};
+                    const amoe_deal::Record r = walk.next(__builtin_amdgcn_readfirstlane(x[2]), per);
+                    if (lane == 0) *(__attribute__((address_space(3))) u32x4_t*)(uintptr_t)(lds + PP_WDEAL + k * 16u) = u32x4_t{r.word(), (uint32_t)r.behind, (uint32_t)r.fill, x[3]};
                 }
             }
             __syncthreads();
+            if (tid < E) {
+                const u32x4_t x = pp_lds<u32x4_t>(lds + PP_WDEAL + tid * 16u);
+                amoe_deal::add_by_depth(amoe_deal::Record::of(x[0], x[1], x[2]), pp_lds<int>(lds + PP_WDEPTH + x[3] * 4u), per, of_depth);
+            }
+            __syncthreads();
+            auto largest = [&](uint32_t at) {
+                const u32x4_t x = pp_lds<u32x4_t>(at + lane * 16u);
+                const int a = x[0], b = a + (int)x[1], c = b + (int)x[2], d = c + (int)x[3];
+                int before = d;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int v = __shfl_up(before, o, 64);
+                    before += lane >= o ? v : 0;
+                }
+                int m = before - d + max(max(a, b), max(c, d));
+#pragma unroll
+                for (int o = 32; o; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+                return __builtin_amdgcn_readfirstlane(m);
+            };
+            by_depth = largest(lds + PP_WLOAD + 1024u) < largest(lds + PP_WLOAD);
         }
     }
-    // this workgroup's place in the dealing: expert (and its position), next tile, and the record's numbers
-    struct { int at, e, i, fill, behind, second; } deal = {-1, 0, 0, 0, 256, 0};
+    // this workgroup's place in the dealing: position of the expert, the expert, and its tiles
+    struct { int at, e; } deal = {-1, 0};
+    amoe_deal::Turns turns({0, 0, 256, 0, 0}, 0);
     // position of the last tile taken in this XCD's queue, and the end of what this workgroup takes
     int q = (int)(blockIdx.x >> 8) * 32 * pp_args().gm + (int)((blockIdx.x >> 3) & 31);
     const int q_end = q + 32 * pp_args().gm;
     q -= 32;
     auto take = [&](Tile& t) -> bool {                // this workgroup's next tile
         if (DEAL && by_depth) {
-            if (deal.i < deal.fill) {
-                deal.i += deal.behind;
-                if (deal.i >= deal.fill) deal.i = deal.second;
-            } else {
-                deal.i += 256;
-            }
-            while (deal.at < 0 || deal.i >= per) {
+            turns.next();
+            while (deal.at < 0 || turns.at >= per) {
                 if (++deal.at >= pp_args().E) return false;
                 const u32x4_t x = pp_lds<u32x4_t>(lds + PP_WDEAL + deal.at * 16u);
-                const int w = __builtin_amdgcn_readfirstlane(x[0]);
-                deal.behind = __builtin_amdgcn_readfirstlane(x[1]);
-                deal.fill = __builtin_amdgcn_readfirstlane(x[2]);
                 deal.e = __builtin_amdgcn_readfirstlane(x[3]);
-                deal.second = deal.fill + ((my - (w >> 16)) & 255);
-                const int place = (my - w) & 255, turn = place - ((w >> 8) & 255);
-                const int first = turn < 0 ? turn + deal.behind : turn;
-                deal.i = place < deal.behind && first < deal.fill ? first : deal.second;
+                turns = amoe_deal::Turns(amoe_deal::Record::of(__builtin_amdgcn_readfirstlane(x[0]), __builtin_amdgcn_readfirstlane(x[1]),
+                                                               __builtin_amdgcn_readfirstlane(x[2])), my);
             }
-            locate(deal.e, deal.i, t);
+            locate(deal.e, turns.at, t);
             return true;
         }
         args_t& p = pp_args();
