@@ -308,11 +308,19 @@ __device__ __forceinline__ void deep_tile(const GemmArgsF32& p, const int4& tm, 
     if constexpr (GATED) store_gated_again(p, m0, mend, n0, 32, 64);
 }
 
-// Up to how many tiles of the last round are worked off in parts, behind `full` others.  8 experts of 512 x 1024 to 1440 x 1024, 4096 rows, down
-// product and data gradient of gate_up (twice as deep, B^T), tiles on a compute unit, us, whole / in parts: 1.12 55 / 44 and 94 / 81, 1.27 56 / 45 and 99 /
-// 81, 1.41 56 / 50 and 97 / 98, 1.55 59 / 61 and 107 / 121; 2.53 101 / 86 and 181 / 180, 2.81 95 / 95 and 176 / 197, 3.2 112 / 103 and 204 /
-// 188; 4.5 (1024 x 2048, K = 2048 and 4096) 271 / 233 and 514 / 453; gate_up (512 x 2048) 4.5 80 / 77, 5.1 89 / 81.
-__host__ __device__ __forceinline__ int most_in_parts(int cus, int full) { return cus * (full > cus ? 10 : 7) / 16; }
+// Up to how many tiles of the last round are worked off in parts, behind `full` others.  A part takes more than a quarter of a tile's time, with B^T, which it
+// reads straight into registers in pieces of a row, more yet.  8 x 512, 8 x 480, 16 x 256 and 39 x 100 rows, K from 512 to 4096, times as fast in parts
+// as whole, A B / A B^T / gated, by the tiles on a compute unit: 1.07 to 1.13 1.18-1.23 / 1.14-1.17 / 1.16-1.25; 1.22 to 1.25 0.98-1.17 / 1.00-1.11 / 1.12-1.17; 1.38
+// 0.91-1.12 (up to K = 1024 0.91-0.98, in another run 1.04-1.10) / 0.87-1.00 / 1.03-1.10; 1.5 0.91-1.16 / 0.75-0.99 / 0.90-1.09; 2.1 1.22-1.29 / 1.18-1.25 / 1.23-1.31; 2.38 to 2.5
+// 1.08-1.14 / 1.02-1.06 / 1.06-1.14; 2.6 1.01-1.06 / 0.91-0.95 / 1.00-1.06; 2.75 1.00-1.06 / 0.88-0.95 / 0.98-1.03; 3.2 1.07-1.17 / 1.03-1.09 / 1.05-1.12; 3.5
+// 0.99-1.10 / 0.92-1.00 / 0.99-1.04; 3.6 0.97-1.03 / 0.88-0.94 / 0.96-1.00; 4.5 1.01-1.05 / 0.97-1.01 / 1.01-1.04; 5.2 1.03-1.08 / 1.00-1.06 / 1.01-1.08;
+// 5.5 1.01-1.03 / 0.92-1.00 / 1.00-1.02; 5.75 0.97-1.00 / 0.93-0.95 / 0.95-1.00.  One line for A B and gated, whose sums are the same.  (us: down product of 8 x 512 rows, K = 1024, 288 tiles 55.4 / 46.1.)
+__host__ __device__ __forceinline__ int most_in_parts(int cus, int full, bool b_kc)
+{
+    const int rounds = full / cus;
+    const int sixteenths = b_kc ? (rounds == 1 ? 4 : rounds == 2 ? 8 : 5) : rounds == 1 ? 7 : rounds == 2 ? 10 : 8;
+    return cus * sixteenths / 16;
+}
 
 // ------------------------------------------------------------------ row-grouped products
 // Four wavefronts of 32 rows x 64 columns.  Each loads its rows of A straight into registers and splits them there; B is
@@ -335,7 +343,7 @@ grouped_gemm_f32_kernel(GemmArgsF32 p)
     if (KG == 1 && p.cus) {
         // The last round's tiles, if they are few, as four workgroups of 32 rows each: a round lasts as long as a tile.
         const int full = total - total % p.cus;
-        if (full && total - full <= most_in_parts(p.cus, full) && tile >= full) {
+        if (full && total - full <= most_in_parts(p.cus, full, B_KC) && tile >= full) {
             const int sub = (tile - full) & 3;
             tile = full + ((tile - full) >> 2);
             if (tile >= total) return;
@@ -714,7 +722,7 @@ int amoe_f32_rows(const void* A, const int32_t* a_row_map, const void* B, const 
     const int cus = device_cu_count();
     if (form == 0 && cus > 0 && grid > cus) {
         a.cus = cus;
-        grid += 3 * most_in_parts(cus, 2 * cus);
+        grid += 3 * most_in_parts(cus, 2 * cus, b_kc);   // (two whole rounds: the most)
     }
     if (inter) launch_rows<false, true>(a, (int)grid, form, s);
     else if (b_kc) launch_rows<true>(a, (int)grid, form, s);
