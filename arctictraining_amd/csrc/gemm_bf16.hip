@@ -1683,12 +1683,13 @@ int amoe_bf16_wgrad(const void* A, const int32_t* a_row_map, const void* B, cons
     if (tile_cfg == 0) {
         // Up to 128 rows per expert the product is bound by the gradients' stores: gemm_short.hip, where its 32-bit tile
         // numbers reach (with a fourth of these tiles' size).  Beyond, gemm_pp.hip, whose tiles are never done in less than three
-        // K tiles and that deals tiles by number: with uneven loads the deep ones fall to a few compute units, four times as large as the
-        // short kernel's.  Steps, us, short / pp: 128 experts of 2048 x 768, even loads, 105 rows 957 / 923, 128 rows 1013 / 949, Zipf loads
-        // 1127 / 1216; 64 of 2048 x 1408, even, 105 rows 822 / 846, 128 rows 891 / 871; 97 of 1856 x 960, 128 rows, even 1058 / 1065,
-        // a sixteenth of the experts with half of the rows 1041 / 1117; 32 of 1024 x 2048, 128 rows, even 403 / 381, a sixteenth
-        // 436 / 463; 27 of 1024 x 4608, 128 rows, even 719 / 670.  The two gradients alone, 64 of 1024 x 2048, 106 rows, all on one expert
-        // 217 / 411, on a quarter of them 201 / 302, even 199 / 218.
+        // K tiles: with uneven loads the deep ones, four times as large as the short kernel's, fall to a few compute units.  (Below 704 rows an expert
+        // it deals tiles by number.)  The two gradients, short / pp, us: 128 experts of 2048 x 768, 96 rows, even 298 / 306, 105 rows 337 / 309, 128 rows 354 /
+        // 317, Zipf loads 342 / 418 and 379 / 454; 64 of 2048 x 1408, even, 96 rows 266 / 283, 105 rows 302 / 286, 128 rows 319 / 290, a sixteenth of the
+        // experts with half of the rows 290 / 308, 302 / 316, 357 / 326, Zipf loads 310 / 338, 321 / 345, 353 / 370; 32 of 1024 x 2048, 105 rows 116 / 114, 105 /
+        // 132, 105 / 139, 128 rows 118 / 113, 123 / 139, 119 / 145; 27 of 1024 x 4608, 105 rows 231 / 207, 241 / 245, 229 / 233.  Of six such layers, from 105
+        // to 128 rows, even loads are 1.00 to 1.13 times as fast on the large tiles, a sixteenth 0.78 to 1.12, Zipf loads 0.73 to 1.03: the line
+        // lies where uneven loads still lose, not where even ones begin to gain.
         if (R <= 128ll * E && offsets32 && 16 * per * per * E < (1ll << 32)) return amoe_short_wgrad(a, s);
         if (offsets32 && per * per * E < (1ll << 32)) return amoe_pp_wgrad(a, s);
         tile_cfg = 5;
