@@ -6,7 +6,8 @@
 // on a compute unit has its own two 8 KB steps in flight.
 //
 // A workgroup owns MT x 16 rows of an expert and 16 * CPL columns, its NW wavefronts take every NW-th step of 32 k; or two groups of
-// NW / 2 wavefronts stand side by side in the columns, and a wavefront takes two such parts of the reduction, one after the other.
+// NW / 2 wavefronts stand side by side in the columns, and a wavefront takes two such parts of the reduction, one after the other
+// (with a barrier in between; skinny_pairs).
 // Lane (lq, l16) loads, for each of the 8 k of its quarter lq, the CPL columns l16 * CPL .. of the row of B (256 or 128
 // contiguous bytes per row and quarter); byte permutes of two such rows give the MFMA operands: fragment j holds column
 // l16 * CPL + j.  The NW parts' sums meet in LDS, in the order of the parts: the two forms give the same bits.
