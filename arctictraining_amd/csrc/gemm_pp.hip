@@ -742,8 +742,8 @@ __device__ __forceinline__ void pp_rows_body()
 // in all, of 2048 that the MFMAs take (in the memory parts, and scalar: 2990).  The loads' place alone, with indices through LDS, gate_up's and
 // down's gradient, us, in the memory parts / so: 128 experts of 2048 x 768, 1024 rows 698 / 688 and 343 / 338; 8 of 4096 x 14336, 2048 rows 2864 / 2805 and
 // 1459 / 1433; 64 of 2048 x 1408, 2048 rows, uneven 1179 / 1154 and 653 / 639, 800 rows 268 / 263; nothing gathered, 32 of 7168 x 2048, 2048 rows 2804 / 2762.
-// The faster the loop, the more is read again, as workgroups with a panel in common get further apart: of the 8 experts' gate_up gradient 2.9, 3.3, 3.4 GB
-// by scalar indices, by these, with the loads behind the MFMAs; of the 128 experts' 0.70, 0.79, 0.79; of the 32 experts' down gradient 1.82, 1.99, 2.01.
+// The faster the loop, the more is read again, as workgroups with a panel in common get further apart: of the 8 experts' gate_up gradient 5.9, 6.6, 6.9 GB
+// by scalar indices, by these, with the loads behind the MFMAs; of the 128 experts' 1.41, 1.59, 1.57; of the 32 experts' down gradient 3.6, 4.0, 4.0.
 // Both together, alone, us, the rows of one operand gathered, gate_up's / down's gradient, before / so: 64 experts of 2048 x 1408, 250 rows 277 / 143 -> 235 / 125, uneven 2048 rows 1472 / 767 -> 1316 / 749; 128 of 2048 x 768,
 // 188 rows 253 / 131 -> 218 / 119, 1024 rows 769 / 439 -> 713 / 426; 8 of 4096 x 14336, 2048 rows 3024 / 1495 -> 2886 / 1457; one of 2048 x 1408, 4001
 // rows 96 / 85 -> 81 / 79.  Stored as lanes 16 apart in pieces of 64 bytes, past no caches, 250 rows were 328 / 173, now 235 / 125.
@@ -794,7 +794,7 @@ __device__ __forceinline__ void pp_wgrad_body()
     // whole rounds, by depth can be the worse one (8 experts, Zipf loads, 253 tiles each 1.01 / 1.08): the largest loads of both orders are
     // worked out, and the smaller one decides.  Alone, us, by number / by depth: 131072 rows as above, 2048 x 1408, gate_up's gradient 1264 / 1164,
     // down's 671 / 644; 65536 rows of 32 experts of 7168 x 2048, Zipf loads (1.06 and 1.08 times the mean / 1.04 and 1.05) 2880 / 2830 and 1478 / 1448 (within
-    // the noise of a whole pass of 13 ms; 3.2 to 3.6 / 3.9 GB read); the 253 tiles 774 / 793 (768 now), 250 765 / 795 (765).  Every workgroup works the dealing out for itself,
+    // the noise of a whole pass of 13 ms; 6.3 to 7.2 / 7.9 GB read); the 253 tiles 774 / 793 (768 now), 250 765 / 795 (765).  Every workgroup works the dealing out for itself,
     // some 10 us for 64 experts: only where the deepest expert has twice the mean, and the work is fifty times that.  To find that it has not takes
     // 0 to 2 us (even loads, without / with it: 64 experts of 2048 x 1408, 800 rows 264.0 / 264.4, 128 of 2048 x 768, 1024 rows 689 / 690 and 337 / 338);
     // in a kernel of its own, as the shallow tiles of two a workgroup took 1 % longer with it.
