@@ -22,9 +22,19 @@ def _chunks(counts, most=128):
     return out
 
 
+def _two_groups(gpu_device, tiles, N, rounds):
+    """whether that many tiles run as workgroups of two column groups, of which `rounds` run on a compute unit at a time"""
+    cus = torch.cuda.get_device_properties(gpu_device).multi_processor_count
+    if cus != 256:
+        pytest.skip(f"sized for 256 compute units, not {cus}")
+    w = tiles * (N // 256)
+    return 2 * w >= 3 * cus and (w > (rounds + 1) * cus or -(-2 * w // cus) % 2 == 0)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("rows", [(0, 1, 2, 16, 3, 0), (17, 0, 1, 16, 5, 4)])   # tiles of 16 and of 32 rows
-@pytest.mark.parametrize("Kd,N", [(32, 1024), (96, 1280), (160, 1024), (224, 1280), (512, 3584), (2048, 1024)])
+@pytest.mark.parametrize("rows,N", [((0, 1, 2, 16, 3, 0), 1536), ((0, 1, 2, 16, 3, 0), 3584), ((0, 1, 2, 16, 3, 0), 1280),   # tiles of 16 rows
+                                    ((17, 0, 1, 16, 5, 4), 1280), ((17, 0, 1, 16, 5, 4), 3584), ((17, 0, 1, 16, 5, 4), 1536)])   # and of 32
+@pytest.mark.parametrize("Kd", [32, 96, 160, 224, 512, 2048])
 def test_rows_of_larger_and_smaller_calls(gpu_device, dtype, rows, Kd, N):
     from arctictraining_amd import ops
 
@@ -33,6 +43,9 @@ def test_rows_of_larger_and_smaller_calls(gpu_device, dtype, rows, Kd, N):
     counts = [rows[e % 6] for e in range(E)]
     counts[5] = 33 if sum(rows) == 22 else 70   # (several tiles)
     R = sum(counts)
+    high = 16 if sum(rows) == 22 else 32
+    two = _two_groups(gpu_device, sum(-(-c // high) for c in counts), N, 4 if high == 16 else 3)
+    assert two == ((high, N) not in ((16, 1280), (32, 1536)))   # (those with one group, as the smaller calls)
     g = torch.Generator(device=gpu_device).manual_seed(Kd + N)
     offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(gpu_device)
     a = torch.randn(R, Kd, device=gpu_device, generator=g).to(dtype)
@@ -61,12 +74,13 @@ def test_map_of_another_bound(gpu_device, plan_rows, call_rows):
     """taller or lower tiles in the map than the call's own rule makes, enough workgroups for two column groups"""
     from arctictraining_amd import ops
 
-    E, Kd, N = 104, 96, 1280
+    E, Kd, N = 104, 96, 1536
     counts = [(0, 1, 2, 7, 3, 0, 5, 0)[e % 8] for e in range(E)]
     counts[3] += 41
     R = sum(counts)
     print("few rows, map of another bound", plan_rows, call_rows, R, flush=True)
     assert R <= min(plan_rows, call_rows) * E and R > 128
+    assert all(_two_groups(gpu_device, sum(-(-c // high) for c in counts), N, rounds) for high, rounds in ((16, 4), (16, 3), (32, 4), (32, 3)))
     g = torch.Generator(device=gpu_device).manual_seed(plan_rows)
     offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(gpu_device)
     x = torch.randn(max(plan_rows, call_rows) * E, Kd, device=gpu_device, generator=g).bfloat16()
@@ -84,8 +98,7 @@ def test_map_of_another_bound(gpu_device, plan_rows, call_rows):
 @pytest.mark.parametrize("rows", [1000, 1900])   # tiles of 16 and of 32 rows
 @pytest.mark.parametrize("on", [1, 7, 64, 100, 130, 180, 205, 230, 260, 275, 300])
 def test_rows_on_some_of_the_experts(gpu_device, rows, on):
-    """one or two column groups by the tiles that there are (256 compute units: from 96 of these on), and every tile by some workgroup:
-    the memory of the output holds NaN before"""
+    """one or two column groups by the tiles that there are, and every tile by some workgroup: the memory of the output holds NaN before"""
     from arctictraining_amd import ops
 
     print("few rows on some of the experts", rows, on, flush=True)
@@ -93,6 +106,9 @@ def test_rows_on_some_of_the_experts(gpu_device, rows, on):
     counts = [0] * E
     for r in range(rows):
         counts[(r % on) * E // on] += 1
+    high, rounds = (16, 4) if rows == 1000 else (32, 3)
+    two = {1000: (100, 180, 230, 300), 1900: (100, 180, 230, 260, 275, 300)}[rows]
+    assert _two_groups(gpu_device, sum(-(-c // high) for c in counts), N, rounds) == (on in two)
     assert sum(c > 0 for c in counts) == on and (rows <= 4 * E) == (rows == 1000) and rows <= 8 * E
     g = torch.Generator(device=gpu_device).manual_seed(on)
     offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(gpu_device)
