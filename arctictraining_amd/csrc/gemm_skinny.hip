@@ -48,18 +48,19 @@ struct MfmaSkinny<f16_t> {
 // source_of(row): the row of A that stands for a row; scale_of(row): its factor in the gated epilogue
 // SHARED: C is stored where workgroups of other XCDs see it (agent scope: through the L2s)
 // PAIRS: two groups of wavefronts stand side by side in the columns, n0 is the first one's
-template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET, bool SHARED = false, bool PAIRS = false, typename SourceOf, typename ScaleOf>
+// FORMS: the kernel holds one or both of the forms in a loop over a tile's parts (0: no loop)
+template <int MT, int CPL, int NW, int EPI, int ACT, bool STREAM, typename ET, bool SHARED = false, bool PAIRS = false, int FORMS = 0, typename SourceOf, typename ScaleOf>
 __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_all)[NW][CPL * 64], int e, int m0, int mend, int n0,
                                             SourceOf source_of, ScaleOf scale_of)
 {
     constexpr int W = CPL / 2, H = CPL / 4;           // dwords of a lane's row, groups of four columns
-    int tid = threadIdx.x;            // (of its own in either form: what both work out ahead of the branch between them is held across the reduction and spills)
-    asm volatile("" : "+v"(tid));
+    int tid = threadIdx.x % (NW * 64);
+    if constexpr (FORMS == 2) asm volatile("" : "+v"(tid));   // (or what both forms need is worked out ahead of the branch between them, held across the reduction, and spills)
     const int lane = tid & 63, l16 = lane & 15, lq = lane >> 4;
     constexpr int GW = PAIRS ? NW / 2 : NW;           // wavefronts of a group
     int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int group = wave / GW;
-    wave %= GW;
+    const int group = PAIRS ? wave / GW : 0;
+    if (PAIRS) wave %= GW;
     static_assert(!PAIRS || (GW == 2 && MT <= GW), "a row of red for every 16 rows");
     sk_f32x4 (*const red)[CPL * 64] = red_all + group * GW;
     n0 += group * 16 * CPL;
@@ -198,8 +199,11 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs& p, sk_f32x4 (&red_al
             sums(i, [&](int u, sk_f32x4 c) { red[wave][u] = c; });
             __syncthreads();
         }
-        int first = threadIdx.x;   // (worked out here: held across the reduction it spills)
-        asm volatile("" : "+v"(first));
+        int first = tid;
+        if constexpr (FORMS > 0) {
+            first = threadIdx.x;   // (worked out here: held across the reduction it spills)
+            asm volatile("" : "+v"(first));
+        }
         for (int u = first % (GW * 64); u < 4 * H * 64; u += GW * 64) {
             sk_f32x4 c = red[PAIRS ? i : 0][u];
             if constexpr (!PAIRS) {
@@ -274,16 +278,28 @@ __device__ __forceinline__ void skinny_body(const GemmArgs& p)
     const int n0 = nt * 16 * CPL;
     const auto source_of = [&](int row) { return p.a_row_map ? p.a_row_map[row] : row; };
     const auto scale_of = [&](int row) { return p.row_scale ? p.row_scale[row] : 1.0f; };
+    auto part = [&](auto TWO) {
+        skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET, false, decltype(TWO)::value, PAIRS ? 2 : 1>(p, red, e, m0, mend, n0, source_of, scale_of);
+    };
     auto walk = [&](auto TWO) {
 #pragma unroll 1
         for (;;) {
-            skinny_tile<MT, CPL, NW, EPI, ACT, STREAM, ET, false, decltype(TWO)::value>(p, red, e, m0, mend, n0, source_of, scale_of);
+            part(TWO);
             if ((m0 += 16 * MT) >= mend) break;
             __syncthreads();   // (the sums are read before the next part's are written)
         }
     };
-    if (two) walk(std::integral_constant<bool, PAIRS>{});
-    else walk(std::integral_constant<bool, false>{});
+    if constexpr (PAIRS) {
+        if (two) walk(std::integral_constant<bool, true>{});
+        else walk(std::integral_constant<bool, false>{});
+    } else {
+        part(std::integral_constant<bool, false>{});
+#pragma unroll 1
+        for (m0 += 16 * MT; m0 < mend; m0 += 16 * MT) {
+            __syncthreads();
+            part(std::integral_constant<bool, false>{});
+        }
+    }
 }
 
 // (at least 4 wavefronts per SIMD with 16 rows, 3 with 32)
